@@ -5,7 +5,7 @@ inference: the four network classes keep the reference's layer names, so a
 reference checkpoint ({'mu', 'sigma', 'model': state_dict}) loads unchanged,
 and `RuntimePredictor.predict(kernel_arguments, device_name)` keeps its
 signature.  The forward pass itself runs in libhabitat_mi.so
-(hbt_mlp_forward: one fused fp32-MFMA kernel for the whole network);
+(hbt_mlp_forward: one launch per layer, on the matrix cores);
 `predict_batch` is the entry that makes it worthwhile.  Training is not part of
 this package.
 """
@@ -104,8 +104,7 @@ class _DeviceMLP:
             ctypes.byref(err))
         if not self.handle:
             raise _lib.HabitatLibraryError(err.value, "hbt_mlp_create")
-        # Batches of up to 7168 rows (and what a larger batch leaves over) run
-        # through scratch memory of the handle, so calls on one handle must not
+        # A forward runs through scratch memory of the handle, so calls on one handle must not
         # overlap.  Calls that follow each other on one stream never do; a call
         # on ANOTHER stream than the one before is made to wait for that stream
         # first, under a lock that also keeps two threads apart.

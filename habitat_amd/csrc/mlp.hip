@@ -1,33 +1,21 @@
-// Per-operation MLP inference on gfx950: the whole network in one kernel.
+// Per-operation MLP inference on gfx950, one launch per layer.
 //
 // Network (analyzer/habitat/analysis/mlp/mlp.py:17-109): fc1 (F -> W), ReLU,
 // `hidden` x [Linear(W, W), ReLU], fc2 (W -> 1), with W = 1024.  Input rows are
 // standardised as RuntimePredictor.predict does (mlp.py:258-264): (x - mu) /
 // sigma in fp64, then cast to fp32.
 //
-// Design.  A workgroup owns 32 input rows for the whole chain.  Their
-// activations (32 x 1024 fp32 = 128 KiB) live in LDS and never touch HBM; the
-// only global traffic in steady state is the weight stream, which every
-// workgroup reads in the same order and therefore mostly finds in L2.  A layer
-// is computed transposed, Out^T[n][m] = sum_k W[n][k] * Act[m][k], with
-// v_mfma_f32_32x32x2_f32: the A operand is a 32(n) x 2(k) weight fragment, the
-// B operand a 2(k) x 32(m) activation fragment.  The 32 n-tiles of a layer are
-// split over the waves; a wave keeps its slice of the output in accumulator
-// registers for the whole K loop and only then, after a barrier, overwrites the
-// LDS activations in place (bias, staged in LDS during the K loop, and ReLU are
-// applied on the way out).
+// Above kLayerMaxRows rows the hidden layers run on the bf16 matrix cores with
+// every fp32 number in three exact pieces (mlp_split.h).  Up to there they run
+// on the fp32 ones (below), with v_mfma_f32_32x32x2_f32: the A operand is a
+// 32(n) x 2(k) weight fragment, the B operand a 2(k) x 32(m) activation
+// fragment.  For these the weights are repacked once, at hbt_mlp_create, so
+// that a fragment for 8 consecutive k is one fully coalesced 1 KiB load (16 B
+// per lane) straight into the registers the MFMA reads: index
+// [n-tile / 8][layer][k/8][n-tile % 8][lane][4] holds
+// W_layer[32 * n-tile + lane%32][8*(k/8) + 4*(lane/32) + e].
 //
-// Weights are repacked once, at hbt_mlp_create, so that a wave's fragment for
-// 8 consecutive k is one fully coalesced 1 KiB load (16 B per lane) straight
-// into the registers the MFMA reads: index [wave][layer][k/8][tile][lane][4]
-// holds W_layer[32*tile_global + lane%32][8*(k/8) + 4*(lane/32) + e].  For one
-// wave the k-groups of all layers form one contiguous stream, so the prefetch
-// ring runs across layer boundaries: the next layer's first weights are already
-// in flight while this layer's results are written back.  The matching
-// activation fragment is one ds_read_b128 of Act[lane%32][8*(k/8) + 4*(lane/32) ..+3];
-// rows are padded by 4 floats so those reads are bank-conflict free.
-//
-// FLOPs per row: 2 * (F*1024 + hidden*1024^2 + 1024); bound: fp32 MFMA rate.
+// FLOPs per row: 2 * (F*1024 + hidden*1024^2 + 1024).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -37,13 +25,13 @@
 #include <vector>
 
 #include "../../include/habitat_mi.h"
+#include "mlp_split.h"
 #include "wave_scale.h"
 
 namespace hbt {
 
 namespace {
 
-using u32x4 = unsigned int __attribute__((ext_vector_type(4)));
 using f32x2 = float __attribute__((ext_vector_type(2)));
 using f32x4 = float __attribute__((ext_vector_type(4)));
 using f32x16 = float __attribute__((ext_vector_type(16)));
@@ -55,240 +43,13 @@ __device__ __forceinline__ float relu(float v) { return v < 0.f ? 0.f : v; }
 
 constexpr int kWidth = 1024;      // hidden width the kernel is built for
 constexpr int kRows = 32;         // rows per workgroup (one MFMA tile of m)
-constexpr int kStride = kWidth + 4;  // LDS row stride in floats
 constexpr int kMaxInPadded = 64;  // in_features padded to a multiple of 32, at most this
-
-struct MlpArgs {
-  const double* raw;     // [n][in_features]
-  float* out;            // [n]
-  int64_t n;
-  int32_t in_features;
-  int32_t in_padded;     // multiple of 32
-  int32_t hidden;
-  const double* mu;      // [in_features]
-  const double* sigma;   // [in_features]
-  const float* w_stream; // packed weights [waves][groups of all layers][tpw][64][4]
-  const float* bias;     // [(hidden + 1)][kWidth]: fc1 bias, then hidden biases
-  const float* w_last;   // fc2.weight [kWidth]
-  float b_last;
-};
-
-// Fragments travel through a ring of four register slots.  Weight fragments are
-// indexed by the wave's global k-group number (all layers, one stream) and are
-// loaded three groups ahead, also across a layer boundary; activation
-// fragments are loaded from LDS three groups ahead within the layer.
-template <int TPW>
-struct Ring {
-  f32x4 w[4][TPW];
-  f32x4 x[4];
-};
-
-// The wave's weight stream as a buffer resource: a load then takes the stream's
-// base from scalar registers, the k-group's offset as a scalar and the lane's
-// 16 bytes as one 32-bit register, with no 64-bit address arithmetic.
-struct WeightStream {
-  __amdgpu_buffer_rsrc_t rsrc;
-  int lane_bytes;  // 16 * lane
-};
-
-__device__ __forceinline__ WeightStream weight_stream(const f32x4* stream, int64_t bytes,
-                                                      int lane) {
-  WeightStream w;
-  w.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<f32x4*>(stream), 0, (int)bytes, 0x00020000);
-  w.lane_bytes = 16 * lane;
-  return w;
-}
-
-template <int TPW, int SLOT>
-__device__ __forceinline__ void ring_load_w(Ring<TPW>& r, const WeightStream& stream, int group,
-                                            int lane) {
-  const int group_bytes = group * (TPW * 64 * 16);
-#pragma unroll
-  for (int t = 0; t < TPW; ++t) {
-    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(stream.rsrc, stream.lane_bytes + t * 1024,
-                                                          group_bytes, 0);
-    r.w[SLOT][t] = __builtin_bit_cast(f32x4, v);
-  }
-}
-
-template <int TPW, int SLOT>
-__device__ __forceinline__ void ring_load_x(Ring<TPW>& r, const float* act_lane, int g) {
-  r.x[SLOT] = *reinterpret_cast<const f32x4*>(act_lane + 8 * g);
-}
-
-template <int TPW, int SLOT>
-__device__ __forceinline__ void ring_mfma(const Ring<TPW>& r, f32x16 (&acc)[TPW]) {
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-#pragma unroll
-    for (int t = 0; t < TPW; ++t)
-      acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(r.w[SLOT][t][e], r.x[SLOT][e], acc[t], 0, 0, 0);
-}
-
-// One layer's K loop: kg groups of 8 k (a multiple of 4) starting at global
-// group `g0` of the wave's stream; `g_end` is the stream's last valid group.
-// On entry ring slots 0..2 hold the weights of groups g0..g0+2.
-template <int TPW>
-__device__ __forceinline__ void layer_k_loop(Ring<TPW>& r, const WeightStream& stream,
-                                             int g0, int kg, int g_end, const float* act_lane,
-                                             f32x16 (&acc)[TPW]) {
-  const int lane = threadIdx.x & 63;
-  const int last = kg - 1;
-  ring_load_x<TPW, 0>(r, act_lane, 0);
-  ring_load_x<TPW, 1>(r, act_lane, min(1, last));
-  ring_load_x<TPW, 2>(r, act_lane, min(2, last));
-  for (int j = 0; j < kg; j += 4) {
-    // The scheduling barriers keep the compiler from sinking a prefetch below
-    // the MFMA block it is meant to overlap with.  Weight groups past the end
-    // of the stream, and activation groups past the end of the layer, reload
-    // the last valid one (unused values).
-    ring_load_w<TPW, 3>(r, stream, min(g0 + j + 3, g_end), lane);
-    ring_load_x<TPW, 3>(r, act_lane, min(j + 3, last));
-    __builtin_amdgcn_sched_barrier(0);
-    ring_mfma<TPW, 0>(r, acc);
-    __builtin_amdgcn_sched_barrier(0);
-    ring_load_w<TPW, 0>(r, stream, min(g0 + j + 4, g_end), lane);
-    ring_load_x<TPW, 0>(r, act_lane, min(j + 4, last));
-    __builtin_amdgcn_sched_barrier(0);
-    ring_mfma<TPW, 1>(r, acc);
-    __builtin_amdgcn_sched_barrier(0);
-    ring_load_w<TPW, 1>(r, stream, min(g0 + j + 5, g_end), lane);
-    ring_load_x<TPW, 1>(r, act_lane, min(j + 5, last));
-    __builtin_amdgcn_sched_barrier(0);
-    ring_mfma<TPW, 2>(r, acc);
-    __builtin_amdgcn_sched_barrier(0);
-    ring_load_w<TPW, 2>(r, stream, min(g0 + j + 6, g_end), lane);
-    ring_load_x<TPW, 2>(r, act_lane, min(j + 6, last));
-    __builtin_amdgcn_sched_barrier(0);
-    ring_mfma<TPW, 3>(r, acc);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-}
-
-template <int WAVES>
-__global__ __launch_bounds__(WAVES * 64, 1) void mlp_fused_kernel(const MlpArgs a) {
-  constexpr int TPW = (kWidth / 32) / WAVES;  // n-tiles per wave
-  constexpr int THREADS = WAVES * 64;
-  extern __shared__ __attribute__((aligned(16))) float lds[];
-  float* act = lds;                           // [kRows][kStride]
-  float* red = lds + kRows * kStride;         // [THREADS / 32][32]
-  float* bias_lds = red + (THREADS / 32) * 32;  // [kWidth]
-  static_assert(THREADS * 4 == kWidth, "one float4 of bias per thread");
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int m = lane & 31, h = lane >> 5;
-  const int64_t row0 = (int64_t)blockIdx.x * kRows;
-
-  // ---- stage standardised inputs: act[r][k], zero beyond in_features / n ----
-  for (int idx = tid; idx < kRows * a.in_padded; idx += THREADS) {
-    const int r = idx / a.in_padded, k = idx - r * a.in_padded;
-    float v = 0.f;
-    if (k < a.in_features && row0 + r < a.n) {
-      const double x = a.raw[(row0 + r) * a.in_features + k];
-      v = (float)((x - a.mu[k]) / a.sigma[k]);
-    }
-    act[r * kStride + k] = v;
-  }
-  // fc1's bias, where the accumulators will pick it up
-  *reinterpret_cast<f32x4*>(bias_lds + 4 * tid) = *reinterpret_cast<const f32x4*>(a.bias + 4 * tid);
-  __syncthreads();
-
-  const float* act_lane = act + m * kStride + 4 * h;
-  const int tile0 = wave * TPW;  // first n-tile of this wave
-
-  // This wave's weight stream: fc1's groups, then 128 groups per hidden layer.
-  const int kg_first = a.in_padded / 8;
-  const int groups = kg_first + a.hidden * (kWidth / 8);
-  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  const int64_t stream_bytes = (int64_t)groups * TPW * 64 * 16;
-  const WeightStream stream = weight_stream(
-      reinterpret_cast<const f32x4*>(a.w_stream) + (size_t)wave_u * groups * TPW * 64, stream_bytes,
-      lane);
-  const int g_end = groups - 1;
-
-  Ring<TPW> ring;
-  ring_load_w<TPW, 0>(ring, stream, 0, lane);
-  ring_load_w<TPW, 1>(ring, stream, min(1, g_end), lane);
-  ring_load_w<TPW, 2>(ring, stream, min(2, g_end), lane);
-
-  f32x16 acc[TPW];
-  int g0 = 0;
-  for (int layer = 0; layer <= a.hidden; ++layer) {
-    // The accumulators start at this layer's bias, which the layer before
-    // parked in LDS; every thread fetches four values of the next layer's now
-    // and parks them after the K loop.  (Adding the bias here instead of in the
-    // write-back leaves room there for a ReLU that hands NaNs on, at no more
-    // instructions than add and max.)
-    const int next_layer = layer < a.hidden ? layer + 1 : layer;
-    const f32x4 bias_part =
-        *reinterpret_cast<const f32x4*>(a.bias + (size_t)next_layer * kWidth + 4 * tid);
-#pragma unroll
-    for (int t = 0; t < TPW; ++t)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x4 b =
-            *reinterpret_cast<const f32x4*>(bias_lds + (tile0 + t) * 32 + 8 * g + 4 * h);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[t][4 * g + e] = b[e];
-      }
-
-    const int kg = (layer == 0) ? kg_first : kWidth / 8;
-    layer_k_loop<TPW>(ring, stream, g0, kg, g_end, act_lane, acc);
-    g0 += kg;
-
-    __syncthreads();  // every wave has finished reading this layer's input and bias
-    *reinterpret_cast<f32x4*>(bias_lds + 4 * tid) = bias_part;
-#pragma unroll
-    for (int t = 0; t < TPW; ++t)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int n = (tile0 + t) * 32 + 8 * g + 4 * h;
-        f32x4 o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = relu(acc[t][4 * g + e]);
-        *reinterpret_cast<f32x4*>(act + m * kStride + n) = o;
-      }
-    __syncthreads();
-  }
-
-  // ---- fc2: out[r] = sum_n act[r][n] * w_last[n] + b_last ----
-  {
-    constexpr int PARTS = THREADS / 32;
-    constexpr int NPP = kWidth / PARTS;
-    const int r = tid & 31, part = tid >> 5;
-    const float* ap = act + r * kStride + part * NPP;
-    const float* wl = a.w_last + part * NPP;
-    float s = 0.f;
-#pragma unroll 8
-    for (int k = 0; k < NPP; k += 4) {
-      const f32x4 x = *reinterpret_cast<const f32x4*>(ap + k);
-      const f32x4 w = *reinterpret_cast<const f32x4*>(wl + k);
-      s = fmaf(x[0], w[0], s);
-      s = fmaf(x[1], w[1], s);
-      s = fmaf(x[2], w[2], s);
-      s = fmaf(x[3], w[3], s);
-    }
-    red[part * 32 + r] = s;
-    __syncthreads();
-    if (tid < 32 && row0 + tid < a.n) {
-      float total = a.b_last;
-#pragma unroll
-      for (int p = 0; p < PARTS; ++p) total += red[p * 32 + tid];
-      a.out[row0 + tid] = total;
-    }
-  }
-}
 
 // ---------------------------------------------------------------------------
 // Up to kLayerMaxRows rows (one prediction, the operations of one trace, a trace
 // for some devices): one launch per layer.
 //
-// The fused kernel gives each workgroup 32 rows and the whole network, so a
-// batch of up to 32 rows runs on ONE compute unit, which has to pull all
-// 33.6 MB of weights through by itself (about 1 ms), and any batch below 8192
-// rows leaves compute units idle for that long.  Here a layer is spread over
-// the chip instead, in one of three shapes:
+// A layer is spread over the chip in one of three shapes:
 //
 //   For a few rows (up to kSplitMaxRows) mlp_layer_kernel with four waves: a
 //   workgroup takes one n-tile x one m-tile and an eighth of K (kSplit: 256
@@ -309,9 +70,7 @@ constexpr int kSplit = 8;            // K-partials per hidden layer, up to kSpli
 // Rows up to which K is split over workgroups (the partials' traffic grows with
 // the rows; beyond this the whole-K shapes are faster).
 constexpr int kSplitMaxRows = 20;
-// Largest batch that takes this path: 224 m-tiles, 7 steps of the tile kernel on
-// 256 compute units, just under what one round of the fused kernel costs
-// whatever it holds.  Tuned on 256 compute units.
+// Largest batch that takes this path.
 constexpr int kLayerMaxRows = 7168;
 // m-tiles up to which the eight-wave shape splits K over two workgroups (128
 // workgroups or fewer per layer would leave half the compute units idle).
@@ -321,8 +80,10 @@ constexpr int kHalfKMaxTiles = 4;
 constexpr int kFirstFmaMaxIn = 16;
 constexpr int kFirstFmaSlices = 8;     // workgroups per m-tile (gridDim.y)
 constexpr int kFirstFmaMinTiles = 64;  // m-tiles from which that kernel is used (2048 rows)
-constexpr size_t kScratchFloats = (size_t)kLayerMaxRows * kWidth;  // each of two buffers (28 MiB)
-static_assert((size_t)kSplit * kRows * kWidth <= kScratchFloats, "the K-partials fit the scratch");
+// Rows per compute unit that the split path takes at a time: two rounds of
+// 256 x 256 workgroups per layer (291 us for two against 145-150 for one), with
+// activations that mostly stay in the 256 MB last-level cache.
+constexpr int64_t kSplitRowsPerUnit = 128;
 
 struct LayerArgs {
   const float* w_stream;   // packed weights, see above
@@ -413,7 +174,7 @@ __global__ __launch_bounds__(WAVES * 64) void mlp_layer_kernel(const LayerArgs a
   int count = per_split - wave * per_wave;
   count = count < 0 ? 0 : (count > per_wave ? per_wave : count);
 
-  // n-tile of the layer -> (stream of the fused kernel's wave, slot in its group)
+  // n-tile of the layer -> (weight stream, slot in its group)
   const int tile = blockIdx.x * NT;  // the first of the workgroup's NT
   const f32x4* w_lane = reinterpret_cast<const f32x4*>(a.w_stream) +
                         ((size_t)(tile >> 3) * a.groups_total + a.g0) * (8 * 64) +
@@ -821,9 +582,7 @@ constexpr size_t kOneDoneOffset = 768;  // and the call number the last kernel p
 constexpr size_t kOneBytes = 1024;
 static_assert(kMaxInPadded * sizeof(double) <= kOneOutOffset, "a raw row fits below the result");
 
-constexpr int kWaves = 4;  // one wave per SIMD: fewer, longer MFMA runs between load bursts than with two
-constexpr size_t kLdsBytes =
-    (size_t)(kRows * kStride + (kWaves * 64 / 32) * 32 + kWidth) * sizeof(float);
+constexpr int kWaves = 4;  // weight streams of 8 n-tiles each
 
 }  // namespace
 
@@ -832,16 +591,19 @@ constexpr size_t kLdsBytes =
 struct hbt_mlp {
   int32_t in_features, in_padded, width, hidden;
   int device;
-  int compute_units;   // of that device: the fused kernel runs one workgroup on each
+  int compute_units;   // of that device
   void* blob;          // one device allocation holding everything below
   const double* mu;
   const double* sigma;
   const float* w_stream;
   const float* bias;
   const float* w_last;
-  const float* w_first_t;  // fc1.weight transposed [kFirstFmaMaxIn][width]; null above that many inputs
+  const float* w_first_t;  // fc1.weight transposed, [kFirstFmaMaxIn or kMaxInPadded][width]
   float b_last;
-  float* scratch[2];   // per-layer path: two buffers of kScratchFloats activations or partials
+  const char* w_split; // the hidden layers' weights in bf16 pieces, kSplitLayerBytes each
+  int64_t chunk_rows;  // rows the split path takes at a time
+  float* scratch[2];   // activations (or K-partials) of one layer and of the next
+  float* part;         // split path: [kWidth / 32][chunk_rows] shares of the final dot product
   // hbt_mlp_predict_one: a pinned, device-visible block (one raw row in, one
   // prediction out at kOneOutOffset) and the lock that serialises its callers
   unsigned char* one_host;
@@ -971,7 +733,7 @@ int forward_layers(hbt_mlp* mlp, const double* raw_features, int64_t n, float* o
     if (layer == 0 && split_k)
       hipLaunchKernelGGL((mlp_layer_kernel<true, 0, true, 4, false, 0>), grid, dim3(256), 0,
                          stream, l);
-    else if (layer == 0 && mlp->w_first_t != nullptr && m_tiles >= kFirstFmaMinTiles) {
+    else if (layer == 0 && mlp->in_features <= kFirstFmaMaxIn && m_tiles >= kFirstFmaMinTiles) {
       hipLaunchKernelGGL(mlp_first_fma_kernel, dim3((unsigned)m_tiles, kFirstFmaSlices), dim3(256), 0,
                          stream, l);
     } else if (layer == 0)
@@ -1018,26 +780,72 @@ int forward_layers(hbt_mlp* mlp, const double* raw_features, int64_t n, float* o
   return hipGetLastError() == hipSuccess ? HBT_OK : HBT_EHIP;
 }
 
-// The fused kernel: one workgroup per 32 rows.
-int forward_fused(hbt_mlp* mlp, const double* raw_features, int64_t n, float* out,
+// The split path's hidden layers (mlp_split.h).
+namespace split = hbt::split;
+using hbt::kWidth;
+constexpr size_t kSplitLayerBytes = (size_t)(kWidth / 32) * split::kTileBytes;
+
+// A workgroup takes 256 outputs x 256 rows.
+struct SplitLarge {
+  using S = split::Large<4, 2, 2, 4, 24>;
+  static constexpr auto kHidden = &split::large_kernel<4, 2, 2, 4, 24, false>;
+  static constexpr auto kLast = &split::large_kernel<4, 2, 2, 4, 24, true>;
+};
+
+template <class C>
+bool split_ready() {
+  const auto set = [](const void* f) {
+    return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, C::S::LDS) ==
+           hipSuccess;
+  };
+  return set(reinterpret_cast<const void*>(C::kHidden)) &&
+         set(reinterpret_cast<const void*>(C::kLast));
+}
+
+template <class C>
+void split_launch(const split::LayerArgs& a, bool last, hipStream_t stream) {
+  const int m_blocks = (a.m_tiles + C::S::BM - 1) / C::S::BM;
+  const dim3 grid((unsigned)((m_blocks + 7) / 8 * 8 * C::S::NBLK));
+  hipLaunchKernelGGL(last ? C::kLast : C::kHidden, grid, dim3(C::S::THREADS), C::S::LDS, stream,
+                     a);
+}
+
+// The split path for up to chunk_rows rows.
+int forward_split(hbt_mlp* mlp, const double* raw_features, int64_t n, float* out,
                   hipStream_t stream) {
   using namespace hbt;
-  const int64_t blocks = (n + kRows - 1) / kRows;
-  MlpArgs a{};
-  a.raw = raw_features;
-  a.out = out;
-  a.n = n;
-  a.in_features = mlp->in_features;
-  a.in_padded = mlp->in_padded;
-  a.hidden = mlp->hidden;
-  a.mu = mlp->mu;
-  a.sigma = mlp->sigma;
-  a.w_stream = mlp->w_stream;
-  a.bias = mlp->bias;
-  a.w_last = mlp->w_last;
-  a.b_last = mlp->b_last;
-  hipLaunchKernelGGL(mlp_fused_kernel<kWaves>, dim3((unsigned)blocks), dim3(kWaves * 64),
-                     kLdsBytes, stream, a);
+  const int m_tiles = (int)((n + kRows - 1) / kRows);
+  char* const buffers[2] = {reinterpret_cast<char*>(mlp->scratch[0]),
+                            reinterpret_cast<char*>(mlp->scratch[1])};
+  split::FirstArgs f{};
+  f.raw = raw_features; f.mu = mlp->mu; f.sigma = mlp->sigma;
+  f.w_t = mlp->w_first_t; f.bias = mlp->bias;
+  f.in_features = mlp->in_features; f.n = n;
+  f.y = buffers[0];
+  const dim3 first_grid((unsigned)m_tiles, split::kFirstSlices);
+  if (mlp->in_features <= kFirstFmaMaxIn)
+    hipLaunchKernelGGL(split::first_kernel<kFirstFmaMaxIn>, first_grid, dim3(256), 0, stream, f);
+  else
+    hipLaunchKernelGGL(split::first_kernel<kMaxInPadded>, first_grid, dim3(256), 0, stream, f);
+  split::LayerArgs l{};
+  l.w_last = mlp->w_last;
+  l.part = mlp->part;
+  l.m_tiles = m_tiles;
+  for (int layer = 0; layer < mlp->hidden; ++layer) {
+    l.w = mlp->w_split + (size_t)layer * kSplitLayerBytes;
+    l.bias = mlp->bias + (size_t)(layer + 1) * kWidth;
+    l.x = buffers[layer & 1];
+    l.y = buffers[(layer + 1) & 1];
+    const bool last = layer + 1 == mlp->hidden;
+    split_launch<SplitLarge>(l, last, stream);
+  }
+  split::FinishArgs z{};
+  z.part = mlp->part;
+  z.rows_pad = m_tiles * kRows;
+  z.b_last = mlp->b_last;
+  z.n = n;
+  z.out = out;
+  hipLaunchKernelGGL(split::finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, z);
   return hipGetLastError() == hipSuccess ? HBT_OK : HBT_EHIP;
 }
 
@@ -1093,13 +901,17 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
   const size_t off_stream = off; off = align_up(off + sizeof(float) * n_stream, 256);
   const size_t off_bias = off; off = align_up(off + sizeof(float) * n_bias, 256);
   const size_t off_last = off; off = align_up(off + sizeof(float) * kWidth, 256);
-  const bool first_fma = in_features <= kFirstFmaMaxIn;
+  const size_t first_t_rows = in_features <= kFirstFmaMaxIn ? kFirstFmaMaxIn : kMaxInPadded;
   const size_t off_first_t = off;
-  if (first_fma) off = align_up(off + sizeof(float) * kFirstFmaMaxIn * kWidth, 256);
+  off = align_up(off + sizeof(float) * first_t_rows * kWidth, 256);
   const size_t image = off;  // what is copied from the host; scratch follows
-  const size_t scratch_bytes = sizeof(float) * kScratchFloats;
+  const int64_t chunk_rows = kSplitRowsPerUnit * compute_units;
+  const size_t scratch_bytes = (size_t)(chunk_rows / kRows) * split::kTileBytes;
+  const size_t off_split = off; off = align_up(off + (size_t)hidden_layers * kSplitLayerBytes, 256);
   const size_t off_scratch0 = off; off = align_up(off + scratch_bytes, 256);
   const size_t off_scratch1 = off; off = align_up(off + scratch_bytes, 256);
+  const size_t off_part = off;
+  off = align_up(off + sizeof(float) * (kWidth / 32) * (size_t)chunk_rows, 256);
   const size_t total = off;
 
   std::vector<unsigned char> host;
@@ -1120,11 +932,10 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
     std::memcpy(host.data() + off_bias + sizeof(float) * (size_t)l * kWidth, b[l],
                 sizeof(float) * kWidth);
   std::memcpy(host.data() + off_last, W[hidden_layers + 1], sizeof(float) * kWidth);
-  if (first_fma) {
-    float* t = reinterpret_cast<float*>(host.data() + off_first_t);  // zero beyond in_features
-    for (int n = 0; n < kWidth; ++n)
-      for (int k = 0; k < in_features; ++k) t[(size_t)k * kWidth + n] = W[0][(size_t)n * in_features + k];
-  }
+  float* first_t = reinterpret_cast<float*>(host.data() + off_first_t);  // zero beyond in_features
+  for (int n = 0; n < kWidth; ++n)
+    for (int k = 0; k < in_features; ++k)
+      first_t[(size_t)k * kWidth + n] = W[0][(size_t)n * in_features + k];
 
   void* blob = nullptr;
   if (hipMalloc(&blob, total) != hipSuccess) {
@@ -1138,9 +949,23 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
     *err = HBT_EHIP;
     return nullptr;
   }
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&mlp_fused_kernel<kWaves>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)kLdsBytes) != hipSuccess) {
+  if (!split_ready<SplitLarge>()) {
+    (void)hipGetLastError();
+    (void)hipFree(blob);
+    *err = HBT_EHIP;
+    return nullptr;
+  }
+  // the hidden layers' weights in bf16 pieces, from the packed fp32 ones
+  for (int l = 0; l < hidden_layers; ++l) {
+    split::PackArgs a{};
+    a.w_stream = reinterpret_cast<const float*>(static_cast<unsigned char*>(blob) + off_stream);
+    a.groups_total = in_padded / 8 + hidden_layers * (kWidth / 8);
+    a.g0 = in_padded / 8 + l * (kWidth / 8);
+    a.w = reinterpret_cast<char*>(blob) + off_split + (size_t)l * kSplitLayerBytes;
+    hipLaunchKernelGGL(split::pack_kernel, dim3((kWidth / 32) * split::kSteps / 4), dim3(256), 0,
+                       nullptr, a);
+  }
+  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
     (void)hipGetLastError();
     (void)hipFree(blob);
     *err = HBT_EHIP;
@@ -1181,7 +1006,10 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
   m->w_stream = reinterpret_cast<const float*>(base + off_stream);
   m->bias = reinterpret_cast<const float*>(base + off_bias);
   m->w_last = reinterpret_cast<const float*>(base + off_last);
-  m->w_first_t = first_fma ? reinterpret_cast<const float*>(base + off_first_t) : nullptr;
+  m->w_first_t = reinterpret_cast<const float*>(base + off_first_t);
+  m->w_split = reinterpret_cast<const char*>(base + off_split);
+  m->chunk_rows = chunk_rows;
+  m->part = reinterpret_cast<float*>(base + off_part);
   m->b_last = b[hidden_layers + 1][0];
   m->scratch[0] = reinterpret_cast<float*>(base + off_scratch0);
   m->scratch[1] = reinterpret_cast<float*>(base + off_scratch1);
@@ -1207,21 +1035,22 @@ int hbt_mlp_forward(hbt_mlp* mlp, const double* raw_features, int64_t n, float* 
   if (device != mlp->device) return HBT_EINVAL;
 
   hipStream_t stream = static_cast<hipStream_t>(hip_stream);
-  // The fused kernel keeps every compute unit busy for whole rounds of
-  // 32 rows x compute units (about 0.94 ms each); what is left over after the
-  // last whole round would cost another one.  Up to kLayerMaxRows leftover rows
-  // go through the per-layer path instead, which takes less for them.
-  const int64_t round_rows = (int64_t)kRows * mlp->compute_units;
-  const int64_t leftover = n % round_rows;
-  if (leftover == 0 || leftover > kLayerMaxRows)
-    return forward_fused(mlp, raw_features, n, out, stream);
-  const int64_t done = n - leftover;
-  if (done > 0) {
-    const int rc = forward_fused(mlp, raw_features, done, out, stream);
+  // Whole rounds of the 256 x 256 workgroups through the split path, two at a
+  // time.  What is left over would cost most of another round: up to
+  // kLayerMaxRows rows go through the fp32 kernels instead.
+  const int64_t round_rows = mlp->chunk_rows / 2;
+  int64_t done = 0;
+  while (done < n) {
+    int64_t rows = n - done < mlp->chunk_rows ? n - done : mlp->chunk_rows;
+    if (rows > round_rows && rows % round_rows <= kLayerMaxRows) rows -= rows % round_rows;
+    const double* raw = raw_features + done * mlp->in_features;
+    const int rc = rows > kLayerMaxRows && mlp->hidden > 0
+                       ? forward_split(mlp, raw, rows, out + done, stream)
+                       : forward_layers(mlp, raw, rows, out + done, mlp->scratch, stream);
     if (rc != HBT_OK) return rc;
+    done += rows;
   }
-  return forward_layers(mlp, raw_features + done * mlp->in_features, leftover, out + done,
-                        mlp->scratch, stream);
+  return HBT_OK;
 }
 
 int hbt_mlp_forward_static(hbt_mlp* mlp, const double* raw_features, int64_t n, float* out,

@@ -1,0 +1,508 @@
+// Hidden layers of the MLP on the bf16 matrix cores, at fp32 precision.
+//
+// What bounds a batch of rows is the matrix cores, and gfx950's do 16 times as
+// many multiply-adds per cycle on bf16 as on fp32.  An fp32 number is the exact
+// sum of three bf16 numbers (8 + 8 + 8 bits of mantissa, bf16 has fp32's range):
+//     x = x0 + x1 + x2,  x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1
+// so weights and activations are kept as three such pieces, and of the nine
+// products of pieces the six that matter are multiplied:
+//     w x = w0 x0 + (w0 x1 + w1 x0) + (w1 x1 + w0 x2 + w2 x0) + ...
+// What is left out, w1 x2 + w2 x1 + w2 x2, is below 2^-23 of the product, with
+// either sign: beside the roundings of a sum of 1024 products it does not show.
+// Products of bf16 are exact in the matrix core and sums are fp32, so the layer
+// is an fp32 layer at 16 / 6 of the fp32 rate.
+//
+// The order of the sum decides its error: the matrix core adds eight products
+// and rounds the running sum, and a rounding costs half an ulp of what the sum
+// has grown to.  Over one layer of 1024 (errors in 2^-24 of the output's rms):
+// fp32 matrix cores 6.7, the six products of each step in turn 7.9, the five
+// small products of all steps before the leading ones 2.4.
+//
+// Included by mlp.hip only.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+#include <type_traits>
+
+namespace hbt {
+namespace split {
+
+using bf16x8 = __bf16 __attribute__((ext_vector_type(8)));
+using f32x4 = float __attribute__((ext_vector_type(4)));
+using f32x16 = float __attribute__((ext_vector_type(16)));
+
+using bf16x2 = __bf16 __attribute__((ext_vector_type(2)));
+using f32x2 = float __attribute__((ext_vector_type(2)));
+
+// Layout.  A layer is computed transposed, Out^T[n][m] = sum_k W[n][k] Act[m][k],
+// with v_mfma_f32_32x32x16_bf16: 32 outputs x 32 rows x 16 k (a k-step).  Weights
+// and activations are both stored as the register image of its operands:
+//     [32-row tile][k-step][piece][lane][8],
+// lane (r, h) = (lane % 32, lane / 32) holding row r of the tile and
+//     k = 16 step + 8 (j / 4) + 4 h + j % 4,  j = 0..7.
+// That order of k within a step is the accumulator's own: register 4 g + e of
+// lane (m, h) is output n = 8 g + 4 h + e of row m, so a lane's registers 8 kk ..
+// 8 kk + 7 are its part of the next layer's k-step 2 tile + kk as they are, and
+// every load and store of a wave is 1 KiB of contiguous memory.
+constexpr int kWidth = 1024;
+constexpr int kRows = 32;                        // rows of a tile
+constexpr int kSteps = kWidth / 16;
+constexpr int kPieces = 3;
+constexpr int kFragBytes = 64 * 16;              // one operand of one MFMA
+constexpr int kStepBytes = kPieces * kFragBytes;
+constexpr int kTileBytes = kSteps * kStepBytes;
+
+// Two floats rounded to bf16 in one register (low half first), and back.
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
+}
+__device__ __forceinline__ float low2(uint32_t v) { return __builtin_bit_cast(float, v << 16); }
+__device__ __forceinline__ float high2(uint32_t v) {
+  return __builtin_bit_cast(float, v & 0xffff0000u);
+}
+
+// The pieces of N values, two to a register.
+template <int N>
+struct Split {
+  uint32_t p[kPieces][N / 2];
+};
+
+// HUGE_VALUES: some of the values are kHuge or more in magnitude, where rounding
+// to bf16 overflows.  A finite one then gets the largest bf16 as its first
+// piece; an infinity becomes its LAST piece alone, which meets nothing but the
+// other operand's first piece, so that inf * w is what it is in fp32 and no
+// inf - inf or inf * 0 comes up that fp32 would not have.
+constexpr float kHuge = 0x1.FFp+127f;
+constexpr float kMaxBf16 = 0x1.FEp+127f;
+
+template <bool HUGE_VALUES, int N>
+__device__ __forceinline__ Split<N> split_values(const float (&values)[N]) {
+  Split<N> s;
+#pragma unroll
+  for (int j = 0; j < N / 2; ++j) {
+    float a = values[2 * j], b = values[2 * j + 1];
+    const bool inf_a = HUGE_VALUES && __builtin_isinf(a), inf_b = HUGE_VALUES && __builtin_isinf(b);
+    if (inf_a) a = 0.f;
+    if (inf_b) b = 0.f;
+    uint32_t hi;
+    if (HUGE_VALUES) {  // (a NaN stays one: it is not beyond either bound)
+      const float ca = a > kMaxBf16 ? kMaxBf16 : a < -kMaxBf16 ? -kMaxBf16 : a;
+      const float cb = b > kMaxBf16 ? kMaxBf16 : b < -kMaxBf16 ? -kMaxBf16 : b;
+      hi = pack2(ca, cb);
+    } else {
+      hi = pack2(a, b);
+    }
+    a -= low2(hi);
+    b -= high2(hi);
+    const uint32_t mid = pack2(a, b);
+    a = inf_a ? values[2 * j] : a - low2(mid);
+    b = inf_b ? values[2 * j + 1] : b - high2(mid);
+    s.p[0][j] = hi;
+    s.p[1][j] = mid;
+    s.p[2][j] = pack2(a, b);
+  }
+  return s;
+}
+
+// Stores a lane's 8 (or first or last 4) values of a fragment in pieces; `out`
+// is their place in the first one.
+template <int N>
+__device__ __forceinline__ void store_split(char* out, const float (&v)[N]) {
+  using V = uint32_t __attribute__((ext_vector_type(N / 2)));
+  float most = 0.f;
+#pragma unroll
+  for (int j = 0; j < N; ++j) most = fmaxf(most, fabsf(v[j]));
+  Split<N> s = split_values<false, N>(v);
+  if (__builtin_expect(most >= kHuge, 0)) s = split_values<true, N>(v);
+#pragma unroll
+  for (int p = 0; p < kPieces; ++p) {
+    V packed;
+#pragma unroll
+    for (int j = 0; j < N / 2; ++j) packed[j] = s.p[p][j];
+    *reinterpret_cast<V*>(out + p * kFragBytes) = packed;
+  }
+}
+
+// Byte offset of k-step `step` of a tile (weights or activations).
+__device__ __forceinline__ size_t tile_offset(int tile, int step) {
+  return (size_t)tile * kTileBytes + (size_t)step * kStepBytes;
+}
+
+struct LayerArgs {
+  const char* w;        // this layer's weights, [32 n-tiles] tiles
+  const char* x;        // activations in, [m_tiles] tiles
+  const float* bias;    // [kWidth]
+  char* y;              // activations out (not LAST)
+  const float* w_last;  // LAST: fc2.weight [kWidth]
+  float* part;          // LAST: [kWidth / 32][m_tiles * 32] shares of the final dot product
+  int32_t m_tiles;
+};
+
+typedef __attribute__((address_space(3))) void lds_void;
+typedef const __attribute__((address_space(1))) void global_void;
+
+// ReLU that hands a NaN on, as torch's does, in one instruction.
+__device__ __forceinline__ float relu_nan(float v) { return __builtin_elementwise_maximum(v, 0.f); }
+
+// Waits until at most N of this wave's fetches are still on their way, and for
+// all of its reads from LDS.
+template <int N>
+__device__ __forceinline__ void wait_fetches() {
+  static_assert(N >= 0 && N < 64, "the counter holds 63");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+
+// Which n-block and m-block a workgroup takes.  Consecutive workgroups go
+// round-robin over the 8 XCDs: XCD x of XN x XM takes every XM-th m-block and
+// an XN-th of the n-blocks.
+template <int NBLK, int XN>
+__device__ __forceinline__ void block_of(int id, int& n_blk, int& m_blk) {
+  constexpr int XM = 8 / XN, PER = NBLK / XN;
+  static_assert(NBLK % XN == 0, "the XCDs share the n-blocks evenly");
+  const int xcd = id & 7, i = id >> 3;
+  n_blk = (xcd % XN) * PER + i % PER;
+  m_blk = (i / PER) * XM + xcd / XN;
+}
+
+// Outputs of one tile: bias is in; ReLU, then stored in pieces, or (LAST) the
+// tile's share of the final dot product.
+template <bool LAST>
+__device__ __forceinline__ void finish_tile(const LayerArgs& a, const f32x16& acc, int n_tile,
+                                            int m_tile, int lane) {
+  const int m = lane & 31, h = lane >> 5;
+  if (LAST) {
+    float sum = 0.f;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 wl = *reinterpret_cast<const f32x4*>(a.w_last + n_tile * 32 + 8 * g + 4 * h);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum = fmaf(relu_nan(acc[4 * g + e]), wl[e], sum);
+    }
+    sum += __shfl_xor(sum, 32);
+    if (h == 0) a.part[(size_t)n_tile * (a.m_tiles * kRows) + m_tile * kRows + m] = sum;
+  } else {
+    char* out = a.y + tile_offset(m_tile, 2 * n_tile) + lane * 16;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = relu_nan(acc[8 * kk + e]);
+      store_split(out + kk * kStepBytes, v);
+    }
+  }
+}
+
+// A hidden layer for thousands of rows.  Bound by the matrix cores, at the clock
+// that the card's power allows them (a loop of nothing but these MFMAs on such
+// data: 1.7 to 1.9 PFLOP/s of the nominal 2.5), and beside them by LDS.
+//
+// A workgroup of WN x WM waves takes BN x BM tiles; the waves' fragments of a
+// k-step (a slab: three fragments per tile) go through LDS, where they are
+// shared, by direct loads (no registers, no instructions but the load's own).
+// 4 x 2 tiles per wave and 2 x 4 waves, 256 outputs x 256 rows: per slab and
+// compute unit 3072 cycles of MFMAs, 1152 of LDS reads and 768 of LDS fills.
+// Two waves per SIMD, so that one's reads and barriers lie beside the other's
+// MFMAs.  Three slabs of LDS: slab s + 3 is fetched when slab s has been read,
+// two thirds of the way through its MFMAs.
+//
+// Order of the sum: for the last SPLIT_STEPS k-steps only the five small
+// products at first, while the sum is still small; then the other steps whole;
+// then the leading products of the last ones, three steps to a slab.  24 of 64
+// steps give an error of 5.5 (see above) for 2.5 % more time than none; all of
+// them 2.4 for 8 % more.
+//
+// 32 768 rows, one layer: 0.28-0.30 ms, 235 TFLOP/s of fp32 work = 1.41 PFLOP/s
+// of bf16 (the fp32 matrix cores: 0.47 ms, 147 TFLOP/s).  Tried and not faster:
+// 128 x 256 and 128 x 128 per workgroup, two workgroups to a compute unit (1.39,
+// 1.45 against 1.55 PFLOP/s without the write-back), four waves of 4 x 4 tiles
+// (1.19), fragments stored by k-step first, fetching a slab earlier.
+template <int TN, int TM, int WN, int WM, int SPLIT_STEPS>
+struct Large {
+  static constexpr int BN = TN * WN, BM = TM * WM, TILES = BN + BM, WAVES = WN * WM;
+  static constexpr int THREADS = WAVES * 64;
+  static constexpr int FRAGS = TILES * kPieces;
+  static constexpr int LPW = FRAGS / WAVES;  // fragments a wave fetches per slab
+  static constexpr int SLAB = FRAGS * kFragBytes;
+  static constexpr int NBUF = 3;
+  static constexpr int LDS = SLAB * NBUF;
+  static constexpr int NBLK = (kWidth / 32) / BN;
+  static_assert(FRAGS % WAVES == 0, "every wave fetches as many fragments");
+  static_assert(SPLIT_STEPS % 3 == 0, "three leading products to a slab");
+};
+
+template <int TN, int TM, int WN, int WM, int SPLIT_STEPS, bool LAST>
+__global__ __launch_bounds__(WN * WM * 64, 2) void large_kernel(const LayerArgs a) {
+  using S = Large<TN, TM, WN, WM, SPLIT_STEPS>;
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = lane >> 5;
+  const int wn = wave % WN, wm = wave / WN;
+  int n_blk, m_blk;
+  block_of<S::NBLK, 1>((int)blockIdx.x, n_blk, m_blk);
+  if (m_blk * S::BM >= a.m_tiles) return;
+  const int n_tile0 = n_blk * S::BN, m_tile0 = m_blk * S::BM;
+
+  // this wave's fragments of a slab (an m-block past the end of the batch reads
+  // its last tile again and stores nothing)
+  const char* src[S::LPW];
+  int q[S::LPW];
+#pragma unroll
+  for (int i = 0; i < S::LPW; ++i) {
+    const int f = wave * S::LPW + i, tile = f / kPieces;
+    q[i] = f % kPieces;
+    const int m_t = m_tile0 + tile - S::BN;
+    src[i] = tile < S::BN ? a.w + tile_offset(n_tile0 + tile, 0)
+                          : a.x + tile_offset(m_t < a.m_tiles ? m_t : a.m_tiles - 1, 0);
+  }
+  constexpr int kFull = kSteps - SPLIT_STEPS, kSlabs = kSteps + SPLIT_STEPS / 3;
+  const uint32_t lane16 = (uint32_t)lane * 16;
+  auto fetch = [&](int slab, int buf) {
+    int step, q_stride = kFragBytes;
+    if (slab < SPLIT_STEPS) step = kFull + slab;
+    else if (slab < kSteps) step = slab - SPLIT_STEPS;
+    else { step = kFull + 3 * (slab - kSteps); q_stride = kStepBytes; }
+    if (slab >= kSlabs) step = 0;  // (not used)
+#pragma unroll
+    for (int i = 0; i < S::LPW; ++i)
+      __builtin_amdgcn_global_load_lds(
+          (global_void*)(src[i] + (uint32_t)(step * kStepBytes + q[i] * q_stride) + lane16),
+          (lds_void*)(lds + buf * S::SLAB + (wave * S::LPW + i) * kFragBytes), 16, 0, 0);
+  };
+
+  f32x16 acc[TN][TM];
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+  const int w_off = wn * TN * kStepBytes + lane * 16;
+  const int x_off = (S::BN + wm * TM) * kStepBytes + lane * 16;
+  bf16x8 w[kPieces][TN], x[kPieces][TM], w_next[TN], x_next[TM];
+  auto load_w = [&](bf16x8(&d)[TN], int buf, int p) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+      d[i] = *reinterpret_cast<const bf16x8*>(lds + buf * S::SLAB + w_off + i * kStepBytes +
+                                              p * kFragBytes);
+  };
+  auto load_x = [&](bf16x8(&d)[TM], int buf, int p) {
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+      d[j] = *reinterpret_cast<const bf16x8*>(lds + buf * S::SLAB + x_off + j * kStepBytes +
+                                              p * kFragBytes);
+  };
+  auto mm = [&](const bf16x8(&p)[TN], const bf16x8(&q)[TM]) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p[i], q[j], acc[i][j], 0, 0, 0);
+  };
+// keeps the compiler from moving a load below the MFMAs it is meant to overlap
+#define HBT_FENCE __builtin_amdgcn_sched_barrier(0)
+
+  fetch(0, 0);
+  fetch(1, 1);
+  fetch(2, 2);
+  wait_fetches<2 * S::LPW>();
+  __builtin_amdgcn_s_barrier();
+  load_w(w[0], 0, 0);
+  load_x(x[0], 0, 0);
+  int buf = 0, s = 0;
+  // Everybody has read slab s, slab s + 1 is there for everybody, slab s + 2 on
+  // its way: slab s + 3 may take the place of slab s.
+  auto turn = [&]() {
+    wait_fetches<S::LPW>();
+    __builtin_amdgcn_s_barrier();
+    fetch(s + 3, buf);
+  };
+  auto body = [&](auto leading) {
+    const int next = buf == 2 ? 0 : buf + 1;
+    load_x(x[1], buf, 1);
+    load_w(w[1], buf, 1);
+    HBT_FENCE;
+    if (leading) mm(w[0], x[0]);
+    HBT_FENCE;
+    load_x(x[2], buf, 2);
+    load_w(w[2], buf, 2);
+    HBT_FENCE;
+    mm(w[0], x[1]);
+    mm(w[1], x[0]);
+    HBT_FENCE;
+    turn();
+    HBT_FENCE;
+    mm(w[1], x[1]);
+    HBT_FENCE;
+    load_w(w_next, next, 0);
+    load_x(x_next, next, 0);
+    HBT_FENCE;
+    mm(w[0], x[2]);
+    mm(w[2], x[0]);
+    HBT_FENCE;
+#pragma unroll
+    for (int i = 0; i < TN; ++i) w[0][i] = w_next[i];
+#pragma unroll
+    for (int j = 0; j < TM; ++j) x[0][j] = x_next[j];
+    buf = next;
+  };
+#pragma unroll 1
+  for (; s < SPLIT_STEPS; ++s) body(std::false_type());
+#pragma unroll 1
+  for (; s < kSteps; ++s) body(std::true_type());
+#pragma unroll 1
+  for (; s < kSlabs; ++s) {
+    const int next = buf == 2 ? 0 : buf + 1;
+    load_x(x[1], buf, 1);
+    load_w(w[1], buf, 1);
+    HBT_FENCE;
+    mm(w[0], x[0]);
+    HBT_FENCE;
+    load_x(x[2], buf, 2);
+    load_w(w[2], buf, 2);
+    turn();
+    HBT_FENCE;
+    mm(w[1], x[1]);
+    HBT_FENCE;
+    load_w(w_next, next, 0);
+    load_x(x_next, next, 0);
+    HBT_FENCE;
+    mm(w[2], x[2]);
+    HBT_FENCE;
+#pragma unroll
+    for (int i = 0; i < TN; ++i) w[0][i] = w_next[i];
+#pragma unroll
+    for (int j = 0; j < TM; ++j) x[0][j] = x_next[j];
+    buf = next;
+  }
+  wait_fetches<0>();
+
+#pragma unroll
+  for (int i = 0; i < TN; ++i) {
+    const int n_tile = n_tile0 + wn * TN + i;
+    f32x4 b[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      b[g] = *reinterpret_cast<const f32x4*>(a.bias + n_tile * 32 + 8 * g + 4 * h);
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] += b[r >> 2][r & 3];
+      const int m_tile = m_tile0 + wm * TM + j;
+      if (m_tile < a.m_tiles) finish_tile<LAST>(a, acc[i][j], n_tile, m_tile, lane);
+    }
+  }
+}
+
+// The packed fp32 weights of one layer (pack_layer in mlp.hip) in pieces; once,
+// when the network is loaded.  One wavefront per (n-tile, k-step).
+struct PackArgs {
+  const float* w_stream;
+  int32_t groups_total;  // k-groups per wave stream
+  int32_t g0;            // first k-group of this layer
+  char* w;
+};
+__global__ __launch_bounds__(256) void pack_kernel(const PackArgs a) {
+  const int lane = threadIdx.x & 63;
+  const int item = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int tile = item / kSteps, step = item % kSteps;
+  const f32x4* in = reinterpret_cast<const f32x4*>(a.w_stream) +
+                    ((size_t)(tile >> 3) * a.groups_total + a.g0 + 2 * step) * (8 * 64) +
+                    (tile & 7) * 64 + lane;
+  float v[8];
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[4 * g + e] = in[g * (8 * 64)][e];
+  store_split(a.w + tile_offset(tile, step) + lane * 16, v);
+}
+
+struct FirstArgs {
+  const double* raw;     // [n][in_features]
+  const double* mu;
+  const double* sigma;
+  const float* w_t;      // fc1.weight transposed, [MAX_IN][kWidth]
+  const float* bias;
+  int32_t in_features;
+  int64_t n;
+  char* y;               // activations out, [m_tiles] tiles
+};
+constexpr int kFirstSlices = 8;
+
+// fc1: K is a dozen, so the layer is its 6 KiB-per-row write and little else, and
+// plain FMAs from LDS do it.  A workgroup takes one m-tile and a slice of the
+// outputs (an eighth: 2 / 8 / 16 / 32 slices took 19.4 / 8.4 / 10.0 / 13.6 us at
+// 4096 rows when the output was fp32).  Sum order: bias, then k ascending.
+// 32 768 rows: 44 us, 4.6 TB/s (a large copy on this card: 4.8).
+template <int MAX_IN>
+__global__ __launch_bounds__(256) void first_kernel(const FirstArgs a) {
+  constexpr int kSlice = kWidth / kFirstSlices;
+  __shared__ float xs[kRows][MAX_IN + 1];
+  __shared__ __attribute__((aligned(16))) float wl[MAX_IN * kSlice];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m = lane & 31, h = lane >> 5;
+  const int m_tile = blockIdx.x, n_base = (int)blockIdx.y * kSlice;
+  for (int idx = tid; idx < kRows * MAX_IN; idx += 256) {
+    const int r = idx / MAX_IN, k = idx - r * MAX_IN;
+    const int64_t row = (int64_t)m_tile * kRows + r;
+    float v = 0.f;
+    if (k < a.in_features && row < a.n)
+      v = (float)((a.raw[row * a.in_features + k] - a.mu[k]) / a.sigma[k]);
+    xs[r][k] = v;
+  }
+  for (int idx = tid; idx < a.in_features * (kSlice / 4); idx += 256) {
+    const int k = idx / (kSlice / 4), c = idx - k * (kSlice / 4);
+    *reinterpret_cast<f32x4*>(wl + k * kSlice + 4 * c) =
+        *reinterpret_cast<const f32x4*>(a.w_t + (size_t)k * kWidth + n_base + 4 * c);
+  }
+  __syncthreads();
+  for (int s = wave; s < kSlice / 16; s += 4) {
+    float v[8];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const f32x4 b = *reinterpret_cast<const f32x4*>(a.bias + n_base + 16 * s + 8 * g + 4 * h);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[4 * g + e] = b[e];
+    }
+    for (int k = 0; k < a.in_features; ++k) {
+      const float x = xs[m][k];
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const f32x4 w = *reinterpret_cast<const f32x4*>(wl + k * kSlice + 16 * s + 8 * g + 4 * h);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[4 * g + e] = fmaf(x, w[e], v[4 * g + e]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = relu_nan(v[j]);
+    store_split(a.y + tile_offset(m_tile, n_base / 16 + s) + lane * 16, v);
+  }
+}
+
+struct FinishArgs {
+  const float* part;  // [kWidth / 32][rows_pad] shares of the final dot product
+  int32_t rows_pad;
+  float b_last;
+  int64_t n;
+  float* out;         // [n]
+};
+
+// fc2: the shares of the final dot product that the last hidden layer left,
+// added in n-tile order.
+__global__ __launch_bounds__(256) void finish_kernel(const FinishArgs a) {
+  const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (row >= a.n) return;
+  float v[kWidth / 32];
+#pragma unroll
+  for (int t = 0; t < kWidth / 32; ++t) v[t] = a.part[(size_t)t * a.rows_pad + row];
+  float sum = 0.f;
+#pragma unroll
+  for (int t = 0; t < kWidth / 32; ++t) sum += v[t];
+  a.out[row] = sum + a.b_last;
+}
+
+}  // namespace split
+}  // namespace hbt

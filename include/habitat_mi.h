@@ -317,18 +317,14 @@ hbt_mlp *hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
  * (un-normalised) features [n][in_features] fp64 — operation features then the
  * four device features — are standardised in fp64, cast to fp32, and run
  * through the network; out[n] receives the fp32 predictions.  Must be called
- * with the device of hbt_mlp_create current.  Large batches go through one
- * fused kernel that runs the whole network with activations on-chip, in whole
- * rounds of 32 rows per compute unit; up to 7168 rows (a single prediction,
- * the operations of one trace, a trace for some devices, or what is left over
- * after the last whole round) each layer is one launch spread over the whole
- * GPU, with activations or partial sums in a scratch buffer that belongs to
- * the handle (2 x 28 MiB, allocated by hbt_mlp_create): calls on ONE handle
- * must therefore not overlap, on any streams; different handles are
- * independent.  Results are reproducible for a given n and position of the
- * row; the paths (per layer with K split over workgroups or waves in several
- * ways by row count, fused) sum in different orders and agree to fp32
- * rounding.
+ * with the device of hbt_mlp_create current.  Each layer is one launch spread
+ * over the whole GPU, with activations or partial sums in scratch memory that
+ * belongs to the handle (allocated by hbt_mlp_create, 13 KiB for each of 128
+ * rows per compute unit: 0.42 GB on 256; longer batches are taken in chunks):
+ * calls on ONE handle must therefore not overlap, on any streams; different
+ * handles are independent.  Results are reproducible for a given n and position
+ * of the row; the kernels for different row counts sum in different orders and
+ * agree to fp32 rounding.
  */
 int hbt_mlp_forward(hbt_mlp *mlp, const double *raw_features, int64_t n, float *out,
                     void *hip_stream);

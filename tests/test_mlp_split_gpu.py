@@ -1,0 +1,94 @@
+"""GPU: the MLP's hidden layers with every fp32 number in three bf16 pieces
+(habitat_amd/csrc/mlp_split.h), at the sizes where its kernels change."""
+import numpy as np
+import pytest
+import torch
+
+from habitat_amd import synthetic
+from habitat_amd.analysis.mlp.mlp import RuntimePredictor
+from oracle import mlp as omlp
+
+pytestmark = pytest.mark.gpu
+
+
+def network(kind, hidden, seed=0):
+    """Weights that keep the activations' size from layer to layer."""
+    torch.manual_seed(seed)
+    rp = RuntimePredictor(kind, hidden, 1024)
+    with torch.no_grad():
+        for name, p in rp.model.named_parameters():
+            if name.endswith("weight") and not name.startswith("fc2"):
+                p.mul_(6.0 ** 0.5)
+    return rp
+
+
+def forward_fp64(rp, x):
+    """oracle.mlp.forward_fp64 on the GPU (float64 matrix products)."""
+    sd = {k: v.double().cuda() for k, v in rp.model.state_dict().items()}
+    h = torch.from_numpy(omlp.standardise(x, rp.mu, rp.sigma)).cuda().double()
+    layers = ["fc1"] + sorted({k[:-7] for k in sd if k.startswith("mlp") and k.endswith("weight")},
+                              key=lambda k: int(k.split(".")[2]))
+    for name in layers:
+        h = torch.relu(h @ sd[name + ".weight"].t() + sd[name + ".bias"])
+    return (h @ sd["fc2.weight"].t() + sd["fc2.bias"]).reshape(-1).cpu().numpy()
+
+
+# around the 32-row tiles, the workgroups' 256 rows, the rounds of 16 384 rows and
+# the chunks of 32 768
+@pytest.mark.parametrize("rows", [7169, 7200, 7424, 7425, 8193, 16383, 16384, 16385, 24001, 32768,
+                                  32769, 40001])
+@pytest.mark.parametrize("hidden", [1, 2])
+def test_rows_around_the_kernels_edges(rows, hidden):
+    rp = network("lstm", hidden)
+    x, mu, sigma = synthetic.mlp_features("lstm", rows, seed=rows)
+    rp.set_normalization(mu, sigma)
+    y = rp.predict_batch(x).cpu().numpy().astype(np.float64)
+    want = forward_fp64(rp, x)
+    # Per layer a sum of 1024 products in fp32: an error of at most 8 x 2^-24 of the
+    # output's rms, as fp32 sums of that length have (7 on the fp32 matrix cores),
+    # each layer's carried through the later ones at the same size; torch's own
+    # float32 forward measures 3e-7 at the worst row here.
+    rms = float(np.sqrt(np.mean((want - want.mean()) ** 2))) + abs(float(want.mean()))
+    err = float(np.sqrt(np.mean((y - want) ** 2)))
+    assert err <= (hidden + 1) * 8 * 2.0 ** -24 * rms
+    assert float(np.max(np.abs(y - want))) <= 6 * (hidden + 1) * 8 * 2.0 ** -24 * rms
+    assert np.array_equal(y, rp.predict_batch(x).cpu().numpy().astype(np.float64))
+
+
+@pytest.mark.parametrize("rows", [9000, 20000])
+def test_values_beyond_bf16(rows):
+    """Activations beyond the largest bf16, up to infinity, and NaN: what fp32
+    arithmetic gives."""
+    rp = network("bmm", 1)
+    big = np.float32(3.4028234663852886e38)
+    finite = np.array([big, np.nextafter(big, np.float32(0)), 3.3961775e38, 3.39617e38, 3.3895e38,
+                       1.0 / 3.0, 2.0 ** -100, 1e-30, 65537.0, -big, 0.0])
+    x = np.zeros((rows, 8))
+    # One unit of fc1 is the feature and one hidden unit an eighth of it, so every
+    # result is exact; a NaN is handed on.
+    with torch.no_grad():
+        for p in rp.model.parameters():
+            p.zero_()
+        rp.model.fc1.weight[7, 2] = 1.0
+        rp.model.mlp.layers[0].weight[100, 7] = 2.0 ** -3
+        rp.model.fc2.weight[0, 100] = 1.0
+    rp.set_normalization(np.zeros(8), np.ones(8))
+    x[:, 2] = np.resize(np.append(finite, np.nan), rows)
+    y = rp.predict_batch(x).cpu().numpy()
+    v = x[:, 2].astype(np.float32)
+    want = np.maximum(v, 0) * np.float32(2.0 ** -3)
+    assert np.array_equal(y, want, equal_nan=True)
+    # An infinite activation whose every weight is positive stays an infinity:
+    # none of its pieces may meet a zero or a negative piece of a weight (0.3 and
+    # 0.7 have both).
+    with torch.no_grad():
+        rp.model.fc1.weight[:, 2] = 1.0
+        rp.model.mlp.layers[0].weight.fill_(0.3)
+        rp.model.mlp.layers[0].weight[:, ::2] = 0.7
+        rp.model.mlp.layers[0].weight[:, ::3] = 0.5
+        rp.model.fc2.weight.fill_(2.0 ** -10)
+    rp.refresh()
+    x[:, 2] = np.resize(np.array([np.inf, 1.0, 1e300, -np.inf]), rows)
+    y = rp.predict_batch(x).cpu().numpy()
+    assert np.array_equal(np.isposinf(y), x[:, 2] > 1.0)
+    assert np.all(y[x[:, 2] < 0] == 0) and np.all(np.isfinite(y[x[:, 2] == 1.0]))
