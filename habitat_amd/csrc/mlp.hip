@@ -70,8 +70,9 @@ constexpr int kSplit = 8;            // K-partials per hidden layer, up to kSpli
 // Rows up to which K is split over workgroups (the partials' traffic grows with
 // the rows; beyond this the whole-K shapes are faster).
 constexpr int kSplitMaxRows = 20;
-// Largest batch that takes this path.
-constexpr int kLayerMaxRows = 7168;
+// Largest batch that takes this path (2048 rows: 33 us a layer here, 39 in the split
+// path, which takes rounds of 4096).
+constexpr int kLayerMaxRows = 2048;
 // m-tiles up to which the eight-wave shape splits K over two workgroups (128
 // workgroups or fewer per layer would leave half the compute units idle).
 constexpr int kHalfKMaxTiles = 4;
@@ -785,12 +786,19 @@ namespace split = hbt::split;
 using hbt::kWidth;
 constexpr size_t kSplitLayerBytes = (size_t)(kWidth / 32) * split::kTileBytes;
 
-// A workgroup takes 256 outputs x 256 rows.
 struct SplitLarge {
   using S = split::Large<4, 2, 2, 4, 24>;
   static constexpr auto kHidden = &split::large_kernel<4, 2, 2, 4, 24, false>;
   static constexpr auto kLast = &split::large_kernel<4, 2, 2, 4, 24, true>;
 };
+template <int TN, int TM, int WN, int WM>
+struct SplitMid {
+  using S = split::Mid<TN, TM, WN, WM, 2, 2>;
+  static constexpr auto kHidden = &split::mid_kernel<TN, TM, WN, WM, 2, 2, false>;
+  static constexpr auto kLast = &split::mid_kernel<TN, TM, WN, WM, 2, 2, true>;
+};
+using SplitMid128 = SplitMid<2, 1, 2, 4>;
+using SplitMid192 = SplitMid<1, 3, 4, 2>;
 
 template <class C>
 bool split_ready() {
@@ -810,6 +818,31 @@ void split_launch(const split::LayerArgs& a, bool last, hipStream_t stream) {
                      a);
 }
 
+// The kernel for a layer of m_tiles m-tiles: each takes rounds of one workgroup
+// per compute unit, whatever the last one holds, so the one whose rounds cost
+// least.  Microseconds of a round measured on 256 compute units; what matters is
+// their ratio.
+using SplitLaunch = void (*)(const split::LayerArgs&, bool, hipStream_t);
+SplitLaunch split_kernel_for(int m_tiles, int compute_units) {
+  struct Choice { int tiles, blocks; float us; SplitLaunch launch; };
+  const Choice choices[] = {
+      {SplitMid128::S::BM, SplitMid128::S::NBLK, 39.f, split_launch<SplitMid128>},
+      {SplitMid192::S::BM, SplitMid192::S::NBLK, 57.f, split_launch<SplitMid192>},
+      {SplitLarge::S::BM, SplitLarge::S::NBLK, 147.f, split_launch<SplitLarge>},
+  };
+  SplitLaunch best = nullptr;
+  float best_us = 0.f;
+  for (const Choice& c : choices) {
+    const int round = c.tiles * (compute_units / c.blocks > 0 ? compute_units / c.blocks : 1);
+    const float us = (float)((m_tiles + round - 1) / round) * c.us;
+    if (best == nullptr || us < best_us) {
+      best = c.launch;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
 // The split path for up to chunk_rows rows.
 int forward_split(hbt_mlp* mlp, const double* raw_features, int64_t n, float* out,
                   hipStream_t stream) {
@@ -827,6 +860,7 @@ int forward_split(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
     hipLaunchKernelGGL(split::first_kernel<kFirstFmaMaxIn>, first_grid, dim3(256), 0, stream, f);
   else
     hipLaunchKernelGGL(split::first_kernel<kMaxInPadded>, first_grid, dim3(256), 0, stream, f);
+  const SplitLaunch launch = split_kernel_for(m_tiles, mlp->compute_units);
   split::LayerArgs l{};
   l.w_last = mlp->w_last;
   l.part = mlp->part;
@@ -837,7 +871,7 @@ int forward_split(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
     l.x = buffers[layer & 1];
     l.y = buffers[(layer + 1) & 1];
     const bool last = layer + 1 == mlp->hidden;
-    split_launch<SplitLarge>(l, last, stream);
+    launch(l, last, stream);
   }
   split::FinishArgs z{};
   z.part = mlp->part;
@@ -949,7 +983,7 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
     *err = HBT_EHIP;
     return nullptr;
   }
-  if (!split_ready<SplitLarge>()) {
+  if (!split_ready<SplitLarge>() || !split_ready<SplitMid128>() || !split_ready<SplitMid192>()) {
     (void)hipGetLastError();
     (void)hipFree(blob);
     *err = HBT_EHIP;
@@ -1035,14 +1069,13 @@ int hbt_mlp_forward(hbt_mlp* mlp, const double* raw_features, int64_t n, float* 
   if (device != mlp->device) return HBT_EINVAL;
 
   hipStream_t stream = static_cast<hipStream_t>(hip_stream);
-  // Whole rounds of the 256 x 256 workgroups through the split path, two at a
-  // time.  What is left over would cost most of another round: up to
-  // kLayerMaxRows rows go through the fp32 kernels instead.
+  // Whole rounds of the 256 x 256 workgroups, two at a time, then what is left
+  // over, with the kernels that suit it.
   const int64_t round_rows = mlp->chunk_rows / 2;
   int64_t done = 0;
   while (done < n) {
     int64_t rows = n - done < mlp->chunk_rows ? n - done : mlp->chunk_rows;
-    if (rows > round_rows && rows % round_rows <= kLayerMaxRows) rows -= rows % round_rows;
+    if (rows > round_rows) rows -= rows % round_rows;
     const double* raw = raw_features + done * mlp->in_features;
     const int rc = rows > kLayerMaxRows && mlp->hidden > 0
                        ? forward_split(mlp, raw, rows, out + done, stream)

@@ -397,6 +397,161 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void large_kernel(const LayerArgs 
   }
 }
 
+// A hidden layer for some thousands of rows, in rounds of one workgroup per
+// compute unit: smaller blocks than large_kernel's, so that a batch fills the
+// card, and for the same reason bound by LDS as much as by the matrix cores
+// (128 x 128: per k-step and compute unit 768 cycles of MFMAs, 576 of reads and
+// 384 of fills).  Eight waves, slabs of KS = 2 k-steps (one barrier for both:
+// 37 us a layer at 4096 rows against 47 with one step), two slabs of LDS.  A
+// wave holds all fragments of a step in registers and reads the next step's
+// during its MFMAs, so a slab's place is free for the next but one at the
+// barrier.  Registers allow two sets of sums, the leading products' and the small
+// ones': the error is 2.4 (see above).
+//
+//   2 x 1 tiles per wave, 2 x 4 waves   128 outputs x 128 rows: a round is 4096
+//                                       rows, 37-41 us, 210-230 TFLOP/s of fp32
+//   1 x 3, 4 x 2                        128 x 192: 6144 rows, 55-57 us, 228
+//
+// against 61 and 90 us on the fp32 matrix cores (mlp_layer_tile_kernel).
+// Tried and not faster: 1 x 2 tiles per wave and 2 x 2 with K over two waves or
+// in a ring of three to six slabs (38-52 us at 4096 rows), 96 rows (36 at 3072),
+// 128 x 256 with 2 x 2 tiles (84 at 8192; 70 with one set of sums, error 7.9).
+template <int TN, int TM, int WN, int WM, int KS, int NBUF>
+struct Mid {
+  static constexpr int BN = TN * WN, BM = TM * WM, TILES = BN + BM, WAVES = WN * WM;
+  static constexpr int THREADS = WAVES * 64;
+  static constexpr int FRAGS = TILES * KS * kPieces;
+  static constexpr int LPW = (FRAGS + WAVES - 1) / WAVES;
+  static constexpr int SLAB = FRAGS * kFragBytes;
+  static constexpr int LDS = SLAB * NBUF;
+  static constexpr int NBLK = (kWidth / 32) / BN;
+  static constexpr int SLABS = kSteps / KS;
+};
+
+template <int TN, int TM, int WN, int WM, int KS, int NBUF, bool LAST>
+__global__ __launch_bounds__(WN * WM * 64, 2) void mid_kernel(const LayerArgs a) {
+  using S = Mid<TN, TM, WN, WM, KS, NBUF>;
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = lane >> 5;
+  const int wn = wave % WN, wm = wave / WN;
+  int n_blk, m_blk;
+  block_of<S::NBLK, 1>((int)blockIdx.x, n_blk, m_blk);
+  if (m_blk * S::BM >= a.m_tiles) return;
+  const int n_tile0 = n_blk * S::BN, m_tile0 = m_blk * S::BM;
+
+  const char* src[S::LPW];
+  int dst[S::LPW];
+#pragma unroll
+  for (int i = 0; i < S::LPW; ++i) {
+    int f = wave * S::LPW + i;
+    if (S::FRAGS % S::WAVES != 0) f = f < S::FRAGS ? f : S::FRAGS - 1;
+    const int tile = f / (KS * kPieces), q = f % (KS * kPieces);
+    const int m_t = m_tile0 + tile - S::BN;
+    src[i] = (tile < S::BN ? a.w + tile_offset(n_tile0 + tile, 0)
+                           : a.x + tile_offset(m_t < a.m_tiles ? m_t : a.m_tiles - 1, 0)) +
+             q * kFragBytes;
+    dst[i] = f * kFragBytes;
+  }
+  const uint32_t lane16 = (uint32_t)lane * 16;
+  auto fetch = [&](int slab, int buf) {
+#pragma unroll
+    for (int i = 0; i < S::LPW; ++i)
+      __builtin_amdgcn_global_load_lds(
+          (global_void*)(src[i] + (uint32_t)slab * (uint32_t)(KS * kStepBytes) + lane16),
+          (lds_void*)(lds + buf * S::SLAB + dst[i]), 16, 0, 0);
+  };
+
+  f32x16 leading[TN][TM], small[TN][TM];
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) leading[i][j][r] = small[i][j][r] = 0.f;
+
+  const int w_off = wn * TN * (KS * kStepBytes) + lane * 16;
+  const int x_off = (S::BN + wm * TM) * (KS * kStepBytes) + lane * 16;
+  bf16x8 w[kPieces][TN], x[kPieces][TM];
+  auto load = [&](bf16x8(&wd)[kPieces][TN], bf16x8(&xd)[kPieces][TM], int buf, int k) {
+    const char* at = lds + buf * S::SLAB + k * kStepBytes;
+#pragma unroll
+    for (int p = 0; p < kPieces; ++p) {
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+        wd[p][i] = *reinterpret_cast<const bf16x8*>(at + w_off + i * (KS * kStepBytes) + p * kFragBytes);
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+        xd[p][j] = *reinterpret_cast<const bf16x8*>(at + x_off + j * (KS * kStepBytes) + p * kFragBytes);
+    }
+  };
+  auto mm = [&](f32x16(&d)[TN][TM], const bf16x8(&p)[TN], const bf16x8(&q)[TM]) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+        d[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p[i], q[j], d[i][j], 0, 0, 0);
+  };
+#pragma unroll
+  for (int s = 0; s < NBUF; ++s) fetch(s, s);
+  wait_fetches<(NBUF - 1) * S::LPW>();
+  __builtin_amdgcn_s_barrier();
+  load(w, x, 0, 0);
+  int buf = 0;
+#pragma unroll 1
+  for (int s = 0; s < S::SLABS; ++s) {
+    const int next = buf + 1 == NBUF ? 0 : buf + 1;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      bf16x8 wf[kPieces][TN], xf[kPieces][TM];
+      if (k == KS - 1) {
+        wait_fetches<(NBUF - 2) * S::LPW>();
+        __builtin_amdgcn_s_barrier();
+        const int ahead = s + NBUF;
+        fetch(ahead < S::SLABS ? ahead : S::SLABS - 1, buf);
+        HBT_FENCE;
+        load(wf, xf, next, 0);
+      } else {
+        load(wf, xf, buf, k + 1);
+      }
+      HBT_FENCE;
+      mm(leading, w[0], x[0]);
+      mm(small, w[0], x[1]);
+      mm(small, w[1], x[0]);
+      mm(small, w[1], x[1]);
+      mm(small, w[0], x[2]);
+      mm(small, w[2], x[0]);
+      HBT_FENCE;
+#pragma unroll
+      for (int p = 0; p < kPieces; ++p) {
+#pragma unroll
+        for (int i = 0; i < TN; ++i) w[p][i] = wf[p][i];
+#pragma unroll
+        for (int j = 0; j < TM; ++j) x[p][j] = xf[p][j];
+      }
+    }
+    buf = next;
+  }
+  wait_fetches<0>();
+
+#pragma unroll
+  for (int i = 0; i < TN; ++i) {
+    const int n_tile = n_tile0 + wn * TN + i;
+    f32x4 b[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      b[g] = *reinterpret_cast<const f32x4*>(a.bias + n_tile * 32 + 8 * g + 4 * h);
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) leading[i][j][r] = (leading[i][j][r] + small[i][j][r]) + b[r >> 2][r & 3];
+      const int m_tile = m_tile0 + wm * TM + j;
+      if (m_tile < a.m_tiles) finish_tile<LAST>(a, leading[i][j], n_tile, m_tile, lane);
+    }
+  }
+}
+
 // The packed fp32 weights of one layer (pack_layer in mlp.hip) in pieces; once,
 // when the network is loaded.  One wavefront per (n-tile, k-step).
 struct PackArgs {

@@ -33,9 +33,9 @@ def forward_fp64(rp, x):
     return (h @ sd["fc2.weight"].t() + sd["fc2.bias"]).reshape(-1).cpu().numpy()
 
 
-# around the 32-row tiles, the workgroups' 256 rows, the rounds of 16 384 rows and
-# the chunks of 32 768
-@pytest.mark.parametrize("rows", [7169, 7200, 7424, 7425, 8193, 16383, 16384, 16385, 24001, 32768,
+# around the 32-row tiles, the workgroups' 128, 192 and 256 rows, the rounds of
+# 4096, 6144 and 16 384 rows and the chunks of 32 768
+@pytest.mark.parametrize("rows", [2049, 2080, 2177, 4095, 4096, 4097, 4161, 6144, 6145, 7169, 7200, 7424, 7425, 8193, 16383, 16384, 16385, 24001, 32768,
                                   32769, 40001])
 @pytest.mark.parametrize("hidden", [1, 2])
 def test_rows_around_the_kernels_edges(rows, hidden):
