@@ -82,6 +82,7 @@ _SIGNATURES = {
     "hbt_mlp_create": (_P, [C.c_int32, C.c_int32, C.c_int32, C.POINTER(_P), C.POINTER(_P), _P, _P,
                             C.POINTER(C.c_int)]),
     "hbt_mlp_forward": (C.c_int, [_P, _P, C.c_int64, _P, _P]),
+    "hbt_mlp_forward_fp32": (C.c_int, [_P, _P, C.c_int64, _P, _P]),
     "hbt_mlp_destroy": (None, [_P]),
     "hbt_mlp_predict_one": (C.c_int, [_P, _P, C.POINTER(C.c_float), _P]),
     "hbt_mlp_forward_static": (C.c_int, [_P, _P, C.c_int64, _P, _P]),

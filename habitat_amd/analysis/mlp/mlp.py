@@ -121,7 +121,7 @@ class _DeviceMLP:
             stream.wait_stream(last)
         self._last_stream = stream
 
-    def forward(self, raw, out=None, stream=None):
+    def forward(self, raw, out=None, stream=None, entry="hbt_mlp_forward"):
         """raw: [n, in_features] float64 GPU tensor -> [n] float32 GPU tensor."""
         if raw.dtype != torch.float64 or raw.dim() != 2 or raw.shape[1] != self.in_features:
             raise TypeError("raw features must be [n, %d] float64" % self.in_features)
@@ -135,10 +135,10 @@ class _DeviceMLP:
             stream = torch.cuda.current_stream(raw.device)
         with self._lock, torch.cuda.device(raw.device):
             self._ordered_after_the_call_before(stream)
-            rc = _lib.lib().hbt_mlp_forward(self.handle, ctypes.c_void_p(raw.data_ptr()), n,
+            rc = getattr(_lib.lib(), entry)(self.handle, ctypes.c_void_p(raw.data_ptr()), n,
                                             ctypes.c_void_p(out.data_ptr()),
                                             ctypes.c_void_p(stream.cuda_stream))
-        _lib.check(rc, "hbt_mlp_forward")
+        _lib.check(rc, entry)
         return out
 
     def predict_one(self, row):
@@ -261,8 +261,16 @@ class RuntimePredictor:
         """raw_features: [n, F+4] float64 (numpy array or GPU tensor): operation
         features in `self.model.features` order followed by the four device
         features.  Returns a float32 GPU tensor of n predictions (not synchronised)."""
+        return self._forward(raw_features, out, stream, "hbt_mlp_forward")
+
+    def predict_batch_fp32(self, raw_features, out=None, stream=None):
+        """predict_batch with the sums of hbt_mlp_forward_fp32: the same last bits at
+        any n, for predictions that are divided by each other."""
+        return self._forward(raw_features, out, stream, "hbt_mlp_forward_fp32")
+
+    def _forward(self, raw_features, out, stream, entry):
         gpu = self._device_mlp()
         if isinstance(raw_features, np.ndarray):
             raw_features = torch.from_numpy(np.ascontiguousarray(raw_features, np.float64)).to(
                 gpu.torch_device)
-        return gpu.forward(raw_features, out=out, stream=stream)
+        return gpu.forward(raw_features, out=out, stream=stream, entry=entry)

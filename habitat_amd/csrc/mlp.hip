@@ -5,13 +5,13 @@
 // standardised as RuntimePredictor.predict does (mlp.py:258-264): (x - mu) /
 // sigma in fp64, then cast to fp32.
 //
-// Above kLayerMaxRows rows the hidden layers run on the bf16 matrix cores with
-// every fp32 number in three exact pieces (mlp_split.h).  Up to there they run
-// on the fp32 ones (below), with v_mfma_f32_32x32x2_f32: the A operand is a
-// 32(n) x 2(k) weight fragment, the B operand a 2(k) x 32(m) activation
-// fragment.  For these the weights are repacked once, at hbt_mlp_create, so
-// that a fragment for 8 consecutive k is one fully coalesced 1 KiB load (16 B
-// per lane) straight into the registers the MFMA reads: index
+// Above kSplitAboveRows rows hbt_mlp_forward's hidden layers run on the bf16 matrix
+// cores with every fp32 number in three exact pieces (mlp_split.h).  Up to there,
+// and in hbt_mlp_forward_fp32, they run on the fp32 ones (below), with
+// v_mfma_f32_32x32x2_f32: the A operand is a 32(n) x 2(k) weight fragment, the B
+// operand a 2(k) x 32(m) activation fragment.  For these the weights are repacked
+// once, at hbt_mlp_create, so that a fragment for 8 consecutive k is one fully
+// coalesced 1 KiB load (16 B per lane) straight into the registers the MFMA reads: index
 // [n-tile / 8][layer][k/8][n-tile % 8][lane][4] holds
 // W_layer[32 * n-tile + lane%32][8*(k/8) + 4*(lane/32) + e].
 //
@@ -32,6 +32,7 @@ namespace hbt {
 
 namespace {
 
+using u32x4 = unsigned int __attribute__((ext_vector_type(4)));
 using f32x2 = float __attribute__((ext_vector_type(2)));
 using f32x4 = float __attribute__((ext_vector_type(4)));
 using f32x16 = float __attribute__((ext_vector_type(16)));
@@ -43,7 +44,235 @@ __device__ __forceinline__ float relu(float v) { return v < 0.f ? 0.f : v; }
 
 constexpr int kWidth = 1024;      // hidden width the kernel is built for
 constexpr int kRows = 32;         // rows per workgroup (one MFMA tile of m)
+constexpr int kStride = kWidth + 4;  // LDS row stride in floats (mlp_fused_kernel)
 constexpr int kMaxInPadded = 64;  // in_features padded to a multiple of 32, at most this
+
+// ---------------------------------------------------------------------------
+// Whole rounds of 32 rows per compute unit on the fp32 matrix cores
+// (hbt_mlp_forward_fp32): one workgroup takes 32 rows through the whole
+// network, with the activations in LDS.  Bound by the fp32 matrix cores: a
+// round of 8192 rows takes 0.94 ms, 146 TFLOP/s of 157.
+struct MlpArgs {
+  const double* raw;     // [n][in_features]
+  float* out;            // [n]
+  int64_t n;
+  int32_t in_features;
+  int32_t in_padded;     // multiple of 32
+  int32_t hidden;
+  const double* mu;      // [in_features]
+  const double* sigma;   // [in_features]
+  const float* w_stream; // packed weights [waves][groups of all layers][tpw][64][4]
+  const float* bias;     // [(hidden + 1)][kWidth]: fc1 bias, then hidden biases
+  const float* w_last;   // fc2.weight [kWidth]
+  float b_last;
+};
+
+// Fragments travel through a ring of four register slots.  Weight fragments are
+// indexed by the wave's global k-group number (all layers, one stream) and are
+// loaded three groups ahead, also across a layer boundary; activation
+// fragments are loaded from LDS three groups ahead within the layer.
+template <int TPW>
+struct Ring {
+  f32x4 w[4][TPW];
+  f32x4 x[4];
+};
+
+// The wave's weight stream as a buffer resource: a load then takes the stream's
+// base from scalar registers, the k-group's offset as a scalar and the lane's
+// 16 bytes as one 32-bit register, with no 64-bit address arithmetic.
+struct WeightStream {
+  __amdgpu_buffer_rsrc_t rsrc;
+  int lane_bytes;  // 16 * lane
+};
+
+__device__ __forceinline__ WeightStream weight_stream(const f32x4* stream, int64_t bytes,
+                                                      int lane) {
+  WeightStream w;
+  w.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<f32x4*>(stream), 0, (int)bytes, 0x00020000);
+  w.lane_bytes = 16 * lane;
+  return w;
+}
+
+template <int TPW, int SLOT>
+__device__ __forceinline__ void ring_load_w(Ring<TPW>& r, const WeightStream& stream, int group,
+                                            int lane) {
+  const int group_bytes = group * (TPW * 64 * 16);
+#pragma unroll
+  for (int t = 0; t < TPW; ++t) {
+    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(stream.rsrc, stream.lane_bytes + t * 1024,
+                                                          group_bytes, 0);
+    r.w[SLOT][t] = __builtin_bit_cast(f32x4, v);
+  }
+}
+
+template <int TPW, int SLOT>
+__device__ __forceinline__ void ring_load_x(Ring<TPW>& r, const float* act_lane, int g) {
+  r.x[SLOT] = *reinterpret_cast<const f32x4*>(act_lane + 8 * g);
+}
+
+template <int TPW, int SLOT>
+__device__ __forceinline__ void ring_mfma(const Ring<TPW>& r, f32x16 (&acc)[TPW]) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int t = 0; t < TPW; ++t)
+      acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(r.w[SLOT][t][e], r.x[SLOT][e], acc[t], 0, 0, 0);
+}
+
+// One layer's K loop: kg groups of 8 k (a multiple of 4) starting at global
+// group `g0` of the wave's stream; `g_end` is the stream's last valid group.
+// On entry ring slots 0..2 hold the weights of groups g0..g0+2.
+template <int TPW>
+__device__ __forceinline__ void layer_k_loop(Ring<TPW>& r, const WeightStream& stream,
+                                             int g0, int kg, int g_end, const float* act_lane,
+                                             f32x16 (&acc)[TPW]) {
+  const int lane = threadIdx.x & 63;
+  const int last = kg - 1;
+  ring_load_x<TPW, 0>(r, act_lane, 0);
+  ring_load_x<TPW, 1>(r, act_lane, min(1, last));
+  ring_load_x<TPW, 2>(r, act_lane, min(2, last));
+  for (int j = 0; j < kg; j += 4) {
+    // The scheduling barriers keep the compiler from sinking a prefetch below
+    // the MFMA block it is meant to overlap with.  Weight groups past the end
+    // of the stream, and activation groups past the end of the layer, reload
+    // the last valid one (unused values).
+    ring_load_w<TPW, 3>(r, stream, min(g0 + j + 3, g_end), lane);
+    ring_load_x<TPW, 3>(r, act_lane, min(j + 3, last));
+    __builtin_amdgcn_sched_barrier(0);
+    ring_mfma<TPW, 0>(r, acc);
+    __builtin_amdgcn_sched_barrier(0);
+    ring_load_w<TPW, 0>(r, stream, min(g0 + j + 4, g_end), lane);
+    ring_load_x<TPW, 0>(r, act_lane, min(j + 4, last));
+    __builtin_amdgcn_sched_barrier(0);
+    ring_mfma<TPW, 1>(r, acc);
+    __builtin_amdgcn_sched_barrier(0);
+    ring_load_w<TPW, 1>(r, stream, min(g0 + j + 5, g_end), lane);
+    ring_load_x<TPW, 1>(r, act_lane, min(j + 5, last));
+    __builtin_amdgcn_sched_barrier(0);
+    ring_mfma<TPW, 2>(r, acc);
+    __builtin_amdgcn_sched_barrier(0);
+    ring_load_w<TPW, 2>(r, stream, min(g0 + j + 6, g_end), lane);
+    ring_load_x<TPW, 2>(r, act_lane, min(j + 6, last));
+    __builtin_amdgcn_sched_barrier(0);
+    ring_mfma<TPW, 3>(r, acc);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 1) void mlp_fused_kernel(const MlpArgs a) {
+  constexpr int TPW = (kWidth / 32) / WAVES;  // n-tiles per wave
+  constexpr int THREADS = WAVES * 64;
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  float* act = lds;                           // [kRows][kStride]
+  float* red = lds + kRows * kStride;         // [THREADS / 32][32]
+  float* bias_lds = red + (THREADS / 32) * 32;  // [kWidth]
+  static_assert(THREADS * 4 == kWidth, "one float4 of bias per thread");
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int m = lane & 31, h = lane >> 5;
+  const int64_t row0 = (int64_t)blockIdx.x * kRows;
+
+  // ---- stage standardised inputs: act[r][k], zero beyond in_features / n ----
+  for (int idx = tid; idx < kRows * a.in_padded; idx += THREADS) {
+    const int r = idx / a.in_padded, k = idx - r * a.in_padded;
+    float v = 0.f;
+    if (k < a.in_features && row0 + r < a.n) {
+      const double x = a.raw[(row0 + r) * a.in_features + k];
+      v = (float)((x - a.mu[k]) / a.sigma[k]);
+    }
+    act[r * kStride + k] = v;
+  }
+  // fc1's bias, where the accumulators will pick it up
+  *reinterpret_cast<f32x4*>(bias_lds + 4 * tid) = *reinterpret_cast<const f32x4*>(a.bias + 4 * tid);
+  __syncthreads();
+
+  const float* act_lane = act + m * kStride + 4 * h;
+  const int tile0 = wave * TPW;  // first n-tile of this wave
+
+  // This wave's weight stream: fc1's groups, then 128 groups per hidden layer.
+  const int kg_first = a.in_padded / 8;
+  const int groups = kg_first + a.hidden * (kWidth / 8);
+  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+  const int64_t stream_bytes = (int64_t)groups * TPW * 64 * 16;
+  const WeightStream stream = weight_stream(
+      reinterpret_cast<const f32x4*>(a.w_stream) + (size_t)wave_u * groups * TPW * 64, stream_bytes,
+      lane);
+  const int g_end = groups - 1;
+
+  Ring<TPW> ring;
+  ring_load_w<TPW, 0>(ring, stream, 0, lane);
+  ring_load_w<TPW, 1>(ring, stream, min(1, g_end), lane);
+  ring_load_w<TPW, 2>(ring, stream, min(2, g_end), lane);
+
+  f32x16 acc[TPW];
+  int g0 = 0;
+  for (int layer = 0; layer <= a.hidden; ++layer) {
+    // The accumulators start at this layer's bias, which the layer before
+    // parked in LDS; every thread fetches four values of the next layer's now
+    // and parks them after the K loop.  (Adding the bias here instead of in the
+    // write-back leaves room there for a ReLU that hands NaNs on, at no more
+    // instructions than add and max.)
+    const int next_layer = layer < a.hidden ? layer + 1 : layer;
+    const f32x4 bias_part =
+        *reinterpret_cast<const f32x4*>(a.bias + (size_t)next_layer * kWidth + 4 * tid);
+#pragma unroll
+    for (int t = 0; t < TPW; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 b =
+            *reinterpret_cast<const f32x4*>(bias_lds + (tile0 + t) * 32 + 8 * g + 4 * h);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[t][4 * g + e] = b[e];
+      }
+
+    const int kg = (layer == 0) ? kg_first : kWidth / 8;
+    layer_k_loop<TPW>(ring, stream, g0, kg, g_end, act_lane, acc);
+    g0 += kg;
+
+    __syncthreads();  // every wave has finished reading this layer's input and bias
+    *reinterpret_cast<f32x4*>(bias_lds + 4 * tid) = bias_part;
+#pragma unroll
+    for (int t = 0; t < TPW; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int n = (tile0 + t) * 32 + 8 * g + 4 * h;
+        f32x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = relu(acc[t][4 * g + e]);
+        *reinterpret_cast<f32x4*>(act + m * kStride + n) = o;
+      }
+    __syncthreads();
+  }
+
+  // ---- fc2: out[r] = sum_n act[r][n] * w_last[n] + b_last ----
+  {
+    constexpr int PARTS = THREADS / 32;
+    constexpr int NPP = kWidth / PARTS;
+    const int r = tid & 31, part = tid >> 5;
+    const float* ap = act + r * kStride + part * NPP;
+    const float* wl = a.w_last + part * NPP;
+    float s = 0.f;
+#pragma unroll 8
+    for (int k = 0; k < NPP; k += 4) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(ap + k);
+      const f32x4 w = *reinterpret_cast<const f32x4*>(wl + k);
+      s = fmaf(x[0], w[0], s);
+      s = fmaf(x[1], w[1], s);
+      s = fmaf(x[2], w[2], s);
+      s = fmaf(x[3], w[3], s);
+    }
+    red[part * 32 + r] = s;
+    __syncthreads();
+    if (tid < 32 && row0 + tid < a.n) {
+      float total = a.b_last;
+#pragma unroll
+      for (int p = 0; p < PARTS; ++p) total += red[p * 32 + tid];
+      a.out[row0 + tid] = total;
+    }
+  }
+}
 
 // ---------------------------------------------------------------------------
 // Up to kLayerMaxRows rows (one prediction, the operations of one trace, a trace
@@ -70,9 +299,13 @@ constexpr int kSplit = 8;            // K-partials per hidden layer, up to kSpli
 // Rows up to which K is split over workgroups (the partials' traffic grows with
 // the rows; beyond this the whole-K shapes are faster).
 constexpr int kSplitMaxRows = 20;
-// Largest batch that takes this path (2048 rows: 33 us a layer here, 39 in the split
-// path, which takes rounds of 4096).
-constexpr int kLayerMaxRows = 2048;
+// Largest batch that takes this path: 224 m-tiles, 7 steps of the tile kernel on
+// 256 compute units, just under what one round of the fused kernel costs
+// whatever it holds.  Tuned on 256 compute units.
+constexpr int kLayerMaxRows = 7168;
+// Largest batch of hbt_mlp_forward that takes this path (2048 rows: 33 us a layer
+// here, 39 in the split path, which takes rounds of 4096).
+constexpr int kSplitAboveRows = 2048;
 // m-tiles up to which the eight-wave shape splits K over two workgroups (128
 // workgroups or fewer per layer would leave half the compute units idle).
 constexpr int kHalfKMaxTiles = 4;
@@ -583,7 +816,11 @@ constexpr size_t kOneDoneOffset = 768;  // and the call number the last kernel p
 constexpr size_t kOneBytes = 1024;
 static_assert(kMaxInPadded * sizeof(double) <= kOneOutOffset, "a raw row fits below the result");
 
-constexpr int kWaves = 4;  // weight streams of 8 n-tiles each
+// Weight streams of 8 n-tiles each, and mlp_fused_kernel's waves: one per SIMD has
+// fewer, longer MFMA runs between load bursts than two.
+constexpr int kWaves = 4;
+constexpr size_t kLdsBytes =
+    (size_t)(kRows * kStride + (kWaves * 64 / 32) * 32 + kWidth) * sizeof(float);
 
 }  // namespace
 
@@ -781,6 +1018,29 @@ int forward_layers(hbt_mlp* mlp, const double* raw_features, int64_t n, float* o
   return hipGetLastError() == hipSuccess ? HBT_OK : HBT_EHIP;
 }
 
+// The fused kernel: one workgroup per 32 rows.
+int forward_fused(hbt_mlp* mlp, const double* raw_features, int64_t n, float* out,
+                  hipStream_t stream) {
+  using namespace hbt;
+  const int64_t blocks = (n + kRows - 1) / kRows;
+  MlpArgs a{};
+  a.raw = raw_features;
+  a.out = out;
+  a.n = n;
+  a.in_features = mlp->in_features;
+  a.in_padded = mlp->in_padded;
+  a.hidden = mlp->hidden;
+  a.mu = mlp->mu;
+  a.sigma = mlp->sigma;
+  a.w_stream = mlp->w_stream;
+  a.bias = mlp->bias;
+  a.w_last = mlp->w_last;
+  a.b_last = mlp->b_last;
+  hipLaunchKernelGGL(mlp_fused_kernel<kWaves>, dim3((unsigned)blocks), dim3(kWaves * 64),
+                     kLdsBytes, stream, a);
+  return hipGetLastError() == hipSuccess ? HBT_OK : HBT_EHIP;
+}
+
 // The split path's hidden layers (mlp_split.h).
 namespace split = hbt::split;
 using hbt::kWidth;
@@ -883,6 +1143,44 @@ int forward_split(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
   return hipGetLastError() == hipSuccess ? HBT_OK : HBT_EHIP;
 }
 
+// Any number of rows on the fp32 matrix cores.  The fused kernel keeps every
+// compute unit busy for whole rounds of 32 rows x compute units (about 0.94 ms
+// each); what is left over after the last whole round would cost another one.
+// Up to kLayerMaxRows leftover rows go through the per-layer path instead, which
+// takes less for them.
+int forward_fp32(hbt_mlp* mlp, const double* raw_features, int64_t n, float* out,
+                 hipStream_t stream) {
+  using namespace hbt;
+  const int64_t round_rows = (int64_t)kRows * mlp->compute_units;
+  const int64_t leftover = n % round_rows;
+  if (leftover == 0 || leftover > kLayerMaxRows)
+    return forward_fused(mlp, raw_features, n, out, stream);
+  const int64_t done = n - leftover;
+  if (done > 0) {
+    const int rc = forward_fused(mlp, raw_features, done, out, stream);
+    if (rc != HBT_OK) return rc;
+  }
+  return forward_layers(mlp, raw_features + done * mlp->in_features, leftover, out + done,
+                        mlp->scratch, stream);
+}
+
+// What hbt_mlp_forward and hbt_mlp_forward_fp32 refuse.
+int check_forward(const hbt_mlp* mlp, const double* raw_features, int64_t n, const float* out) {
+  if (mlp == nullptr || n < 0) return HBT_EINVAL;
+  if (n == 0) return HBT_OK;
+  if (raw_features == nullptr || out == nullptr) return HBT_EINVAL;
+  if ((reinterpret_cast<uintptr_t>(raw_features) % 8) != 0 ||
+      (reinterpret_cast<uintptr_t>(out) % 4) != 0)
+    return HBT_EALIGN;
+  if ((n + hbt::kRows - 1) / hbt::kRows > 0x7fffffff) return HBT_ESIZE;
+  int device = -1;
+  if (hipGetDevice(&device) != hipSuccess) {
+    (void)hipGetLastError();
+    return HBT_EHIP;
+  }
+  return device != mlp->device ? HBT_EINVAL : HBT_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -940,7 +1238,9 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
   off = align_up(off + sizeof(float) * first_t_rows * kWidth, 256);
   const size_t image = off;  // what is copied from the host; scratch follows
   const int64_t chunk_rows = kSplitRowsPerUnit * compute_units;
-  const size_t scratch_bytes = (size_t)(chunk_rows / kRows) * split::kTileBytes;
+  size_t scratch_bytes = (size_t)(chunk_rows / kRows) * split::kTileBytes;
+  const size_t layer_bytes = sizeof(float) * (size_t)kLayerMaxRows * kWidth;  // forward_layers
+  if (scratch_bytes < layer_bytes) scratch_bytes = layer_bytes;
   const size_t off_split = off; off = align_up(off + (size_t)hidden_layers * kSplitLayerBytes, 256);
   const size_t off_scratch0 = off; off = align_up(off + scratch_bytes, 256);
   const size_t off_scratch1 = off; off = align_up(off + scratch_bytes, 256);
@@ -983,7 +1283,10 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
     *err = HBT_EHIP;
     return nullptr;
   }
-  if (!split_ready<SplitLarge>() || !split_ready<SplitMid128>() || !split_ready<SplitMid192>()) {
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&mlp_fused_kernel<kWaves>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize,
+                          (int)kLdsBytes) != hipSuccess ||
+      !split_ready<SplitLarge>() || !split_ready<SplitMid128>() || !split_ready<SplitMid192>()) {
     (void)hipGetLastError();
     (void)hipFree(blob);
     *err = HBT_EHIP;
@@ -1053,21 +1356,8 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
 int hbt_mlp_forward(hbt_mlp* mlp, const double* raw_features, int64_t n, float* out,
                     void* hip_stream) {
   using namespace hbt;
-  if (mlp == nullptr || n < 0) return HBT_EINVAL;
-  if (n == 0) return HBT_OK;
-  if (raw_features == nullptr || out == nullptr) return HBT_EINVAL;
-  if ((reinterpret_cast<uintptr_t>(raw_features) % 8) != 0 ||
-      (reinterpret_cast<uintptr_t>(out) % 4) != 0)
-    return HBT_EALIGN;
-  const int64_t blocks = (n + kRows - 1) / kRows;
-  if (blocks > 0x7fffffff) return HBT_ESIZE;
-  int device = -1;
-  if (hipGetDevice(&device) != hipSuccess) {
-    (void)hipGetLastError();
-    return HBT_EHIP;
-  }
-  if (device != mlp->device) return HBT_EINVAL;
-
+  const int bad = check_forward(mlp, raw_features, n, out);
+  if (bad != HBT_OK || n == 0) return bad;
   hipStream_t stream = static_cast<hipStream_t>(hip_stream);
   // Whole rounds of the 256 x 256 workgroups, two at a time, then what is left
   // over, with the kernels that suit it.
@@ -1077,13 +1367,20 @@ int hbt_mlp_forward(hbt_mlp* mlp, const double* raw_features, int64_t n, float* 
     int64_t rows = n - done < mlp->chunk_rows ? n - done : mlp->chunk_rows;
     if (rows > round_rows) rows -= rows % round_rows;
     const double* raw = raw_features + done * mlp->in_features;
-    const int rc = rows > kLayerMaxRows && mlp->hidden > 0
+    const int rc = rows > kSplitAboveRows && mlp->hidden > 0
                        ? forward_split(mlp, raw, rows, out + done, stream)
-                       : forward_layers(mlp, raw, rows, out + done, mlp->scratch, stream);
+                       : forward_fp32(mlp, raw, rows, out + done, stream);
     if (rc != HBT_OK) return rc;
     done += rows;
   }
   return HBT_OK;
+}
+
+int hbt_mlp_forward_fp32(hbt_mlp* mlp, const double* raw_features, int64_t n, float* out,
+                         void* hip_stream) {
+  const int bad = check_forward(mlp, raw_features, n, out);
+  if (bad != HBT_OK || n == 0) return bad;
+  return forward_fp32(mlp, raw_features, n, out, static_cast<hipStream_t>(hip_stream));
 }
 
 int hbt_mlp_forward_static(hbt_mlp* mlp, const double* raw_features, int64_t n, float* out,

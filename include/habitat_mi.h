@@ -328,6 +328,17 @@ hbt_mlp *hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
  */
 int hbt_mlp_forward(hbt_mlp *mlp, const double *raw_features, int64_t n, float *out,
                     void *hip_stream);
+
+/*
+ * hbt_mlp_forward with every product and sum on the fp32 matrix cores at any n
+ * (hbt_mlp_forward takes large batches in bf16 pieces: faster, closer to an
+ * exact evaluation, other last bits).  For callers that divide predictions by
+ * each other and hold the quotients against earlier ones, as a device sweep does:
+ * where predictions cancel, a quotient shows another order of sums in its fifth
+ * digit.  Arguments, limits and scratch as hbt_mlp_forward.
+ */
+int hbt_mlp_forward_fp32(hbt_mlp *mlp, const double *raw_features, int64_t n, float *out,
+                         void *hip_stream);
 void hbt_mlp_destroy(hbt_mlp *mlp);
 
 /*

@@ -92,3 +92,46 @@ def test_values_beyond_bf16(rows):
     y = rp.predict_batch(x).cpu().numpy()
     assert np.array_equal(np.isposinf(y), x[:, 2] > 1.0)
     assert np.all(y[x[:, 2] < 0] == 0) and np.all(np.isfinite(y[x[:, 2] == 1.0]))
+
+
+# hbt_mlp_forward_fp32 (device sweeps): around its per-layer path's end at 7168 rows, the
+# fused kernel's rounds of 8192 and what such a round leaves over
+@pytest.mark.parametrize("rows", [2048, 2049, 7168, 7169, 8192, 8193, 16384, 20001])
+def test_fp32_sums_at_any_row_count(rows):
+    rp = network("linear", 2)
+    x, mu, sigma = synthetic.mlp_features("linear", rows, seed=rows)
+    rp.set_normalization(mu, sigma)
+    y = rp.predict_batch_fp32(x).cpu().numpy()
+    want = forward_fp64(rp, x)
+    rms = float(np.sqrt(np.mean(want ** 2)))
+    # the bound of test_rows_around_the_kernels_edges
+    assert float(np.sqrt(np.mean((y - want) ** 2))) <= 3 * 8 * 2.0 ** -24 * rms
+    # a row's sums do not depend on the rows after it: whole rounds, then the rest
+    whole = rows - rows % 8192 if rows % 8192 <= 7168 else rows
+    if whole:
+        assert np.array_equal(y[:whole], rp.predict_batch_fp32(x[:whole]).cpu().numpy())
+    if whole < rows:
+        assert np.array_equal(y[whole:], rp.predict_batch_fp32(x[whole:]).cpu().numpy())
+
+
+def test_a_sweep_divides_predictions_with_fp32_sums():
+    from habitat_amd import Device
+    from habitat_amd.analysis.predictor import Predictor
+    preds = {kind: network(kind, 2) for kind in ("conv2d", "linear")}
+    for kind, rp in preds.items():
+        _, mu, sigma = synthetic.mlp_features(kind, 2048, seed=1)
+        rp.set_normalization(mu, sigma)
+        with torch.no_grad():
+            rp.model.fc2.bias.fill_(4.0)
+        rp.refresh()
+    trace = synthetic.resnet50_trace(Device.V100, batch=32, seed=3)
+    devices, feats = synthetic.device_sweep(120, seed=3)     # 2783 convolution rows
+    features = {d.name: list(f) for d, f in zip(devices, feats)}
+    features[Device.V100.name] = [16, 900, 80, 14.028]
+    plan = Predictor(mlp_predictors=preds).plan_trace(trace)
+    sweep = plan.prepare(devices, features)
+    res = sweep.launch()
+    for kind, (_, rp, op_feats, ms, op_row) in plan.special.items():
+        y = rp.predict_batch_fp32(sweep.rows[kind]).double().view(121, -1)[:, op_row.long()]
+        want = torch.clamp(ms * y[:120] / y[120], min=0.0)
+        assert torch.equal(res.special_ms[kind], want)
