@@ -303,12 +303,12 @@ constexpr int kSplitMaxRows = 20;
 // 256 compute units, just under what one round of the fused kernel costs
 // whatever it holds.  Tuned on 256 compute units.
 constexpr int kLayerMaxRows = 7168;
-// Largest batch of hbt_mlp_forward that takes this path (2048 rows: 33 us a layer
-// here, 39 in the split path, which takes rounds of 4096).
-constexpr int kSplitAboveRows = 2048;
 // m-tiles up to which the eight-wave shape splits K over two workgroups (128
 // workgroups or fewer per layer would leave half the compute units idle).
 constexpr int kHalfKMaxTiles = 4;
+// Largest batch of hbt_mlp_forward that takes this path (256 rows: 7.6 us a layer
+// here, 6.8 in the split path; 700 rows: 15.3 and 11.8).
+constexpr int kSplitAboveRows = kHalfKMaxTiles * kRows;
 // Input features up to which fc1 of a batch stored by k-group is computed with
 // plain FMAs (mlp_first_fma_kernel); the reference's networks have 8 to 12.
 constexpr int kFirstFmaMaxIn = 16;
@@ -876,18 +876,22 @@ size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 }  // namespace
 }  // namespace hbt
 
-// Scratch memory of hbt_mlp_forward_static: the per-layer path's two buffers
-// for up to HBT_MLP_STATIC_MAX_ROWS rows, part of the code object (each GPU the
-// library runs on holds its own copy until the process ends).  In host code
-// this name is only a handle for hipGetSymbolAddress: kernels and copies get
-// the per-device address kept in static_scratch_of().
+// Scratch memory of hbt_mlp_forward_static: two buffers of activations (or
+// K-partials) for up to HBT_MLP_STATIC_MAX_ROWS rows and the split path's shares
+// of the final dot product, part of the code object (each GPU the library runs on
+// holds its own copy until the process ends).  In host code this name is only a
+// handle for hipGetSymbolAddress: kernels and copies get the per-device address
+// kept in static_scratch_of().
 constexpr int kStaticMaxRows = HBT_MLP_STATIC_MAX_ROWS;
-constexpr size_t kStaticFloats = (size_t)kStaticMaxRows * hbt::kWidth;  // each of the two
+constexpr size_t kStaticFloats =   // each of the two
+    (size_t)(kStaticMaxRows / hbt::kRows) * hbt::split::kTileBytes / sizeof(float);
+constexpr size_t kStaticShares = (size_t)(hbt::kWidth / 32) * kStaticMaxRows;
 static_assert((size_t)hbt::kSplit * hbt::kRows * hbt::kWidth <= kStaticFloats &&
                   2 * (size_t)hbt::kHalfKMaxTiles * hbt::kRows * hbt::kWidth <= kStaticFloats &&
+                  (size_t)kStaticMaxRows * hbt::kWidth <= kStaticFloats &&
                   kStaticMaxRows % hbt::kRows == 0 && kStaticMaxRows <= hbt::kLayerMaxRows,
               "the K-partials of the small shapes and the padded rows fit the static scratch");
-static __device__ __align__(256) float scratch[2 * kStaticFloats];
+static __device__ __align__(256) float scratch[2 * kStaticFloats + kStaticShares];
 
 namespace {
 
@@ -1051,17 +1055,27 @@ struct SplitLarge {
   static constexpr auto kHidden = &split::large_kernel<4, 2, 2, 4, 24, false>;
   static constexpr auto kLast = &split::large_kernel<4, 2, 2, 4, 24, true>;
 };
-template <int TN, int TM, int WN, int WM>
-struct SplitMid {
-  using S = split::Mid<TN, TM, WN, WM, 2, 2>;
-  static constexpr auto kHidden = &split::mid_kernel<TN, TM, WN, WM, 2, 2, false>;
-  static constexpr auto kLast = &split::mid_kernel<TN, TM, WN, WM, 2, 2, true>;
+struct SplitMid192 {
+  using S = split::Mid<1, 3, 4, 2, 2, 2>;
+  static constexpr auto kHidden = &split::mid_kernel<1, 3, 4, 2, 2, 2, false>;
+  static constexpr auto kLast = &split::mid_kernel<1, 3, 4, 2, 2, 2, true>;
 };
-using SplitMid128 = SplitMid<2, 1, 2, 4>;
-using SplitMid192 = SplitMid<1, 3, 4, 2>;
+template <int TN, int TM, int WAVES, int RING, int SETS>
+struct SplitSmall {
+  using S = split::Small<TN, TM, WAVES, RING, 4, SETS>;
+  static constexpr auto kHidden = &split::small_kernel<TN, TM, WAVES, RING, 4, SETS, false>;
+  static constexpr auto kLast = &split::small_kernel<TN, TM, WAVES, RING, 4, SETS, true>;
+};
+using SplitSmall1x1 = SplitSmall<1, 1, 8, 4, 2>;
+using SplitSmall1x2 = SplitSmall<1, 2, 8, 3, 2>;
+using SplitSmall2x2 = SplitSmall<2, 2, 8, 2, 2>;
+using SplitSmall2x3 = SplitSmall<2, 3, 4, 2, 2>;
+using SplitSmall2x4 = SplitSmall<2, 4, 4, 2, 2>;
+using SplitSmall4x3 = SplitSmall<4, 3, 4, 2, 1>;
+using SplitSmall4x4 = SplitSmall<4, 4, 4, 2, 1>;
 
 template <class C>
-bool split_ready() {
+bool split_ready_one() {
   const auto set = [](const void* f) {
     return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, C::S::LDS) ==
            hipSuccess;
@@ -1070,46 +1084,57 @@ bool split_ready() {
          set(reinterpret_cast<const void*>(C::kLast));
 }
 
+template <class... C>
+bool split_ready() {
+  return (split_ready_one<C>() && ...);
+}
+
 template <class C>
 void split_launch(const split::LayerArgs& a, bool last, hipStream_t stream) {
   const int m_blocks = (a.m_tiles + C::S::BM - 1) / C::S::BM;
-  const dim3 grid((unsigned)((m_blocks + 7) / 8 * 8 * C::S::NBLK));
+  const dim3 grid((unsigned)((m_blocks + C::S::XM - 1) / C::S::XM * C::S::XM * C::S::NBLK));
   hipLaunchKernelGGL(last ? C::kLast : C::kHidden, grid, dim3(C::S::THREADS), C::S::LDS, stream,
                      a);
 }
 
 // The kernel for a layer of m_tiles m-tiles: each takes rounds of one workgroup
 // per compute unit, whatever the last one holds, so the one whose rounds cost
-// least.  Microseconds of a round measured on 256 compute units; what matters is
-// their ratio.
+// least.  Microseconds on 256 compute units (start + per round, fitted to 1 to 4
+// rounds); what matters is their ratio.
 using SplitLaunch = void (*)(const split::LayerArgs&, bool, hipStream_t);
 SplitLaunch split_kernel_for(int m_tiles, int compute_units) {
-  struct Choice { int tiles, blocks; float us; SplitLaunch launch; };
-  const Choice choices[] = {
-      {SplitMid128::S::BM, SplitMid128::S::NBLK, 39.f, split_launch<SplitMid128>},
-      {SplitMid192::S::BM, SplitMid192::S::NBLK, 57.f, split_launch<SplitMid192>},
-      {SplitLarge::S::BM, SplitLarge::S::NBLK, 147.f, split_launch<SplitLarge>},
-  };
   SplitLaunch best = nullptr;
   float best_us = 0.f;
-  for (const Choice& c : choices) {
-    const int round = c.tiles * (compute_units / c.blocks > 0 ? compute_units / c.blocks : 1);
-    const float us = (float)((m_tiles + round - 1) / round) * c.us;
+  const auto consider = [&](auto kernel, float start, float round_us) {
+    using C = decltype(kernel);
+    const int per_round = C::S::BM * (compute_units / C::S::NBLK > 0 ? compute_units / C::S::NBLK : 1);
+    const float us = start + round_us * (float)((m_tiles + per_round - 1) / per_round);
     if (best == nullptr || us < best_us) {
-      best = c.launch;
+      best = split_launch<C>;
       best_us = us;
     }
-  }
+  };
+  consider(SplitSmall1x1(), 2.7f, 4.05f);   // rounds of 256 rows
+  consider(SplitSmall1x2(), 2.f, 6.9f);     // 512
+  consider(SplitSmall2x2(), 2.5f, 9.5f);    // 1024
+  consider(SplitSmall2x3(), 2.5f, 13.5f);   // 1536
+  consider(SplitSmall2x4(), 4.f, 18.f);     // 2048
+  consider(SplitSmall4x3(), 4.f, 24.5f);    // 3072
+  consider(SplitSmall4x4(), 3.f, 32.f);     // 4096
+  consider(SplitMid192(), 6.f, 44.f);       // 6144
+  consider(SplitLarge(), 0.f, 122.f);       // 16 384
   return best;
 }
 
-// The split path for up to chunk_rows rows.
+// The split path for up to chunk_rows rows, through two buffers of activations in
+// pieces (kTileBytes per m-tile) and one of the final dot product's shares
+// ([kWidth / 32][m_tiles * 32]): the handle's, or the library's static ones.
 int forward_split(hbt_mlp* mlp, const double* raw_features, int64_t n, float* out,
-                  hipStream_t stream) {
+                  float* const scratch[2], float* part, hipStream_t stream) {
   using namespace hbt;
   const int m_tiles = (int)((n + kRows - 1) / kRows);
-  char* const buffers[2] = {reinterpret_cast<char*>(mlp->scratch[0]),
-                            reinterpret_cast<char*>(mlp->scratch[1])};
+  char* const buffers[2] = {reinterpret_cast<char*>(scratch[0]),
+                            reinterpret_cast<char*>(scratch[1])};
   split::FirstArgs f{};
   f.raw = raw_features; f.mu = mlp->mu; f.sigma = mlp->sigma;
   f.w_t = mlp->w_first_t; f.bias = mlp->bias;
@@ -1123,7 +1148,7 @@ int forward_split(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
   const SplitLaunch launch = split_kernel_for(m_tiles, mlp->compute_units);
   split::LayerArgs l{};
   l.w_last = mlp->w_last;
-  l.part = mlp->part;
+  l.part = part;
   l.m_tiles = m_tiles;
   for (int layer = 0; layer < mlp->hidden; ++layer) {
     l.w = mlp->w_split + (size_t)layer * kSplitLayerBytes;
@@ -1134,7 +1159,7 @@ int forward_split(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
     launch(l, last, stream);
   }
   split::FinishArgs z{};
-  z.part = mlp->part;
+  z.part = part;
   z.rows_pad = m_tiles * kRows;
   z.b_last = mlp->b_last;
   z.n = n;
@@ -1286,7 +1311,8 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(&mlp_fused_kernel<kWaves>),
                           hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)kLdsBytes) != hipSuccess ||
-      !split_ready<SplitLarge>() || !split_ready<SplitMid128>() || !split_ready<SplitMid192>()) {
+      !split_ready<SplitSmall1x1, SplitSmall1x2, SplitSmall2x2, SplitSmall2x3, SplitSmall2x4,
+                   SplitSmall4x3, SplitSmall4x4, SplitMid192, SplitLarge>()) {
     (void)hipGetLastError();
     (void)hipFree(blob);
     *err = HBT_EHIP;
@@ -1368,7 +1394,7 @@ int hbt_mlp_forward(hbt_mlp* mlp, const double* raw_features, int64_t n, float* 
     if (rows > round_rows) rows -= rows % round_rows;
     const double* raw = raw_features + done * mlp->in_features;
     const int rc = rows > kSplitAboveRows && mlp->hidden > 0
-                       ? forward_split(mlp, raw, rows, out + done, stream)
+                       ? forward_split(mlp, raw, rows, out + done, mlp->scratch, mlp->part, stream)
                        : forward_fp32(mlp, raw, rows, out + done, stream);
     if (rc != HBT_OK) return rc;
     done += rows;
@@ -1406,7 +1432,10 @@ int hbt_mlp_forward_static(hbt_mlp* mlp, const double* raw_features, int64_t n, 
   // (rows past n within the last 32-row tile included), so nothing needs
   // clearing between calls.
   float* const buffers[2] = {base, base + kStaticFloats};
-  return forward_layers(mlp, raw_features, n, out, buffers, static_cast<hipStream_t>(hip_stream));
+  hipStream_t stream = static_cast<hipStream_t>(hip_stream);
+  return n > kSplitAboveRows && mlp->hidden > 0
+             ? forward_split(mlp, raw_features, n, out, buffers, base + 2 * kStaticFloats, stream)
+             : forward_layers(mlp, raw_features, n, out, buffers, stream);
 }
 
 int hbt_mlp_predict_one(hbt_mlp* mlp, const double* raw_row, float* out, void* hip_stream) {

@@ -227,7 +227,7 @@ struct Large {
   static constexpr int SLAB = FRAGS * kFragBytes;
   static constexpr int NBUF = 3;
   static constexpr int LDS = SLAB * NBUF;
-  static constexpr int NBLK = (kWidth / 32) / BN;
+  static constexpr int NBLK = (kWidth / 32) / BN, XM = 8;
   static_assert(FRAGS % WAVES == 0, "every wave fetches as many fragments");
   static_assert(SPLIT_STEPS % 3 == 0, "three leading products to a slab");
 };
@@ -397,25 +397,17 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void large_kernel(const LayerArgs 
   }
 }
 
-// A hidden layer for some thousands of rows, in rounds of one workgroup per
-// compute unit: smaller blocks than large_kernel's, so that a batch fills the
-// card, and for the same reason bound by LDS as much as by the matrix cores
-// (128 x 128: per k-step and compute unit 768 cycles of MFMAs, 576 of reads and
-// 384 of fills).  Eight waves, slabs of KS = 2 k-steps (one barrier for both:
-// 37 us a layer at 4096 rows against 47 with one step), two slabs of LDS.  A
-// wave holds all fragments of a step in registers and reads the next step's
-// during its MFMAs, so a slab's place is free for the next but one at the
-// barrier.  Registers allow two sets of sums, the leading products' and the small
-// ones': the error is 2.4 (see above).
-//
-//   2 x 1 tiles per wave, 2 x 4 waves   128 outputs x 128 rows: a round is 4096
-//                                       rows, 37-41 us, 210-230 TFLOP/s of fp32
-//   1 x 3, 4 x 2                        128 x 192: 6144 rows, 55-57 us, 228
-//
-// against 61 and 90 us on the fp32 matrix cores (mlp_layer_tile_kernel).
-// Tried and not faster: 1 x 2 tiles per wave and 2 x 2 with K over two waves or
-// in a ring of three to six slabs (38-52 us at 4096 rows), 96 rows (36 at 3072),
-// 128 x 256 with 2 x 2 tiles (84 at 8192; 70 with one set of sums, error 7.9).
+// A hidden layer for 4097 to 6144 rows (and multiples), in rounds of one workgroup
+// per compute unit: smaller blocks than large_kernel's, so that a batch fills the
+// card, and for the same reason bound by LDS as much as by the matrix cores.
+// 1 x 3 tiles per wave, 4 x 2 waves, 128 outputs x 192 rows: 6144 rows in 50-57
+// us, 228-250 TFLOP/s of fp32 (the fp32 matrix cores: 90 us; small_kernel in two
+// rounds: 54).  Slabs of KS = 2 k-steps (one barrier for both: 37 us a layer at
+// 4096 rows against 47 with one step), two slabs of LDS.  A wave holds all
+// fragments of a step in registers and reads the next step's during its MFMAs, so
+// a slab's place is free for the next but one at the barrier.  Registers allow
+// two sets of sums, the leading products' and the small ones': the error is 2.4
+// (see above).
 template <int TN, int TM, int WN, int WM, int KS, int NBUF>
 struct Mid {
   static constexpr int BN = TN * WN, BM = TM * WM, TILES = BN + BM, WAVES = WN * WM;
@@ -424,7 +416,7 @@ struct Mid {
   static constexpr int LPW = (FRAGS + WAVES - 1) / WAVES;
   static constexpr int SLAB = FRAGS * kFragBytes;
   static constexpr int LDS = SLAB * NBUF;
-  static constexpr int NBLK = (kWidth / 32) / BN;
+  static constexpr int NBLK = (kWidth / 32) / BN, XM = 8;
   static constexpr int SLABS = kSteps / KS;
 };
 
@@ -548,6 +540,182 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void mid_kernel(const LayerArgs a)
       for (int r = 0; r < 16; ++r) leading[i][j][r] = (leading[i][j][r] + small[i][j][r]) + b[r >> 2][r & 3];
       const int m_tile = m_tile0 + wm * TM + j;
       if (m_tile < a.m_tiles) finish_tile<LAST>(a, leading[i][j], n_tile, m_tile, lane);
+    }
+  }
+}
+
+// A hidden layer for some hundreds to 4096 rows: one workgroup per compute unit of
+// TN x TM tiles, K split over its waves.  A wave multiplies all of the
+// workgroup's tiles over its part of K, so no fragment is wanted by two waves:
+// they come straight from L2 into a ring of RING k-steps of registers (no LDS,
+// no barrier until the end), where the waves' sums then meet in wave order.
+// What bounds it is the L2 of those loads, (TN + TM) x 192 KiB per workgroup,
+// beside TN x TM x 1.3 us of MFMAs and some 3 us to start and to write back.
+// Microseconds per layer at a full round, and on the fp32 matrix cores:
+//
+//   tiles  waves  rows    here  fp32        tiles  waves  rows    here  fp32
+//   1 x 1    8     256     6.8   7.6        2 x 4    4    2048    19-24   33
+//   1 x 2    8     512     8.9  12          4 x 3    4    3072    28      47
+//   2 x 2    8    1024    12    18          4 x 4    4    4096    32-34   61
+//   2 x 3    4    1536    15.5  26
+//
+// (mid_kernel with 128 x 128 blocks took 37-40 at 3072 and 4096 rows.)  Four
+// waves have twice the registers each: room for more tiles, where one wave per
+// SIMD and a ring of two k-steps keep the matrix cores fed.  With 12 and 16 tiles
+// there is room for one set of sums only; K in four parts still keeps its error
+// below the fp32 kernels' (1.0e-7 of an fp64 evaluation against 1.6e-7; with two
+// sets 4.6e-8 against 0.9-1.2e-7).
+// XN = 4: an XCD reads a quarter of the weights and half of the activations
+// (1, 2 and 8 are within 5 %).  Tried and not faster: 16 waves (6.9 us at 160
+// rows, 16.8 at 700), 2 x 4 tiles on eight waves (out of registers), four waves
+// of 2 x 2 (12.4), 1 x 3 on eight (11.1 at 700 rows, 2 x 2 11.4), deeper rings.
+template <int TN, int TM, int WAVES, int RING, int XN, int SETS = 2>
+struct Small {
+  static constexpr int BN = TN, BM = TM, TILES = TN * TM, XM = 8 / XN;
+  static constexpr int THREADS = WAVES * 64;
+  static constexpr int STEPS = kSteps / WAVES;     // per wave
+  static constexpr int PHASES = WAVES * TILES > 40 ? 2 : 1;  // the sums meet in as many parts
+  static constexpr int PART = TILES / PHASES;      // tiles of a part
+  static constexpr int HALVES = 2 * PART;          // half tiles: a k-step of the next layer
+  static constexpr int LDS = WAVES * PART * 16 * 64 * (int)sizeof(float);
+  static constexpr int NBLK = (kWidth / 32) / BN;
+  static_assert(kSteps % WAVES == 0 && RING <= STEPS, "every wave has as many steps");
+  static_assert(TILES % PHASES == 0 && LDS <= 160 * 1024, "the sums of all waves fit the LDS");
+};
+
+template <int TN, int TM, int WAVES, int RING, int XN, int SETS, bool LAST>
+__global__ __launch_bounds__(WAVES * 64, WAVES / 4) void small_kernel(const LayerArgs a) {
+  using S = Small<TN, TM, WAVES, RING, XN, SETS>;
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  float* const red = reinterpret_cast<float*>(lds);  // [wave][tile][register][lane]
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m = lane & 31, h = lane >> 5;
+  int n_blk, m_blk;
+  block_of<S::NBLK, XN>((int)blockIdx.x, n_blk, m_blk);
+  if (m_blk * TM >= a.m_tiles) return;
+  const int n_tile0 = n_blk * TN, m_tile0 = m_blk * TM;
+
+  const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<char*>(a.w), 0, (kWidth / 32) * kTileBytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<char*>(a.x), 0, a.m_tiles * kTileBytes, 0x00020000);
+  const int step0 = wave * S::STEPS * kStepBytes;
+  int x_base[TM];  // (a tile past the end of the batch: the last one again, nothing stored)
+#pragma unroll
+  for (int j = 0; j < TM; ++j)
+    x_base[j] = (m_tile0 + j < a.m_tiles ? m_tile0 + j : a.m_tiles - 1) * kTileBytes + step0;
+  const int w_base = n_tile0 * kTileBytes + step0;
+
+  bf16x8 w[RING][kPieces][TN], x[RING][kPieces][TM];
+  auto load = [&](int slot, int step) {
+#pragma unroll
+    for (int p = 0; p < kPieces; ++p) {
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+        w[slot][p][i] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
+            w_rsrc, lane * 16 + p * kFragBytes, w_base + i * kTileBytes + step * kStepBytes, 0));
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+        x[slot][p][j] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
+            x_rsrc, lane * 16 + p * kFragBytes, x_base[j] + step * kStepBytes, 0));
+    }
+  };
+  f32x16 acc[SETS][TN][TM];  // with two: the leading products' and the small ones'
+#pragma unroll
+  for (int t = 0; t < SETS; ++t)
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[t][i][j][r] = 0.f;
+  auto mm = [&](f32x16(&d)[TN][TM], const bf16x8(&p)[TN], const bf16x8(&q)[TM]) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+        d[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p[i], q[j], d[i][j], 0, 0, 0);
+  };
+#pragma unroll
+  for (int s = 0; s < RING - 1; ++s) load(s, s);
+#pragma unroll
+  for (int s = 0; s < S::STEPS; ++s) {
+    const int c = s % RING;
+    if (s + RING - 1 < S::STEPS) load((s + RING - 1) % RING, s + RING - 1);
+    HBT_FENCE;
+    mm(acc[0], w[c][0], x[c][0]);
+    mm(acc[SETS - 1], w[c][0], x[c][1]);
+    mm(acc[SETS - 1], w[c][1], x[c][0]);
+    mm(acc[SETS - 1], w[c][1], x[c][1]);
+    mm(acc[SETS - 1], w[c][0], x[c][2]);
+    mm(acc[SETS - 1], w[c][2], x[c][0]);
+    HBT_FENCE;
+  }
+
+#pragma unroll
+  for (int phase = 0; phase < S::PHASES; ++phase) {
+    if (phase > 0) __syncthreads();
+#pragma unroll
+    for (int t = 0; t < S::PART; ++t) {
+      const int i = (phase * S::PART + t) / TM, j = (phase * S::PART + t) % TM;
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        red[((wave * S::PART + t) * 16 + r) * 64 + lane] =
+            SETS == 2 ? acc[0][i][j][r] + acc[SETS - 1][i][j][r] : acc[0][i][j][r];
+    }
+    __syncthreads();
+    // half tiles go round the waves: accumulator registers 8 kk .. 8 kk + 7 of a tile
+    constexpr int kPerWave = (S::HALVES + WAVES - 1) / WAVES;
+    float share[kPerWave];
+#pragma unroll
+    for (int q = 0; q < kPerWave; ++q) {
+      const int half = wave + q * WAVES;
+      share[q] = 0.f;
+      if (S::HALVES % WAVES != 0 && half >= S::HALVES) continue;
+      const int t = half >> 1, kk = half & 1, tile = phase * S::PART + t;
+      const int n_tile = n_tile0 + tile / TM, m_tile = m_tile0 + tile % TM;
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float sum = red[(t * 16 + 8 * kk + e) * 64 + lane];
+#pragma unroll
+        for (int p = 1; p < WAVES; ++p) sum += red[((p * S::PART + t) * 16 + 8 * kk + e) * 64 + lane];
+        v[e] = sum;
+      }
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const int n = n_tile * 32 + 16 * kk + 8 * g + 4 * h;
+        const f32x4 b = *reinterpret_cast<const f32x4*>(a.bias + n);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[4 * g + e] = relu_nan(v[4 * g + e] + b[e]);
+        if (LAST) {
+          const f32x4 wl = *reinterpret_cast<const f32x4*>(a.w_last + n);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) share[q] = fmaf(v[4 * g + e], wl[e], share[q]);
+        }
+      }
+      if (LAST)
+        share[q] += __shfl_xor(share[q], 32);
+      else if (m_tile < a.m_tiles)
+        store_split(a.y + tile_offset(m_tile, 2 * n_tile + kk) + lane * 16, v);
+    }
+    if (LAST) {
+      // a tile's two half shares of the final dot product
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < kPerWave; ++q) {
+        const int half = wave + q * WAVES;
+        if (half < S::HALVES && h == 0) red[half * 32 + m] = share[q];
+      }
+      __syncthreads();
+      for (int i = threadIdx.x; i < S::PART * 32; i += S::THREADS) {
+        const int t = i >> 5, row = i & 31, tile = phase * S::PART + t;
+        const int n_tile = n_tile0 + tile / TM, m_tile = m_tile0 + tile % TM;
+        if (m_tile < a.m_tiles)
+          a.part[(size_t)n_tile * (a.m_tiles * kRows) + m_tile * kRows + row] =
+              red[(2 * t) * 32 + row] + red[(2 * t + 1) * 32 + row];
+      }
     }
   }
 }

@@ -364,8 +364,8 @@ int hbt_mlp_predict_one(hbt_mlp *mlp, const double *raw_row, float *out, void *h
  * harnesses that forbid hipMalloc.  No counterpart in the reference.  The same
  * per-layer kernels as hbt_mlp_forward runs for such row counts (and therefore
  * bit-identical results), but their scratch (activations or partial sums
- * between the layer launches) lives in a static device array of the library, 2
- * x 4 MiB per GPU for the life of the process, not in memory of the handle; the
+ * between the layer launches) lives in a static device array of the library, 12
+ * MiB per GPU for the life of the process, not in memory of the handle; the
  * call allocates and frees nothing.  n > HBT_MLP_STATIC_MAX_ROWS returns
  * HBT_ESIZE.  All calls on one GPU share that array, whatever handle or stream
  * they use: calls that overlap on one GPU race; calls that follow each other on

@@ -33,10 +33,12 @@ def forward_fp64(rp, x):
     return (h @ sd["fc2.weight"].t() + sd["fc2.bias"]).reshape(-1).cpu().numpy()
 
 
-# around the 32-row tiles, the workgroups' 128, 192 and 256 rows, the rounds of
-# 4096, 6144 and 16 384 rows and the chunks of 32 768
-@pytest.mark.parametrize("rows", [2049, 2080, 2177, 4095, 4096, 4097, 4161, 6144, 6145, 7169, 7200, 7424, 7425, 8193, 16383, 16384, 16385, 24001, 32768,
-                                  32769, 40001])
+# around the 32-row tiles, the workgroups' 32 to 256 rows, the rounds of 256, 512,
+# 1024, 1536, 2048, 3072, 4096, 6144 and 16 384 rows and the chunks of 32 768
+@pytest.mark.parametrize("rows", [129, 160, 161, 255, 256, 257, 480, 511, 512, 513, 700, 1023, 1024,
+                                  1025, 1500, 1536, 1537, 2048, 2049, 2080, 2177, 3071, 3072, 3073,
+                                  4095, 4096, 4097, 4161, 6144, 6145, 7169, 7200, 7424, 7425, 8193,
+                                  16383, 16384, 16385, 24001, 32768, 32769, 40001])
 @pytest.mark.parametrize("hidden", [1, 2])
 def test_rows_around_the_kernels_edges(rows, hidden):
     rp = network("lstm", hidden)
@@ -55,7 +57,7 @@ def test_rows_around_the_kernels_edges(rows, hidden):
     assert np.array_equal(y, rp.predict_batch(x).cpu().numpy().astype(np.float64))
 
 
-@pytest.mark.parametrize("rows", [9000, 20000])
+@pytest.mark.parametrize("rows", [200, 400, 800, 1400, 2000, 3000, 4000, 6000, 9000, 20000])
 def test_values_beyond_bf16(rows):
     """Activations beyond the largest bf16, up to infinity, and NaN: what fp32
     arithmetic gives."""
