@@ -65,7 +65,7 @@ __device__ __forceinline__ void vec_set(typename VecOf<T, N>::type& v, int k, T 
 //
 // Every column is read once and every output written once, so both directions
 // carry the non-temporal hint: the lines are not kept in L2 or the last-level
-// cache at the expense of each other.
+// cache at the expense of each other.  (PLAIN stores do without it, see kMergeChunks.)
 template <class T, int R, class Index>
 __device__ __forceinline__ void load_r(const T* __restrict__ p, Index i, T (&out)[R]) {
   using V = typename VecOf<T, R>::type;
@@ -76,27 +76,43 @@ __device__ __forceinline__ void load_r(const T* __restrict__ p, Index i, T (&out
   for (int k = 0; k < R; ++k) out[k] = vec_get<T, R>(v, k);
 }
 
-template <class T, int R, class Index>
+template <bool PLAIN, class T, int R, class Index>
 __device__ __forceinline__ void store_r(T* __restrict__ p, Index i, const T (&in)[R]) {
   using V = typename VecOf<T, R>::type;
   V v;
 #pragma unroll
   for (int k = 0; k < R; ++k) vec_set<T, R>(v, k, in[k]);
   const Index byte = i * (Index)sizeof(T);
-  __builtin_nontemporal_store(v, reinterpret_cast<V*>(reinterpret_cast<char*>(p) + (size_t)byte));
+  V* at = reinterpret_cast<V*>(reinterpret_cast<char*>(p) + (size_t)byte);
+  if (PLAIN) *at = v;
+  else __builtin_nontemporal_store(v, at);
 }
 
 // An optional output column (null = the caller does not want it).
-template <class T, int R, class Index>
+template <bool PLAIN, class T, int R, class Index>
 __device__ __forceinline__ void store_out(T* __restrict__ p, Index i, const T (&in)[R]) {
-  if (p != nullptr) store_r<T, R>(p, i, in);
+  if (p != nullptr) store_r<PLAIN, T, R>(p, i, in);
 }
+
+// Several destinations whose rows do not begin at 128-byte lines (an odd number of
+// records): a wavefront's stores then end in the middle of a line, the next
+// wavefront writes the rest, and where the two sit on different XCDs, as
+// neighbouring workgroups do, each half goes to memory from an L2 of its own.  So
+// such launches give each XCD runs of this many neighbouring workgroups (4096
+// records) and store without the non-temporal hint: its L2 then holds the lines
+// until they are whole.  To seven destinations, 1 000 003 records: 46.5 -> 34 us,
+// 4 000 003: 176 -> 128, 8 000 003: 341 -> 244; 524 291: 26.6 -> 23.4, where 262 147
+// gain nothing (13.2, 13.9).  (Runs of 8 / 16 / 64: 133 / 130 /
+// 126 us at 4 000 003; with the hint 161-167.)  With rows at lines it is the
+// other way round, 110 us with the hint at 4 000 000 and 117-120 without.
+constexpr int kMergeChunks = 32;
+constexpr int64_t kMergeMinRecords = (int64_t)1 << 19;
 
 // Records i .. i+R-1 (all below n) for every destination of the launch.
 // SINGLE: the launch has one destination; its constants then sit at fixed
 // offsets of the argument segment and are fetched once, up front, instead of
 // inside a loop over destinations.
-template <int R, int MODEL, bool PERMUTE, bool SINGLE, class Index>
+template <int R, int MODEL, bool PERMUTE, bool SINGLE, bool MERGE, class Index>
 __device__ __forceinline__ void process(const WaveScaleArgs& a, Index i) {
   const double log2_lane = PERMUTE ? kLog2Int[threadIdx.x & 63] : 0.0;
   int32_t nb[R], block[R], dyn[R], stat[R], regs[R], dregs[R];
@@ -187,10 +203,10 @@ __device__ __forceinline__ void process(const WaveScaleArgs& a, Index i) {
       in_order = in_order || o.in_order;
     }
     const DestOut& w = a.out[d];
-    store_r<double, R>(w.time_ns, i, ot);
-    store_out<int32_t, R>(w.occ, i, occ_d);
-    store_out<int32_t, R>(w.wave, i, wave_d);
-    store_out<uint8_t, R>(w.status, i, st);
+    store_r<MERGE, double, R>(w.time_ns, i, ot);
+    store_out<MERGE, int32_t, R>(w.occ, i, occ_d);
+    store_out<MERGE, int32_t, R>(w.wave, i, wave_d);
+    store_out<MERGE, uint8_t, R>(w.status, i, st);
     // Run times beyond 2^+-500 ns (see dest_scale): the time is formed again in
     // the reference's order of operations and stored over the first one, after
     // everything else, where the rare call costs the other records nothing.
@@ -199,7 +215,7 @@ __device__ __forceinline__ void process(const WaveScaleArgs& a, Index i) {
       for (int k = 0; k < R; ++k)
         if (gamma[k] == gamma[k])
           ot[k] = scaled_time_in_order(rin[k].t, gamma[k], p.log2_bw, p.log2_clk, p.log2_clk_sm);
-      store_r<double, R>(w.time_ns, i, ot);
+      store_r<MERGE, double, R>(w.time_ns, i, ot);
     }
   }
 
@@ -210,14 +226,18 @@ __device__ __forceinline__ void process(const WaveScaleArgs& a, Index i) {
     int32_t occ_o[R], wave_o[R];
 #pragma unroll
     for (int k = 0; k < R; ++k) { occ_o[k] = mid[k].occ_o; wave_o[k] = mid[k].wave_o; }
-    store_out<int32_t, R>(a.out_occ_origin, i, occ_o);
-    store_out<int32_t, R>(a.out_wave_origin, i, wave_o);
+    store_out<MERGE, int32_t, R>(a.out_occ_origin, i, occ_o);
+    store_out<MERGE, int32_t, R>(a.out_wave_origin, i, wave_o);
   }
 }
 
-template <int R, int MODEL, bool SINGLE, class Index>
+template <int R, int MODEL, bool SINGLE, bool MERGE, class Index>
 __global__ __launch_bounds__(kBlock) void wave_scale_kernel(const WaveScaleArgs a) {
-  const Index thread = (Index)blockIdx.x * kBlock + threadIdx.x;
+  unsigned chunk = blockIdx.x;
+  if (MERGE)  // consecutive workgroups go round-robin over the 8 XCDs
+    chunk = (chunk / (8 * kMergeChunks)) * (8 * kMergeChunks) + (chunk % 8) * kMergeChunks +
+            chunk / 8 % kMergeChunks;
+  const Index thread = (Index)chunk * kBlock + threadIdx.x;
   const Index i = thread * R;
   const Index n = (Index)a.n;
   // A wavefront whose 64 * R records are all in range takes the vector path
@@ -225,10 +245,10 @@ __global__ __launch_bounds__(kBlock) void wave_scale_kernel(const WaveScaleArgs 
   // record at a time.
   const Index wave_end = ((thread | 63) + 1) * R;
   if (wave_end <= n) {
-    process<R, MODEL, true, SINGLE, Index>(a, i);
+    process<R, MODEL, true, SINGLE, MERGE, Index>(a, i);
   } else {
     const Index end = (i + R < n) ? i + R : n;
-    for (Index j = i; j < end; ++j) process<1, MODEL, false, SINGLE, Index>(a, j);
+    for (Index j = i; j < end; ++j) process<1, MODEL, false, SINGLE, MERGE, Index>(a, j);
   }
 }
 
@@ -236,12 +256,24 @@ template <int R, int MODEL, class Index>
 void launch(const WaveScaleArgs& args, hipStream_t stream) {
   const int64_t threads = (args.n + R - 1) / R;
   const int64_t blocks = (threads + kBlock - 1) / kBlock;
+  bool merge = args.n_dest > 1 && args.n >= kMergeMinRecords;
+  if (merge) {
+    bool lines = true;
+    for (int d = 0; d < args.n_dest; ++d)
+      lines = lines && reinterpret_cast<uintptr_t>(args.out[d].time_ns) % 128 == 0;
+    merge = !lines;
+  }
+  constexpr int64_t kRun = 8 * kMergeChunks;
+  const dim3 grid((unsigned)(merge ? (blocks + kRun - 1) / kRun * kRun : blocks));
   if (args.n_dest == 1)
-    hipLaunchKernelGGL((wave_scale_kernel<R, MODEL, true, Index>), dim3((unsigned)blocks),
-                       dim3(kBlock), 0, stream, args);
+    hipLaunchKernelGGL((wave_scale_kernel<R, MODEL, true, false, Index>), grid, dim3(kBlock), 0,
+                       stream, args);
+  else if (merge)
+    hipLaunchKernelGGL((wave_scale_kernel<R, MODEL, false, true, Index>), grid, dim3(kBlock), 0,
+                       stream, args);
   else
-    hipLaunchKernelGGL((wave_scale_kernel<R, MODEL, false, Index>), dim3((unsigned)blocks),
-                       dim3(kBlock), 0, stream, args);
+    hipLaunchKernelGGL((wave_scale_kernel<R, MODEL, false, false, Index>), grid, dim3(kBlock), 0,
+                       stream, args);
 }
 
 template <int R, int MODEL>

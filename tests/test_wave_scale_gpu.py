@@ -473,6 +473,28 @@ def test_ragged_sizes_single_and_multi_destination(n):
     check(rec, Device.V100, dests, wave_scale(kr, Device.V100, dests))
 
 
+# destinations' rows off the 128-byte lines, around the 524 288 records from which
+# workgroups then go to the XCDs in runs of 4096 records, and the end of such a run;
+# 524 304 has its rows at lines
+@pytest.mark.parametrize("n", [524287, 524289, 524304, 528383, 528385, 557057])
+def test_rows_off_the_lines(n):
+    rec, _ = synthetic.kernel_records(n, Device.V100, seed=n, metrics_fraction=0.5)
+    dests = [Device.MI355X, Device.T4, Device.P100]
+    kr = KernelRecords.from_numpy(rec)
+    out = WaveScaleOutput(n, 3, kr.device)
+    for t in (out.time_ns, out.occ_dest, out.wave_dest, out.status, out.occ_origin):
+        t.fill_(77)
+    wave_scale(kr, Device.V100, dests, out=out)
+    check(rec, Device.V100, dests, out)
+    # bit for bit what a launch with its rows at lines gives the same records
+    m = n - n % 16
+    lines = wave_scale(KernelRecords.from_numpy({k: v[:m] for k, v in rec.items()}), Device.V100,
+                       dests)
+    for name in ("time_ns", "occ_dest", "wave_dest", "status"):
+        a, b = getattr(out, name)[:, :m].cpu().contiguous().numpy(), getattr(lines, name).cpu().numpy()
+        assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), name
+
+
 def test_roofline_gamma_alone():
     """Row a-4 on its own: gamma of every record against the oracle's Python
     (bit-identical operation order), NaN exactly where the reference asserts."""
