@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "../../include/habitat_mi.h"
+#include "mlp_chain.h"
 #include "mlp_split.h"
 #include "wave_scale.h"
 
@@ -299,6 +300,9 @@ constexpr int kSplit = 8;            // K-partials per hidden layer, up to kSpli
 // Rows up to which K is split over workgroups (the partials' traffic grows with
 // the rows; beyond this the whole-K shapes are faster).
 constexpr int kSplitMaxRows = 20;
+// Rows that go through all layers in one launch (mlp_chain.h).
+constexpr int kChainMaxRows = chain::kMaxRows;
+constexpr size_t kChainHeader = 32;  // words before a handle's activations: the tickets
 // Largest batch that takes this path: 224 m-tiles, 7 steps of the tile kernel on
 // 256 compute units, just under what one round of the fused kernel costs
 // whatever it holds.  Tuned on 256 compute units.
@@ -840,6 +844,9 @@ struct hbt_mlp {
   float b_last;
   const char* w_split; // the hidden layers' weights in bf16 pieces, kSplitLayerBytes each
   int64_t chunk_rows;  // rows the split path takes at a time
+  // the words of chain::Args of hbt_mlp_forward and hbt_mlp_predict_one, and of
+  // hbt_mlp_forward_static; the counter of tickets comes first, in a block of its own
+  uint64_t* chain[2];
   float* scratch[2];   // activations (or K-partials) of one layer and of the next
   float* part;         // split path: [kWidth / 32][chunk_rows] shares of the final dot product
   // hbt_mlp_predict_one: a pinned, device-visible block (one raw row in, one
@@ -941,13 +948,48 @@ int tile_k_parts(int m_tiles, int compute_units) {
   return best;
 }
 
+// Up to kChainMaxRows rows through the whole network in one launch (mlp_chain.h).
+template <int ROWS>
+void launch_chain(const hbt::chain::Args& a, hipStream_t stream) {
+  hipLaunchKernelGGL(hbt::chain::chain_kernel<ROWS>, dim3((unsigned)(a.hidden * hbt::chain::kTiles + 1)),
+                     dim3(1024), 0, stream, a);
+}
+
+int forward_chain(hbt_mlp* mlp, const double* raw_features, int64_t n, float* out, uint64_t* chain,
+                  hipStream_t stream, uint32_t* done_flag, uint32_t done_value) {
+  hbt::chain::Args a{};
+  a.w_stream = mlp->w_stream;
+  a.first_groups = mlp->in_padded / 8;
+  a.groups_total = a.first_groups + mlp->hidden * (hbt::kWidth / 8);
+  a.hidden = mlp->hidden;
+  a.w_first_t = mlp->w_first_t;
+  a.bias = mlp->bias;
+  a.w_last = mlp->w_last;
+  a.b_last = mlp->b_last;
+  a.raw = raw_features; a.mu = mlp->mu; a.sigma = mlp->sigma;
+  a.in_features = mlp->in_features;
+  a.n = (int32_t)n;
+  a.out = out;
+  a.done_flag = done_flag;
+  a.done_value = done_value;
+  a.tickets = chain;
+  a.words = chain + hbt::kChainHeader;
+  if (n == 1) launch_chain<1>(a, stream);
+  else if (n == 2) launch_chain<2>(a, stream);
+  else launch_chain<4>(a, stream);
+  return hipGetLastError() == hipSuccess ? HBT_OK : HBT_EHIP;
+}
+
 // One launch per layer for n <= kLayerMaxRows rows, through two buffers of
 // activations or K-partials (each at least max(n rounded up to 32, kSplit * 32)
-// x kWidth floats): the handle's, or the library's static ones.
+// x kWidth floats): the handle's, or the library's static ones.  The fewest rows
+// take one launch for all layers.
 int forward_layers(hbt_mlp* mlp, const double* raw_features, int64_t n, float* out,
-                   float* const buffers[2], hipStream_t stream, uint32_t* done_flag = nullptr,
-                   uint32_t done_value = 0) {
+                   float* const buffers[2], uint64_t* chain, hipStream_t stream,
+                   uint32_t* done_flag = nullptr, uint32_t done_value = 0) {
   using namespace hbt;
+  if (n <= kChainMaxRows && mlp->hidden > 0)
+    return forward_chain(mlp, raw_features, n, out, chain, stream, done_flag, done_value);
   const int m_tiles = (int)((n + kRows - 1) / kRows);
   const bool split_k = n <= kSplitMaxRows;
   // with a few m-tiles the eight-wave shape splits K in two as well
@@ -1186,7 +1228,7 @@ int forward_fp32(hbt_mlp* mlp, const double* raw_features, int64_t n, float* out
     if (rc != HBT_OK) return rc;
   }
   return forward_layers(mlp, raw_features + done * mlp->in_features, leftover, out + done,
-                        mlp->scratch, stream);
+                        mlp->scratch, mlp->chain[0], stream);
 }
 
 // What hbt_mlp_forward and hbt_mlp_forward_fp32 refuse.
@@ -1271,6 +1313,9 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
   const size_t off_scratch1 = off; off = align_up(off + scratch_bytes, 256);
   const size_t off_part = off;
   off = align_up(off + sizeof(float) * (kWidth / 32) * (size_t)chunk_rows, 256);
+  const size_t chain_bytes = align_up(sizeof(uint64_t) *
+      (kChainHeader + (size_t)hidden_layers * chain::kMaxRows * kWidth), 256);
+  const size_t off_chain = off; off += 2 * chain_bytes;
   const size_t total = off;
 
   std::vector<unsigned char> host;
@@ -1313,6 +1358,12 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
                           (int)kLdsBytes) != hipSuccess ||
       !split_ready<SplitSmall1x1, SplitSmall1x2, SplitSmall2x2, SplitSmall2x3, SplitSmall2x4,
                    SplitSmall4x3, SplitSmall4x4, SplitMid192, SplitLarge>()) {
+    (void)hipGetLastError();
+    (void)hipFree(blob);
+    *err = HBT_EHIP;
+    return nullptr;
+  }
+  if (hipMemset(static_cast<unsigned char*>(blob) + off_chain, 0, 2 * chain_bytes) != hipSuccess) {
     (void)hipGetLastError();
     (void)hipFree(blob);
     *err = HBT_EHIP;
@@ -1372,6 +1423,8 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
   m->w_first_t = reinterpret_cast<const float*>(base + off_first_t);
   m->w_split = reinterpret_cast<const char*>(base + off_split);
   m->chunk_rows = chunk_rows;
+  for (int i = 0; i < 2; ++i)
+    m->chain[i] = reinterpret_cast<uint64_t*>(base + off_chain + i * chain_bytes);
   m->part = reinterpret_cast<float*>(base + off_part);
   m->b_last = b[hidden_layers + 1][0];
   m->scratch[0] = reinterpret_cast<float*>(base + off_scratch0);
@@ -1435,7 +1488,7 @@ int hbt_mlp_forward_static(hbt_mlp* mlp, const double* raw_features, int64_t n, 
   hipStream_t stream = static_cast<hipStream_t>(hip_stream);
   return n > kSplitAboveRows && mlp->hidden > 0
              ? forward_split(mlp, raw_features, n, out, buffers, base + 2 * kStaticFloats, stream)
-             : forward_layers(mlp, raw_features, n, out, buffers, stream);
+             : forward_layers(mlp, raw_features, n, out, buffers, mlp->chain[1], stream);
 }
 
 int hbt_mlp_predict_one(hbt_mlp* mlp, const double* raw_row, float* out, void* hip_stream) {
@@ -1461,7 +1514,7 @@ int hbt_mlp_predict_one(hbt_mlp* mlp, const double* raw_row, float* out, void* h
   const uint32_t call = ++mlp->one_calls;
   const int rc = forward_layers(mlp, reinterpret_cast<const double*>(mlp->one_device), 1,
                                 reinterpret_cast<float*>(mlp->one_device + kOneOutOffset),
-                                mlp->scratch, stream,
+                                mlp->scratch, mlp->chain[0], stream,
                                 reinterpret_cast<uint32_t*>(mlp->one_device + kOneDoneOffset), call);
   if (rc != HBT_OK) return rc;
   // The last kernel publishes the call's number once the prediction is in the

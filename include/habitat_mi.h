@@ -317,8 +317,8 @@ hbt_mlp *hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
  * (un-normalised) features [n][in_features] fp64 — operation features then the
  * four device features — are standardised in fp64, cast to fp32, and run
  * through the network; out[n] receives the fp32 predictions.  Must be called
- * with the device of hbt_mlp_create current.  Each layer is one launch spread
- * over the whole GPU, with activations or partial sums in scratch memory that
+ * with the device of hbt_mlp_create current.  Up to 4 rows the network is one
+ * launch, above that each layer is one, spread over the whole GPU, with activations or partial sums in scratch memory that
  * belongs to the handle (allocated by hbt_mlp_create, 13 KiB for each of 128
  * rows per compute unit: 0.42 GB on 256; longer batches are taken in chunks):
  * calls on ONE handle must therefore not overlap, on any streams; different
@@ -347,9 +347,9 @@ void hbt_mlp_destroy(hbt_mlp *mlp);
  * twice per MLP-predicted operation (analysis/predictor.py:177-180), as one C
  * call.  raw_row [in_features] and out are HOST memory.  The row goes through
  * a pinned, device-visible block of the handle (1 KiB, allocated by
- * hbt_mlp_create), the per-layer kernels of hbt_mlp_forward read it and write
+ * hbt_mlp_create), the kernel of hbt_mlp_forward reads it there and writes
  * the prediction there, and the call waits for `hip_stream` before it returns:
- * about 40 us of GPU time, launch-bound.  The result is bit-identical to
+ * about 20 us of GPU time.  The result is bit-identical to
  * hbt_mlp_forward with n = 1.  Uses the handle's scratch like hbt_mlp_forward:
  * the call must not overlap other calls on the same handle from other streams;
  * concurrent hbt_mlp_predict_one calls on one handle are serialised inside the
@@ -362,10 +362,11 @@ int hbt_mlp_predict_one(hbt_mlp *mlp, const double *raw_row, float *out, void *h
  * hbt_mlp_forward for callers that cannot allocate device memory or tolerate a
  * library that does: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc.  No counterpart in the reference.  The same
- * per-layer kernels as hbt_mlp_forward runs for such row counts (and therefore
+ * kernels as hbt_mlp_forward runs for such row counts (and therefore
  * bit-identical results), but their scratch (activations or partial sums
  * between the layer launches) lives in a static device array of the library, 12
- * MiB per GPU for the life of the process, not in memory of the handle; the
+ * MiB per GPU for the life of the process, not in memory of the handle (up to 4
+ * rows: in a part of the handle that only this entry point uses); the
  * call allocates and frees nothing.  n > HBT_MLP_STATIC_MAX_ROWS returns
  * HBT_ESIZE.  All calls on one GPU share that array, whatever handle or stream
  * they use: calls that overlap on one GPU race; calls that follow each other on

@@ -1,0 +1,105 @@
+"""GPU: a few rows through the whole network in one launch
+(habitat_amd/csrc/mlp_chain.h)."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from habitat_amd import _lib, synthetic
+from habitat_amd.analysis.mlp import mlp as mlp_module
+from habitat_amd.analysis.mlp.mlp import RuntimePredictor
+from oracle import mlp as omlp
+
+pytestmark = pytest.mark.gpu
+
+
+def network(kind, hidden, seed=0):
+    torch.manual_seed(seed)
+    rp = RuntimePredictor(kind, hidden, 1024)
+    with torch.no_grad():
+        for name, p in rp.model.named_parameters():
+            if name.endswith("weight") and not name.startswith("fc2"):
+                p.mul_(6.0 ** 0.5)
+    x, mu, sigma = synthetic.mlp_features(kind, 64, seed=seed)
+    rp.set_normalization(mu, sigma)
+    return rp, x
+
+
+# 5 rows and more take a launch per layer, whose sums the one launch repeats: the
+# same bits.  Every row count of it, between other counts.
+@pytest.mark.parametrize("kind,hidden", [("conv2d", 8), ("lstm", 1), ("bmm", 3), ("linear", 20)])
+def test_the_bits_of_the_launches_per_layer(kind, hidden):
+    rp, x = network(kind, hidden)
+    x[3] = 0.0
+    x[5, 1] = np.inf        # NaN and infinities travel as in the per-layer kernels
+    x[7, 0] = np.nan
+    x[11] *= 1e-3
+    want = rp.predict_batch(x[:16]).cpu().numpy()
+    exact = omlp.forward_fp64(rp.model.state_dict(), x[:16], rp.mu, rp.sigma)
+    ok = np.isfinite(exact)
+    # fp32 sums of 1024 products: at most 8 x 2^-24 of the output's size per layer
+    size = np.sqrt(np.mean(exact[ok] ** 2))
+    assert np.max(np.abs(want[ok] - exact[ok])) <= 6 * (hidden + 1) * 8 * 2.0 ** -24 * size
+    for rows in (1, 4, 3, 2, 5, 4, 2, 3, 1):
+        for first in (0, 16 - rows):
+            got = rp.predict_batch(x[first:first + rows]).cpu().numpy()
+            assert np.array_equal(got, want[first:first + rows], equal_nan=True), (rows, first)
+    gpu = rp._device_mlp()
+    raw = torch.from_numpy(x).cuda()
+    for rows in (1, 3):
+        out = torch.empty((rows,), dtype=torch.float32, device="cuda")
+        assert _lib.lib().hbt_mlp_forward_static(
+            gpu.handle, ctypes.c_void_p(raw.data_ptr()), rows, ctypes.c_void_p(out.data_ptr()),
+            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+        assert np.array_equal(out.cpu().numpy(), want[:rows], equal_nan=True)
+    assert gpu.predict_one(np.ascontiguousarray(x[11])) == want[11]
+
+
+def test_more_input_features_than_32():
+    class Wide(mlp_module._OperationMLP):
+        features = ["f%d" % i for i in range(36)]
+    torch.manual_seed(3)
+    rp = RuntimePredictor("conv2d", 2, 1024)
+    rp.model = Wide(2, 1024)
+    rp.set_normalization(np.arange(40) / 10.0, np.ones(40))
+    x = np.random.default_rng(3).normal(size=(12, 40))
+    want = rp.predict_batch(x).cpu().numpy()
+    for rows in (1, 2, 4):
+        assert np.array_equal(rp.predict_batch(x[:rows]).cpu().numpy(), want[:rows])
+
+
+def test_two_networks_on_two_streams():
+    """Launches that share the GPU: each waits only for its own workgroups."""
+    nets = [network("conv2d", 8, seed=s) for s in (1, 2)]
+    want = [rp.predict_batch(x[:12]).cpu().numpy() for rp, x in nets]
+    raw = [torch.from_numpy(x).cuda() for _, x in nets]
+    streams = [torch.cuda.Stream() for _ in nets]
+    torch.cuda.synchronize()
+    got = []
+    for i in range(40):
+        for (rp, _), r, s, w in zip(nets, raw, streams, want):
+            rows = 1 + i % 5
+            with torch.cuda.stream(s):
+                got.append((rp.predict_batch(r[:rows]), w[:rows]))
+    torch.cuda.synchronize()
+    for y, w in got:
+        assert np.array_equal(y.cpu().numpy(), w)
+
+
+def test_replayed_from_a_graph():
+    rp, x = network("linear", 8)
+    rows = torch.from_numpy(x).cuda()
+    raw, out = rows[:3].clone(), torch.zeros((3,), dtype=torch.float32, device="cuda")
+    rp.predict_batch(raw, out=out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        rp.predict_batch(raw, out=out)
+    for i in range(6):
+        raw.copy_(rows[3 * i:3 * i + 3])
+        graph.replay()
+        torch.cuda.synchronize()
+        replayed = out.clone()
+        assert torch.equal(replayed, rp.predict_batch(rows[3 * i:3 * i + 3]))
+        torch.cuda.synchronize()
