@@ -866,16 +866,20 @@ namespace {
 void pack_layer(const float* W, int k_in, int k_padded, int waves, float* dst, size_t wave_stride) {
   const int tpw = (kWidth / 32) / waves;
   const int kg = k_padded / 8;
+  // (a tile's 32 rows at a time, each read through: 6.5 ms for eight hidden layers, 18 with
+  // k outermost)
   for (int w = 0; w < waves; ++w)
-    for (int j = 0; j < kg; ++j)
-      for (int t = 0; t < tpw; ++t)
-        for (int lane = 0; lane < 64; ++lane)
-          for (int e = 0; e < 4; ++e) {
-            const int n = (w * tpw + t) * 32 + (lane & 31);
-            const int k = 8 * j + 4 * (lane >> 5) + e;
-            const float v = (k < k_in) ? W[(size_t)n * k_in + k] : 0.f;
-            dst[(size_t)w * wave_stride + (((size_t)j * tpw + t) * 64 + lane) * 4 + e] = v;
-          }
+    for (int t = 0; t < tpw; ++t)
+      for (int j = 0; j < kg; ++j)
+        for (int lane = 0; lane < 64; ++lane) {
+          const int n = (w * tpw + t) * 32 + (lane & 31);
+          const int k = 8 * j + 4 * (lane >> 5);
+          float* out = dst + (size_t)w * wave_stride + (((size_t)j * tpw + t) * 64 + lane) * 4;
+          const float* in = W + (size_t)n * k_in;
+          if (k + 4 <= k_in) std::memcpy(out, in + k, 4 * sizeof(float));
+          else
+            for (int e = 0; e < 4; ++e) out[e] = k + e < k_in ? in[k + e] : 0.f;
+        }
 }
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
