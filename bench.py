@@ -146,8 +146,8 @@ def tile_records(rec, n):
 
 
 def mlp_bench(args):
-    """configs[2] (and the other kinds of configs[3], one step each): the fused
-    MLP at full size, the per-layer path (up to 7168 rows), and a torch CPU baseline."""
+    """configs[2] (and the other kinds of configs[3], one step each): the MLP at
+    full size, fewer rows, and a torch CPU baseline."""
     import numpy as np
     import torch
     from habitat_amd import synthetic
@@ -234,9 +234,9 @@ def mlp_bench(args):
         mlp["parity"] = {"max_rel_error_vs_fp64": worst, "tolerance": 1e-4,
                          "floor_on_reference_magnitude": 1e-3,
                          "against": "oracle/mlp.py forward_fp64 on the first %d rows" % m}
-    few["note"] = ("rows_N_us: GPU time of one forward (HIP events); up to 7168 rows one "
-                   "launch per layer over the whole GPU (mlp_layer_kernel up to 128 rows, "
-                   "mlp_layer_tile_kernel above); predict_wall_us: wall time of one "
+    few["note"] = ("rows_N_us: GPU time of one forward (HIP events); up to 4 rows one launch "
+                   "(chain_kernel), above that one per layer over the whole GPU "
+                   "(mlp_layer_kernel up to 128 rows, split:: kernels above); predict_wall_us: wall time of one "
                    "RuntimePredictor.predict call, predict_again_wall_us: of one with arguments "
                    "asked before; cpu_rows_1_us: torch CPU fp32, batch 1, as the reference "
                    "predicts")
