@@ -122,9 +122,11 @@ __device__ __forceinline__ void put(uint64_t* word, float value, uint32_t call) 
 // The values of ROWS words `stride` apart once all of the first n carry the number
 // of this call (or a later one).  While the first is not there only that one is
 // asked for, and after kBusyLooks looks only now and then: all workgroups wait at
-// a time, and asking for every row at full rate (twice as many workgroups of half
-// a tile and eight rows, 33 MB a look) kept the writes that they waited for from
-// getting through.  (One row is 2 MB a look.)
+// a time, and where they asked for every row at full rate (twice as many, of half
+// a tile, and eight rows: 33 MB a look) some waits ran into their bound, as if the
+// reads had kept the write waited for from getting through.  One row is 2 MB a
+// look; 32 000 calls, half of them beside a kernel that takes all of the memory's
+// bandwidth, then all took their usual time.
 template <int ROWS>
 __device__ __forceinline__ void get(const uint64_t* words, int stride, int n, uint32_t call,
                                     float (&value)[ROWS]) {
