@@ -318,10 +318,10 @@ constexpr int kSplitAboveRows = kHalfKMaxTiles * kRows;
 constexpr int kFirstFmaMaxIn = 16;
 constexpr int kFirstFmaSlices = 8;     // workgroups per m-tile (gridDim.y)
 constexpr int kFirstFmaMinTiles = 64;  // m-tiles from which that kernel is used (2048 rows)
-// Rows per compute unit that the split path takes at a time: two rounds of
-// 256 x 256 workgroups per layer (291 us for two against 145-150 for one), with
-// activations that mostly stay in the 256 MB last-level cache.
-constexpr int64_t kSplitRowsPerUnit = 128;
+// Rows per compute unit that the split path takes at a time: one round of
+// 256 x 256 workgroups per layer, with activations that stay in the 256 MB
+// last-level cache: 1 M rows 72.9 ms, with two rounds 74.3 (and twice the scratch).
+constexpr int64_t kSplitRowsPerUnit = 64;
 
 struct LayerArgs {
   const float* w_stream;   // packed weights, see above
@@ -1442,13 +1442,11 @@ int hbt_mlp_forward(hbt_mlp* mlp, const double* raw_features, int64_t n, float* 
   const int bad = check_forward(mlp, raw_features, n, out);
   if (bad != HBT_OK || n == 0) return bad;
   hipStream_t stream = static_cast<hipStream_t>(hip_stream);
-  // Whole rounds of the 256 x 256 workgroups, two at a time, then what is left
-  // over, with the kernels that suit it.
-  const int64_t round_rows = mlp->chunk_rows / 2;
+  // Whole rounds of the 256 x 256 workgroups, then what is left over, with the
+  // kernels that suit it.
   int64_t done = 0;
   while (done < n) {
-    int64_t rows = n - done < mlp->chunk_rows ? n - done : mlp->chunk_rows;
-    if (rows > round_rows) rows -= rows % round_rows;
+    const int64_t rows = n - done < mlp->chunk_rows ? n - done : mlp->chunk_rows;
     const double* raw = raw_features + done * mlp->in_features;
     const int rc = rows > kSplitAboveRows && mlp->hidden > 0
                        ? forward_split(mlp, raw, rows, out + done, mlp->scratch, mlp->part, stream)

@@ -213,7 +213,7 @@ __device__ __forceinline__ void finish_tile(const LayerArgs& a, const f32x16& ac
 // steps give an error of 5.5 (see above) for 2.5 % more time than none; all of
 // them 2.4 for 8 % more.
 //
-// 32 768 rows, one layer: 0.28-0.30 ms, 235 TFLOP/s of fp32 work = 1.41 PFLOP/s
+// 32 768 rows in two rounds, one layer: 0.28-0.30 ms, 235 TFLOP/s of fp32 work = 1.41 PFLOP/s
 // of bf16 (the fp32 matrix cores: 0.47 ms, 147 TFLOP/s).  Tried and not faster:
 // 128 x 256 and 128 x 128 per workgroup, two workgroups to a compute unit (1.39,
 // 1.45 against 1.55 PFLOP/s without the write-back), four waves of 4 x 4 tiles

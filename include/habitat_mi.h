@@ -319,8 +319,8 @@ hbt_mlp *hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
  * through the network; out[n] receives the fp32 predictions.  Must be called
  * with the device of hbt_mlp_create current.  Up to 4 rows the network is one
  * launch, above that each layer is one, spread over the whole GPU, with activations or partial sums in scratch memory that
- * belongs to the handle (allocated by hbt_mlp_create, 13 KiB for each of 128
- * rows per compute unit: 0.42 GB on 256; longer batches are taken in chunks):
+ * belongs to the handle (allocated by hbt_mlp_create, 13 KiB for each of 64
+ * rows per compute unit: 0.21 GB on 256; longer batches are taken in chunks):
  * calls on ONE handle must therefore not overlap, on any streams; different
  * handles are independent.  Results are reproducible for a given n and position
  * of the row; the kernels for different row counts sum in different orders and

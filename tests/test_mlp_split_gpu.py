@@ -34,7 +34,7 @@ def forward_fp64(rp, x):
 
 
 # around the 32-row tiles, the workgroups' 32 to 256 rows, the rounds of 256, 512,
-# 1024, 1536, 2048, 3072, 4096, 6144 and 16 384 rows and the chunks of 32 768
+# 1024, 1536, 2048, 3072, 4096, 6144 and 16 384 rows, and chunks of 16 384
 @pytest.mark.parametrize("rows", [129, 160, 161, 255, 256, 257, 480, 511, 512, 513, 700, 1023, 1024,
                                   1025, 1500, 1536, 1537, 2048, 2049, 2080, 2177, 3071, 3072, 3073,
                                   4095, 4096, 4097, 4161, 6144, 6145, 7169, 7200, 7424, 7425, 8193,
