@@ -953,12 +953,6 @@ int tile_k_parts(int m_tiles, int compute_units) {
 }
 
 // Up to kChainMaxRows rows through the whole network in one launch (mlp_chain.h).
-template <int ROWS>
-void launch_chain(const hbt::chain::Args& a, hipStream_t stream) {
-  hipLaunchKernelGGL(hbt::chain::chain_kernel<ROWS>, dim3((unsigned)(a.hidden * hbt::chain::kTiles + 1)),
-                     dim3(1024), 0, stream, a);
-}
-
 int forward_chain(hbt_mlp* mlp, const double* raw_features, int64_t n, float* out, uint64_t* chain,
                   hipStream_t stream, uint32_t* done_flag, uint32_t done_value) {
   hbt::chain::Args a{};
@@ -978,10 +972,7 @@ int forward_chain(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
   a.done_value = done_value;
   a.tickets = chain;
   a.words = chain + hbt::kChainHeader;
-  if (n == 1) launch_chain<1>(a, stream);
-  else if (n == 2) launch_chain<2>(a, stream);
-  else launch_chain<4>(a, stream);
-  return hipGetLastError() == hipSuccess ? HBT_OK : HBT_EHIP;
+  return hbt::chain::launch(a, stream) == hipSuccess ? HBT_OK : HBT_EHIP;
 }
 
 // One launch per layer for n <= kLayerMaxRows rows, through two buffers of

@@ -7,7 +7,9 @@
 // for the activations of the layer before.  Those come as 8-byte words of a value
 // and the number of the call, written and read with single atomic accesses, so a
 // word that carries this call's number is the value itself: one trip through
-// memory per layer, no fence, no counter, no clearing between calls.
+// memory per layer, no fence, no counter, no clearing between calls.  Every
+// kNumberAll-th call numbers the words of all kMaxRows rows, also those past its own:
+// no word is older than that, and 32 bits of the number are enough for good.
 //
 // Order of workgroups: each takes the next ticket of the handle's counter when it
 // starts, and the ticket says which tile of which layer it is.  So a workgroup
@@ -43,6 +45,7 @@ constexpr int kTiles = kWidth / 32;
 // and 44.2).  What a row adds is its share of the multiply-adds on a layer's 32
 // compute units, 0.2 us, and the reads of the next layer.
 constexpr int kMaxRows = 4;
+constexpr uint32_t kNumberAll = 1u << 16;
 constexpr int kMaxIn = 64;
 constexpr int kFewIn = 16;   // rows that w_first_t has at least, zero beyond the features
 constexpr int kChains = 32;  // sums of 32 products that an output is added up from
@@ -114,13 +117,20 @@ __device__ __forceinline__ float add_products(const f32x4 (&w)[4][2], float x, f
 
 __device__ __forceinline__ float relu(float v) { return v < 0.f ? 0.f : v; }
 
+// Whether a word was written by this call.  Until then it holds the number of one of
+// the 2 kNumberAll calls before, or the 0 of a new handle, whose first calls have
+// other numbers.
+__device__ __host__ constexpr bool carries(uint64_t word, uint32_t call) {
+  return (uint32_t)(word >> 32) == call;
+}
+
 __device__ __forceinline__ void put(uint64_t* word, float value, uint32_t call) {
   __hip_atomic_store(word, (uint64_t)call << 32 | __builtin_bit_cast(uint32_t, value),
                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // The values of ROWS words `stride` apart once all of the first n carry the number
-// of this call (or a later one).  While the first is not there only that one is
+// of this call.  While the first is not there only that one is
 // asked for, and after kBusyLooks looks only now and then: all workgroups wait at
 // a time, and where they asked for every row at full rate (twice as many, of half
 // a tile, and eight rows: 33 MB a look) some waits ran into their bound, as if the
@@ -135,7 +145,7 @@ __device__ __forceinline__ void get(const uint64_t* words, int stride, int n, ui
     v[r] = __hip_atomic_load(words + (r < n ? r : 0) * stride, __ATOMIC_RELAXED,
                              __HIP_MEMORY_SCOPE_AGENT);
   };
-  const auto there = [&](int r) { return (int32_t)((uint32_t)(v[r] >> 32) - call) >= 0; };
+  const auto there = [&](int r) { return carries(v[r], call); };
   for (int look = 0; look < kMaxLooks; ++look) {
     ask(0);
     if (there(0)) {
@@ -189,6 +199,8 @@ __global__ __launch_bounds__(1024) void chain_kernel(const Args a) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) w[j][h] = at[j * (8 * 64) + 32 * h];
   }
+  if (__builtin_expect(call % kNumberAll == 0, 0) && layer < a.hidden && c >= a.n && c < kMaxRows)
+    put(a.words + ((size_t)layer * kMaxRows + c) * kWidth + tile * 32 + n, 0.f, call);
 
   if (layer == 0) {
     // fc1, by each of the first layer's workgroups for itself: thread = output;
@@ -297,6 +309,17 @@ __global__ __launch_bounds__(1024) void chain_kernel(const Args a) {
       __hip_atomic_store(a.done_flag, a.done_value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
   }
+}
+
+// The network for a.n rows, 1 to kMaxRows; hidden > 0.
+inline hipError_t launch(const Args& a, hipStream_t stream) {
+  const auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(a.hidden * kTiles + 1)), dim3(1024), 0, stream, a);
+  };
+  if (a.n == 1) go(chain_kernel<1>);
+  else if (a.n == 2) go(chain_kernel<2>);
+  else go(chain_kernel<4>);
+  return hipGetLastError();
 }
 
 }  // namespace chain

@@ -448,3 +448,22 @@ def test_gpu_selftest_library_builds_and_exports_its_checkers():
     for name in ("arith_fast_div", "arith_ceil_div", "arith_div_const", "arith_exp2",
                  "arith_exp2_at", "arith_occupancy_lattice"):
         assert hasattr(lib, name), name
+
+
+def test_few_row_mlp_words_count_for_their_own_call_only():
+    """tests/native/mlp_chain.hip: the few-row MLP kernel takes a word of value and
+    call number for this call's only at that number.  A signed distance took
+    whatever lay up to 2^31 numbers ahead, which is where words of rows that no
+    call had written for that long, or ever, end up.  Nothing is launched here."""
+    import ctypes
+    import subprocess
+    native = os.path.join(ROOT, "tests", "native")
+    subprocess.check_call(["make", "-s", "-C", native])
+    lib = ctypes.CDLL(os.path.join(native, "_build", "libmlp_chain.so"))
+    assert hasattr(lib, "chain_forward")
+    lib.chain_carries.argtypes = [ctypes.c_uint64, ctypes.c_uint32]
+    numbers = [0, 1, 2, 1000, 2 ** 31 - 1, 2 ** 31, 2 ** 31 + 1, 2 ** 32 - 2, 2 ** 32 - 1]
+    for call in numbers:
+        for written in numbers:
+            for bits in (0, 0x3f800000, 0x7fc00000, 0xffffffff):
+                assert bool(lib.chain_carries(written << 32 | bits, call)) == (written == call)

@@ -1,6 +1,7 @@
 """GPU: a few rows through the whole network in one launch
 (habitat_amd/csrc/mlp_chain.h)."""
 import ctypes
+import os
 
 import numpy as np
 import pytest
@@ -12,6 +13,9 @@ from habitat_amd.analysis.mlp.mlp import RuntimePredictor
 from oracle import mlp as omlp
 
 pytestmark = pytest.mark.gpu
+
+NATIVE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "_build",
+                      "libmlp_chain.so")
 
 
 def network(kind, hidden, seed=0):
@@ -103,3 +107,73 @@ def test_replayed_from_a_graph():
         replayed = out.clone()
         assert torch.equal(replayed, rp.predict_batch(rows[3 * i:3 * i + 3]))
         torch.cuda.synchronize()
+
+
+class Chain:
+    """A network of eight features and up to 16 for hbt::chain::launch, with the
+    hand-over's counter and words in tensors of the test's."""
+
+    def __init__(self, rp):
+        if not os.path.exists(NATIVE):
+            pytest.fail("tests/native/_build/libmlp_chain.so is not built: run "
+                        "`make -C tests/native` (or __graft_entry__.build()) first")
+        lib = ctypes.CDLL(NATIVE)
+        P, I, F = ctypes.c_void_p, ctypes.c_int32, ctypes.c_float
+        lib.chain_forward.argtypes = [P, I, I, P, P, P, F, P, P, P, I, I, P, P, P, P]
+        self.lib, self.max_rows = lib, lib.chain_max_rows()
+        sd = {k: v.numpy() for k, v in rp.model.state_dict().items()}
+        names = ["fc1"] + sorted({k[:-7] for k in sd if k.startswith("mlp") and "weight" in k},
+                                 key=lambda k: int(k.split(".")[2]))
+        self.hidden = len(names) - 1
+        self.blocks = 32 * self.hidden + 1
+        fc1 = sd["fc1.weight"]
+        self.f = fc1.shape[1]
+        assert self.f <= 16
+        packed, first_t = [], np.zeros((16, 1024), np.float32)
+        first_t[:self.f] = fc1.T
+        for name in names:
+            w = sd[name + ".weight"]
+            w = np.pad(w, ((0, 0), (0, (-w.shape[1]) % 32)))
+            # [stream][k-group][n-tile % 8][half][row][4]
+            packed.append(w.reshape(4, 8, 32, -1, 2, 4).transpose(0, 3, 1, 4, 2, 5))
+        up = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+        self.w, self.first_t = up(np.concatenate(packed, axis=1)), up(first_t)
+        self.bias = up(np.stack([sd[n + ".bias"] for n in names]))
+        self.w_last, self.b_last = up(sd["fc2.weight"].reshape(-1)), float(sd["fc2.bias"][0])
+        self.mu, self.sigma = up(rp.mu), up(rp.sigma)
+        self.tickets = torch.zeros(1, dtype=torch.int64, device="cuda")
+        self.words = torch.zeros((self.hidden, self.max_rows, 1024), dtype=torch.int64,
+                                 device="cuda")
+
+    def __call__(self, raw):
+        out = torch.full((raw.shape[0],), -1.0, dtype=torch.float32, device="cuda")
+        p = lambda t: ctypes.c_void_p(t.data_ptr())
+        rc = self.lib.chain_forward(
+            p(self.w), 4, self.hidden, p(self.first_t), p(self.bias), p(self.w_last), self.b_last,
+            p(raw), p(self.mu), p(self.sigma), self.f, raw.shape[0], p(out), p(self.tickets),
+            p(self.words), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert rc == 0
+        return out.cpu().numpy()
+
+
+def test_words_of_older_calls_are_never_taken():
+    """A word counts when it carries this call's number: not one that was never
+    written, or by a call 2^31 numbers ago, nor where the number's 32 bits turn over."""
+    rp, x = network("conv2d", 3)
+    want = rp.predict_batch(x[:20]).cpu().numpy()
+    chain, raw = Chain(rp), torch.from_numpy(x).cuda()
+    assert np.array_equal(chain(raw[:4]), want[:4])
+    for before in (2 ** 31 - 2, 2 ** 31 + 5, 2 ** 32 - 3, 3 * 2 ** 31):
+        for left in (0, 0x7fc00000, (7 << 32) + 0x3f800000):   # unwritten, NaN, call 7's 1.0
+            chain.tickets.fill_(before * chain.blocks)
+            chain.words.fill_(left)
+            for i, rows in enumerate((4, 1, 1, 3, 1, 2, 4)):
+                got = chain(raw[i:i + rows])
+                assert np.array_equal(got, want[i:i + rows]), (before, left, i)
+                call = (before + i + 1) % 2 ** 32
+                numbered = ((chain.words >> 32) & 0xffffffff) == call
+                assert bool(torch.all(numbered[:, :rows]))
+                if call % 2 ** 16 == 0:    # every so often all rows', so that none gets old
+                    assert bool(torch.all(numbered))
+                else:
+                    assert not bool(torch.any(numbered[:, rows:]))
