@@ -972,6 +972,7 @@ int forward_chain(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
   a.done_value = done_value;
   a.tickets = chain;
   a.words = chain + hbt::kChainHeader;
+  a.looks = hbt::chain::kMaxLooks;
   return hbt::chain::launch(a, stream) == hipSuccess ? HBT_OK : HBT_EHIP;
 }
 

@@ -14,7 +14,9 @@
 // Order of workgroups: each takes the next ticket of the handle's counter when it
 // starts, and the ticket says which tile of which layer it is.  So a workgroup
 // waits only for ones that have started before it: nothing has to be resident
-// together, and several such launches may share the GPU.
+// together, and several such launches may share the GPU.  A workgroup that has
+// waited too long computes its input by itself (alone()), in the same order of
+// sums: a result never depends on how the waits went.
 //
 // The sums are those of mlp_layer_kernel and mlp_last_kernel for up to
 // kSplitMaxRows rows, in the same order and as fused multiply-adds, which is how
@@ -40,20 +42,19 @@ using f32x4 = float __attribute__((ext_vector_type(4)));
 
 constexpr int kWidth = 1024;
 constexpr int kTiles = kWidth / 32;
-// Rows up to which this is the faster way: 19.8 / 25.6 / 30.1 / 32.7 us for 1 to 4
-// (launches per layer 38.8 / 39.6 / 40.9 / 41.6), 39.5 and 46.0 for 5 and 8 (42.0
-// and 44.2).  What a row adds is its share of the multiply-adds on a layer's 32
+// Rows up to which this is the faster way: 19.2 / 23.9 / 27.6 / 29.9 us for 1 to 4
+// (launches per layer 38.8 / 39.6 / 40.9 / 41.6); an earlier form took 39.5 and 46.0
+// for 5 and 8 (42.0 and 44.2).  What a row adds is its share of the multiply-adds on a layer's 32
 // compute units, 0.2 us, and the reads of the next layer.
 constexpr int kMaxRows = 4;
-constexpr uint32_t kNumberAll = 1u << 16;
+constexpr uint32_t kNumberAll = 1u << 16;  // calls
 constexpr int kMaxIn = 64;
 constexpr int kFewIn = 16;   // rows that w_first_t has at least, zero beyond the features
 constexpr int kChains = 32;  // sums of 32 products that an output is added up from
-// Looks at a word at full rate (about 200 us), and before a wait is given up
-// (some seconds): only calls that overlap on one handle, which its users must not
-// do, could get there.
+// Looks at a word at full rate (about 200 us), and before a wait is given up (about
+// 15 ms; a call in which every wait was given up at once took 0.4 ms).
 constexpr int kBusyLooks = 256;
-constexpr int kMaxLooks = 1 << 20;
+constexpr int kMaxLooks = 1 << 12;
 
 struct Args {
   const float* w_stream;   // packed weights (mlp.hip)
@@ -74,6 +75,7 @@ struct Args {
   uint32_t done_value;
   uint64_t* tickets;       // counts all workgroups of all calls
   uint64_t* words;         // [hidden][kMaxRows][kWidth] activations and call numbers
+  int32_t looks;           // at a word before a wait is given up (kMaxLooks)
 };
 
 // The i-th k that a sum takes: of each 8, the pairs (e, 4 + e) that the matrix core
@@ -129,53 +131,171 @@ __device__ __forceinline__ void put(uint64_t* word, float value, uint32_t call) 
                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// The values of ROWS words `stride` apart once all of the first n carry the number
-// of this call.  While the first is not there only that one is
+// The values of ROWS words `stride` apart once all of the first n, for every lane of
+// the wave, carry the number of this call (a loop for the wave: with one for each
+// lane 2 to 4 rows took 1 us more).  While the first is not there only that one is
 // asked for, and after kBusyLooks looks only now and then: all workgroups wait at
 // a time, and where they asked for every row at full rate (twice as many, of half
-// a tile, and eight rows: 33 MB a look) some waits ran into their bound, as if the
-// reads had kept the write waited for from getting through.  One row is 2 MB a
-// look; 32 000 calls, half of them beside a kernel that takes all of the memory's
-// bandwidth, then all took their usual time.
+// a tile, and eight rows: 33 MB a look) some waits did not end in a second, as if the
+// reads had kept the write waited for from getting through (the cause was not
+// found).  One row is 2 MB a look; 32 000 calls, half of them beside a kernel that
+// takes all of the memory's bandwidth, then all took their usual time.  False, and
+// no values, where the wait was given up after `looks`.
 template <int ROWS>
-__device__ __forceinline__ void get(const uint64_t* words, int stride, int n, uint32_t call,
-                                    float (&value)[ROWS]) {
-  uint64_t v[ROWS];
+__device__ __forceinline__ bool get(const uint64_t* words, int stride, int n, uint32_t call,
+                                    int looks, float (&value)[ROWS]) {
+  uint64_t v[ROWS] = {};
   const auto ask = [&](int r) {
     v[r] = __hip_atomic_load(words + (r < n ? r : 0) * stride, __ATOMIC_RELAXED,
                              __HIP_MEMORY_SCOPE_AGENT);
   };
-  const auto there = [&](int r) { return carries(v[r], call); };
-  for (int look = 0; look < kMaxLooks; ++look) {
+  bool ready = false;
+  for (int look = 0; !ready; ++look) {
+    if (__builtin_expect(look == looks, 0)) break;
+    if (look > 0) {
+      if (look <= kBusyLooks) __builtin_amdgcn_s_sleep(1);
+      else __builtin_amdgcn_s_sleep(127);
+    }
     ask(0);
-    if (there(0)) {
-      bool ready = true;
+    ready = __all(carries(v[0], call));
+    if (ROWS > 1 && ready) {
+      bool all = true;
 #pragma unroll
       for (int r = 1; r < ROWS; ++r) ask(r);
 #pragma unroll
-      for (int r = 1; r < ROWS; ++r) ready = ready && there(r);
-      if (ready) {
-#pragma unroll
-        for (int r = 0; r < ROWS; ++r) value[r] = __builtin_bit_cast(float, (uint32_t)v[r]);
-        return;
-      }
+      for (int r = 1; r < ROWS; ++r) all = all && carries(v[r], call);
+      ready = __all(all);
     }
-    if (look < kBusyLooks) __builtin_amdgcn_s_sleep(1);
-    else __builtin_amdgcn_s_sleep(127);
   }
 #pragma unroll
-  for (int r = 0; r < ROWS; ++r) value[r] = __builtin_nanf("");
+  for (int r = 0; r < ROWS; ++r) value[r] = __builtin_bit_cast(float, (uint32_t)v[r]);
+  return ready;
+}
+
+// The packed weights of an output of a hidden layer, its k-groups 8 * 64 apart and
+// the upper four k of a group 32 further.
+__device__ __forceinline__ const f32x4* weights_of(const Args& a, int layer, int tile, int n) {
+  return reinterpret_cast<const f32x4*>(a.w_stream) +
+         ((size_t)(tile >> 3) * a.groups_total + a.first_groups + layer * (kWidth / 8)) * (8 * 64) +
+         (tile & 7) * 64 + n;
+}
+
+// The rows standardised, zeros beyond them; thread = (row, feature).
+template <int ROWS>
+__device__ __forceinline__ void standardise(const Args& a, int tid, float (&xs)[ROWS][kMaxIn]) {
+  if (tid < ROWS * kMaxIn) {
+    const int r = tid / kMaxIn, k = tid % kMaxIn;
+    float v = 0.f;
+    if (r < a.n && k < a.in_features)
+      v = (float)((a.raw[(size_t)r * a.in_features + k] - a.mu[k]) / a.sigma[k]);
+    xs[r][k] = v;
+  }
+}
+
+// One output of fc1: four sums, each of a quarter of the k-groups, as
+// mlp_layer_kernel's waves.  wk: its weights, where in_features <= kFewIn.
+template <int ROWS>
+__device__ __forceinline__ void first_layer(const Args& a, int out, const float (&wk)[kFewIn],
+                                            const float (&xs)[ROWS][kMaxIn], float (&v)[ROWS]) {
+  float sum[ROWS];
+  if (a.in_features <= kFewIn) {
+    // two k-groups, each a sum of its own (the other two sums are zero)
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      float part[2] = {0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < kFewIn; ++i) {
+        const int k = product(i);
+        part[k >> 3] = fmaf(wk[k], xs[r][k], part[k >> 3]);
+      }
+      sum[r] = part[0] + part[1];
+    }
+  } else {
+    const int per_sum = (a.first_groups + 3) / 4;
+    for (int s = 0; s < 4; ++s) {
+      float part[ROWS];
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) part[r] = 0.f;
+      for (int i = 8 * s * per_sum; i < 8 * (s + 1) * per_sum; ++i) {
+        const int k = product(i);
+        const float w1 = k < a.in_features ? a.w_first_t[(size_t)k * kWidth + out] : 0.f;
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) part[r] = fmaf(w1, k < a.in_features ? xs[r][k] : 0.f, part[r]);
+      }
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) sum[r] = s == 0 ? part[r] : sum[r] + part[r];
+    }
+  }
+  const float b = a.bias[out];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) v[r] = relu(sum[r] + b);
+}
+
+// The input of layer `layer` into act, by this workgroup without any other: thread =
+// output, its sums in the order of chain_kernel.  About 40 us a layer where all
+// workgroups do it; it is there for waits that were given up and nothing else.
+template <int ROWS>
+__device__ __forceinline__ void alone(const Args& a, int layer, int tid, float (&xs)[ROWS][kMaxIn],
+                                      float (&act)[ROWS][kWidth]) {
+  float wk[kFewIn], v[ROWS];
+  for (int k = 0; k < kFewIn; ++k) wk[k] = a.w_first_t[(size_t)k * kWidth + tid];
+  standardise<ROWS>(a, tid, xs);
+  __syncthreads();
+  first_layer<ROWS>(a, tid, wk, xs, v);
+#pragma unroll 1
+  for (int l = 0; l < layer; ++l) {
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) act[r][tid] = v[r];
+    __syncthreads();
+    const f32x4* at = weights_of(a, l, tid >> 5, tid & 31);
+    const float b = a.bias[(size_t)(l + 1) * kWidth + tid];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) v[r] = b;
+#pragma unroll 1
+    for (int p = 0; p < kChains; p += 4) {
+      float part[ROWS];
+#pragma unroll 1
+      for (int c = p; c < p + 4; ++c) {
+        float sum[ROWS];
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) sum[r] = 0.f;
+#pragma unroll 1
+        for (int j = 4 * c; j < 4 * c + 4; ++j) {
+          const f32x4 lower = at[(size_t)j * (8 * 64)], upper = at[(size_t)j * (8 * 64) + 32];
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {
+              sum[r] = fmaf(lower[e], act[r][8 * j + e], sum[r]);
+              sum[r] = fmaf(upper[e], act[r][8 * j + 4 + e], sum[r]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) part[r] = c == p ? sum[r] : part[r] + sum[r];
+      }
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) v[r] += part[r];
+    }
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) v[r] = relu(v[r]);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) act[r][tid] = v[r];
+  __syncthreads();
 }
 
 template <int ROWS>
 __global__ __launch_bounds__(1024) void chain_kernel(const Args a) {
   __shared__ uint32_t taken[2];
+  __shared__ uint32_t late;  // a thread's wait was given up
   __shared__ float xs[ROWS][kMaxIn];
   __shared__ __attribute__((aligned(16))) float act[ROWS][kWidth];
   __shared__ float red[ROWS][kChains][32];
   const int tid = threadIdx.x;
   const int blocks = a.hidden * kTiles + 1;
   if (tid == 0) {
+    late = 0;
     const uint64_t t =
         __hip_atomic_fetch_add(a.tickets, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     taken[0] = (uint32_t)(t % (uint32_t)blocks);
@@ -190,105 +310,78 @@ __global__ __launch_bounds__(1024) void chain_kernel(const Args a) {
   // k-groups 4 c .. 4 c + 3
   const int n = tid & 31, c = tid >> 5;
   f32x4 w[4][2];
-  if (layer < a.hidden) {
-    const f32x4* at = reinterpret_cast<const f32x4*>(a.w_stream) +
-                      ((size_t)(tile >> 3) * a.groups_total + a.first_groups +
-                       layer * (kWidth / 8) + 4 * c) * (8 * 64) + (tile & 7) * 64 + n;
+  const auto load_weights = [&]() {
+    const f32x4* at = weights_of(a, layer, tile, n) + 4 * c * (8 * 64);
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int h = 0; h < 2; ++h) w[j][h] = at[j * (8 * 64) + 32 * h];
-  }
+  };
+  if (layer < a.hidden) load_weights();
   if (__builtin_expect(call % kNumberAll == 0, 0) && layer < a.hidden && c >= a.n && c < kMaxRows)
     put(a.words + ((size_t)layer * kMaxRows + c) * kWidth + tile * 32 + n, 0.f, call);
 
   if (layer == 0) {
-    // fc1, by each of the first layer's workgroups for itself: thread = output;
-    // four sums, each of a quarter of the k-groups, as mlp_layer_kernel's waves
-    float wk[kFewIn];
+    // fc1, by each of the first layer's workgroups for itself: thread = output
+    float wk[kFewIn], v[ROWS];
 #pragma unroll
     for (int k = 0; k < kFewIn; ++k) wk[k] = a.w_first_t[(size_t)k * kWidth + tid];
-    if (tid < ROWS * kMaxIn) {
-      const int r = tid / kMaxIn, k = tid % kMaxIn;
-      float v = 0.f;
-      if (r < a.n && k < a.in_features)
-        v = (float)((a.raw[(size_t)r * a.in_features + k] - a.mu[k]) / a.sigma[k]);
-      xs[r][k] = v;
-    }
+    standardise<ROWS>(a, tid, xs);
     __syncthreads();
-    float sum[ROWS];
-    if (a.in_features <= kFewIn) {
-      // two k-groups, each a sum of its own (the other two sums are zero)
+    first_layer<ROWS>(a, tid, wk, xs, v);
 #pragma unroll
-      for (int r = 0; r < ROWS; ++r) {
-        float part[2] = {0.f, 0.f};
-#pragma unroll
-        for (int i = 0; i < kFewIn; ++i) {
-          const int k = product(i);
-          part[k >> 3] = fmaf(wk[k], xs[r][k], part[k >> 3]);
-        }
-        sum[r] = part[0] + part[1];
-      }
-    } else {
-      const int per_sum = (a.first_groups + 3) / 4;
-      for (int s = 0; s < 4; ++s) {
-        float part[ROWS];
-#pragma unroll
-        for (int r = 0; r < ROWS; ++r) part[r] = 0.f;
-        for (int i = 8 * s * per_sum; i < 8 * (s + 1) * per_sum; ++i) {
-          const int k = product(i);
-          const float w1 = k < a.in_features ? a.w_first_t[(size_t)k * kWidth + tid] : 0.f;
-#pragma unroll
-          for (int r = 0; r < ROWS; ++r) part[r] = fmaf(w1, k < a.in_features ? xs[r][k] : 0.f, part[r]);
-        }
-#pragma unroll
-        for (int r = 0; r < ROWS; ++r) sum[r] = s == 0 ? part[r] : sum[r] + part[r];
-      }
-    }
-    const float b = a.bias[tid];
-#pragma unroll
-    for (int r = 0; r < ROWS; ++r) act[r][tid] = relu(sum[r] + b);
+    for (int r = 0; r < ROWS; ++r) act[r][tid] = v[r];
   } else {
     float v[ROWS];
-    get<ROWS>(a.words + (size_t)(layer - 1) * kMaxRows * kWidth + tid, kWidth, a.n, call, v);
+    if (!get<ROWS>(a.words + (size_t)(layer - 1) * kMaxRows * kWidth + tid, kWidth, a.n, call,
+                   a.looks, v))
+      late = 1;
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) act[r][tid] = v[r];
   }
   __syncthreads();
 
   if (layer < a.hidden) {
+    const auto finish_tile = [&](const uint32_t& given_up) {
 #pragma unroll
-    for (int r = 0; r < ROWS; ++r) {
-      if (r >= a.n) break;
-      // (16 lanes share the values that they all want: read from LDS by every lane
-      // they took 0.4 us a row)
-      const float* x = &act[r][32 * c + product(tid & 15)];
-      const float sum = add_products<0>(w, x[0], 0.f);
-      red[r][c][n] = add_products<16>(w, x[16], sum);
-    }
-    __syncthreads();
-    // a wave per row: four sums make a K-partial, the eight partials follow the
-    // bias; lanes 0 to 31 add the first four, lanes 32 to 63 the others
-    const int row = tid >> 6, upper = c & 1;
-    if (row >= ROWS || row >= a.n) return;
-    float p[kChains / 2];
+      for (int r = 0; r < ROWS; ++r) {
+        if (r >= a.n) break;
+        // (16 lanes share the values that they all want: read from LDS by every lane
+        // they took 0.4 us a row)
+        const float* x = &act[r][32 * c + product(tid & 15)];
+        const float sum = add_products<0>(w, x[0], 0.f);
+        red[r][c][n] = add_products<16>(w, x[16], sum);
+      }
+      __syncthreads();
+      // a wave per row: four sums make a K-partial, the eight partials follow the
+      // bias; lanes 0 to 31 add the first four, lanes 32 to 63 the others
+      const int row = tid >> 6, upper = c & 1;
+      if (row >= ROWS || row >= a.n) return;
+      float p[kChains / 2];
 #pragma unroll
-    for (int i = 0; i < kChains / 2; ++i) p[i] = red[row][upper * (kChains / 2) + i][n];
-    float v = a.bias[(size_t)(layer + 1) * kWidth + tile * 32 + n];
+      for (int i = 0; i < kChains / 2; ++i) p[i] = red[row][upper * (kChains / 2) + i][n];
+      float v = a.bias[(size_t)(layer + 1) * kWidth + tile * 32 + n];
 #pragma unroll
-    for (int s = 0; s < kChains / 4 / 2; ++s)
-      p[s] = ((p[4 * s] + p[4 * s + 1]) + p[4 * s + 2]) + p[4 * s + 3];
+      for (int s = 0; s < kChains / 4 / 2; ++s)
+        p[s] = ((p[4 * s] + p[4 * s + 1]) + p[4 * s + 2]) + p[4 * s + 3];
 #pragma unroll
-    for (int s = 0; s < kChains / 4 / 2; ++s) v += p[s];
-    v = __shfl_up(v, 32);   // the lower half's sum, for the upper half
+      for (int s = 0; s < kChains / 4 / 2; ++s) v += p[s];
+      v = __shfl_up(v, 32);   // the lower half's sum, for the upper half
 #pragma unroll
-    for (int s = 0; s < kChains / 4 / 2; ++s) v += p[s];
-    if (upper)
-      put(a.words + ((size_t)layer * kMaxRows + row) * kWidth + tile * 32 + n, relu(v), call);
+      for (int s = 0; s < kChains / 4 / 2; ++s) v += p[s];
+      if (upper && given_up == 0)
+        put(a.words + ((size_t)layer * kMaxRows + row) * kWidth + tile * 32 + n, relu(v), call);
+    };
+    finish_tile(late);
+    if (__builtin_expect(late == 0, 1)) return;
+    alone<ROWS>(a, layer, tid, xs, act);
+    load_weights();
+    finish_tile(0);
     return;
   }
 
   // fc2: a wave per row, summed as in mlp_last_kernel
+  if (__builtin_expect(late != 0, 0)) alone<ROWS>(a, layer, tid, xs, act);
   const int lane = tid & 63, row = tid >> 6;
   if (row >= a.n) return;
   float sum = 0.f;

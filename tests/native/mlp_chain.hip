@@ -12,13 +12,15 @@ extern "C" {
 int chain_carries(uint64_t word, uint32_t call) { return hbt::chain::carries(word, call); }
 
 int chain_max_rows() { return hbt::chain::kMaxRows; }
+int chain_max_looks() { return hbt::chain::kMaxLooks; }
 
 // Device pointers; the shapes are those of hbt::chain::Args.
 int chain_forward(const float* w_stream, int32_t first_groups, int32_t hidden,
                   const float* w_first_t, const float* bias, const float* w_last, float b_last,
                   const double* raw, const double* mu, const double* sigma, int32_t in_features,
-                  int32_t n, float* out, uint64_t* tickets, uint64_t* words, void* stream) {
-  if (n < 1 || n > hbt::chain::kMaxRows || hidden < 1 || in_features < 1 ||
+                  int32_t n, float* out, uint64_t* tickets, uint64_t* words, int32_t looks,
+                  void* stream) {
+  if (looks < 0 || looks > hbt::chain::kMaxLooks || n < 1 || n > hbt::chain::kMaxRows || hidden < 1 || in_features < 1 ||
       in_features > 8 * first_groups || 8 * first_groups > hbt::chain::kMaxIn)
     return -1;
   hbt::chain::Args a{};
@@ -36,6 +38,7 @@ int chain_forward(const float* w_stream, int32_t first_groups, int32_t hidden,
   a.out = out;
   a.tickets = tickets;
   a.words = words;
+  a.looks = looks;
   return hbt::chain::launch(a, static_cast<hipStream_t>(stream)) == hipSuccess ? 0 : -2;
 }
 

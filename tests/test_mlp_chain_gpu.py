@@ -119,7 +119,7 @@ class Chain:
                         "`make -C tests/native` (or __graft_entry__.build()) first")
         lib = ctypes.CDLL(NATIVE)
         P, I, F = ctypes.c_void_p, ctypes.c_int32, ctypes.c_float
-        lib.chain_forward.argtypes = [P, I, I, P, P, P, F, P, P, P, I, I, P, P, P, P]
+        lib.chain_forward.argtypes = [P, I, I, P, P, P, F, P, P, P, I, I, P, P, P, I, P]
         self.lib, self.max_rows = lib, lib.chain_max_rows()
         sd = {k: v.numpy() for k, v in rp.model.state_dict().items()}
         names = ["fc1"] + sorted({k[:-7] for k in sd if k.startswith("mlp") and "weight" in k},
@@ -145,13 +145,14 @@ class Chain:
         self.words = torch.zeros((self.hidden, self.max_rows, 1024), dtype=torch.int64,
                                  device="cuda")
 
-    def __call__(self, raw):
+    def __call__(self, raw, looks=None):
+        looks = self.lib.chain_max_looks() if looks is None else looks
         out = torch.full((raw.shape[0],), -1.0, dtype=torch.float32, device="cuda")
         p = lambda t: ctypes.c_void_p(t.data_ptr())
         rc = self.lib.chain_forward(
             p(self.w), 4, self.hidden, p(self.first_t), p(self.bias), p(self.w_last), self.b_last,
             p(raw), p(self.mu), p(self.sigma), self.f, raw.shape[0], p(out), p(self.tickets),
-            p(self.words), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+            p(self.words), looks, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
         assert rc == 0
         return out.cpu().numpy()
 
@@ -177,3 +178,19 @@ def test_words_of_older_calls_are_never_taken():
                     assert bool(torch.all(numbered))
                 else:
                     assert not bool(torch.any(numbered[:, rows:]))
+
+
+@pytest.mark.parametrize("kind,hidden", [("conv2d", 1), ("lstm", 4), ("bmm", 8)])
+def test_a_wait_that_is_given_up_changes_no_bit(kind, hidden):
+    """The bound on a wait at nothing (every workgroup computes its input by itself)
+    and at a few looks (some do): the results of calls that wait, NaN handed on."""
+    rp, x = network(kind, hidden)
+    x[3] = 0.0
+    x[5, 1] = np.inf
+    x[7, 0] = np.nan
+    want = rp.predict_batch(x[:16]).cpu().numpy()
+    chain, raw = Chain(rp), torch.from_numpy(x).cuda()
+    for looks in (0, 1, 2, 5, 20, 0):
+        for rows, first in ((1, 0), (4, 2), (3, 9), (2, 6), (1, 7), (4, 12)):
+            got = chain(raw[first:first + rows], looks=looks)
+            assert np.array_equal(got, want[first:first + rows], equal_nan=True), (looks, rows)
