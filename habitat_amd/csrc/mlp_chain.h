@@ -109,7 +109,7 @@ __device__ __forceinline__ float add_products(const f32x4 (&w)[4][2], float x, f
       "v_fmac_f32_dpp %0, %1, %15 row_newbcast:13 row_mask:0xf bank_mask:0xf\n\t"
       "v_fmac_f32_dpp %0, %1, %16 row_newbcast:14 row_mask:0xf bank_mask:0xf\n\t"
       "v_fmac_f32_dpp %0, %1, %17 row_newbcast:15 row_mask:0xf bank_mask:0xf"
-      : "+v"(sum)
+      : "+&v"(sum)
       : "v"(x), "v"(w[j][0][0]), "v"(w[j][1][0]), "v"(w[j][0][1]), "v"(w[j][1][1]),
         "v"(w[j][0][2]), "v"(w[j][1][2]), "v"(w[j][0][3]), "v"(w[j][1][3]),
         "v"(w[j + 1][0][0]), "v"(w[j + 1][1][0]), "v"(w[j + 1][0][1]), "v"(w[j + 1][1][1]),
