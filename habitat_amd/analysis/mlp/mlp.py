@@ -10,6 +10,7 @@ signature.  The forward pass itself runs in libhabitat_mi.so
 this package.
 """
 import collections
+import contextvars
 import ctypes
 import threading
 
@@ -175,6 +176,24 @@ class _DeviceMLP:
             pass
 
 
+# Whether predict_batch, in this thread, runs with the sums of hbt_mlp_forward_fp32.
+_fp32_sums = contextvars.ContextVar("habitat_amd_fp32_sums", default=False)
+
+
+def predict_for_quotients(pred, rows):
+    """pred.predict_batch(rows) for predictions that are divided by each other (those
+    of a trace and of a sweep): with the products and sums of hbt_mlp_forward_fp32,
+    also below a subclass's or an instance's own predict_batch.  On devices far from
+    those a network was trained on both predictions can be small differences of large
+    sums, where another order of the sums shows in the quotient's fifth digit (5e-5
+    seen); so a trace's and a sweep's results stay those of fp32 sums at any size."""
+    token = _fp32_sums.set(True)
+    try:
+        return pred.predict_batch(rows)
+    finally:
+        _fp32_sums.reset(token)
+
+
 class RuntimePredictor:
     # predictions `predict` remembers: the reference asks for every operation
     # twice, once with the origin's device features (predictor.py:177-180), and
@@ -261,11 +280,13 @@ class RuntimePredictor:
         """raw_features: [n, F+4] float64 (numpy array or GPU tensor): operation
         features in `self.model.features` order followed by the four device
         features.  Returns a float32 GPU tensor of n predictions (not synchronised)."""
-        return self._forward(raw_features, out, stream, "hbt_mlp_forward")
+        return self._forward(raw_features, out, stream, "hbt_mlp_forward_fp32"
+                             if _fp32_sums.get() else "hbt_mlp_forward")
 
     def predict_batch_fp32(self, raw_features, out=None, stream=None):
-        """predict_batch with the sums of hbt_mlp_forward_fp32: the same last bits at
-        any n, for predictions that are divided by each other."""
+        """predict_batch with the products and sums of hbt_mlp_forward_fp32 at any n, for
+        predictions that are divided by each other.  (The order of its sums, and so the
+        last bits, depend on n and on the row's position.)"""
         return self._forward(raw_features, out, stream, "hbt_mlp_forward_fp32")
 
     def _forward(self, raw_features, out, stream, entry):

@@ -19,7 +19,7 @@ import torch
 from habitat_amd.analysis import SPECIAL_OPERATIONS
 from habitat_amd.analysis.metrics import Metric
 from habitat_amd.analysis.mlp.devices import get_device_features
-from habitat_amd.analysis.mlp.mlp import RuntimePredictor
+from habitat_amd.analysis.mlp.mlp import RuntimePredictor, predict_for_quotients
 from habitat_amd.analysis.operation import PredictedOperation
 from habitat_amd.analysis.run_time import (RunTimePrediction, RunTimePurePrediction, ms_to_ns)
 from habitat_amd.analysis.wave_scaling.batch import KernelRecords, wave_scale
@@ -360,7 +360,7 @@ class Predictor:
                 rows.append(feats + dest_feats)
                 rows.append(feats + get_device_features(op.device.name, pred.device_params))
             pairs.append(pair_of[key])
-        return pred.predict_batch(np.asarray(rows, np.float64)), pairs
+        return predict_for_quotients(pred, np.asarray(rows, np.float64)), pairs
 
     @staticmethod
     def _special_finish(operations, enqueued):

@@ -23,7 +23,7 @@ import torch
 
 from habitat_amd.analysis import SPECIAL_OPERATIONS
 from habitat_amd.analysis.mlp.devices import get_device_features
-from habitat_amd.analysis.mlp.mlp import RuntimePredictor
+from habitat_amd.analysis.mlp.mlp import predict_for_quotients
 from habitat_amd.analysis.run_time import ms_to_ns
 from habitat_amd.analysis.wave_scaling.batch import DeviceTable, ratio_scale, wave_scale_sum
 
@@ -141,17 +141,6 @@ class TracePlan:
         return self.prepare(dest_devices, device_features).launch()
 
 
-def _predict_rows(pred):
-    """The forward that a sweep runs on `pred`.  It divides each prediction by the
-    origin's, and on devices far from those a network was trained on both can be
-    small differences of large sums, where another order of the sums shows in the
-    quotient's fifth digit (5e-5 seen): the fp32 sums then keep a sweep's results
-    what they have been.  A caller's own predict_batch is called as it is."""
-    own = (isinstance(pred, RuntimePredictor) and "predict_batch" not in vars(pred)
-           and type(pred).predict_batch is RuntimePredictor.predict_batch)
-    return pred.predict_batch_fp32 if own else pred.predict_batch
-
-
 class SweepCall:
     """A prepared sweep: `launch()` enqueues its kernels on the current stream
     and returns a TraceSweep of GPU tensors, without synchronising and without
@@ -217,7 +206,7 @@ class SweepCall:
             U = op_feats.shape[0]
             side.wait_stream(main)
             with torch.cuda.stream(side):
-                y = _predict_rows(pred)(self.rows[kind]).view(D + 1, U)
+                y = predict_for_quotients(pred, self.rows[kind]).view(D + 1, U)
             y.record_stream(main)
             preds[kind] = y
         total = torch.full((D,), plan.const_ms, dtype=torch.float64, device=plan.gpu)

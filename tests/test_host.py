@@ -467,3 +467,49 @@ def test_few_row_mlp_words_count_for_their_own_call_only():
         for written in numbers:
             for bits in (0, 0x3f800000, 0x7fc00000, 0xffffffff):
                 assert bool(lib.chain_carries(written << 32 | bits, call)) == (written == call)
+
+
+@pytest.mark.parametrize("batches", [(32,), (16, 32, 64)])     # 23 and 69 distinct convolutions
+def test_a_traces_quotients_are_of_fp32_sums(batches):
+    """The two predictions of an operation that Trace.to_device divides come from
+    hbt_mlp_forward_fp32 at any number of operations (hbt_mlp_forward takes 129 rows
+    and more in bf16 pieces), also where a subclass or an instance has a
+    predict_batch of its own; a batch asked for directly does not."""
+    import torch
+    from habitat_amd.analysis.mlp.mlp import RuntimePredictor
+    from habitat_amd.analysis.predictor import Predictor
+
+    class Handle:
+        torch_device = torch.device("cpu")
+
+        def __init__(self):
+            self.calls = []
+
+        def forward(self, raw, out=None, stream=None, entry="hbt_mlp_forward"):
+            self.calls.append((entry, raw.shape[0]))
+            return torch.ones(raw.shape[0])
+
+    class Logging(RuntimePredictor):
+        seen = 0
+
+        def predict_batch(self, raw_features, out=None, stream=None):
+            self.seen += 1
+            return super().predict_batch(raw_features, out, stream)
+
+    operations = [op for b in batches
+                  for op in synthetic.resnet50_trace(Device.V100, batch=b).operations
+                  if op.name == "conv2d"]
+    for make in (RuntimePredictor, Logging):
+        pred = make("conv2d", 8, 1024)
+        pred._gpu = Handle()
+        predictor = Predictor(mlp_predictors={"conv2d": pred})
+        times = predictor._special_scale_many("conv2d", operations, Device.T4)
+        assert times == [op.run_time_ms for op in operations]
+        own = pred.predict_batch
+        pred.predict_batch = lambda rows: own(rows)
+        predictor._special_scale_many("conv2d", operations, Device.T4)
+        rows = 2 * 23 * len(batches)
+        assert pred._gpu.calls == [("hbt_mlp_forward_fp32", rows)] * 2
+        pred.predict_batch(np.zeros((rows, 12)))
+        assert pred._gpu.calls[2:] == [("hbt_mlp_forward", rows)]
+        assert make is RuntimePredictor or pred.seen == 3

@@ -137,3 +137,31 @@ def test_a_sweep_divides_predictions_with_fp32_sums():
         y = rp.predict_batch_fp32(sweep.rows[kind]).double().view(121, -1)[:, op_row.long()]
         want = torch.clamp(ms * y[:120] / y[120], min=0.0)
         assert torch.equal(res.special_ms[kind], want)
+
+
+def test_a_trace_divides_predictions_with_fp32_sums():
+    """From 65 distinct operations of a kind on (129 rows) hbt_mlp_forward takes the
+    pieces; a trace's quotients do not."""
+    from habitat_amd import Device
+    from habitat_amd.analysis.predictor import Predictor
+    rp = network("conv2d", 2)
+    _, mu, sigma = synthetic.mlp_features("conv2d", 2048, seed=1)
+    rp.set_normalization(mu, sigma)
+    with torch.no_grad():
+        rp.model.fc2.bias.fill_(4.0)
+    rp.refresh()
+    predictor = Predictor(mlp_predictors={"conv2d": rp})
+    ops = [op for b in (16, 32, 64)
+           for op in synthetic.resnet50_trace(Device.V100, batch=b, seed=3).operations
+           if op.name == "conv2d"]
+    gpu, seen = rp._device_mlp(), []
+    forward = gpu.forward
+    gpu.forward = lambda raw, **kw: seen.append(raw) or forward(raw, **kw)
+    y, pairs = predictor._special_enqueue("conv2d", ops, Device.T4)
+    predicted = predictor.predict_operations(ops, Device.T4)
+    assert seen[0].shape[0] == 138 and torch.equal(seen[0], seen[1])
+    assert torch.equal(y, rp.predict_batch_fp32(seen[0]))
+    assert not torch.equal(y, rp.predict_batch(seen[0]))
+    pair = y.cpu().numpy().astype(np.float64).reshape(-1, 2)
+    for op, i, got in zip(ops, pairs, predicted):
+        assert got.run_time_ms == op.run_time_ms * pair[i, 0] / pair[i, 1]
