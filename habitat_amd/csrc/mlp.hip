@@ -6,8 +6,9 @@
 // sigma in fp64, then cast to fp32.
 //
 // Above kSplitAboveRows rows hbt_mlp_forward's hidden layers run on the bf16 matrix
-// cores with every fp32 number in three exact pieces (mlp_split.h).  Up to there,
-// and in hbt_mlp_forward_fp32, they run on the fp32 ones (below), with
+// cores with every fp32 number in three pieces (mlp_split.h).  Up to there, in
+// hbt_mlp_forward_fp32 and for networks whose weights do not fit that (fits_pieces),
+// they run on the fp32 ones (below), with
 // v_mfma_f32_32x32x2_f32: the A operand is a 32(n) x 2(k) weight fragment, the B
 // operand a 2(k) x 32(m) activation fragment.  For these the weights are repacked
 // once, at hbt_mlp_create, so that a fragment for 8 consecutive k is one fully
@@ -843,6 +844,7 @@ struct hbt_mlp {
   const float* w_first_t;  // fc1.weight transposed, [kFirstFmaMaxIn or kMaxInPadded][width]
   float b_last;
   const char* w_split; // the hidden layers' weights in bf16 pieces, kSplitLayerBytes each
+  bool takes_pieces;   // whether they fit, and there are any
   int64_t chunk_rows;  // rows the split path takes at a time
   // the words of chain::Args of hbt_mlp_forward and hbt_mlp_predict_one, and of
   // hbt_mlp_forward_static; the counter of tickets comes first, in a block of its own
@@ -1312,6 +1314,7 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
   const size_t chain_bytes = align_up(sizeof(uint64_t) *
       (kChainHeader + (size_t)hidden_layers * chain::kMaxRows * kWidth), 256);
   const size_t off_chain = off; off += 2 * chain_bytes;
+  const size_t off_outside = off; off += 256;  // cleared with the above
   const size_t total = off;
 
   std::vector<unsigned char> host;
@@ -1359,7 +1362,7 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
     *err = HBT_EHIP;
     return nullptr;
   }
-  if (hipMemset(static_cast<unsigned char*>(blob) + off_chain, 0, 2 * chain_bytes) != hipSuccess) {
+  if (hipMemset(static_cast<unsigned char*>(blob) + off_chain, 0, total - off_chain) != hipSuccess) {
     (void)hipGetLastError();
     (void)hipFree(blob);
     *err = HBT_EHIP;
@@ -1372,10 +1375,14 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
     a.groups_total = in_padded / 8 + hidden_layers * (kWidth / 8);
     a.g0 = in_padded / 8 + l * (kWidth / 8);
     a.w = reinterpret_cast<char*>(blob) + off_split + (size_t)l * kSplitLayerBytes;
+    a.outside = reinterpret_cast<uint32_t*>(static_cast<unsigned char*>(blob) + off_outside);
     hipLaunchKernelGGL(split::pack_kernel, dim3((kWidth / 32) * split::kSteps / 4), dim3(256), 0,
                        nullptr, a);
   }
-  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
+  uint32_t outside = 0;
+  if (hipGetLastError() != hipSuccess ||
+      hipMemcpy(&outside, static_cast<unsigned char*>(blob) + off_outside, sizeof outside,
+                hipMemcpyDeviceToHost) != hipSuccess) {
     (void)hipGetLastError();
     (void)hipFree(blob);
     *err = HBT_EHIP;
@@ -1418,6 +1425,7 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
   m->w_last = reinterpret_cast<const float*>(base + off_last);
   m->w_first_t = reinterpret_cast<const float*>(base + off_first_t);
   m->w_split = reinterpret_cast<const char*>(base + off_split);
+  m->takes_pieces = hidden_layers > 0 && outside == 0;
   m->chunk_rows = chunk_rows;
   for (int i = 0; i < 2; ++i)
     m->chain[i] = reinterpret_cast<uint64_t*>(base + off_chain + i * chain_bytes);
@@ -1440,7 +1448,7 @@ int hbt_mlp_forward(hbt_mlp* mlp, const double* raw_features, int64_t n, float* 
   while (done < n) {
     const int64_t rows = n - done < mlp->chunk_rows ? n - done : mlp->chunk_rows;
     const double* raw = raw_features + done * mlp->in_features;
-    const int rc = rows > kSplitAboveRows && mlp->hidden > 0
+    const int rc = rows > kSplitAboveRows && mlp->takes_pieces
                        ? forward_split(mlp, raw, rows, out + done, mlp->scratch, mlp->part, stream)
                        : forward_fp32(mlp, raw, rows, out + done, stream);
     if (rc != HBT_OK) return rc;
@@ -1480,7 +1488,7 @@ int hbt_mlp_forward_static(hbt_mlp* mlp, const double* raw_features, int64_t n, 
   // clearing between calls.
   float* const buffers[2] = {base, base + kStaticFloats};
   hipStream_t stream = static_cast<hipStream_t>(hip_stream);
-  return n > kSplitAboveRows && mlp->hidden > 0
+  return n > kSplitAboveRows && mlp->takes_pieces
              ? forward_split(mlp, raw_features, n, out, buffers, base + 2 * kStaticFloats, stream)
              : forward_layers(mlp, raw_features, n, out, buffers, mlp->chain[1], stream);
 }

@@ -720,6 +720,17 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void small_kernel(const Laye
   }
 }
 
+// Whether a layer may hold this weight and still be an fp32 layer in pieces.  Below
+// kLeastWeight the third piece falls under bf16's smallest number and the sum of the
+// three is no longer exact.  From kMostWeight on (an infinity too) the products of
+// its smaller pieces with a large activation's can overflow with another sign than
+// the leading product's: NaN where fp32 has an infinity.
+constexpr float kLeastWeight = 0x1p-110f, kMostWeight = 0x1p7f;
+__device__ __host__ constexpr bool fits_pieces(float w) {
+  const float size = w < 0.f ? -w : w;
+  return size == 0.f || (size >= kLeastWeight && size < kMostWeight);
+}
+
 // The packed fp32 weights of one layer (pack_layer in mlp.hip) in pieces; once,
 // when the network is loaded.  One wavefront per (n-tile, k-step).
 struct PackArgs {
@@ -727,6 +738,7 @@ struct PackArgs {
   int32_t groups_total;  // k-groups per wave stream
   int32_t g0;            // first k-group of this layer
   char* w;
+  uint32_t* outside;     // set where a weight does not fit
 };
 __global__ __launch_bounds__(256) void pack_kernel(const PackArgs a) {
   const int lane = threadIdx.x & 63;
@@ -740,6 +752,10 @@ __global__ __launch_bounds__(256) void pack_kernel(const PackArgs a) {
   for (int g = 0; g < 2; ++g)
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[4 * g + e] = in[g * (8 * 64)][e];
+  bool fits = true;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) fits = fits && fits_pieces(v[j]);
+  if (!fits) *a.outside = 1;  // (every such lane the same value)
   store_split(a.w + tile_offset(tile, step) + lane * 16, v);
 }
 

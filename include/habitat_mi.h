@@ -324,7 +324,10 @@ hbt_mlp *hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
  * calls on ONE handle must therefore not overlap, on any streams; different
  * handles are independent.  Results are reproducible for a given n and position
  * of the row; the kernels for different row counts sum in different orders and
- * agree to fp32 rounding.
+ * agree to fp32 rounding.  From 129 rows on the hidden layers' products are formed
+ * from bf16 pieces (see hbt_mlp_forward_fp32), unless a hidden weight is infinite,
+ * NaN, 2^7 or more in magnitude or, not being zero, less than 2^-110: such a network
+ * is hbt_mlp_forward_fp32 at any n.
  */
 int hbt_mlp_forward(hbt_mlp *mlp, const double *raw_features, int64_t n, float *out,
                     void *hip_stream);

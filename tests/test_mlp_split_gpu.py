@@ -96,6 +96,47 @@ def test_values_beyond_bf16(rows):
     assert np.all(y[x[:, 2] < 0] == 0) and np.all(np.isfinite(y[x[:, 2] == 1.0]))
 
 
+@pytest.mark.parametrize("rows", [200, 400, 800, 1400, 2000, 3000, 4000, 6000, 9000, 13000])
+def test_infinite_and_huge_weights(rows):
+    """One weight that is infinite, huge or tiny against activations that are
+    infinite, huge and zero: infinities and NaN where fp32 has them."""
+    rp = network("bmm", 1)
+    x = np.abs(np.random.default_rng(rows).normal(size=(rows, 8)))
+    x[:, 2] = np.resize([10.0, 1.0, 0.5, 0.0, -1.0], rows)
+    rp.set_normalization(np.zeros(8), np.ones(8))
+    with torch.no_grad():
+        for p in rp.model.parameters():
+            p.abs_()
+        rp.model.fc1.weight[:, 2] = 0.0
+        rp.model.fc1.weight[7] = torch.tensor([0, 0, 3e38, 0, 0, 0, 0, 0])   # unit 7 alone
+        rp.model.fc1.bias[7] = 0.0
+        rp.model.mlp.layers[0].weight[:, 7] = -0.3     # dead where unit 7 is large
+        rp.model.fc2.weight.zero_()
+        rp.model.fc2.weight[0, 100] = 1.0
+        rp.model.fc2.bias.zero_()
+    with np.errstate(all="ignore"):
+        unit7 = np.maximum(np.float32(3e38) * x[:, 2].astype(np.float32), 0)
+        assert np.isposinf(unit7[0]) and unit7[1] > 1e38 and unit7[4] == 0
+        for special in (np.inf, -np.inf, 3e38, -3e38, 128.0, 127.0, -127.0, 2.0 ** -100,
+                        -2.0 ** -100, 2.0 ** -120):
+            with torch.no_grad():
+                rp.model.mlp.layers[0].weight[100, 7] = special
+            rp.refresh()
+            big = np.float32(special) * unit7
+            pieces, fp32 = rp.predict_batch(x).cpu().numpy(), rp.predict_batch_fp32(x).cpu().numpy()
+            # a network with a weight that does not fit the pieces takes the fp32 kernels
+            if not 2.0 ** -110 <= abs(special) < 128:
+                assert np.array_equal(pieces, fp32, equal_nan=True)
+            else:
+                assert not np.array_equal(pieces, fp32, equal_nan=True)
+            for y in (pieces, fp32):
+                assert np.array_equal(np.isnan(y), np.isnan(big)), special
+                assert np.array_equal(np.isposinf(y), np.isposinf(big)), special
+                assert np.all(y[big < -1e8] == 0) and np.all(y[big == 0] > 0), special
+                large = (big > 1e8) & np.isfinite(big)   # the other units give some hundreds
+                assert np.all(np.abs(y[large] / big[large] - 1) < 1e-5), special
+
+
 # hbt_mlp_forward_fp32 (device sweeps): around its per-layer path's end at 7168 rows, the
 # fused kernel's rounds of 8192 and what such a round leaves over
 @pytest.mark.parametrize("rows", [2048, 2049, 7168, 7169, 8192, 8193, 16384, 20001])
