@@ -100,13 +100,29 @@ __device__ __forceinline__ void store_out(T* __restrict__ p, Index i, const T (&
 // neighbouring workgroups do, each half goes to memory from an L2 of its own.  So
 // such launches give each XCD runs of this many neighbouring workgroups (4096
 // records) and store without the non-temporal hint: its L2 then holds the lines
-// until they are whole.  To seven destinations, 1 000 003 records: 46.5 -> 34 us,
-// 4 000 003: 176 -> 128, 8 000 003: 341 -> 244; 524 291: 26.6 -> 23.4, where 262 147
-// gain nothing (13.2, 13.9).  (Runs of 8 / 16 / 64: 133 / 130 /
-// 126 us at 4 000 003; with the hint 161-167.)  With rows at lines it is the
-// other way round, 110 us with the hint at 4 000 000 and 117-120 without.
+// until they are whole.  (Runs of 8 / 16 / 64: 133 / 130 / 126 us at 4 000 003
+// records to seven destinations, 129 with these; with the hint 161-167.)
+//
+// Only the times' rows are asked about, which are most of the bytes: with those at
+// lines and the others within (a multiple of 16 records that is none of 128) it goes
+// either way, 4 000 016 records to seven with all outputs 153 us before and 161 so,
+// 1 000 016 39.4 and 36.7; with all rows at lines 111 us with the hint at 4 000 000
+// and 120 without.  From how many records on depends on how much of a line the
+// wavefronts share, us before and so, to 4 / 5 / 7 destinations:
+//
+//   records + 1 (8 bytes)           + 4 (32 bytes)                  + 8 (64 bytes)
+//   524 k   15.2 19.2 26.0 / 15.4 18.9 23.0   14.9 17.8 24.1 / 15.4 18.9 22.9   14.3 17.2 21.0 / 15.4 18.8 22.9
+//   614 k   17.1 21.1 26.9 / 17.1 21.0 24.7   16.8 20.4 25.2 / 16.9 21.0 24.8   16.3 19.5 23.3 / 16.9 21.0 24.8
+//   700 k   19.5 23.5 30.8 / 18.7 22.3 26.6   19.1 22.4 28.9 / 18.7 22.3 26.6   18.1 21.3 25.8 / 18.6 22.2 26.6
+//   800 k   21.8 27.0 36.6 / 20.2 24.2 28.9   21.3 25.5 33.8 / 20.2 24.1 28.8   20.0 24.1 30.0 / 20.3 24.0 28.8
+//   1.2 M   32.8 40.4 55.5 / 26.0 31.4 38.1   31.9 37.0 51.2 / 26.0 31.4 38.2   29.5 34.3 45.2 / 26.0 31.1 38.0
+//
+// (two destinations never lose more than 2 %; below 2^19 records little is gained).
+// With wave numbers, another two rows a destination, four and more gain from 2^19 on
+// whatever the offset: 524 296 records to seven 25.9 / 24.8, to four 16.9 / 17.4,
+// 614 408 29.1 / 27.2 and 19.2 / 19.5; three lose (13.8 / 14.9).
 constexpr int kMergeChunks = 32;
-constexpr int64_t kMergeMinRecords = (int64_t)1 << 19;
+constexpr int64_t kMergeMinRecords[3] = {32 << 14, 40 << 14, 50 << 14};  // odd, 32, 64 bytes
 
 // Records i .. i+R-1 (all below n) for every destination of the launch.
 // SINGLE: the launch has one destination; its constants then sit at fixed
@@ -256,13 +272,12 @@ template <int R, int MODEL, class Index>
 void launch(const WaveScaleArgs& args, hipStream_t stream) {
   const int64_t threads = (args.n + R - 1) / R;
   const int64_t blocks = (threads + kBlock - 1) / kBlock;
-  bool merge = args.n_dest > 1 && args.n >= kMergeMinRecords;
-  if (merge) {
-    bool lines = true;
-    for (int d = 0; d < args.n_dest; ++d)
-      lines = lines && reinterpret_cast<uintptr_t>(args.out[d].time_ns) % 128 == 0;
-    merge = !lines;
-  }
+  uintptr_t within = 0;  // of a line: where the times' rows begin
+  for (int d = 0; d < args.n_dest; ++d)
+    within |= reinterpret_cast<uintptr_t>(args.out[d].time_ns) % 128;
+  const bool many_rows = args.n_dest >= 4 && args.out[0].wave != nullptr;
+  const int offset = many_rows ? 0 : within % 64 == 0 ? 2 : within % 32 == 0 ? 1 : 0;
+  const bool merge = args.n_dest > 1 && within != 0 && args.n >= kMergeMinRecords[offset];
   constexpr int64_t kRun = 8 * kMergeChunks;
   const dim3 grid((unsigned)(merge ? (blocks + kRun - 1) / kRun * kRun : blocks));
   if (args.n_dest == 1)

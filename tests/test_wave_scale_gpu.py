@@ -473,15 +473,18 @@ def test_ragged_sizes_single_and_multi_destination(n):
     check(rec, Device.V100, dests, wave_scale(kr, Device.V100, dests))
 
 
-# destinations' rows off the 128-byte lines, around the 524 288 records from which
-# workgroups then go to the XCDs in runs of 4096 records, and the end of such a run;
-# 524 304 has its rows at lines
-@pytest.mark.parametrize("n", [524287, 524289, 524304, 528383, 528385, 557057])
-def test_rows_off_the_lines(n):
+# destinations' rows off the 128-byte lines, around the 524 288, 655 360 (rows at 32
+# bytes) and 819 200 records (at 64) from which workgroups then go to the XCDs in runs
+# of 4096 records, and the end of such a run; four destinations with wave numbers do
+# from 524 288 on at any offset; 524 304 has its rows at lines
+@pytest.mark.parametrize("n,n_dest", [(524287, 3), (524289, 3), (524304, 3), (528383, 3),
+                                      (528385, 3), (557057, 3), (655356, 3), (655364, 3),
+                                      (819192, 3), (819208, 3), (524280, 4), (524296, 4)])
+def test_rows_off_the_lines(n, n_dest):
     rec, _ = synthetic.kernel_records(n, Device.V100, seed=n, metrics_fraction=0.5)
-    dests = [Device.MI355X, Device.T4, Device.P100]
+    dests = [Device.MI355X, Device.T4, Device.P100, Device.P4000][:n_dest]
     kr = KernelRecords.from_numpy(rec)
-    out = WaveScaleOutput(n, 3, kr.device)
+    out = WaveScaleOutput(n, n_dest, kr.device)
     for t in (out.time_ns, out.occ_dest, out.wave_dest, out.status, out.occ_origin):
         t.fill_(77)
     wave_scale(kr, Device.V100, dests, out=out)
