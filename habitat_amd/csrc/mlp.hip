@@ -7,7 +7,7 @@
 //
 // Above kSplitAboveRows rows hbt_mlp_forward's hidden layers run on the bf16 matrix
 // cores with every fp32 number in three pieces (mlp_split.h).  Up to there, in
-// hbt_mlp_forward_fp32 and for networks whose weights do not fit that (fits_pieces),
+// hbt_mlp_forward_fp32 and for networks whose weights are not for that (check_kernel),
 // they run on the fp32 ones (below), with
 // v_mfma_f32_32x32x2_f32: the A operand is a 32(n) x 2(k) weight fragment, the B
 // operand a 2(k) x 32(m) activation fragment.  For these the weights are repacked
@@ -1375,8 +1375,16 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
     a.groups_total = in_padded / 8 + hidden_layers * (kWidth / 8);
     a.g0 = in_padded / 8 + l * (kWidth / 8);
     a.w = reinterpret_cast<char*>(blob) + off_split + (size_t)l * kSplitLayerBytes;
-    a.outside = reinterpret_cast<uint32_t*>(static_cast<unsigned char*>(blob) + off_outside);
     hipLaunchKernelGGL(split::pack_kernel, dim3((kWidth / 32) * split::kSteps / 4), dim3(256), 0,
+                       nullptr, a);
+  }
+  if (hidden_layers > 0) {
+    split::CheckArgs a{};
+    a.w_stream = reinterpret_cast<const float*>(static_cast<unsigned char*>(blob) + off_stream);
+    a.groups_total = in_padded / 8 + hidden_layers * (kWidth / 8);
+    a.g0 = in_padded / 8;
+    a.outside = reinterpret_cast<uint32_t*>(static_cast<unsigned char*>(blob) + off_outside);
+    hipLaunchKernelGGL(split::check_kernel, dim3(kWidth / 32, (unsigned)hidden_layers), dim3(64), 0,
                        nullptr, a);
   }
   uint32_t outside = 0;

@@ -720,17 +720,6 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void small_kernel(const Laye
   }
 }
 
-// Whether a layer may hold this weight and still be an fp32 layer in pieces.  Below
-// kLeastWeight the third piece falls under bf16's smallest number and the sum of the
-// three is no longer exact.  From kMostWeight on (an infinity too) the products of
-// its smaller pieces with a large activation's can overflow with another sign than
-// the leading product's: NaN where fp32 has an infinity.
-constexpr float kLeastWeight = 0x1p-110f, kMostWeight = 0x1p7f;
-__device__ __host__ constexpr bool fits_pieces(float w) {
-  const float size = w < 0.f ? -w : w;
-  return size == 0.f || (size >= kLeastWeight && size < kMostWeight);
-}
-
 // The packed fp32 weights of one layer (pack_layer in mlp.hip) in pieces; once,
 // when the network is loaded.  One wavefront per (n-tile, k-step).
 struct PackArgs {
@@ -738,7 +727,6 @@ struct PackArgs {
   int32_t groups_total;  // k-groups per wave stream
   int32_t g0;            // first k-group of this layer
   char* w;
-  uint32_t* outside;     // set where a weight does not fit
 };
 __global__ __launch_bounds__(256) void pack_kernel(const PackArgs a) {
   const int lane = threadIdx.x & 63;
@@ -752,11 +740,54 @@ __global__ __launch_bounds__(256) void pack_kernel(const PackArgs a) {
   for (int g = 0; g < 2; ++g)
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[4 * g + e] = in[g * (8 * 64)][e];
-  bool fits = true;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) fits = fits && fits_pieces(v[j]);
-  if (!fits) *a.outside = 1;  // (every such lane the same value)
   store_split(a.w + tile_offset(tile, step) + lane * 16, v);
+}
+
+// Whether a layer may hold this weight and still be an fp32 layer in pieces.  Below
+// kLeastWeight the third piece falls under bf16's smallest number and the sum of the
+// three is no longer exact.  From kMostWeight on (an infinity too) the products of
+// its smaller pieces with a large activation's can overflow with another sign than
+// the leading product's: NaN where fp32 has an infinity.
+constexpr float kLeastWeight = 0x1p-110f, kMostWeight = 0x1p7f;
+// Nonzero weights that an output has at least, or none.  A nonzero product takes up
+// to six roundings of the running sum here and one on the fp32 matrix cores; over a
+// whole row those are more, because they add two products at a time and not eight.
+// Errors in 2^-24 of the output's rms, here and there, for the kernels with one set
+// of sums, weights of both signs: 0.95 / 1.13 and 0.85 / 0.82 with 32 and 64, 1.10 /
+// 0.94 with 128, 0.88 / 0.99 with 192, 1.22 / 2.29 with all; large_kernel, all positive: 1.57 /
+// 1.41 with 32, 1.97 / 1.97 with 64, 3.83 / 7.82 with all.
+constexpr int kLeastNonzero = 192;
+__device__ __host__ constexpr bool fits_pieces(float w) {
+  const float size = w < 0.f ? -w : w;
+  return size == 0.f || (size >= kLeastWeight && size < kMostWeight);
+}
+
+// Sets *outside where a layer's weights are not for pieces; once, when the network
+// is loaded.  One wavefront per n-tile (blockIdx.x) and layer (blockIdx.y).
+struct CheckArgs {
+  const float* w_stream;
+  int32_t groups_total;  // k-groups per wave stream
+  int32_t g0;            // first k-group of the first layer
+  uint32_t* outside;
+};
+__global__ __launch_bounds__(64) void check_kernel(const CheckArgs a) {
+  const int lane = threadIdx.x, tile = blockIdx.x;
+  const f32x4* in = reinterpret_cast<const f32x4*>(a.w_stream) +
+                    ((size_t)(tile >> 3) * a.groups_total + a.g0 + blockIdx.y * (kWidth / 8)) * (8 * 64) +
+                    (tile & 7) * 64 + lane;
+  bool fits = true;
+  int nonzero = 0;
+#pragma unroll 8
+  for (int g = 0; g < kWidth / 8; ++g) {
+    const f32x4 v = in[(size_t)g * (8 * 64)];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      fits = fits && fits_pieces(v[e]);
+      nonzero += v[e] != 0.f;
+    }
+  }
+  nonzero += __shfl_xor(nonzero, 32);
+  if (!fits || (nonzero > 0 && nonzero < kLeastNonzero)) *a.outside = 1;  // (all the same value)
 }
 
 struct FirstArgs {

@@ -326,8 +326,8 @@ hbt_mlp *hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
  * of the row; the kernels for different row counts sum in different orders and
  * agree to fp32 rounding.  From 129 rows on the hidden layers' products are formed
  * from bf16 pieces (see hbt_mlp_forward_fp32), unless a hidden weight is infinite,
- * NaN, 2^7 or more in magnitude or, not being zero, less than 2^-110: such a network
- * is hbt_mlp_forward_fp32 at any n.
+ * NaN, 2^7 or more in magnitude or, not being zero, less than 2^-110, or a hidden
+ * unit has 1 to 191 nonzero weights: such a network is hbt_mlp_forward_fp32 at any n.
  */
 int hbt_mlp_forward(hbt_mlp *mlp, const double *raw_features, int64_t n, float *out,
                     void *hip_stream);

@@ -137,6 +137,23 @@ def test_infinite_and_huge_weights(rows):
                 assert np.all(np.abs(y[large] / big[large] - 1) < 1e-5), special
 
 
+@pytest.mark.parametrize("rows", [129, 3000, 13000])
+def test_sparse_weights_keep_fp32_sums(rows):
+    """One output with fewer nonzero weights than the pieces need: the fp32 kernels."""
+    rp = network("linear", 2)
+    x, mu, sigma = synthetic.mlp_features("linear", rows, seed=rows)
+    rp.set_normalization(mu, sigma)
+    weight = rp.model.mlp.layers[2].weight
+    whole = weight.detach()[1023].clone()
+    for nonzero, pieces in ((1024, True), (1, False), (191, False), (192, True), (0, True)):
+        with torch.no_grad():
+            weight[1023] = whole
+            weight[1023, torch.randperm(1024)[nonzero:]] = 0.0
+        rp.refresh()
+        y, fp32 = rp.predict_batch(x), rp.predict_batch_fp32(x)
+        assert torch.equal(y, fp32) != pieces, nonzero
+
+
 # hbt_mlp_forward_fp32 (device sweeps): around its per-layer path's end at 7168 rows, the
 # fused kernel's rounds of 8192 and what such a round leaves over
 @pytest.mark.parametrize("rows", [2048, 2049, 7168, 7169, 8192, 8193, 16384, 20001])
