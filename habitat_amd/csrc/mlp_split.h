@@ -213,8 +213,8 @@ __device__ __forceinline__ void finish_tile(const LayerArgs& a, const f32x16& ac
 // steps give an error of 5.5 (see above) for 2.5 % more time than none; all of
 // them 2.4 for 8 % more.
 //
-// 32 768 rows in two rounds, one layer: 0.28-0.30 ms, 235 TFLOP/s of fp32 work = 1.41 PFLOP/s
-// of bf16 (the fp32 matrix cores: 0.47 ms, 147 TFLOP/s).  Tried and not faster:
+// 16 384 rows, one layer: 0.143-0.15 ms, 235 TFLOP/s of fp32 work = 1.41 PFLOP/s
+// of bf16 (the fp32 matrix cores: 0.235 ms, 147 TFLOP/s).  From 12 289 rows on.  Tried and not faster:
 // 128 x 256 and 128 x 128 per workgroup, two workgroups to a compute unit (1.39,
 // 1.45 against 1.55 PFLOP/s without the write-back), four waves of 4 x 4 tiles
 // (1.19), fragments stored by k-step first, fetching a slab earlier.
@@ -397,12 +397,13 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void large_kernel(const LayerArgs 
   }
 }
 
-// A hidden layer for 4097 to 6144 rows (and multiples), in rounds of one workgroup
+// A hidden layer for 4609 to 6144 and 10 241 to 12 288 rows, in rounds of one workgroup
 // per compute unit: smaller blocks than large_kernel's, so that a batch fills the
 // card, and for the same reason bound by LDS as much as by the matrix cores.
 // 1 x 3 tiles per wave, 4 x 2 waves, 128 outputs x 192 rows: 6144 rows in 50-57
 // us, 228-250 TFLOP/s of fp32 (the fp32 matrix cores: 90 us; small_kernel in two
-// rounds: 54).  Slabs of KS = 2 k-steps (one barrier for both: 37 us a layer at
+// rounds: 54; whole forwards of 4700 to 6144 rows are within 4 % of those with its 4 x 3
+// tiles, which have one set of sums).  Slabs of KS = 2 k-steps (one barrier for both: 37 us a layer at
 // 4096 rows against 47 with one step), two slabs of LDS.  A wave holds all
 // fragments of a step in registers and reads the next step's during its MFMAs, so
 // a slab's place is free for the next but one at the barrier.  Registers allow
@@ -544,8 +545,8 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void mid_kernel(const LayerArgs a)
   }
 }
 
-// A hidden layer for some hundreds to 4096 rows: one workgroup per compute unit of
-// TN x TM tiles, K split over its waves.  A wave multiplies all of the
+// A hidden layer for 129 to 4608 and 6145 to 10 240 rows, in rounds of one workgroup
+// per compute unit of TN x TM tiles, K split over its waves.  A wave multiplies all of the
 // workgroup's tiles over its part of K, so no fragment is wanted by two waves:
 // they come straight from L2 into a ring of RING k-steps of registers (no LDS,
 // no barrier until the end), where the waves' sums then meet in wave order.

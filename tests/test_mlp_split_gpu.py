@@ -154,6 +154,51 @@ def test_sparse_weights_keep_fp32_sums(rows):
         assert torch.equal(y, fp32) != pieces, nonzero
 
 
+def whole_numbers(seed):
+    """Two dense hidden layers of whole numbers, 11 bits wide in the first, whose sums
+    are exact in any order: below 2^24 in every partial sum, activations of up to
+    three pieces and weights of two."""
+    rng = np.random.default_rng(seed)
+    rp = RuntimePredictor("bmm", 2, 1024)
+    first = rng.integers(1, 2048, (1024, 1024)) * rng.choice([-1, 1], (1024, 1024))
+    second = rng.choice([-1, 1], (1024, 1024)) * (rng.random((1024, 1024)) < 0.3)
+    last = np.zeros(1024)
+    last[rng.choice(1024, 16, replace=False)] = rng.choice([-1, 1], 16)
+    with torch.no_grad():
+        for p in rp.model.parameters():
+            p.zero_()
+        rp.model.fc1.weight.copy_(torch.from_numpy(rng.integers(-1, 2, (1024, 8))))
+        rp.model.mlp.layers[0].weight.copy_(torch.from_numpy(first))
+        rp.model.mlp.layers[2].weight.copy_(torch.from_numpy(second))
+        rp.model.mlp.layers[0].bias.copy_(torch.from_numpy(rng.integers(-2048, 2048, 1024)))
+        rp.model.mlp.layers[2].bias.copy_(torch.from_numpy(rng.integers(-2048, 2048, 1024)))
+        rp.model.fc2.weight.copy_(torch.from_numpy(last)[None])
+    rp.set_normalization(np.zeros(8), np.ones(8))
+    return rp, rng
+
+
+# Every kernel of split_kernel_for (256 compute units) at the ends of its ranges and
+# between: 1 x 1, 1 x 2, 2 x 2, 2 x 3, 2 x 4, 4 x 3 and 4 x 4 tiles, mid_kernel from 4609
+# and 10 241 rows, large_kernel from 12 289; whole and partial last blocks of each.
+@pytest.mark.parametrize("rows", [129, 191, 256, 257, 500, 513, 1000, 1025, 1505, 1537, 1950, 2049, 2900,
+                                  3073, 4000, 4097, 4605, 4609, 5121, 5911, 6113, 6144, 6145, 7300,
+                                  8193, 9100, 9217, 10200, 10241, 11000, 12288, 12289, 13000, 14433,
+                                  16351, 16384, 16384 + 12500])
+def test_every_weight_position_is_wired_in_pieces(rows):
+    rp, rng = whole_numbers(rows)
+    x = rng.integers(-1, 2, (rows, 8)).astype(np.float64)
+    sd = {k: v.double().cuda() for k, v in rp.model.state_dict().items()}
+    h = torch.relu(torch.from_numpy(x).cuda() @ sd["fc1.weight"].t())
+    for name in ("mlp.layers.0", "mlp.layers.2", "fc2"):
+        w = sd[name + ".weight"]
+        assert float((h @ w.abs().t()).max()) + 2048 < 2 ** 24
+        h = h @ w.t() + sd[name + ".bias"]
+        h = torch.relu(h) if name != "fc2" else h
+    pieces, fp32 = rp.predict_batch(x).double(), rp.predict_batch_fp32(x).double()
+    assert torch.equal(fp32, h.reshape(-1))
+    assert torch.equal(pieces, h.reshape(-1))
+
+
 # hbt_mlp_forward_fp32 (device sweeps): around its per-layer path's end at 7168 rows, the
 # fused kernel's rounds of 8192 and what such a round leaves over
 @pytest.mark.parametrize("rows", [2048, 2049, 7168, 7169, 8192, 8193, 16384, 20001])
