@@ -37,8 +37,9 @@ def forward_fp64(rp, x):
 # 1024, 1536, 2048, 3072, 4096, 6144 and 16 384 rows, and chunks of 16 384
 @pytest.mark.parametrize("rows", [129, 160, 161, 255, 256, 257, 480, 511, 512, 513, 700, 1023, 1024,
                                   1025, 1500, 1536, 1537, 2048, 2049, 2080, 2177, 3071, 3072, 3073,
-                                  4095, 4096, 4097, 4161, 6144, 6145, 7169, 7200, 7424, 7425, 8193,
-                                  16383, 16384, 16385, 24001, 32768, 32769, 40001])
+                                  4095, 4096, 4097, 4161, 4608, 4609, 5911, 6113, 6144, 6145, 7169,
+                                  7200, 7424, 7425, 8193, 9217, 10241, 11000, 12288, 12289, 13000,
+                                  16351, 16383, 16384, 16385, 24001, 32768, 32769, 40001])
 @pytest.mark.parametrize("hidden", [1, 2])
 def test_rows_around_the_kernels_edges(rows, hidden):
     rp = network("lstm", hidden)
@@ -94,6 +95,36 @@ def test_values_beyond_bf16(rows):
     y = rp.predict_batch(x).cpu().numpy()
     assert np.array_equal(np.isposinf(y), x[:, 2] > 1.0)
     assert np.all(y[x[:, 2] < 0] == 0) and np.all(np.isfinite(y[x[:, 2] == 1.0]))
+
+
+@pytest.mark.parametrize("rows", [200, 400, 800, 1400, 2000, 3000, 4000, 6000, 9000, 11000, 13000,
+                                  16351])
+def test_values_beyond_bf16_among_dense_weights(rows):
+    """As above where the network takes the pieces: one unit of fc1 is the feature,
+    the others are zero, and the hidden weights are dense.  NaN and infinities too."""
+    rp = network("bmm", 1)
+    big = np.float32(3.4028234663852886e38)
+    values = np.array([big, np.nextafter(big, np.float32(0)), 3.3961775e38, 3.39617e38, 3.3895e38,
+                       1.0 / 3.0, 2.0 ** -100, 1e-30, 65537.0, -big, 0.0, np.nan, np.inf, -np.inf])
+    with torch.no_grad():
+        rp.model.fc1.weight.zero_()
+        rp.model.fc1.bias.zero_()
+        rp.model.fc1.weight[7, 2] = 1.0
+        hidden = rp.model.mlp.layers[0]
+        hidden.bias.zero_()
+        hidden.weight[:, 7] = -0.7                 # the other units are dead
+        hidden.weight[100, 7] = 2.0 ** -3
+        rp.model.fc2.weight.fill_(1.0)
+        rp.model.fc2.bias.zero_()
+    rp.set_normalization(np.zeros(8), np.ones(8))
+    x = np.zeros((rows, 8))
+    x[:, 2] = np.resize(values, rows)
+    v = x[:, 2].astype(np.float32)
+    with np.errstate(invalid="ignore"):
+        # a NaN or an infinity of the feature is NaN in every unit of fc1 (0 x inf)
+        want = np.where(np.isfinite(v), np.maximum(v, 0) * np.float32(2.0 ** -3), np.nan)
+    for y in (rp.predict_batch(x), rp.predict_batch_fp32(x)):
+        assert np.array_equal(y.cpu().numpy(), want, equal_nan=True)
 
 
 @pytest.mark.parametrize("rows", [200, 400, 800, 1400, 2000, 3000, 4000, 6000, 9000, 13000])
@@ -201,10 +232,14 @@ def test_every_weight_position_is_wired_in_pieces(rows):
 
 # hbt_mlp_forward_fp32 (device sweeps): around its per-layer path's end at 7168 rows, the
 # fused kernel's rounds of 8192 and what such a round leaves over
-@pytest.mark.parametrize("rows", [2048, 2049, 7168, 7169, 8192, 8193, 16384, 20001])
-def test_fp32_sums_at_any_row_count(rows):
-    rp = network("linear", 2)
-    x, mu, sigma = synthetic.mlp_features("linear", rows, seed=rows)
+@pytest.mark.parametrize("kind,rows", [("linear", r) for r in (2048, 2049, 7168, 7169, 8192, 8193,
+                                                                16384, 20001)] +
+                         [(("conv2d", "linear", "bmm", "lstm")[r % 4], r)
+                          for r in (129, 160, 161, 255, 511, 512, 513, 1000, 1025, 1503, 2047,
+                                    4095, 4096, 4097, 5002)])
+def test_fp32_sums_at_any_row_count(kind, rows):
+    rp = network(kind, 2)
+    x, mu, sigma = synthetic.mlp_features(kind, rows, seed=rows)
     rp.set_normalization(mu, sigma)
     y = rp.predict_batch_fp32(x).cpu().numpy()
     want = forward_fp64(rp, x)
@@ -217,6 +252,34 @@ def test_fp32_sums_at_any_row_count(rows):
         assert np.array_equal(y[:whole], rp.predict_batch_fp32(x[:whole]).cpu().numpy())
     if whole < rows:
         assert np.array_equal(y[whole:], rp.predict_batch_fp32(x[whole:]).cpu().numpy())
+
+
+@pytest.mark.parametrize("zero_sigma", [False, True])
+def test_fp32_sums_hand_on_nan_and_infinities(zero_sigma):
+    """test_nan_and_infinite_features_give_what_torch_gives for hbt_mlp_forward_fp32:
+    K over workgroups, K in 4, 2 and 1 parts, and the fused kernel."""
+    rp = network("conv2d", 4)
+    x, mu, sigma = synthetic.mlp_features("conv2d", 9000, seed=2)
+    rng, x = np.random.default_rng(1), x.copy()
+    special = np.array([np.nan, np.inf, -np.inf, 1e300, -1e300, 3e38, 1e-300, 0.0])
+    for r in rng.choice(9000, 900, replace=False):
+        x[r, rng.integers(0, x.shape[1])] = rng.choice(special)
+    if zero_sigma:
+        sigma = np.where(np.arange(sigma.shape[0]) == 3, 0.0, sigma)
+    rp.set_normalization(mu, sigma)
+    with np.errstate(all="ignore"):
+        every = omlp.forward_fp32(rp.model.state_dict(), x, mu, sigma)
+    for rows in (20, 100, 300, 3000, 5000, 9000):
+        want, got = every[:rows], rp.predict_batch_fp32(x[:rows]).cpu().numpy()
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        assert np.array_equal(np.isposinf(got), np.isposinf(want))
+        assert np.array_equal(np.isneginf(got), np.isneginf(want))
+        fin = np.isfinite(want) & (np.abs(want) < 1e3)    # (a feature of 3e38 gives more)
+        # the bound of test_rows_around_the_kernels_edges at the worst row, for each of
+        # the two orders of fp32 sums
+        rms = np.sqrt(np.mean(want[fin].astype(np.float64) ** 2)) if fin.any() else 0.0
+        assert np.all(np.abs(got[fin] - want[fin]) <= 2 * 6 * 5 * 8 * 2.0 ** -24 * rms)
+        assert not zero_sigma or np.all(np.isnan(want))
 
 
 def test_a_sweep_divides_predictions_with_fp32_sums():
