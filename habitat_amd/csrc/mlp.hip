@@ -1466,13 +1466,14 @@ int hbt_mlp_forward(hbt_mlp* mlp, const double* raw_features, int64_t n, float* 
   const int bad = check_forward(mlp, raw_features, n, out);
   if (bad != HBT_OK || n == 0) return bad;
   hipStream_t stream = static_cast<hipStream_t>(hip_stream);
+  if (!mlp->takes_pieces) return forward_fp32(mlp, raw_features, n, out, stream);
   // Whole rounds of the 256 x 256 workgroups, then what is left over, with the
   // kernels that suit it.
   int64_t done = 0;
   while (done < n) {
     const int64_t rows = n - done < mlp->chunk_rows ? n - done : mlp->chunk_rows;
     const double* raw = raw_features + done * mlp->in_features;
-    const int rc = rows > kSplitAboveRows && mlp->takes_pieces
+    const int rc = rows > kSplitAboveRows
                        ? forward_split(mlp, raw, rows, out + done, mlp->scratch, mlp->part, stream)
                        : forward_fp32(mlp, raw, rows, out + done, stream);
     if (rc != HBT_OK) return rc;
