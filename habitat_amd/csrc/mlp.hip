@@ -818,6 +818,7 @@ __global__ __launch_bounds__(256) void mlp_last_km_kernel(const LastArgs a) {
 
 constexpr size_t kOneOutOffset = 512;   // hbt_mlp_predict_one's result within its staging block
 constexpr size_t kOneDoneOffset = 768;  // and the call number the last kernel publishes after it
+constexpr size_t kOneOutsideOffset = 896;  // and what hbt_mlp_create's check_kernel leaves
 constexpr size_t kOneBytes = 1024;
 static_assert(kMaxInPadded * sizeof(double) <= kOneOutOffset, "a raw row fits below the result");
 
@@ -1330,7 +1331,6 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
   const size_t chain_bytes = align_up(sizeof(uint64_t) *
       (kChainHeader + (size_t)hidden_layers * chain::kMaxRows * kWidth), 256);
   const size_t off_chain = off; off += 2 * chain_bytes;
-  const size_t off_outside = off; off += 256;  // cleared with the above
   const size_t total = off;
 
   std::vector<unsigned char> host;
@@ -1378,12 +1378,24 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
     *err = HBT_EHIP;
     return nullptr;
   }
-  if (hipMemset(static_cast<unsigned char*>(blob) + off_chain, 0, total - off_chain) != hipSuccess) {
+  if (hipMemset(static_cast<unsigned char*>(blob) + off_chain, 0, 2 * chain_bytes) != hipSuccess) {
     (void)hipGetLastError();
     (void)hipFree(blob);
     *err = HBT_EHIP;
     return nullptr;
   }
+  void* one_host = nullptr;
+  void* one_device = nullptr;
+  if (hipHostMalloc(&one_host, kOneBytes, hipHostMallocDefault) != hipSuccess ||
+      hipHostGetDevicePointer(&one_device, one_host, 0) != hipSuccess || one_device == nullptr) {
+    (void)hipGetLastError();
+    if (one_host != nullptr) (void)hipHostFree(one_host);
+    (void)hipFree(blob);
+    *err = HBT_ENOMEM;
+    return nullptr;
+  }
+  std::memset(one_host, 0, kOneBytes);
+
   // the hidden layers' weights in bf16 pieces, from the packed fp32 ones
   for (int l = 0; l < hidden_layers; ++l) {
     split::PackArgs a{};
@@ -1399,31 +1411,21 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
     a.w_stream = reinterpret_cast<const float*>(static_cast<unsigned char*>(blob) + off_stream);
     a.groups_total = in_padded / 8 + hidden_layers * (kWidth / 8);
     a.g0 = in_padded / 8;
-    a.outside = reinterpret_cast<uint32_t*>(static_cast<unsigned char*>(blob) + off_outside);
+    // (through host memory: a copy back made the next call from an idle GPU 10 us slower)
+    a.outside = reinterpret_cast<uint32_t*>(static_cast<unsigned char*>(one_device) +
+                                            kOneOutsideOffset);
     hipLaunchKernelGGL(split::check_kernel, dim3(kWidth / 32, (unsigned)hidden_layers), dim3(64), 0,
                        nullptr, a);
   }
-  uint32_t outside = 0;
-  if (hipGetLastError() != hipSuccess ||
-      hipMemcpy(&outside, static_cast<unsigned char*>(blob) + off_outside, sizeof outside,
-                hipMemcpyDeviceToHost) != hipSuccess) {
+  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
     (void)hipGetLastError();
+    (void)hipHostFree(one_host);
     (void)hipFree(blob);
     *err = HBT_EHIP;
     return nullptr;
   }
-
-  void* one_host = nullptr;
-  void* one_device = nullptr;
-  if (hipHostMalloc(&one_host, kOneBytes, hipHostMallocDefault) != hipSuccess ||
-      hipHostGetDevicePointer(&one_device, one_host, 0) != hipSuccess || one_device == nullptr) {
-    (void)hipGetLastError();
-    if (one_host != nullptr) (void)hipHostFree(one_host);
-    (void)hipFree(blob);
-    *err = HBT_ENOMEM;
-    return nullptr;
-  }
-  std::memset(one_host, 0, kOneBytes);
+  uint32_t outside = 0;
+  std::memcpy(&outside, static_cast<unsigned char*>(one_host) + kOneOutsideOffset, sizeof outside);
 
   hbt_mlp* m = new (std::nothrow) hbt_mlp();
   if (m == nullptr) {
