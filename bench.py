@@ -3,9 +3,8 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W]
 
-A step is one pass of wave scaling over the 1 M synthetic kernel records of
-BASELINE.json's configs[1] (V100-like origin -> MI355X-like destination),
-inputs resident in HBM.  Prints ONE JSON line:
+A step is one pass of wave scaling over 1 M synthetic kernel records (V100-like
+origin -> MI355X-like destination), inputs resident in HBM.  Prints ONE JSON line:
   value         whole-job wave-scaled kernel records per second (K steps, wall clock)
   roofline      the wave-scaling kernel against HBM bandwidth: 68 algorithmic
                 bytes per record / average launch duration (HIP events on the
@@ -20,12 +19,12 @@ inputs resident in HBM.  Prints ONE JSON line:
                 device table in one launch (records read once)
   large         the same kernel at 64 M records (beyond the 256 MB last-level cache);
                 large_16M: at 16 M records
-  mlp           the MLP (configs[2], conv2d, 1 M rows): rows/s, its roofline
+  mlp           the MLP (conv2d, 1 M rows): rows/s, its roofline
                 against the bf16 matrix peak at six products per fp32 product and a torch-CPU fp32 baseline
   scalar_strategy  the reference's one-kernel strategy call through the same kernel
   host_records  the same records as an array of structures in HOST memory, results
                 back in host memory, copies and wait included
-  sweep         configs[4]: one ResNet-50-shaped trace predicted for 256 devices
+  sweep         one ResNet-50-shaped trace predicted for 256 devices
                 (fused per-pass sums + MLP rows + ratio kernel), eager and as a
                 replayed HIP graph, next to the per-device CPU path
 Only one GPU is used; --gpus above 1 exits.
@@ -73,7 +72,7 @@ def parse():
     ap.add_argument("--no-large", action="store_true")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-sweep", action="store_true",
-                    help="skip configs[4] (one ResNet-50-shaped trace against 256 devices)")
+                    help="skip the sweep (one ResNet-50-shaped trace against 256 devices)")
     ap.add_argument("--sweep-devices", type=int, default=256)
     ap.add_argument("--no-ceilings", action="store_true",
                     help="skip measuring the box's own copy bandwidth and FMA/MFMA rates")
@@ -146,7 +145,7 @@ def tile_records(rec, n):
 
 
 def mlp_bench(args):
-    """configs[2] (and the other kinds of configs[3], one step each): the MLP at
+    """The conv2d MLP (and the other kinds, one step each) at
     full size, fewer rows, and a torch CPU baseline."""
     import numpy as np
     import torch
@@ -166,7 +165,7 @@ def mlp_bench(args):
     tflops = flops_per_row * args.mlp_rows / (m_launch * 1e-3) / 1e12
     mlp = {"metric": "MLP op-predictions/s", "value": args.mlp_rows / (m_wall * 1e-3),
            "unit": "rows/s", "steps": args.mlp_steps, "ms_per_step": m_wall, "dtype": "f32",
-           "config": {"workload": "configs[2]: %s MLP, %d rows x %d raw fp64 features, "
+           "config": {"workload": "%s MLP, %d rows x %d raw fp64 features, "
                                   "fc1 + 8 x 1024 hidden + fc2, seed-0 random init"
                                   % (kind, args.mlp_rows, f_in)},
            "roofline": {"bound": "mfma", "achieved": tflops, "peak": MFMA_SPLIT_PEAK_TFLOPS,
@@ -198,7 +197,7 @@ def mlp_bench(args):
         few["rows_%d_us" % rows] = f_launch * 1e3
     # RuntimePredictor.predict as the reference calls it (mlp.py:252-267): what a
     # caller waits per call, wall clock, for arguments not asked before (one
-    # hbt_mlp_predict_one: a row through pinned memory, ten launches, a wait) and
+    # hbt_mlp_predict_one: a row through pinned memory, one launch, a wait) and
     # for arguments asked before (answered from the predictor's table)
     n_feat = len(rp.model.features)
     ops = [list(map(float, x[i, :n_feat])) for i in range(400)]
@@ -261,7 +260,7 @@ def mlp_bench(args):
 
 
 def sweep_bench(args, origin):
-    """predicted iteration time of one trace on D devices."""
+    """Predicted iteration time of one trace on D devices."""
     import numpy as np
     import torch
     from habitat_amd import synthetic
@@ -304,7 +303,7 @@ def sweep_bench(args, origin):
     same = bool(torch.allclose(captured.total_ms, totals, rtol=1e-12, atol=0))
     n_kernels = len(plan.kernels)
     n_special = sum(len(v[0]) for v in plan.special.values())
-    out = {"workload": "configs[4]: ResNet-50-shaped trace (%d operations, %d kernel records in "
+    out = {"workload": "ResNet-50-shaped trace (%d operations, %d kernel records in "
                        "%d passes, %d MLP-predicted operations), V100 origin, %d synthetic devices"
                        % (len(trace.operations), n_kernels, len(plan.pass_owner), n_special, D),
            "devices": D, "prepare_ms_once": prepare_ms,
@@ -406,7 +405,7 @@ def main():
         del src, dst
         torch.cuda.empty_cache()
 
-    # ---------------- wave scaling, configs[1] ----------------
+    # ---------------- wave scaling ----------------
     rec, stats = synthetic.kernel_records(args.records, origin, seed=0)
     records = KernelRecords.from_numpy(rec)
     out = WaveScaleOutput(records.n, 1, records.device, waves=False, status=True)
@@ -424,7 +423,7 @@ def main():
         "warmup": args.warmup, "ms_per_step": wall_ms,
         "higher_is_better": True,
         "scaling": "weak", "vs_baseline": None, "dtype": "f64", "data": "synthetic",
-        "config": {"workload": "configs[1]: wave scaling, %d kernel records (SoA, int32 launch "
+        "config": {"workload": "wave scaling, %d kernel records (SoA, int32 launch "
                                "params, fp64 times/metrics), V100 -> MI355X-like, outputs time + "
                                "2 occupancies + status" % args.records,
                    "records": args.records, "origin": origin.name, "dest": dest.name,
@@ -443,7 +442,7 @@ def main():
                      "traffic_source": "constant from profiles/wave_scale_kernel_1M_and_64M_"
                                        "records.md (rocprofv3 FETCH_SIZE + WRITE_SIZE per "
                                        "record, copy-calibrated), not measured in this run",
-                     "kernel": "wave_scale_kernel<1, 1, true, unsigned int>", "launch_us": launch_ms * 1e3,
+                     "kernel": "wave_scale_kernel<1, 1, true, false, unsigned int>", "launch_us": launch_ms * 1e3,
                      "bytes_per_record": BYTES_PER_RECORD},
     }
     if args.steps < 1000:
@@ -703,11 +702,11 @@ def main():
             attempt("large_16M", lambda: large_section(16_000_000))
             torch.cuda.empty_cache()
 
-    # ---------------- MLP, configs[2] ----------------
+    # ---------------- MLP ----------------
     if not args.no_mlp:
         attempt("mlp", lambda: mlp_bench(args))
 
-    # ---------------- configs[4]: one trace, a sweep of destination devices ----------------
+    # ---------------- one trace, a sweep of destination devices ----------------
     if not args.no_sweep:
         attempt("sweep", lambda: sweep_bench(args, origin))
 

@@ -5,7 +5,7 @@ inference: the four network classes keep the reference's layer names, so a
 reference checkpoint ({'mu', 'sigma', 'model': state_dict}) loads unchanged,
 and `RuntimePredictor.predict(kernel_arguments, device_name)` keeps its
 signature.  The forward pass itself runs in libhabitat_mi.so
-(hbt_mlp_forward: one launch per layer, on the matrix cores);
+(hbt_mlp_forward: up to 4 rows one launch, above that one per layer);
 `predict_batch` is the entry that makes it worthwhile.  Training is not part of
 this package.
 """

@@ -2,7 +2,7 @@
 //
 // What bounds a batch of rows is the matrix cores, and gfx950's do 16 times as
 // many multiply-adds per cycle on bf16 as on fp32.  An fp32 number is the exact
-// sum of three bf16 numbers (8 + 8 + 8 bits of mantissa, bf16 has fp32's range):
+// sum of three bf16 numbers (8 + 8 + 8 bits of mantissa):
 //     x = x0 + x1 + x2,  x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1
 // so weights and activations are kept as three such pieces, and of the nine
 // products of pieces the six that matter are multiplied:
@@ -11,6 +11,18 @@
 // either sign: beside the roundings of a sum of 1024 products it does not show.
 // Products of bf16 are exact in the matrix core and sums are fp32, so the layer
 // is an fp32 layer at 16 / 6 of the fp32 rate.
+//
+// Where it is not: below 2^-110 the third piece falls under bf16's smallest number,
+// 2^-133, and a number is held to 2^-134 and no longer to 24 bits (a single product
+// with an activation of 2^-114: off by 1e-6, of 2^-122 by 2.4e-4; products and sums
+// that small are kept otherwise, the matrix core does not flush them).  A layer with
+// bias or weights of ordinary size never shows it; weights below it, and weights whose
+// products could overflow, do not come here (fits_pieces).  And a product takes more
+// roundings than on the fp32 matrix cores, so that with a few nonzero products to a
+// sum the error is larger: for a single one up to 1.7 x 2^-24 with two sets of sums (small_kernel
+// to 2 x 4 tiles, mid_kernel), 3.7 with one (the larger tiles, large_kernel), 1.0 in
+// fp32.  Sparse weights therefore do not come here either (kLeastNonzero); a layer
+// whose input has fewer than some 100 active units of 1024 can see it.
 //
 // The order of the sum decides its error: the matrix core adds eight products
 // and rounds the running sum, and a rounding costs half an ulp of what the sum
@@ -807,7 +819,7 @@ constexpr int kFirstSlices = 8;
 // plain FMAs from LDS do it.  A workgroup takes one m-tile and a slice of the
 // outputs (an eighth: 2 / 8 / 16 / 32 slices took 19.4 / 8.4 / 10.0 / 13.6 us at
 // 4096 rows when the output was fp32).  Sum order: bias, then k ascending.
-// 32 768 rows: 44 us, 4.6 TB/s (a large copy on this card: 4.8).
+// 16 384 rows: 20.5 us, 4.9 TB/s (a large copy on this card: 4.8).
 template <int MAX_IN>
 __global__ __launch_bounds__(256) void first_kernel(const FirstArgs a) {
   constexpr int kSlice = kWidth / kFirstSlices;

@@ -318,9 +318,11 @@ hbt_mlp *hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
  * four device features — are standardised in fp64, cast to fp32, and run
  * through the network; out[n] receives the fp32 predictions.  Must be called
  * with the device of hbt_mlp_create current.  Up to 4 rows the network is one
- * launch, above that each layer is one, spread over the whole GPU, with activations or partial sums in scratch memory that
- * belongs to the handle (allocated by hbt_mlp_create, 13 KiB for each of 64
- * rows per compute unit: 0.21 GB on 256; longer batches are taken in chunks):
+ * launch, above that each layer is one, spread over the whole GPU, with activations
+ * or partial sums in scratch memory that belongs to the handle (allocated by
+ * hbt_mlp_create, 13 KiB for each of 64 rows per compute unit: 0.21 GB on 256;
+ * longer batches are taken in chunks.  With its weights a handle of eight hidden
+ * layers holds 0.29 GB of device memory from the start):
  * calls on ONE handle must therefore not overlap, on any streams; different
  * handles are independent.  Results are reproducible for a given n and position
  * of the row; the kernels for different row counts sum in different orders and
@@ -333,12 +335,14 @@ int hbt_mlp_forward(hbt_mlp *mlp, const double *raw_features, int64_t n, float *
                     void *hip_stream);
 
 /*
- * hbt_mlp_forward with every product and sum on the fp32 matrix cores at any n
- * (hbt_mlp_forward takes large batches in bf16 pieces: faster, closer to an
- * exact evaluation, other last bits).  For callers that divide predictions by
- * each other and hold the quotients against earlier ones, as a device sweep does:
- * where predictions cancel, a quotient shows another order of sums in its fifth
- * digit.  Arguments, limits and scratch as hbt_mlp_forward.
+ * hbt_mlp_forward with fp32 products and sums at any n; their order, and so the
+ * last bits, depends on n and on the position of the row.  (hbt_mlp_forward takes
+ * batches from 129 rows on in bf16 pieces: faster, sums of some hundred products
+ * and more closer to an exact evaluation, other last bits; a single product is held
+ * to 2^-23, an activation below 2^-110 to 2^-134.)  For callers that divide
+ * predictions by each other and hold the quotients against earlier ones, as a trace
+ * and a device sweep do: where predictions cancel, a quotient shows another order of
+ * sums in its fifth digit.  Arguments, limits and scratch as hbt_mlp_forward.
  */
 int hbt_mlp_forward_fp32(hbt_mlp *mlp, const double *raw_features, int64_t n, float *out,
                          void *hip_stream);

@@ -330,7 +330,7 @@ def test_scalar_predict_and_checkpoint_round_trip(tmp_path):
 
 @pytest.mark.parametrize("kind", ["conv2d", "linear", "bmm", "lstm"])
 def test_config2_and_config3_full_size_properties(kind):
-    # 1M rows (configs[2]: conv2d; configs[3]: the other three): the oracle is
+    # 1M rows of each kind: the oracle is
     # too slow for all of them, so check a strided sample against it and, over
     # the whole batch, invariance to row order.
     rp = make(kind)

@@ -1,6 +1,5 @@
 """GPU: the fused per-pass sums (hbt_wave_scale_sum), the ratio kernel
-(hbt_ratio_scale) and the 256-device sweep of BASELINE's end-to-end
-configuration, against the CPU oracle."""
+(hbt_ratio_scale) and a 256-device sweep end to end, against the CPU oracle."""
 import numpy as np
 import pytest
 import torch
@@ -230,7 +229,7 @@ def test_sweep_shares_rows_of_equal_operations_and_counts_clamped_ones(caplog):
 
 
 def test_end_to_end_256_device_sweep():
-    """a ResNet-50-shaped trace against 256 destinations."""
+    """A ResNet-50-shaped trace against 256 destinations."""
     origin = Device.V100
     trace = synthetic.resnet50_trace(origin, batch=32, seed=3)
     preds = {}
