@@ -13,11 +13,12 @@
 // is an fp32 layer at 16 / 6 of the fp32 rate.
 //
 // Where it is not: below 2^-110 the third piece falls under bf16's smallest number,
-// 2^-133, and a number is held to 2^-134 and no longer to 24 bits (a single product
-// with an activation of 2^-114: off by 1e-6, of 2^-122 by 2.4e-4; products and sums
-// that small are kept otherwise, the matrix core does not flush them).  A layer with
-// bias or weights of ordinary size never shows it; weights below it, and weights whose
-// products could overflow, do not come here (fits_pieces).  And a product takes more
+// 2^-133, and a weight or activation is held to 2^-134 and no longer to 24 bits (a
+// single product with an activation of 2^-114: off by 1e-6, of 2^-122 by 2.4e-4;
+// products and sums that small are kept otherwise, the matrix core does not flush
+// them).  Beside a bias or another product of ordinary size that does not show: what
+// is lost is 2^-134 of the other operand.  Weights whose products could overflow do
+// not come here (fits_pieces).  And a product takes more
 // roundings than on the fp32 matrix cores, so that with a few nonzero products to a
 // sum the error is larger: for a single one up to 1.7 x 2^-24 with two sets of sums (small_kernel
 // to 2 x 4 tiles, mid_kernel), 3.7 with one (the larger tiles, large_kernel), 1.0 in
@@ -756,12 +757,12 @@ __global__ __launch_bounds__(256) void pack_kernel(const PackArgs a) {
   store_split(a.w + tile_offset(tile, step) + lane * 16, v);
 }
 
-// Whether a layer may hold this weight and still be an fp32 layer in pieces.  Below
-// kLeastWeight the third piece falls under bf16's smallest number and the sum of the
-// three is no longer exact.  From kMostWeight on (an infinity too) the products of
-// its smaller pieces with a large activation's can overflow with another sign than
-// the leading product's: NaN where fp32 has an infinity.
-constexpr float kLeastWeight = 0x1p-110f, kMostWeight = 0x1p7f;
+// Whether a layer may hold this weight and be an fp32 layer in pieces.  From
+// kMostWeight on (an infinity too) the products of its smaller pieces with a large
+// activation's can overflow with another sign than the leading product's: NaN where
+// fp32 has an infinity.
+constexpr float kMostWeight = 0x1p7f;
+__device__ __host__ constexpr bool fits_pieces(float w) { return w < kMostWeight && w > -kMostWeight; }
 // Nonzero weights that an output has at least, or none.  A nonzero product takes up
 // to six roundings of the running sum here and one on the fp32 matrix cores; over a
 // whole row those are more, because they add two products at a time and not eight.
@@ -770,10 +771,6 @@ constexpr float kLeastWeight = 0x1p-110f, kMostWeight = 0x1p7f;
 // 0.94 with 128, 0.88 / 0.99 with 192, 1.22 / 2.29 with all; large_kernel, all positive: 1.57 /
 // 1.41 with 32, 1.97 / 1.97 with 64, 3.83 / 7.82 with all.
 constexpr int kLeastNonzero = 192;
-__device__ __host__ constexpr bool fits_pieces(float w) {
-  const float size = w < 0.f ? -w : w;
-  return size == 0.f || (size >= kLeastWeight && size < kMostWeight);
-}
 
 // Sets *outside where a layer's weights are not for pieces; once, when the network
 // is loaded.  One wavefront per n-tile (blockIdx.x) and layer (blockIdx.y).

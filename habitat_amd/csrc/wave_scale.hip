@@ -108,14 +108,15 @@ __device__ __forceinline__ void store_out(T* __restrict__ p, Index i, const T (&
 // either way, 4 000 016 records to seven with all outputs 153 us before and 161 so,
 // 1 000 016 39.4 and 36.7; with all rows at lines 111 us with the hint at 4 000 000
 // and 120 without.  From how many records on depends on how much of a line the
-// wavefronts share, us before and so, to 4 / 5 / 7 destinations:
+// wavefronts share.  To 4, 5 and 7 destinations, us so, and before with rows 8, 32 and
+// 64 bytes into a line (1, 4 and 8 records more):
 //
-//   records + 1 (8 bytes)           + 4 (32 bytes)                  + 8 (64 bytes)
-//   524 k   15.2 19.2 26.0 / 15.4 18.9 23.0   14.9 17.8 24.1 / 15.4 18.9 22.9   14.3 17.2 21.0 / 15.4 18.8 22.9
-//   614 k   17.1 21.1 26.9 / 17.1 21.0 24.7   16.8 20.4 25.2 / 16.9 21.0 24.8   16.3 19.5 23.3 / 16.9 21.0 24.8
-//   700 k   19.5 23.5 30.8 / 18.7 22.3 26.6   19.1 22.4 28.9 / 18.7 22.3 26.6   18.1 21.3 25.8 / 18.6 22.2 26.6
-//   800 k   21.8 27.0 36.6 / 20.2 24.2 28.9   21.3 25.5 33.8 / 20.2 24.1 28.8   20.0 24.1 30.0 / 20.3 24.0 28.8
-//   1.2 M   32.8 40.4 55.5 / 26.0 31.4 38.1   31.9 37.0 51.2 / 26.0 31.4 38.2   29.5 34.3 45.2 / 26.0 31.1 38.0
+//   records   so               8 bytes          32               64
+//   524 k     15.4 18.9 23.0   15.2 19.2 26.0   14.9 17.8 24.1   14.3 17.2 21.0
+//   614 k     17.1 21.0 24.7   17.1 21.1 26.9   16.8 20.4 25.2   16.3 19.5 23.3
+//   700 k     18.7 22.3 26.6   19.5 23.5 30.8   19.1 22.4 28.9   18.1 21.3 25.8
+//   800 k     20.2 24.2 28.9   21.8 27.0 36.6   21.3 25.5 33.8   20.0 24.1 30.0
+//   1.2 M     26.0 31.4 38.1   32.8 40.4 55.5   31.9 37.0 51.2   29.5 34.3 45.2
 //
 // (two destinations never lose more than 2 %; below 2^19 records little is gained).
 // With wave numbers, another two rows a destination, four and more gain from 2^19 on

@@ -328,8 +328,8 @@ hbt_mlp *hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
  * of the row; the kernels for different row counts sum in different orders and
  * agree to fp32 rounding.  From 129 rows on the hidden layers' products are formed
  * from bf16 pieces (see hbt_mlp_forward_fp32), unless a hidden weight is infinite,
- * NaN, 2^7 or more in magnitude or, not being zero, less than 2^-110, or a hidden
- * unit has 1 to 191 nonzero weights: such a network is hbt_mlp_forward_fp32 at any n.
+ * NaN or 2^7 or more in magnitude, or a hidden unit has 1 to 191 nonzero weights:
+ * such a network is hbt_mlp_forward_fp32 at any n.
  */
 int hbt_mlp_forward(hbt_mlp *mlp, const double *raw_features, int64_t n, float *out,
                     void *hip_stream);
@@ -339,7 +339,7 @@ int hbt_mlp_forward(hbt_mlp *mlp, const double *raw_features, int64_t n, float *
  * last bits, depends on n and on the position of the row.  (hbt_mlp_forward takes
  * batches from 129 rows on in bf16 pieces: faster, sums of some hundred products
  * and more closer to an exact evaluation, other last bits; a single product is held
- * to 2^-23, an activation below 2^-110 to 2^-134.)  For callers that divide
+ * to 2^-23, a weight or activation below 2^-110 to 2^-134.)  For callers that divide
  * predictions by each other and hold the quotients against earlier ones, as a trace
  * and a device sweep do: where predictions cancel, a quotient shows another order of
  * sums in its fifth digit.  Arguments, limits and scratch as hbt_mlp_forward.

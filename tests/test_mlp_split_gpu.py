@@ -156,7 +156,7 @@ def test_infinite_and_huge_weights(rows):
             big = np.float32(special) * unit7
             pieces, fp32 = rp.predict_batch(x).cpu().numpy(), rp.predict_batch_fp32(x).cpu().numpy()
             # a network with a weight that does not fit the pieces takes the fp32 kernels
-            if not 2.0 ** -110 <= abs(special) < 128:
+            if abs(special) >= 128:
                 assert np.array_equal(pieces, fp32, equal_nan=True)
             else:
                 assert not np.array_equal(pieces, fp32, equal_nan=True)
@@ -166,6 +166,36 @@ def test_infinite_and_huge_weights(rows):
                 assert np.all(y[big < -1e8] == 0) and np.all(y[big == 0] > 0), special
                 large = (big > 1e8) & np.isfinite(big)   # the other units give some hundreds
                 assert np.all(np.abs(y[large] / big[large] - 1) < 1e-5), special
+
+
+@pytest.mark.parametrize("tiny", ["weights", "activations"])
+@pytest.mark.parametrize("rows", [200, 3000, 5911, 13000])
+def test_numbers_below_the_third_piece(rows, tiny):
+    """Weights or activations around 2^-115 lose at most 2^-134 of each product's
+    other operand, beside the roundings of the sum."""
+    rp = network("bmm", 1)
+    x = np.random.default_rng(rows).normal(size=(rows, 8))
+    rp.set_normalization(np.zeros(8), np.ones(8))
+    with torch.no_grad():
+        hidden = rp.model.mlp.layers[0]
+        hidden.bias.zero_()
+        for p in ((hidden.weight,) if tiny == "weights" else (rp.model.fc1.weight, rp.model.fc1.bias)):
+            p.mul_(2.0 ** -115)
+        rp.model.fc2.weight.zero_()
+        rp.model.fc2.weight[0, 5] = 2.0 ** 100
+        rp.model.fc2.bias.zero_()
+    rp.refresh()
+    y, want = rp.predict_batch(x).double().cpu().numpy(), forward_fp64(rp, x)
+    sd = {k: v.double() for k, v in rp.model.state_dict().items()}
+    act = torch.relu(torch.from_numpy(x) @ sd["fc1.weight"].t() + sd["fc1.bias"])
+    weight = sd["mlp.layers.0.weight"][5].abs()
+    other = float(act.sum(1).max()) if tiny == "weights" else float(weight.sum())
+    # (the bound of test_rows_around_the_kernels_edges on the largest possible sum)
+    size = float((act @ weight).max())
+    assert 0 < size < 2.0 ** -100
+    bound = 2.0 ** 100 * (2.0 ** -134 * other + 8 * 2.0 ** -24 * size)
+    assert float(np.max(np.abs(y - want))) <= bound
+    assert not torch.equal(rp.predict_batch(x), rp.predict_batch_fp32(x))
 
 
 @pytest.mark.parametrize("rows", [129, 3000, 13000])
