@@ -1,10 +1,12 @@
 """GPU: the MLP's hidden layers with every fp32 number in three bf16 pieces
 (habitat_amd/csrc/mlp_split.h), at the sizes where its kernels change."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
-from habitat_amd import synthetic
+from habitat_amd import _lib, synthetic
 from habitat_amd.analysis.mlp.mlp import RuntimePredictor
 from oracle import mlp as omlp
 
@@ -198,9 +200,21 @@ def test_numbers_below_the_third_piece(rows, tiny):
     assert not torch.equal(rp.predict_batch(x), rp.predict_batch_fp32(x))
 
 
-@pytest.mark.parametrize("rows", [129, 3000, 13000])
+def static_forward(rp, x):
+    """hbt_mlp_forward_static."""
+    raw = torch.from_numpy(x).cuda()
+    out = torch.empty((raw.shape[0],), dtype=torch.float32, device="cuda")
+    assert _lib.lib().hbt_mlp_forward_static(
+        rp._device_mlp().handle, ctypes.c_void_p(raw.data_ptr()), raw.shape[0],
+        ctypes.c_void_p(out.data_ptr()),
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    return out
+
+
+@pytest.mark.parametrize("rows", [129, 1000, 3000, 13000])
 def test_sparse_weights_keep_fp32_sums(rows):
-    """One output with fewer nonzero weights than the pieces need: the fp32 kernels."""
+    """One output with fewer nonzero weights than the pieces need: the fp32 kernels,
+    also through the library's static scratch."""
     rp = network("linear", 2)
     x, mu, sigma = synthetic.mlp_features("linear", rows, seed=rows)
     rp.set_normalization(mu, sigma)
@@ -213,6 +227,7 @@ def test_sparse_weights_keep_fp32_sums(rows):
         rp.refresh()
         y, fp32 = rp.predict_batch(x), rp.predict_batch_fp32(x)
         assert torch.equal(y, fp32) != pieces, nonzero
+        assert rows > 1024 or torch.equal(static_forward(rp, x), y)
 
 
 def whole_numbers(seed):
