@@ -28,7 +28,7 @@
 // is done, longer pauses between looks; activations read from LDS by every lane
 // instead of shared among 16 (21 us; the compiler's own sharing, 21.6).
 //
-// Included by mlp.hip only.
+// Included by mlp.hip, and by its test (tests/native/mlp_chain.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -44,8 +44,8 @@ constexpr int kWidth = 1024;
 constexpr int kTiles = kWidth / 32;
 // Rows up to which this is the faster way: 19.2 / 23.9 / 27.6 / 29.9 us for 1 to 4
 // (launches per layer 38.8 / 39.6 / 40.9 / 41.6); an earlier form took 39.5 and 46.0
-// for 5 and 8 (42.0 and 44.2).  What a row adds is its share of the multiply-adds on a layer's 32
-// compute units, 0.2 us, and the reads of the next layer.
+// for 5 and 8 (42.0 and 44.2).  What a row adds is its share of the multiply-adds on
+// a layer's 32 compute units, 0.2 us, and the reads of the next layer.
 constexpr int kMaxRows = 4;
 constexpr uint32_t kNumberAll = 1u << 16;  // calls
 constexpr int kMaxIn = 64;
