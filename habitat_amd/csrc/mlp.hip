@@ -5,8 +5,9 @@
 // standardised as RuntimePredictor.predict does (mlp.py:258-264): (x - mu) /
 // sigma in fp64, then cast to fp32.
 //
-// Above kSplitAboveRows rows hbt_mlp_forward's hidden layers run on the bf16 matrix
-// cores with every fp32 number in three pieces (mlp_split.h).  Up to there, in
+// Above kSplitAboveRows rows hbt_mlp_forward's hidden layers run on the 16-bit matrix
+// cores: with every fp32 number in three bf16 pieces (mlp_split.h) or, from some 2000 rows
+// on, as a pair of fp16 numbers (mlp_pairs.h; takes_pairs).  Up to there, in
 // hbt_mlp_forward_fp32 and for networks whose weights are not for that (check_kernel),
 // they run on the fp32 ones (below), with
 // v_mfma_f32_32x32x2_f32: the A operand is a 32(n) x 2(k) weight fragment, the B
@@ -27,6 +28,7 @@
 
 #include "../../include/habitat_mi.h"
 #include "mlp_chain.h"
+#include "mlp_pairs.h"
 #include "mlp_split.h"
 #include "wave_scale.h"
 
@@ -819,6 +821,7 @@ __global__ __launch_bounds__(256) void mlp_last_km_kernel(const LastArgs a) {
 constexpr size_t kOneOutOffset = 512;   // hbt_mlp_predict_one's result within its staging block
 constexpr size_t kOneDoneOffset = 768;  // and the call number the last kernel publishes after it
 constexpr size_t kOneOutsideOffset = 896;  // and what hbt_mlp_create's check_kernel leaves
+constexpr size_t kOneOutsidePairsOffset = kOneOutsideOffset + 4;  // and its prepare kernels
 constexpr size_t kOneBytes = 1024;
 static_assert(kMaxInPadded * sizeof(double) <= kOneOutOffset, "a raw row fits below the result");
 
@@ -846,6 +849,15 @@ struct hbt_mlp {
   float b_last;
   const char* w_split; // the hidden layers' weights in bf16 pieces, kSplitLayerBytes each
   bool takes_pieces;   // whether they fit, and there are any
+  // the same as fp16 pairs (mlp_pairs.h): weights, kPairsLayerBytes each, and the exponents
+  // of the units' scales, F [hidden][kWidth] and G [hidden + 1][kWidth]
+  const char* w_pairs;
+  const int32_t* F;
+  const int32_t* G;
+  const int32_t* bias_most; // [hidden + 1]
+  bool takes_pairs;
+  int32_t* row_scales[2];   // of a layer's rows and of the next one's: [chunk_rows]
+  int32_t* row_most[2];     // [kWidth / 32][chunk_rows]
   int64_t chunk_rows;  // rows the split path takes at a time
   // the words of chain::Args of hbt_mlp_forward and hbt_mlp_predict_one, and of
   // hbt_mlp_forward_static; the counter of tickets comes first, in a block of its own
@@ -1088,6 +1100,7 @@ int forward_fused(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
 
 // The split path's hidden layers (mlp_split.h).
 namespace split = hbt::split;
+namespace pairs = hbt::pairs;
 using hbt::kWidth;
 constexpr size_t kSplitLayerBytes = (size_t)(kWidth / 32) * split::kTileBytes;
 
@@ -1158,28 +1171,31 @@ void split_launch(const split::LayerArgs& a, bool last, hipStream_t stream) {
 //
 // Where mid_kernel and the 4 x 3 and 4 x 4 tiles are within 2 %, it is taken for its
 // second set of sums (errors of 0.8 and 1.2 in 2^-24 of a layer's output).
-using SplitLaunch = void (*)(const split::LayerArgs&, bool, hipStream_t);
-SplitLaunch split_kernel_for(int m_tiles, int compute_units) {
-  SplitLaunch best = nullptr;
+struct SplitKernel {
+  void (*launch)(const split::LayerArgs&, bool, hipStream_t);
+  bool nearest;   // its sums are the nearest to exact ones (1.3 in 2^-24 of a layer's output)
+};
+SplitKernel split_kernel_for(int m_tiles, int compute_units) {
+  SplitKernel best{};
   float best_us = 0.f;
-  const auto consider = [&](auto kernel, float start, float round_us) {
+  const auto consider = [&](auto kernel, float start, float round_us, bool nearest) {
     using C = decltype(kernel);
     const int per_round = C::S::BM * (compute_units / C::S::NBLK > 0 ? compute_units / C::S::NBLK : 1);
     const float us = start + round_us * (float)((m_tiles + per_round - 1) / per_round);
-    if (best == nullptr || us < best_us) {
-      best = split_launch<C>;
+    if (best.launch == nullptr || us < best_us) {
+      best = {split_launch<C>, nearest};
       best_us = us;
     }
   };
-  consider(SplitSmall1x1(), 2.7f, 4.05f);   // rounds of 256 rows
-  consider(SplitSmall1x2(), 2.f, 6.9f);     // 512
-  consider(SplitSmall2x2(), 3.5f, 10.f);    // 1024
-  consider(SplitSmall2x3(), 2.5f, 13.5f);   // 1536
-  consider(SplitSmall2x4(), 4.f, 18.f);     // 2048
-  consider(SplitSmall4x3(), 4.f, 24.5f);    // 3072
-  consider(SplitSmall4x4(), 3.f, 32.f);     // 4096
-  consider(SplitMid192(), 6.f, 44.f);       // 6144
-  consider(SplitLarge(), 0.f, 122.f);       // 16 384
+  consider(SplitSmall1x1(), 2.7f, 4.05f, true);   // rounds of 256 rows
+  consider(SplitSmall1x2(), 2.f, 6.9f, true);     // 512
+  consider(SplitSmall2x2(), 3.5f, 10.f, true);    // 1024
+  consider(SplitSmall2x3(), 2.5f, 13.5f, true);   // 1536
+  consider(SplitSmall2x4(), 4.f, 18.f, true);     // 2048
+  consider(SplitSmall4x3(), 4.f, 24.5f, false);   // 3072
+  consider(SplitSmall4x4(), 3.f, 32.f, false);    // 4096
+  consider(SplitMid192(), 6.f, 44.f, false);      // 6144
+  consider(SplitLarge(), 0.f, 122.f, false);      // 16 384
   return best;
 }
 
@@ -1202,7 +1218,7 @@ int forward_split(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
     hipLaunchKernelGGL(split::first_kernel<kFirstFmaMaxIn>, first_grid, dim3(256), 0, stream, f);
   else
     hipLaunchKernelGGL(split::first_kernel<kMaxInPadded>, first_grid, dim3(256), 0, stream, f);
-  const SplitLaunch launch = split_kernel_for(m_tiles, mlp->compute_units);
+  const SplitKernel kernel = split_kernel_for(m_tiles, mlp->compute_units);
   split::LayerArgs l{};
   l.w_last = mlp->w_last;
   l.part = part;
@@ -1213,7 +1229,7 @@ int forward_split(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
     l.x = buffers[layer & 1];
     l.y = buffers[(layer + 1) & 1];
     const bool last = layer + 1 == mlp->hidden;
-    launch(l, last, stream);
+    kernel.launch(l, last, stream);
   }
   split::FinishArgs z{};
   z.part = part;
@@ -1223,6 +1239,117 @@ int forward_split(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
   z.out = out;
   hipLaunchKernelGGL(split::finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, z);
   return hipGetLastError() == hipSuccess ? HBT_OK : HBT_EHIP;
+}
+
+// The pairs' hidden layers (mlp_pairs.h).
+constexpr size_t kPairsLayerBytes = (size_t)(kWidth / 32) * pairs::kTileBytes;
+
+template <int TN, int TM, int KS, int NBUF, int RING, int XB, int FLUSH, int SPLIT>
+struct PairsWide {
+  using S = pairs::Wide<TN, TM, KS, NBUF, RING, XB, FLUSH, SPLIT>;
+  static constexpr auto kHidden = &pairs::wide_kernel<TN, TM, KS, NBUF, RING, XB, FLUSH, SPLIT, false>;
+  static constexpr auto kLast = &pairs::wide_kernel<TN, TM, KS, NBUF, RING, XB, FLUSH, SPLIT, true>;
+};
+using PairsWide1x2 = PairsWide<1, 2, 4, 3, 4, 2, 8, 0>;
+using PairsWide1x3 = PairsWide<1, 3, 8, 2, 4, 2, 8, 0>;
+using PairsWide2x4 = PairsWide<2, 4, 4, 3, 2, 2, 64, 24>;
+
+template <class C>
+void pairs_launch(const pairs::LayerArgs& a, bool last, hipStream_t stream) {
+  const int m_blocks = (a.m_tiles + C::S::BM - 1) / C::S::BM;
+  const dim3 grid((unsigned)((m_blocks + C::S::XM - 1) / C::S::XM * C::S::XM * C::S::NBLK));
+  hipLaunchKernelGGL(last ? C::kLast : C::kHidden, grid, dim3(C::S::THREADS), C::S::LDS, stream,
+                     a);
+}
+
+// The kernel for a layer of m_tiles m-tiles, as split_kernel_for: in rounds of one
+// workgroup per compute unit, the one whose rounds cost least, microseconds on 256 compute
+// units.  Whole forwards of ten layers, us, in turn on one card:
+//
+//    rows   1x2   1x3   2x4   (three bf16 pieces)
+//    4096   222   244   492    326
+//    5911   362   293   499    482
+//    8192   389   471   540    653
+//   12288   630   579   567    962
+//   16384   814   803   686   1196
+//
+// At 9217 to 12 288 rows 2 x 4 tiles are 2 % faster than 1 x 3; the sums of these are nearer.
+struct PairsKernel {
+  void (*launch)(const pairs::LayerArgs&, bool, hipStream_t);
+  int parts;   // in which a layer leaves the rows' largest outputs
+};
+PairsKernel pairs_kernel_for(int m_tiles, int compute_units) {
+  PairsKernel best{};
+  float best_us = 0.f;
+  const auto consider = [&](auto kernel, float start, float round_us) {
+    using C = decltype(kernel);
+    const int per_round = C::S::BM * (compute_units / C::S::NBLK > 0 ? compute_units / C::S::NBLK : 1);
+    const float us = start + round_us * (float)((m_tiles + per_round - 1) / per_round);
+    if (best.launch == nullptr || us < best_us) {
+      best = {pairs_launch<C>, C::S::PARTS};
+      best_us = us;
+    }
+  };
+  consider(PairsWide1x2(), 1.5f, 22.5f);   // rounds of 4096 rows
+  consider(PairsWide1x3(), 0.5f, 32.5f);   // 6144
+  consider(PairsWide2x4(), 0.f, 81.f);     // 16 384
+  return best;
+}
+
+// The same with pairs, through the handle's scratch.
+int forward_pairs(hbt_mlp* mlp, const double* raw_features, int64_t n, float* out,
+                  hipStream_t stream) {
+  using namespace hbt;
+  const int m_tiles = (int)((n + kRows - 1) / kRows);
+  char* const buffers[2] = {reinterpret_cast<char*>(mlp->scratch[0]),
+                            reinterpret_cast<char*>(mlp->scratch[1])};
+  pairs::FirstArgs f{};
+  f.raw = raw_features; f.mu = mlp->mu; f.sigma = mlp->sigma;
+  f.w_t = mlp->w_first_t;
+  f.units = {mlp->bias, nullptr, mlp->G, mlp->bias_most};
+  f.in_features = mlp->in_features; f.n = n;
+  f.y = buffers[0]; f.e_out = mlp->row_scales[0]; f.most_out = mlp->row_most[0];
+  const dim3 first_grid((unsigned)m_tiles, split::kFirstSlices);
+  if (mlp->in_features <= kFirstFmaMaxIn)
+    hipLaunchKernelGGL(pairs::first_kernel<kFirstFmaMaxIn>, first_grid, dim3(256), 0, stream, f);
+  else
+    hipLaunchKernelGGL(pairs::first_kernel<kMaxInPadded>, first_grid, dim3(256), 0, stream, f);
+  const PairsKernel kernel = pairs_kernel_for(m_tiles, mlp->compute_units);
+  pairs::LayerArgs l{};
+  l.w_last = mlp->w_last;
+  l.part = mlp->part;
+  l.m_tiles = m_tiles;
+  l.most_count = pairs::kFirstParts;
+  for (int layer = 0; layer < mlp->hidden; ++layer) {
+    const int in = layer & 1, to = in ^ 1;
+    l.w = mlp->w_pairs + (size_t)layer * kPairsLayerBytes;
+    l.units = {mlp->bias + (size_t)(layer + 1) * kWidth, mlp->F + (size_t)layer * kWidth,
+               mlp->G + (size_t)(layer + 1) * kWidth, mlp->bias_most + layer + 1};
+    l.x = buffers[in]; l.e_in = mlp->row_scales[in]; l.most_in = mlp->row_most[in];
+    l.y = buffers[to]; l.e_out = mlp->row_scales[to]; l.most_out = mlp->row_most[to];
+    kernel.launch(l, layer + 1 == mlp->hidden, stream);
+    l.most_count = kernel.parts;
+  }
+  split::FinishArgs z{};
+  z.part = mlp->part;
+  z.rows_pad = m_tiles * kRows;
+  z.b_last = mlp->b_last;
+  z.n = n;
+  z.out = out;
+  hipLaunchKernelGGL(split::finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, z);
+  return hipGetLastError() == hipSuccess ? HBT_OK : HBT_EHIP;
+}
+
+// Whether a batch goes through pairs: from 2049 rows on they are faster everywhere (3072
+// rows 264 -> 190 us, 5911 488 -> 293, 16 384 1196 -> 686), and nearer to fp64 except where
+// the pieces are multiplied with two sets of sums and K over the waves (on 256 compute units
+// up to 2048 rows, at 4097 to 4608 and 9217 to 10 240): predictions of four networks, 2-norm
+// of the error over that of the result, pairs 6.5e-8 to 12 288 rows and 1.26e-7 above, these
+// pieces 5.0e-8, the other kernels of pieces 1.13e-7 (4 x 3 and 4 x 4 tiles), 6.8e-8
+// (mid_kernel) and 1.41e-7 (large_kernel).
+bool takes_pairs(const hbt_mlp* mlp, int64_t n) {
+  const int m_tiles = (int)((n + hbt::kRows - 1) / hbt::kRows);
+  return mlp->takes_pairs && !split_kernel_for(m_tiles, mlp->compute_units).nearest;
 }
 
 // Any number of rows on the fp32 matrix cores.  The fused kernel keeps every
@@ -1318,12 +1445,20 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
   const size_t first_t_rows = in_features <= kFirstFmaMaxIn ? kFirstFmaMaxIn : kMaxInPadded;
   const size_t off_first_t = off;
   off = align_up(off + sizeof(float) * first_t_rows * kWidth, 256);
+  const size_t off_bias_most = off; off = align_up(off + sizeof(int32_t) * (hidden_layers + 1), 256);
   const size_t image = off;  // what is copied from the host; scratch follows
   const int64_t chunk_rows = kSplitRowsPerUnit * compute_units;
   size_t scratch_bytes = (size_t)(chunk_rows / kRows) * split::kTileBytes;
   const size_t layer_bytes = sizeof(float) * (size_t)kLayerMaxRows * kWidth;  // forward_layers
   if (scratch_bytes < layer_bytes) scratch_bytes = layer_bytes;
   const size_t off_split = off; off = align_up(off + (size_t)hidden_layers * kSplitLayerBytes, 256);
+  const size_t off_pairs = off; off = align_up(off + (size_t)hidden_layers * kPairsLayerBytes, 256);
+  const size_t unit_ints = (size_t)(hidden_layers + 1) * kWidth;
+  const size_t off_F = off; off += sizeof(int32_t) * unit_ints;
+  const size_t off_G = off; off += sizeof(int32_t) * unit_ints;
+  const size_t off_sizes = off; off = align_up(off + sizeof(float) * unit_ints, 256);
+  const size_t off_row_scales = off;
+  off = align_up(off + sizeof(int32_t) * 2 * (1 + kWidth / 32) * (size_t)chunk_rows, 256);
   const size_t off_scratch0 = off; off = align_up(off + scratch_bytes, 256);
   const size_t off_scratch1 = off; off = align_up(off + scratch_bytes, 256);
   const size_t off_part = off;
@@ -1356,6 +1491,9 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
     for (int k = 0; k < in_features; ++k)
       first_t[(size_t)k * kWidth + n] = W[0][(size_t)n * in_features + k];
 
+  for (int l = 0; l <= hidden_layers; ++l)
+    reinterpret_cast<int32_t*>(host.data() + off_bias_most)[l] = -pairs::kNotFinite;
+
   void* blob = nullptr;
   if (hipMalloc(&blob, total) != hipSuccess) {
     (void)hipGetLastError();
@@ -1372,7 +1510,7 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
                           hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)kLdsBytes) != hipSuccess ||
       !split_ready<SplitSmall1x1, SplitSmall1x2, SplitSmall2x2, SplitSmall2x3, SplitSmall2x4,
-                   SplitSmall4x3, SplitSmall4x4, SplitMid192, SplitLarge>()) {
+                   SplitSmall4x3, SplitSmall4x4, SplitMid192, SplitLarge, PairsWide1x2, PairsWide1x3, PairsWide2x4>()) {
     (void)hipGetLastError();
     (void)hipFree(blob);
     *err = HBT_EHIP;
@@ -1416,6 +1554,40 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
                                             kOneOutsideOffset);
     hipLaunchKernelGGL(split::check_kernel, dim3(kWidth / 32, (unsigned)hidden_layers), dim3(64), 0,
                        nullptr, a);
+    // and as fp16 pairs, after the sizes of the units, a layer after the other
+    unsigned char* const base = static_cast<unsigned char*>(blob);
+    pairs::PrepareArgs p{};
+    p.w_stream = a.w_stream;
+    p.groups_total = a.groups_total;
+    p.w_first_t = reinterpret_cast<const float*>(base + off_first_t);
+    p.in_features = in_features;
+    p.bias = reinterpret_cast<const float*>(base + off_bias);
+    p.G = reinterpret_cast<int32_t*>(base + off_G);
+    p.bias_most = reinterpret_cast<int32_t*>(base + off_bias_most);
+    p.size = reinterpret_cast<float*>(base + off_sizes);
+    p.outside = reinterpret_cast<uint32_t*>(static_cast<unsigned char*>(one_device) +
+                                            kOneOutsidePairsOffset);
+    hipLaunchKernelGGL(pairs::prepare_first, dim3(kWidth / 256), dim3(256), 0, nullptr, p);
+    for (int l = 0; l < hidden_layers; ++l) {
+      p.g0 = in_padded / 8 + l * (kWidth / 8);
+      p.G_in = p.G;
+      p.size_in = p.size;
+      p.F = reinterpret_cast<int32_t*>(base + off_F) + (size_t)l * kWidth;
+      p.G += kWidth;
+      p.size += kWidth;
+      p.bias += kWidth;
+      ++p.bias_most;
+      hipLaunchKernelGGL(pairs::prepare_layer, dim3(kWidth / 32), dim3(1024), 0, nullptr, p);
+      pairs::PackArgs k{};
+      k.w_stream = a.w_stream;
+      k.groups_total = a.groups_total;
+      k.g0 = p.g0;
+      k.G_in = p.G_in;
+      k.F = p.F;
+      k.w = reinterpret_cast<char*>(base) + off_pairs + (size_t)l * kPairsLayerBytes;
+      hipLaunchKernelGGL(pairs::pack_kernel, dim3((kWidth / 32) * split::kSteps / 4), dim3(256), 0,
+                         nullptr, k);
+    }
   }
   if (hipGetLastError() != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
     (void)hipGetLastError();
@@ -1424,8 +1596,8 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
     *err = HBT_EHIP;
     return nullptr;
   }
-  uint32_t outside = 0;
-  std::memcpy(&outside, static_cast<unsigned char*>(one_host) + kOneOutsideOffset, sizeof outside);
+  uint32_t outside[2] = {};
+  std::memcpy(outside, static_cast<unsigned char*>(one_host) + kOneOutsideOffset, sizeof outside);
 
   hbt_mlp* m = new (std::nothrow) hbt_mlp();
   if (m == nullptr) {
@@ -1451,7 +1623,18 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
   m->w_last = reinterpret_cast<const float*>(base + off_last);
   m->w_first_t = reinterpret_cast<const float*>(base + off_first_t);
   m->w_split = reinterpret_cast<const char*>(base + off_split);
-  m->takes_pieces = hidden_layers > 0 && outside == 0;
+  m->takes_pieces = hidden_layers > 0 && outside[0] == 0;
+  m->w_pairs = reinterpret_cast<const char*>(base + off_pairs);
+  m->F = reinterpret_cast<const int32_t*>(base + off_F);
+  m->G = reinterpret_cast<const int32_t*>(base + off_G);
+  m->bias_most = reinterpret_cast<const int32_t*>(base + off_bias_most);
+  m->takes_pairs = m->takes_pieces && outside[1] == 0;
+  for (int i = 0; i < 2; ++i) {
+    int32_t* const rows = reinterpret_cast<int32_t*>(base + off_row_scales) +
+                          (size_t)i * (1 + kWidth / 32) * (size_t)chunk_rows;
+    m->row_scales[i] = rows;
+    m->row_most[i] = rows + chunk_rows;
+  }
   m->chunk_rows = chunk_rows;
   for (int i = 0; i < 2; ++i)
     m->chain[i] = reinterpret_cast<uint64_t*>(base + off_chain + i * chain_bytes);
@@ -1475,9 +1658,10 @@ int hbt_mlp_forward(hbt_mlp* mlp, const double* raw_features, int64_t n, float* 
   while (done < n) {
     const int64_t rows = n - done < mlp->chunk_rows ? n - done : mlp->chunk_rows;
     const double* raw = raw_features + done * mlp->in_features;
-    const int rc = rows > kSplitAboveRows
-                       ? forward_split(mlp, raw, rows, out + done, mlp->scratch, mlp->part, stream)
-                       : forward_fp32(mlp, raw, rows, out + done, stream);
+    const int rc = rows <= kSplitAboveRows ? forward_fp32(mlp, raw, rows, out + done, stream)
+                   : takes_pairs(mlp, rows)
+                       ? forward_pairs(mlp, raw, rows, out + done, stream)
+                       : forward_split(mlp, raw, rows, out + done, mlp->scratch, mlp->part, stream);
     if (rc != HBT_OK) return rc;
     done += rows;
   }

@@ -156,6 +156,9 @@ struct LayerArgs {
 typedef __attribute__((address_space(3))) void lds_void;
 typedef const __attribute__((address_space(1))) void global_void;
 
+// Keeps the compiler from moving a load below the MFMAs it is meant to overlap.
+#define HBT_FENCE __builtin_amdgcn_sched_barrier(0)
+
 // ReLU that hands a NaN on, as torch's does, in one instruction.
 __device__ __forceinline__ float relu_nan(float v) { return __builtin_elementwise_maximum(v, 0.f); }
 
@@ -315,9 +318,6 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void large_kernel(const LayerArgs 
       for (int j = 0; j < TM; ++j)
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p[i], q[j], acc[i][j], 0, 0, 0);
   };
-// keeps the compiler from moving a load below the MFMAs it is meant to overlap
-#define HBT_FENCE __builtin_amdgcn_sched_barrier(0)
-
   fetch(0, 0);
   fetch(1, 1);
   fetch(2, 2);

@@ -1,0 +1,134 @@
+"""GPU: the MLP's hidden layers with every fp32 number as a pair of fp16 numbers
+(habitat_amd/csrc/mlp_pairs.h): scales, and what has no scale."""
+import numpy as np
+import pytest
+import torch
+
+from habitat_amd import synthetic
+from habitat_amd.analysis.mlp.mlp import RuntimePredictor
+from tests.test_mlp_split_gpu import forward_fp64, network
+
+pytestmark = pytest.mark.gpu
+
+# 1 x 2 tiles in one and two rounds, 1 x 3 in one and two, 2 x 4, a second chunk; whole
+# and partial last blocks of each
+ROWS = [2049, 3071, 4096, 4609, 5911, 6144, 6145, 8192, 8193, 10241, 12288, 12289, 13001, 16384,
+        16384 + 2100]
+
+
+def scaled(rp, units, rows):
+    """The same network with everything 2^rows as large, the prediction too, and unit n of
+    every layer 2^units[n] as large, which the next layer's weights undo."""
+    sd = {k: v.clone() for k, v in rp.model.state_dict().items()}
+    out = RuntimePredictor(rp.model_name, rp.layers, 1024)
+    layers = ["fc1"] + ["mlp.layers.%d" % (2 * i) for i in range(rp.layers)] + ["fc2"]
+    by = torch.ldexp(torch.ones(1024), units)
+    for i, name in enumerate(layers):
+        w, b = sd[name + ".weight"], sd[name + ".bias"]
+        if i > 0:
+            w /= by
+        else:
+            w *= 2.0 ** rows
+        if i < len(layers) - 1:
+            w *= by[:, None]
+            b *= by * 2.0 ** rows
+        else:
+            b *= 2.0 ** rows
+    out.model.load_state_dict(sd)
+    out.set_normalization(rp.mu, rp.sigma)
+    return out
+
+
+@pytest.mark.parametrize("rows", ROWS)
+def test_powers_of_two_change_no_bit(rows):
+    rp = network("lstm", 3)
+    x, mu, sigma = synthetic.mlp_features("lstm", rows, seed=rows)
+    rp.set_normalization(mu, sigma)
+    want = rp.predict_batch(x)
+    units = torch.from_numpy(np.random.default_rng(rows).integers(-5, 5, 1024)).to(torch.int32)
+    assert torch.equal(scaled(rp, units, 0).predict_batch(x), want)
+    for size in (40, -40):
+        assert torch.equal(scaled(rp, units, size).predict_batch(x), want * 2.0 ** size)
+
+
+@pytest.mark.parametrize("rows", ROWS)
+def test_rows_of_all_sizes_in_one_batch(rows):
+    """Without biases a row 2^k as large gives 2^k the prediction, bit for bit, beside
+    rows of any other size: every row has a scale of its own."""
+    rp = network("bmm", 2)
+    with torch.no_grad():
+        for name, p in rp.model.named_parameters():
+            if name.endswith("bias"):
+                p.zero_()
+    rp.set_normalization(np.zeros(8), np.ones(8))
+    rng = np.random.default_rng(rows)
+    x = rng.normal(size=(rows, 8)).astype(np.float32).astype(np.float64)
+    size = rng.integers(-60, 60, rows)
+    y = rp.predict_batch(x).cpu().numpy()
+    assert np.array_equal(rp.predict_batch(np.ldexp(x, size[:, None])).cpu().numpy(), np.ldexp(y, size))
+    want = forward_fp64(rp, x)
+    # 8 x 2^-24 of the output's rms for each layer's sum (tests/test_mlp_split_gpu.py)
+    assert np.sqrt(np.mean((y - want) ** 2)) <= \
+        3 * 8 * 2.0 ** -24 * np.sqrt(np.mean(want ** 2))
+
+
+@pytest.mark.parametrize("rows", ROWS)
+def test_whole_numbers_are_exact(rows):
+    """Weights of 11 bits in the first hidden layer and activations of up to 23 in the
+    second, with sums below 2^24 in any order: every number is held and every position wired."""
+    rng = np.random.default_rng(rows)
+    rp = RuntimePredictor("bmm", 2, 1024)
+    last = np.zeros(1024)
+    last[rng.choice(1024, 16, replace=False)] = rng.choice([-1, 1], 16)
+    with torch.no_grad():
+        for p in rp.model.parameters():
+            p.zero_()
+        rp.model.fc1.weight.copy_(torch.from_numpy(rng.choice([-1, 1], (1024, 8))))
+        rp.model.mlp.layers[0].weight.copy_(torch.from_numpy(
+            rng.integers(1, 256, (1024, 1024)) * rng.choice([-1, 1], (1024, 1024)) / 4))
+        rp.model.mlp.layers[2].weight.copy_(torch.from_numpy(rng.choice([-1, 1], (1024, 1024))))
+        rp.model.mlp.layers[0].bias.copy_(torch.from_numpy(rng.integers(-2048, 2048, 1024)))
+        rp.model.fc2.weight.copy_(torch.from_numpy(last)[None])
+    rp.set_normalization(np.zeros(8), np.ones(8))
+    x = rng.integers(-1, 2, (rows, 8)).astype(np.float64)
+    assert np.array_equal(rp.predict_batch(x).double().cpu().numpy(), forward_fp64(rp, x))
+
+
+@pytest.mark.parametrize("rows", [2100, 5000, 13000])
+def test_infinities_and_nan_among_finite_rows(rows):
+    """Where fp32 gives an infinity, zero or NaN for a row, and nothing in the rows beside it."""
+    rp = network("conv2d", 3)
+    x, mu, sigma = synthetic.mlp_features("conv2d", rows, seed=3)
+    rp.set_normalization(mu, sigma)
+    plain = rp.predict_batch(x).cpu().numpy()
+    rng, x = np.random.default_rng(rows), x.copy()
+    at = rng.choice(rows, rows // 10, replace=False)
+    x[at, rng.integers(0, x.shape[1], at.size)] = np.resize(
+        [np.nan, np.inf, -np.inf, 1e300, -1e300], at.size)
+    got, want = rp.predict_batch(x).cpu().numpy(), rp.predict_batch_fp32(x).cpu().numpy()
+    for of in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(of(got), of(want))
+    others = np.setdiff1d(np.arange(rows), at)
+    assert np.array_equal(got[others], plain[others])
+
+
+def test_units_on_few_inputs_are_not_for_pairs():
+    """A unit of which one input makes nearly all: what the pairs would lose of the others
+    shows where that one is off.  The bf16 pieces take the network then, and give the same
+    for its rows whether others with that input on are beside them."""
+    rp = network("linear", 1)
+    with torch.no_grad():
+        for p in rp.model.parameters():
+            p.zero_() if p.dim() == 1 else p.abs_()
+        rp.model.fc1.weight[:, 0] = 0.0
+        rp.model.fc1.weight[7] = 0.0
+        rp.model.fc1.weight[7, 0] = 1.0            # unit 7 is feature 0 alone
+        hidden = rp.model.mlp.layers[0].weight
+        hidden.mul_(2.0 ** -24)
+        hidden[:, 7] = 1.0
+    rp.set_normalization(np.zeros(8), np.ones(8))
+    x = np.abs(np.random.default_rng(1).normal(size=(6000, 8)))
+    x[:, 0] = 0.0
+    want = forward_fp64(rp, x)
+    y = rp.predict_batch(x).double().cpu().numpy()
+    assert np.max(np.abs(y / want - 1)) <= 6 * 2 * 8 * 2.0 ** -24
