@@ -6,8 +6,8 @@
 // sigma in fp64, then cast to fp32.
 //
 // Above kSplitAboveRows rows hbt_mlp_forward's hidden layers run on the 16-bit matrix
-// cores: with every fp32 number in three bf16 pieces (mlp_split.h) or, from some 2000 rows
-// on, as a pair of fp16 numbers (mlp_pairs.h; takes_pairs).  Up to there, in
+// cores: with every fp32 number in three bf16 pieces (mlp_split.h) or, from 1025 rows
+// on, as a pair of fp16 numbers (mlp_pairs.h).  Up to there, in
 // hbt_mlp_forward_fp32 and for networks whose weights are not for that (check_kernel),
 // they run on the fp32 ones (below), with
 // v_mfma_f32_32x32x2_f32: the A operand is a 32(n) x 2(k) weight fragment, the B
@@ -1244,15 +1244,16 @@ int forward_split(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
 // The pairs' hidden layers (mlp_pairs.h).
 constexpr size_t kPairsLayerBytes = (size_t)(kWidth / 32) * pairs::kTileBytes;
 
-template <int TN, int TM, int KS, int NBUF, int RING, int XB, int FLUSH, int SPLIT>
+template <class T, int TN, int TM, int KS, int NBUF, int RING, int XB, int FLUSH, int SPLIT>
 struct PairsWide {
   using S = pairs::Wide<TN, TM, KS, NBUF, RING, XB, FLUSH, SPLIT>;
-  static constexpr auto kHidden = &pairs::wide_kernel<TN, TM, KS, NBUF, RING, XB, FLUSH, SPLIT, false>;
-  static constexpr auto kLast = &pairs::wide_kernel<TN, TM, KS, NBUF, RING, XB, FLUSH, SPLIT, true>;
+  static constexpr auto kHidden = &pairs::wide_kernel<T, TN, TM, KS, NBUF, RING, XB, FLUSH, SPLIT, false>;
+  static constexpr auto kLast = &pairs::wide_kernel<T, TN, TM, KS, NBUF, RING, XB, FLUSH, SPLIT, true>;
 };
-using PairsWide1x2 = PairsWide<1, 2, 4, 3, 4, 2, 8, 0>;
-using PairsWide1x3 = PairsWide<1, 3, 8, 2, 4, 2, 8, 0>;
-using PairsWide2x4 = PairsWide<2, 4, 4, 3, 2, 2, 64, 24>;
+using PairsWide1x1 = PairsWide<double, 1, 1, 4, 3, 4, 2, 4, 0>;
+using PairsWide1x2 = PairsWide<float, 1, 2, 4, 3, 4, 2, 8, 0>;
+using PairsWide1x3 = PairsWide<float, 1, 3, 8, 2, 4, 2, 8, 0>;
+using PairsWide2x4 = PairsWide<float, 2, 4, 4, 3, 2, 2, 64, 24>;
 
 template <class C>
 void pairs_launch(const pairs::LayerArgs& a, bool last, hipStream_t stream) {
@@ -1266,19 +1267,28 @@ void pairs_launch(const pairs::LayerArgs& a, bool last, hipStream_t stream) {
 // workgroup per compute unit, the one whose rounds cost least, microseconds on 256 compute
 // units.  Whole forwards of ten layers, us, in turn on one card:
 //
-//    rows   1x2   1x3   2x4   (three bf16 pieces)
-//    4096   222   244   492    326
-//    5911   362   293   499    482
-//    8192   389   471   540    653
-//   12288   630   579   567    962
-//   16384   814   803   686   1196
+//    rows   1x1   1x2   1x3   2x4   (three bf16 pieces)
+//    1500   144                       155
+//    2048   164   173                 196
+//    4096         222   244   492     326
+//    4500   370                       420
+//    5911         362   293   499     482
+//    8192         389   471   540     653
+//   12288         630   579   567     962
+//   16384         814   803   686    1196
 //
 // At 9217 to 12 288 rows 2 x 4 tiles are 2 % faster than 1 x 3; the sums of these are nearer.
+// 1 x 1 tiles, with totals in double, are for the batches whose bf16 pieces have their
+// nearest sums (split_kernel_for): errors of a prediction (eight networks, 2-norm, relative)
+// 4.8e-8 both; 1 x 2 and 1 x 3 have 5.8e-8 (mid_kernel 6.5e-8, one set of pieces' sums
+// 1.07e-7), 2 x 4 1.17e-7 (large_kernel 1.41e-7).
 struct PairsKernel {
   void (*launch)(const pairs::LayerArgs&, bool, hipStream_t);
   int parts;   // in which a layer leaves the rows' largest outputs
 };
 PairsKernel pairs_kernel_for(int m_tiles, int compute_units) {
+  if (split_kernel_for(m_tiles, compute_units).nearest)
+    return {pairs_launch<PairsWide1x1>, PairsWide1x1::S::PARTS};
   PairsKernel best{};
   float best_us = 0.f;
   const auto consider = [&](auto kernel, float start, float round_us) {
@@ -1340,17 +1350,10 @@ int forward_pairs(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
   return hipGetLastError() == hipSuccess ? HBT_OK : HBT_EHIP;
 }
 
-// Whether a batch goes through pairs: from 2049 rows on they are faster everywhere (3072
-// rows 264 -> 190 us, 5911 488 -> 293, 16 384 1196 -> 686), and nearer to fp64 except where
-// the pieces are multiplied with two sets of sums and K over the waves (on 256 compute units
-// up to 2048 rows, at 4097 to 4608 and 9217 to 10 240): predictions of four networks, 2-norm
-// of the error over that of the result, pairs 6.5e-8 to 12 288 rows and 1.26e-7 above, these
-// pieces 5.0e-8, the other kernels of pieces 1.13e-7 (4 x 3 and 4 x 4 tiles), 6.8e-8
-// (mid_kernel) and 1.41e-7 (large_kernel).
-bool takes_pairs(const hbt_mlp* mlp, int64_t n) {
-  const int m_tiles = (int)((n + hbt::kRows - 1) / hbt::kRows);
-  return mlp->takes_pairs && !split_kernel_for(m_tiles, mlp->compute_units).nearest;
-}
+// Rows up to which the pieces stay: a layer there is a launch's start, loads' latency and
+// the meeting of the sums, and pairs, with half the products and two thirds of the bytes,
+// gain nothing (700 rows: 96 us in the form of split::small_kernel, 99 with pieces).
+constexpr int kPairsAboveRows = 1024;
 
 // Any number of rows on the fp32 matrix cores.  The fused kernel keeps every
 // compute unit busy for whole rounds of 32 rows x compute units (about 0.94 ms
@@ -1510,7 +1513,7 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
                           hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)kLdsBytes) != hipSuccess ||
       !split_ready<SplitSmall1x1, SplitSmall1x2, SplitSmall2x2, SplitSmall2x3, SplitSmall2x4,
-                   SplitSmall4x3, SplitSmall4x4, SplitMid192, SplitLarge, PairsWide1x2, PairsWide1x3, PairsWide2x4>()) {
+                   SplitSmall4x3, SplitSmall4x4, SplitMid192, SplitLarge, PairsWide1x1, PairsWide1x2, PairsWide1x3, PairsWide2x4>()) {
     (void)hipGetLastError();
     (void)hipFree(blob);
     *err = HBT_EHIP;
@@ -1659,7 +1662,7 @@ int hbt_mlp_forward(hbt_mlp* mlp, const double* raw_features, int64_t n, float* 
     const int64_t rows = n - done < mlp->chunk_rows ? n - done : mlp->chunk_rows;
     const double* raw = raw_features + done * mlp->in_features;
     const int rc = rows <= kSplitAboveRows ? forward_fp32(mlp, raw, rows, out + done, stream)
-                   : takes_pairs(mlp, rows)
+                   : rows > kPairsAboveRows && mlp->takes_pairs
                        ? forward_pairs(mlp, raw, rows, out + done, stream)
                        : forward_split(mlp, raw, rows, out + done, mlp->scratch, mlp->part, stream);
     if (rc != HBT_OK) return rc;

@@ -73,26 +73,28 @@ __device__ __forceinline__ void fetch_fragment(const char* tiles, int count, cha
                                            offset, 0, 0);
 }
 
-// Stores a lane's 8 scaled values of a fragment as pairs; `most` is the largest.
-__device__ __forceinline__ void store_pairs(char* out, const float (&v)[8], float most) {
+// Stores a lane's 8 scaled values of a fragment as pairs; `most` is the largest.  rest:
+// what the values have beyond fp32 (nullable).
+__device__ __forceinline__ void store_pairs(char* out, const float (&v)[8], const float* rest,
+                                            float most) {
   using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
   u32x4 first, second;
-  const auto put = [&](const float (&a)[8], const float (&b)[8]) {
+  const auto put = [&](const float (&a)[8], const float* r) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const half2 p = __builtin_convertvector((f32x2){a[2 * j], a[2 * j + 1]}, half2);
-      const half2 q = __builtin_convertvector(
-          (f32x2){fmaf((float)p[0], -1.f, b[2 * j]), fmaf((float)p[1], -1.f, b[2 * j + 1])}, half2);
+      f32x2 q = {v[2 * j] - (float)p[0], v[2 * j + 1] - (float)p[1]};
+      if (r != nullptr) q += (f32x2){r[2 * j], r[2 * j + 1]};
       first[j] = __builtin_bit_cast(uint32_t, p);
-      second[j] = __builtin_bit_cast(uint32_t, q);
+      second[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(q, half2));
     }
   };
-  put(v, v);
+  put(v, rest);
   if (__builtin_expect(!(most < 65504.f), 0)) {  // an infinity or a NaN
     float a[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) a[j] = __builtin_isinf(v[j]) ? 0.f : v[j];
-    put(a, v);
+    put(a, nullptr);
   }
   *reinterpret_cast<u32x4*>(out) = first;
   *reinterpret_cast<u32x4*>(out + kFragBytes) = second;
@@ -137,27 +139,39 @@ struct LayerArgs {
   int32_t m_tiles;
 };
 
-// The exponents of a block's rows, in and out, into LDS.
+// The exponents of a block's rows, in and out, into LDS.  Some lanes to a row, each with its
+// share of the parts, all loads at once: this comes before the first MFMA.
 template <int ROWS, int THREADS, bool LAST>
 __device__ __forceinline__ void row_scales(const LayerArgs& a, int m_tile0, bool store_out,
                                            int (*scales)[2]) {
+  constexpr int kLanes = ROWS <= THREADS / 16 ? 16 : ROWS <= THREADS / 8 ? 8 : 4;
+  constexpr int kLoads = kWidth / 32 / kLanes;
+  static_assert(ROWS * kLanes <= THREADS, "one pass");
   const int rows = a.m_tiles * kRows, bias_most = *a.units.bias_most;
-  for (int r = threadIdx.x; r < ROWS; r += THREADS) {
-    const int row = m_tile0 * kRows + r < rows ? m_tile0 * kRows + r : rows - 1;
-    scales[r][0] = a.e_in[row];
-    if (LAST) continue;
-    int most = -kNotFinite;
-    for (int c = 0; c < a.most_count; c += 8) {
-      int v[8];
+  const int r = threadIdx.x / kLanes, part = threadIdx.x % kLanes;
+  const int row = m_tile0 * kRows + r < rows ? m_tile0 * kRows + r : rows - 1;
+  const int e_in = a.e_in[row];
+  int most = -kNotFinite;
+  if (!LAST) {
+    int v[kLoads];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = a.most_in[(size_t)(c + j) * rows + row];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) most = v[j] > most ? v[j] : most;
+    for (int j = 0; j < kLoads; ++j) {
+      const int p = part + j * kLanes < a.most_count ? part + j * kLanes : 0;
+      v[j] = a.most_in[(size_t)p * rows + row];
     }
-    const int e = row_exponent(most, bias_most);
-    scales[r][1] = e;
-    if (store_out && m_tile0 * kRows + r < rows) a.e_out[row] = e;
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) most = v[j] > most ? v[j] : most;
+#pragma unroll
+    for (int d = 1; d < kLanes; d *= 2) {
+      const int other = __shfl_xor(most, d);
+      most = other > most ? other : most;
+    }
   }
+  if (part != 0 || r >= ROWS) return;
+  const int e = row_exponent(most, bias_most);
+  scales[r][0] = e_in;
+  scales[r][1] = e;
+  if (!LAST && store_out && m_tile0 * kRows + r < rows) a.e_out[row] = e;
 }
 
 // The largest of a row's outputs in part `part` of them.
@@ -168,49 +182,64 @@ __device__ __forceinline__ void put_most(const LayerArgs& a, int part, int m_til
     a.most_out[(size_t)part * (a.m_tiles * kRows) + m_tile * kRows + lane] = exponent_of(most, e_out);
 }
 
-// Outputs of one tile from its sums.  most: the largest of a row's so far.
-template <bool LAST>
-__device__ __forceinline__ void finish_tile(const LayerArgs& a, const f32x16& acc, int n_tile,
-                                            int m_tile, int lane, int e_in, int e_out,
-                                            float& most) {
-  const int m = lane & 31, h = lane >> 5;
-  float v[16];
-  float share = 0.f;
+// A lane's 8 outputs of a k-step of the next layer, registers 8 kk .. 8 kk + 7 of a tile,
+// from their sums.  most: the largest of a row's so far; share (LAST): of the final dot
+// product.  Sums in double leave the pair one rounding, not an fp32 number's and its own.
+template <bool LAST, class T>
+__device__ __forceinline__ void finish_half(const LayerArgs& a, const T (&sums)[8], int n_tile, int kk,
+                                            int m_tile, int lane, int e_in, int e_out, float& most,
+                                            float& share) {
+  const int h = lane >> 5;
+  float v[8], rest[8], largest = 0.f;
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const int n = n_tile * 32 + 8 * g + 4 * h;
+  for (int g = 0; g < 2; ++g) {
+    const int n = n_tile * 32 + 16 * kk + 8 * g + 4 * h;
     const f32x4 b = *reinterpret_cast<const f32x4*>(a.units.bias + n);
     const i32x4 F = *reinterpret_cast<const i32x4*>(a.units.F + n);
+    const i32x4 G = *reinterpret_cast<const i32x4*>(a.units.G + n);
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      v[4 * g + e] = relu_nan(__builtin_ldexpf(acc[4 * g + e], F[e] - e_in) + b[e]);
+    for (int e = 0; e < 4; ++e) {
+      if constexpr (std::is_same_v<T, double>) {
+        double y = __builtin_ldexp(sums[4 * g + e], F[e] - e_in) + (double)b[e];
+        y = y < 0. ? 0. : y;
+        if (!LAST) y = __builtin_ldexp(y, G[e] + e_out);
+        v[4 * g + e] = (float)y;
+        rest[4 * g + e] = (float)(y - (double)v[4 * g + e]);
+      } else {
+        const float y = relu_nan(__builtin_ldexpf(sums[4 * g + e], F[e] - e_in) + b[e]);
+        v[4 * g + e] = LAST ? y : __builtin_ldexpf(y, G[e] + e_out);
+      }
+    }
     if (LAST) {
       const f32x4 wl = *reinterpret_cast<const f32x4*>(a.w_last + n);
 #pragma unroll
       for (int e = 0; e < 4; ++e) share = fmaf(v[4 * g + e], wl[e], share);
-    } else {
-      const i32x4 G = *reinterpret_cast<const i32x4*>(a.units.G + n);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        v[4 * g + e] = __builtin_ldexpf(v[4 * g + e], G[e] + e_out);
     }
+  }
+  if (LAST) return;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) largest = __builtin_elementwise_maximum(largest, v[e]);
+  store_pairs(a.y + tile_offset(m_tile, 2 * n_tile + kk) + lane * 16, v,
+              std::is_same_v<T, double> ? rest : nullptr, largest);
+  most = __builtin_elementwise_maximum(most, largest);
+}
+
+// Outputs of one tile from its sums.
+template <bool LAST, class T>
+__device__ __forceinline__ void finish_tile(const LayerArgs& a, const T (&sums)[16], int n_tile,
+                                            int m_tile, int lane, int e_in, int e_out,
+                                            float& most) {
+  float share = 0.f;
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+    T half[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) half[e] = sums[8 * kk + e];
+    finish_half<LAST, T>(a, half, n_tile, kk, m_tile, lane, e_in, e_out, most, share);
   }
   if (LAST) {
     share += __shfl_xor(share, 32);
-    if (h == 0) a.part[(size_t)n_tile * (a.m_tiles * kRows) + m_tile * kRows + m] = share;
-  } else {
-    char* out = a.y + tile_offset(m_tile, 2 * n_tile) + lane * 16;
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      float u[8], largest = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        u[e] = v[8 * kk + e];
-        largest = __builtin_elementwise_maximum(largest, u[e]);
-      }
-      store_pairs(out + kk * kStepBytes, u, largest);
-      most = __builtin_elementwise_maximum(most, largest);
-    }
+    if (lane < 32) a.part[(size_t)n_tile * (a.m_tiles * kRows) + m_tile * kRows + lane] = share;
   }
 }
 
@@ -231,14 +260,17 @@ __device__ __forceinline__ void finish_tile(const LayerArgs& a, const f32x16& ac
 // rounding costs half an ulp of what the sum has grown to (errors in 2^-24 of the output's
 // rms, from a model of it that agrees with the matrix core in 94 of 100 sums):
 //   FLUSH < 64: three sets of sums, for TN x TM <= 3.  The small products have one of their
-//     own, the leading ones another that is added to the third every FLUSH k-steps.  With
-//     FLUSH = 8 the error is 2.0 (three bf16 pieces with two sets 2.3, fp32 matrix cores 6.8).
+//     own, the leading ones another that is added to the third, the total, every FLUSH
+//     k-steps.  With FLUSH = 8 the error is 2.0 (three bf16 pieces with two sets 2.3, fp32
+//     matrix cores 6.8).  A total in double (T) and FLUSH = 4 leave little but the pairs'
+//     own error, 1.2.
 //   FLUSH = 64: one set, for 2 x 4 tiles.  The last SPLIT_STEPS k-steps come for their small
 //     products first, while the sum is small, and for their leading ones at the end, two to a
 //     unit of the loop.  With 24 the error is 4.8 (three bf16 pieces in this order 5.2), with
 //     none 6.0 and 2.5 % less time, with all 3.7.
 //
 //   TN x TM  rows of a round  us a layer  PFLOP/s of fp16  three bf16 pieces
+//   1 x 1 double  2048           16-18        0.7            19-24
 //   1 x 2         4096           24            1.1            34
 //   1 x 3         6144           32            1.2            52
 //   2 x 4        16384           81            1.27          143
@@ -259,7 +291,8 @@ struct Wide {
   static_assert(KS % RING == 0 && KS % XB == 0, "the rings turn a whole number of times in a slab");
 };
 
-template <int TN, int TM, int KS, int NBUF, int RING, int XB, int FLUSH, int SPLIT_STEPS, bool LAST>
+template <class T, int TN, int TM, int KS, int NBUF, int RING, int XB, int FLUSH, int SPLIT_STEPS,
+          bool LAST>
 __global__ __launch_bounds__(512, 2) void wide_kernel(const LayerArgs a) {
   using S = Wide<TN, TM, KS, NBUF, RING, XB, FLUSH, SPLIT_STEPS>;
   constexpr bool PARTED = FLUSH < kSteps;   // three sets of sums
@@ -314,16 +347,20 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const LayerArgs a) {
   for (int s = 0; s < RING - 1; ++s) load_w(s, s);
   row_scales<S::BM * kRows, S::THREADS, LAST>(a, m_tile0, n_blk == 0, scales);
 
-  f32x16 sums[PARTED ? 3 : 1][TN][TM];   // leading products', small ones', finished parts'
+  f32x16 sums[PARTED ? 2 : 1][TN][TM];   // leading products', small ones'
+  T total[TN][TM][16];                   // PARTED: finished parts'
   f32x16(&leading)[TN][TM] = sums[0], (&small)[TN][TM] = sums[PARTED ? 1 : 0];
 #pragma unroll
-  for (int t = 0; t < (PARTED ? 3 : 1); ++t)
+  for (int t = 0; t < (PARTED ? 2 : 1); ++t)
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
       for (int j = 0; j < TM; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) sums[t][i][j][r] = 0.f;
+        for (int r = 0; r < 16; ++r) {
+          sums[t][i][j][r] = 0.f;
+          total[i][j][r] = 0;
+        }
 
   half8 x[XB][2][TM];
   auto load_x = [&](half8(&d)[2][TM], int buf, int k) {
@@ -386,7 +423,7 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const LayerArgs a) {
         for (int j = 0; j < TM; ++j)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            sums[2][i][j][r] += leading[i][j][r];
+            total[i][j][r] += (T)leading[i][j][r];
             leading[i][j][r] = 0.f;
           }
     }
@@ -410,11 +447,9 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const LayerArgs a) {
     float most = 0.f;
 #pragma unroll
     for (int i = 0; i < TN; ++i) {
-      f32x16& acc = sums[PARTED ? 2 : 0][i][j];
-      if (PARTED)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[r] += small[i][j][r];
-      finish_tile<LAST>(a, acc, n_tile0 + i, m_tile, lane, e_in, e_out, most);
+      for (int r = 0; r < 16; ++r) total[i][j][r] += (T)small[i][j][r];
+      finish_tile<LAST, T>(a, total[i][j], n_tile0 + i, m_tile, lane, e_in, e_out, most);
     }
     if (!LAST) put_most(a, n_blk * S::WAVES + wave, m_tile, lane, most, e_out);
   }
@@ -617,7 +652,7 @@ __global__ __launch_bounds__(256) void first_kernel(const FirstArgs a) {
         largest = __builtin_elementwise_maximum(largest, v[4 * g + e]);
       }
     }
-    store_pairs(a.y + tile_offset(m_tile, n_base / 16 + s) + lane * 16, v, largest);
+    store_pairs(a.y + tile_offset(m_tile, n_base / 16 + s) + lane * 16, v, nullptr, largest);
     most = __builtin_elementwise_maximum(most, largest);
   }
   most = __builtin_elementwise_maximum(most, __shfl_xor(most, 32));

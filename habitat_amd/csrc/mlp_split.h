@@ -870,18 +870,18 @@ struct FinishArgs {
   float* out;         // [n]
 };
 
-// fc2: the shares of the final dot product that the last hidden layer left,
-// added in n-tile order.
+// fc2: the shares of the final dot product that the last hidden layer left, added in
+// n-tile order, in double: in fp32 these 32 sums were half of a prediction's error.
 __global__ __launch_bounds__(256) void finish_kernel(const FinishArgs a) {
   const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (row >= a.n) return;
   float v[kWidth / 32];
 #pragma unroll
   for (int t = 0; t < kWidth / 32; ++t) v[t] = a.part[(size_t)t * a.rows_pad + row];
-  float sum = 0.f;
+  double sum = a.b_last;
 #pragma unroll
-  for (int t = 0; t < kWidth / 32; ++t) sum += v[t];
-  a.out[row] = sum + a.b_last;
+  for (int t = 0; t < kWidth / 32; ++t) sum += (double)v[t];
+  a.out[row] = (float)sum;
 }
 
 }  // namespace split

@@ -10,9 +10,9 @@ from tests.test_mlp_split_gpu import forward_fp64, network
 
 pytestmark = pytest.mark.gpu
 
-# 1 x 2 tiles in one and two rounds, 1 x 3 in one and two, 2 x 4, a second chunk; whole
-# and partial last blocks of each
-ROWS = [2049, 3071, 4096, 4609, 5911, 6144, 6145, 8192, 8193, 10241, 12288, 12289, 13001, 16384,
+# 1 x 1 tiles in one round and in several, 1 x 2 in one and two, 1 x 3 in one and two, 2 x 4,
+# a second chunk; whole and partial last blocks of each
+ROWS = [1025, 1500, 2048, 4097, 4600, 9217, 10240, 2049, 3071, 4096, 4609, 5911, 6144, 6145, 8192, 8193, 10241, 12288, 12289, 13001, 16384,
         16384 + 2100]
 
 
