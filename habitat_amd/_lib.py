@@ -42,6 +42,15 @@ class KernelRecord(C.Structure):
     ]
 
 
+class RatioKind(C.Structure):
+    """hbt_ratio_kind."""
+    _fields_ = [("pred", C.c_void_p), ("op_row", C.c_void_p), ("run_time_ms", C.c_void_p),
+                ("out_ms", C.c_void_p), ("n_rows", C.c_int32), ("n_ops", C.c_int32)]
+
+
+RATIO_MAX_KINDS = 8   # HBT_RATIO_MAX_KINDS
+
+
 class HabitatLibraryError(RuntimeError):
     def __init__(self, code, what):
         self.code = code
@@ -76,9 +85,12 @@ _SIGNATURES = {
     "hbt_wave_scale_sum": (C.c_int, [_P, C.c_int64] + [_P] * 12 + [C.c_int32, _P, _P, _P]),
     "hbt_wave_scale_sum_ordered": (C.c_int, [_P, C.c_int64] + [_P] * 12 + [C.c_int32, _P, _P, _P,
                                                                             _P]),
+    "hbt_wave_scale_sum_totals": (C.c_int, [_P, C.c_int64] + [_P] * 12 +
+                                  [C.c_int32, _P, _P, C.c_int32, C.c_double, _P, _P, _P, _P]),
     "hbt_roofline_gamma": (C.c_int, [C.POINTER(DeviceSpec), C.POINTER(DeviceSpec), C.c_int64,
                                      _P, _P, _P, _P, _P, _P]),
     "hbt_ratio_scale": (C.c_int, [_P, C.c_int32, C.c_int32, _P, C.c_int32, _P, _P, _P, _P, _P]),
+    "hbt_ratio_scale_kinds": (C.c_int, [C.POINTER(RatioKind), C.c_int32, C.c_int32, _P, _P, _P]),
     "hbt_mlp_create": (_P, [C.c_int32, C.c_int32, C.c_int32, C.POINTER(_P), C.POINTER(_P), _P, _P,
                             C.POINTER(C.c_int)]),
     "hbt_mlp_forward": (C.c_int, [_P, _P, C.c_int64, _P, _P]),

@@ -9,12 +9,11 @@ analysis/run_time.py:50-58, analysis/predictor.py:111-148)
 
 `overhead_p = max(0, ms_p * 1e6 - sum_k t_k)` depends on the origin only, so it
 is computed once on the host.  The per-destination parts run on the GPU: one
-hbt_wave_scale_sum_ordered launch over all kernel records of the trace (scaled
-times are summed per pass on the fly, in the kernels' order, and never written
-out), one MLP launch per
+hbt_wave_scale_sum_totals call over all kernel records of the trace (scaled
+times are summed per pass, in the kernels' order), one MLP forward per
 operation kind over (destinations + origin) x distinct feature rows (a network
 repeats layer shapes: ResNet-50's 53 convolutions have 23 distinct rows), and
-hbt_ratio_scale for the ratio, clamp and sum.
+one hbt_ratio_scale_kinds launch for the ratios, clamps and sums of all kinds.
 """
 import logging
 
@@ -25,7 +24,7 @@ from habitat_amd.analysis import SPECIAL_OPERATIONS
 from habitat_amd.analysis.mlp.devices import get_device_features
 from habitat_amd.analysis.mlp.mlp import predict_for_quotients
 from habitat_amd.analysis.run_time import ms_to_ns
-from habitat_amd.analysis.wave_scaling.batch import DeviceTable, ratio_scale, wave_scale_sum
+from habitat_amd.analysis.wave_scaling.batch import DeviceTable, TotalsCall, ratio_scale_kinds
 
 logger = logging.getLogger(__name__)
 
@@ -169,12 +168,12 @@ class SweepCall:
                 rec = plan._records_for(dests[idxs[0]])
                 table = DeviceTable(P.occupancy_device(plan.origin, plan.mode),
                                     [P.occupancy_device(dests[i], plan.mode) for i in idxs])
-                at = None if whole else torch.tensor(idxs, device=plan.gpu)
+                at = None if whole else torch.tensor(idxs, dtype=torch.int32, device=plan.gpu)
                 # where the scaled times pass through on their way to the ordered sums
                 work = torch.empty((len(idxs), max(rec.n, 1)), dtype=torch.float64,
                                    device=plan.gpu)
-                self.groups.append((rec, table, at, work))
-        self.streams = [torch.cuda.Stream(plan.gpu) for _ in plan.special]   # default priority
+                self.groups.append(TotalsCall(rec, table, plan.segment_start, plan.n_seg, work,
+                                              at, len(dests), plan.const_ms))
         # The MLP input rows of every kind, (destinations + origin) x distinct
         # operation rows: they depend on the plan and the destinations only, so
         # they are laid out here, once, and `launch` just runs the networks.
@@ -190,52 +189,52 @@ class SweepCall:
                     [op_feats.unsqueeze(0).expand(D + 1, U, -1),
                      dev_feats.unsqueeze(1).expand(D + 1, U, 4)], dim=2).reshape((D + 1) * U, -1)
 
+        # The kind with the most rows runs on the caller's stream, so that what decides the
+        # time waits for no other stream, each other kind beside it on one of its own (of
+        # default priority).  The passes' sums come before them: 25 us with the GPU to
+        # themselves; beside a network's launches they are as slow as those (256 devices:
+        # 836 us a sweep and 878, 60: 274 and 314).
+        kinds = sorted(self.rows, key=lambda kind: -self.rows[kind].shape[0])
+        self.kinds = [(kind, torch.cuda.Stream(plan.gpu) if i else None)
+                      for i, kind in enumerate(kinds)]
+        self.streams = [stream for _, stream in self.kinds if stream is not None]
+
     def launch(self):
         plan, D = self.plan, len(self.dests)
         res = TraceSweep()
         res.pass_overhead_ns = plan.pass_overhead_ns
         res.pass_owner = plan.pass_owner
-        # One MLP forward per kind, each on a stream of its own and enqueued
-        # first: a kind with few operations fills a fraction of the GPU, so the
-        # kinds run side by side, and the wave-scaling sums of the main stream
-        # run beside them instead of in front of them.
         main = torch.cuda.current_stream(plan.gpu)
-        preds = {}
-        for (kind, (idxs, pred, op_feats, ms, op_row)), side in zip(plan.special.items(),
-                                                                    self.streams):
-            U = op_feats.shape[0]
+        for side in self.streams:
             side.wait_stream(main)
-            with torch.cuda.stream(side):
-                y = predict_for_quotients(pred, self.rows[kind]).view(D + 1, U)
-            y.record_stream(main)
-            preds[kind] = y
-        total = torch.full((D,), plan.const_ms, dtype=torch.float64, device=plan.gpu)
         if self.groups:
-            if len(self.groups) == 1 and self.groups[0][2] is None:
-                rec, table, _, work = self.groups[0]
-                res.pass_kernel_ns, res.bad_records = wave_scale_sum(
-                    rec, table, n_segments=plan.n_seg, segment_start=plan.segment_start,
-                    workspace=work)
-            else:
-                res.pass_kernel_ns = torch.zeros((D, plan.n_seg), dtype=torch.float64,
-                                                 device=plan.gpu)
-                res.bad_records = torch.zeros((D,), dtype=torch.int32, device=plan.gpu)
-                for rec, table, at, work in self.groups:
-                    sums, bad = wave_scale_sum(rec, table, n_segments=plan.n_seg,
-                                               segment_start=plan.segment_start, workspace=work)
-                    res.pass_kernel_ns[at] = sums
-                    res.bad_records[at] = bad
-            total += res.pass_kernel_ns.sum(dim=1) / 1e6
-            total = torch.where(res.bad_records > 0, torch.full_like(total, float("nan")), total)
+            total = torch.empty((D,), dtype=torch.float64, device=plan.gpu)
+            res.pass_kernel_ns = torch.empty((D, plan.n_seg), dtype=torch.float64, device=plan.gpu)
+            res.bad_records = torch.empty((D,), dtype=torch.int32, device=plan.gpu)
+            for call in self.groups:
+                call(res.pass_kernel_ns, res.bad_records, total, main)
         else:
+            total = torch.full((D,), plan.const_ms, dtype=torch.float64, device=plan.gpu)
             res.pass_kernel_ns = torch.zeros((D, plan.n_seg), dtype=torch.float64, device=plan.gpu)
             res.bad_records = torch.zeros((D,), dtype=torch.int32, device=plan.gpu)
-        res.clamped_ops = torch.zeros((D,), dtype=torch.int32, device=plan.gpu)
+        preds = {}
+        for kind, stream in self.kinds:
+            pred = plan.special[kind][1]
+            if stream is None:
+                y = predict_for_quotients(pred, self.rows[kind])
+            else:
+                with torch.cuda.stream(stream):
+                    y = predict_for_quotients(pred, self.rows[kind])
+                y.record_stream(main)
+            preds[kind] = y.view(D + 1, -1)
         for side in self.streams:
             main.wait_stream(side)
-        for kind, (idxs, pred, op_feats, ms, op_row) in plan.special.items():
-            res.special_ms[kind] = ratio_scale(preds[kind], ms, D, totals=total, op_row=op_row,
-                                               clamped=res.clamped_ops)
+        # what is left once the networks are done: one launch
+        res.special_ms, res.clamped_ops = ratio_scale_kinds(
+            [(kind, preds[kind], ms, op_row)
+             for kind, (idxs, pred, op_feats, ms, op_row) in plan.special.items()],
+            D, total, main)
+        for kind, (idxs, *_) in plan.special.items():
             res.special_owner[kind] = idxs
         res.total_ms = total
         return res

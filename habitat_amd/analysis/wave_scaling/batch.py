@@ -239,6 +239,79 @@ def wave_scale_sum(records, table, segment=None, n_segments=1, stream=None, segm
     return sums, bad
 
 
+class TotalsCall:
+    """hbt_wave_scale_sum_totals for records and destinations that stay the same: what the
+    call is made of is looked over and laid out once.  `rows`: int32 GPU tensor naming each
+    destination's row of the outputs (None: row d)."""
+
+    def __init__(self, records, table, segment_start, n_segments, workspace, rows, n_rows,
+                 constant_ms):
+        if records.device != table.torch_device:
+            raise ValueError("records and device table live on different GPUs")
+        if (segment_start.dtype != torch.int64 or segment_start.shape != (n_segments + 1,)
+                or workspace.dtype != torch.float64
+                or workspace.numel() < len(table) * records.n
+                or (rows is not None and (rows.dtype != torch.int32 or len(rows) != len(table)))
+                or any(t.device != records.device or not t.is_contiguous()
+                       for t in (segment_start, workspace) + (() if rows is None else (rows,)))):
+            raise TypeError("segment_start must be int64 [%d], workspace float64 [%d] and rows "
+                            "int32 [%d], on the records' GPU"
+                            % (n_segments + 1, len(table) * records.n, len(table)))
+        self.shape = (n_rows, n_segments)
+        self._keep = (records, table, segment_start, workspace, rows)
+        self._device = records.device
+        c = records.columns
+        self._args = (
+            table.handle, records.n,
+            _ptr(c["num_blocks"]), _ptr(c["block_size"]), _ptr(c["dynamic_smem"]),
+            _ptr(c["static_smem"]), _ptr(c["regs_per_thread"]), _ptr(records.dest_regs),
+            _ptr(c["run_time_ns"]), _ptr(c["flop_sp_efficiency"]),
+            _ptr(c["dram_read_bytes"]), _ptr(c["dram_write_bytes"]),
+            _ptr(records.has_metrics), _ptr(segment_start), n_segments, _ptr(workspace),
+            _ptr(rows), n_rows, constant_ms)
+
+    def __call__(self, sums, bad, totals, stream):
+        """sums float64 [n_rows, n_segments], bad int32 [n_rows], totals float64 [n_rows]:
+        contiguous GPU tensors; only the rows of this call are written."""
+        if (sums.shape != self.shape or bad.shape != self.shape[:1] or totals.shape != bad.shape
+                or sums.dtype != torch.float64 or bad.dtype != torch.int32
+                or totals.dtype != torch.float64):
+            raise TypeError("sums must be float64 %s, bad int32 and totals float64 of its rows"
+                            % (list(self.shape),))
+        with torch.cuda.device(self._device):
+            rc = _lib.lib().hbt_wave_scale_sum_totals(
+                *self._args, sums.data_ptr(), bad.data_ptr(), totals.data_ptr(),
+                stream.cuda_stream)
+        _lib.check(rc, "hbt_wave_scale_sum_totals")
+
+
+def ratio_scale_kinds(kinds, n_dest, totals, stream):
+    """ratio_scale for several kinds of operation in one launch.  kinds: (name, pred,
+    run_time_ms, op_row) each, as there.  Adds to `totals`; returns ({name: ms [n_dest,
+    n_ops]}, clamped int32 [n_dest])."""
+    clamped = torch.empty((n_dest,), dtype=torch.int32, device=totals.device)
+    array = (_lib.RatioKind * max(len(kinds), 1))()
+    out, keep = {}, []
+    for entry, (name, pred, run_time_ms, op_row) in zip(array, kinds):
+        n_ops = run_time_ms.shape[0]
+        if pred.dtype != torch.float32 or pred.dim() != 2 or pred.shape[0] != n_dest + 1:
+            raise TypeError("pred must be float32 [%d, rows]" % (n_dest + 1))
+        if (run_time_ms.dtype != torch.float64 or op_row.dtype != torch.int32
+                or op_row.shape != (n_ops,)):
+            raise TypeError("run_time_ms must be float64 and op_row int32, both [%d]" % n_ops)
+        pred, run_time_ms, op_row = pred.contiguous(), run_time_ms.contiguous(), op_row.contiguous()
+        out[name] = torch.empty((n_dest, n_ops), dtype=torch.float64, device=pred.device)
+        keep.append((pred, run_time_ms, op_row))
+        entry.pred, entry.op_row = pred.data_ptr(), op_row.data_ptr()
+        entry.run_time_ms, entry.out_ms = run_time_ms.data_ptr(), out[name].data_ptr()
+        entry.n_rows, entry.n_ops = pred.shape[1], n_ops
+    with torch.cuda.device(totals.device):
+        rc = _lib.lib().hbt_ratio_scale_kinds(array, len(kinds), n_dest, totals.data_ptr(),
+                                              clamped.data_ptr(), stream.cuda_stream)
+    _lib.check(rc, "hbt_ratio_scale_kinds")
+    return out, clamped
+
+
 def ratio_scale(pred, run_time_ms, n_dest, totals=None, want_ms=True, stream=None, op_row=None,
                 clamped=None):
     """MLP-predicted operations on a sweep (see hbt_ratio_scale).  pred: float32

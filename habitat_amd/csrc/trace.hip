@@ -18,10 +18,17 @@
 //                        adds them, without atomics: the scaled times pass
 //                        through a caller's workspace and one thread per
 //                        (segment, destination) adds them up.
+//   hbt_wave_scale_sum_totals
+//                        the same with each destination's total, for some rows of a
+//                        sweep's destinations.
 //   hbt_ratio_scale      per destination and MLP-predicted operation:
 //                        run_time_ms * pred_dest / pred_origin, negative -> 0
 //                        (predictor.py:132-148 and :182,218,238,283), the
-//                        per-destination sum of those and the number replaced.
+//                        per-destination sum of those and the number replaced;
+//   hbt_ratio_scale_kinds
+//                        for all kinds of operation in one launch: all that a sweep
+//                        does once its networks are done (five launches of 4 to 11 us
+//                        each before, and the sums' seven).
 //
 // Destinations live in a device-resident table (hbt_device_table) so that one
 // launch covers all of them: blockIdx.y is a group of destinations, and their
@@ -61,6 +68,17 @@ constexpr int kBlock = 256;
 // equal occupancy constants within the group.
 constexpr int kSumGroup = 8;
 
+// Where destination d's results go: row d of the outputs, or the row that `rows` names;
+// -1 where there is no such row.
+struct OutputRows {
+  const int32_t* rows;  // [n_dest], nullable
+  int32_t count;        // of the outputs' rows
+  __device__ int of(int d) const {
+    const int row = rows != nullptr ? rows[d] : d;
+    return row >= 0 && row < count ? row : -1;
+  }
+};
+
 struct SumArgs {
   int64_t n;
   int32_t n_segments;
@@ -82,12 +100,20 @@ struct SumArgs {
   double* work;                // ORDERED: [n_dest][n]
   const DestArgs* dests;
   OriginArgs origin;
+  OutputRows out;              // ORDERED: rows of out_bad
 };
 
 __global__ void fill_zero_kernel(double* sums, int64_t n_sums, int32_t* bad, int32_t n_bad) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n_sums) sums[i] = 0.0;
   if (bad != nullptr && i < n_bad) bad[i] = 0;
+}
+
+__global__ void zero_rows_kernel(int32_t* bad, int32_t n_dest, OutputRows out) {
+  const int d = (int)blockIdx.x * blockDim.x + threadIdx.x;
+  if (d >= n_dest) return;
+  const int row = out.of(d);
+  if (row >= 0) bad[row] = 0;
 }
 
 // One thread per record and group of kSumGroup destinations.  Within a
@@ -149,7 +175,8 @@ __global__ __launch_bounds__(kBlock) void wave_scale_sum_kernel(const SumArgs a)
     double v = ok ? o.t : 0.0;
     if (a.out_bad != nullptr) {
       const unsigned long long bad = __ballot(in_range && o.status != HBT_ST_OK);
-      if (lane == 0 && bad != 0) atomicAdd(a.out_bad + d, (int32_t)__popcll(bad));
+      const int row = ORDERED ? a.out.of(d) : d;
+      if (lane == 0 && bad != 0 && row >= 0) atomicAdd(a.out_bad + row, (int32_t)__popcll(bad));
     }
     if (ORDERED) {
       if (in_range) a.work[(int64_t)d * a.n + i] = v;
@@ -170,27 +197,84 @@ struct OrderedSumArgs {
   int32_t n_segments;
   const double* work;            // [n_dest][n], from wave_scale_sum_kernel<., true>
   const int64_t* segment_start;  // [n_segments + 1]
-  double* out_sum;               // [n_dest][n_segments]
+  double* out_sum;               // [rows][n_segments]
+  OutputRows out;
+  // a sweep's totals: constant_ms + the segments' sums in milliseconds, NaN where a record
+  // was bad
+  double* out_total;             // [rows], nullable
+  const int32_t* out_bad;        // [rows], with out_total
+  double constant_ms;
 };
 
-// One thread per (segment, destination = blockIdx.y): it adds the segment's
-// scaled times one after the other in the records' order, as the reference
-// adds a pass's kernels (run_time.py:50-58).  No floating-point atomics: the
-// sum is the same every time, and the same as a sequential sum of the
-// per-record kernel's times.  (The loads do not depend on the running sum, so
-// they run ahead of the additions.)
+// Sum of `v` over the workgroup, in one order; for thread 0.
+__device__ __forceinline__ double block_sum(double v, double (&part)[kBlock / 64]) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double total = 0.0;
+#pragma unroll
+  for (int w = 0; w < kBlock / 64; ++w) total += part[w];
+  return total;
+}
+
+// One workgroup per destination, a thread per segment: it adds the segment's scaled times
+// one after the other in the records' order, as the reference adds a pass's kernels
+// (run_time.py:50-58).  No floating-point atomics: the sum is the same every time, and the
+// same as a sequential sum of the per-record kernel's times.  Bound by that chain of
+// additions for the longest segment (an optimizer pass is several hundred kernels): the
+// times come through LDS, kStage of them at a time, so that no addition waits for memory
+// (256 destinations of a ResNet-50's records: 21 us with loads of their own, 8 us).
+constexpr int kStage = 2048;
 __global__ __launch_bounds__(kBlock) void segment_sum_ordered_kernel(const OrderedSumArgs a) {
-  const int s = blockIdx.x * kBlock + threadIdx.x;
-  if (s >= a.n_segments) return;
-  // (clamped to the columns: a wrong boundary must not become a stray read)
-  int64_t begin = a.segment_start[s], end = a.segment_start[s + 1];
-  begin = begin < 0 ? 0 : begin;
-  end = end > a.n ? a.n : end;
-  const double* v = a.work + (int64_t)blockIdx.y * a.n;
-  double sum = 0.0;
+  __shared__ double staged[kStage];
+  __shared__ double part[kBlock / 64];
+  __shared__ long long range[2];
+  const int d = blockIdx.x, row = a.out.of(d);
+  if (row < 0) return;
+  const double* v = a.work + (int64_t)d * a.n;
+  double mine = 0.0;
+  for (int s0 = 0; s0 < a.n_segments; s0 += kBlock) {
+    const int s = s0 + (int)threadIdx.x;
+    // (clamped to the columns: a wrong boundary must not become a stray read)
+    int64_t begin = 0, end = 0;
+    if (s < a.n_segments) {
+      begin = a.segment_start[s];
+      end = a.segment_start[s + 1];
+      begin = begin < 0 ? 0 : begin;
+      end = end > a.n ? a.n : end;
+    }
+    if (threadIdx.x == 0) {
+      range[0] = a.n;
+      range[1] = 0;
+    }
+    __syncthreads();
+    if (begin < end) {
+      atomicMin(&range[0], (long long)begin);
+      atomicMax(&range[1], (long long)end);
+    }
+    __syncthreads();
+    const int64_t first = range[0], last = range[1];
+    double sum = 0.0;
+    for (int64_t c = first; c < last; c += kStage) {
+      const int count = (int)(last - c < kStage ? last - c : kStage);
+      __syncthreads();
+      for (int j = threadIdx.x; j < count; j += kBlock) staged[j] = v[c + j];
+      __syncthreads();
+      const int from = (int)(begin > c ? (begin - c < count ? begin - c : count) : 0);
+      const int to = (int)(end > c ? (end - c < count ? end - c : count) : 0);
 #pragma unroll 8
-  for (int64_t j = begin; j < end; ++j) sum += v[j];
-  a.out_sum[(int64_t)blockIdx.y * a.n_segments + s] = sum;
+      for (int j = from; j < to; ++j) sum += staged[j];
+    }
+    if (s < a.n_segments) a.out_sum[(int64_t)row * a.n_segments + s] = sum;
+    mine += sum;
+    __syncthreads();   // range is read above and set again
+  }
+  if (a.out_total == nullptr) return;
+  const double total = block_sum(mine, part);
+  if (threadIdx.x == 0)
+    a.out_total[row] = a.out_bad[row] > 0 ? __builtin_nan("") : a.constant_ms + total / 1e6;
 }
 
 struct GammaArgs {
@@ -220,60 +304,49 @@ __global__ __launch_bounds__(kBlock) void roofline_gamma_kernel(const GammaArgs 
 }
 
 struct RatioArgs {
-  const float* pred;          // [(n_dest + 1)][n_rows]; the last row is the origin
-  const double* run_time_ms;  // [n_ops]
-  const int32_t* op_row;      // [n_ops], nullable: operation o reads column o
-  int32_t n_dest, n_rows, n_ops;
-  double* out_ms;             // [n_dest][n_ops], nullable
+  hbt_ratio_kind kinds[HBT_RATIO_MAX_KINDS];
+  int32_t n_kinds, n_dest;
   double* out_total;          // [n_dest], nullable; added to
-  int32_t* out_clamped;       // [n_dest], nullable; added to
+  int32_t* out_clamped;       // [n_dest], nullable
+  bool add_clamped;           // added to, or written
 };
 
-// blockIdx.x = destination; the block's threads stride over the operations.
-// Operations with equal features share one column of pred.
+// blockIdx.x = destination; the block's threads stride over the operations of one kind
+// after the other.  Operations with equal features share one column of pred.
 __global__ __launch_bounds__(kBlock) void ratio_scale_kernel(const RatioArgs a) {
-  const int d = blockIdx.x;
-  const float* dest = a.pred + (int64_t)d * a.n_rows;
-  const float* orig = a.pred + (int64_t)a.n_dest * a.n_rows;
-  double acc = 0.0;
-  int32_t clamped = 0;
-  for (int o = threadIdx.x; o < a.n_ops; o += kBlock) {
-    const int32_t row = a.op_row != nullptr ? a.op_row[o] : o;
-    double ms = __builtin_nan("");
-    if (row >= 0 && row < a.n_rows) {
-      // predictor.py:182: operation.run_time_ms * pred_dest / pred_orig, in fp64
-      ms = a.run_time_ms[o] * (double)dest[row] / (double)orig[row];
-      if (ms < 0) {   // predictor.py:135-141: warned about and replaced by 0
-        ms = 0.;
-        ++clamped;
-      }
-    }
-    if (a.out_ms != nullptr) a.out_ms[(int64_t)d * a.n_ops + o] = ms;
-    acc += ms;
-  }
-  if (a.out_total == nullptr && a.out_clamped == nullptr) return;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    acc += __shfl_down(acc, off);
-    clamped += __shfl_down(clamped, off);
-  }
   __shared__ double part[kBlock / 64];
-  __shared__ int32_t part_clamped[kBlock / 64];
-  if ((threadIdx.x & 63) == 0) {
-    part[threadIdx.x >> 6] = acc;
-    part_clamped[threadIdx.x >> 6] = clamped;
+  __shared__ int32_t count;
+  const int d = blockIdx.x;
+  if (threadIdx.x == 0) count = 0;
+  __syncthreads();
+  double total = a.out_total != nullptr ? a.out_total[d] : 0.0;
+  for (int k = 0; k < a.n_kinds; ++k) {
+    const hbt_ratio_kind& kind = a.kinds[k];
+    const float* dest = kind.pred + (int64_t)d * kind.n_rows;
+    const float* orig = kind.pred + (int64_t)a.n_dest * kind.n_rows;
+    double acc = 0.0;
+    int32_t clamped = 0;
+    for (int o = threadIdx.x; o < kind.n_ops; o += kBlock) {
+      const int32_t row = kind.op_row != nullptr ? kind.op_row[o] : o;
+      double ms = __builtin_nan("");
+      if (row >= 0 && row < kind.n_rows) {
+        // predictor.py:182: operation.run_time_ms * pred_dest / pred_orig, in fp64
+        ms = kind.run_time_ms[o] * (double)dest[row] / (double)orig[row];
+        if (ms < 0) {   // predictor.py:135-141: warned about and replaced by 0
+          ms = 0.;
+          ++clamped;
+        }
+      }
+      if (kind.out_ms != nullptr) kind.out_ms[(int64_t)d * kind.n_ops + o] = ms;
+      acc += ms;
+    }
+    if (a.out_total != nullptr) total += block_sum(acc, part);
+    if (clamped > 0) atomicAdd(&count, clamped);
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double total = 0.0;
-    int32_t count = 0;
-    for (int w = 0; w < kBlock / 64; ++w) {
-      total += part[w];
-      count += part_clamped[w];
-    }
-    if (a.out_total != nullptr) a.out_total[d] += total;
-    if (a.out_clamped != nullptr) a.out_clamped[d] += count;
-  }
+  if (threadIdx.x != 0) return;
+  if (a.out_total != nullptr) a.out_total[d] = total;
+  if (a.out_clamped != nullptr) a.out_clamped[d] = a.add_clamped ? a.out_clamped[d] + count : count;
 }
 
 }  // namespace
@@ -404,17 +477,20 @@ int hbt_wave_scale_sum(const hbt_device_table* table, int64_t n, const int32_t* 
   return hipGetLastError() == hipSuccess ? HBT_OK : HBT_EHIP;
 }
 
-int hbt_wave_scale_sum_ordered(const hbt_device_table* table, int64_t n, const int32_t* num_blocks,
-                               const int32_t* block_size, const int32_t* dynamic_smem,
-                               const int32_t* static_smem, const int32_t* regs,
-                               const int32_t* dest_regs, const double* run_time_ns,
-                               const double* flop_sp_efficiency, const double* dram_read_bytes,
-                               const double* dram_write_bytes, const uint8_t* has_metrics,
-                               const int64_t* segment_start, int32_t n_segments, double* workspace,
-                               double* out_sum, int32_t* out_bad, void* hip_stream) {
+int hbt_wave_scale_sum_totals(const hbt_device_table* table, int64_t n, const int32_t* num_blocks,
+                              const int32_t* block_size, const int32_t* dynamic_smem,
+                              const int32_t* static_smem, const int32_t* regs,
+                              const int32_t* dest_regs, const double* run_time_ns,
+                              const double* flop_sp_efficiency, const double* dram_read_bytes,
+                              const double* dram_write_bytes, const uint8_t* has_metrics,
+                              const int64_t* segment_start, int32_t n_segments, double* workspace,
+                              const int32_t* out_rows, int32_t n_rows, double constant_ms,
+                              double* out_sum, int32_t* out_bad, double* out_total,
+                              void* hip_stream) {
   using namespace hbt;
   if (table == nullptr || n < 0 || n_segments <= 0 || out_sum == nullptr ||
-      segment_start == nullptr)
+      segment_start == nullptr || n_rows < 0 || (out_total != nullptr && out_bad == nullptr) ||
+      (out_rows == nullptr && n_rows != table->n_dest))
     return HBT_EINVAL;
   if (n > 0 && (!num_blocks || !block_size || !dynamic_smem || !static_smem || !regs ||
                 !run_time_ns || !flop_sp_efficiency || !dram_read_bytes || !dram_write_bytes ||
@@ -430,10 +506,10 @@ int hbt_wave_scale_sum_ordered(const hbt_device_table* table, int64_t n, const i
   }
   if (device != table->device) return HBT_EINVAL;
   hipStream_t stream = static_cast<hipStream_t>(hip_stream);
+  const OutputRows out{out_rows, n_rows};
   if (out_bad != nullptr) {
-    hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((table->n_dest + kBlock - 1) / kBlock)),
-                       dim3(kBlock), 0, stream, static_cast<double*>(nullptr), (int64_t)0, out_bad,
-                       table->n_dest);
+    hipLaunchKernelGGL(zero_rows_kernel, dim3((unsigned)((table->n_dest + kBlock - 1) / kBlock)),
+                       dim3(kBlock), 0, stream, out_bad, table->n_dest, out);
     if (hipGetLastError() != hipSuccess) return HBT_EHIP;
   }
   if (n > 0) {
@@ -447,6 +523,7 @@ int hbt_wave_scale_sum_ordered(const hbt_device_table* table, int64_t n, const i
     a.dram_read_bytes = dram_read_bytes; a.dram_write_bytes = dram_write_bytes;
     a.has_metrics = has_metrics;
     a.out_bad = out_bad;
+    a.out = out;
     a.work = workspace;
     a.dests = table->dests;
     a.origin = table->origin;
@@ -463,10 +540,28 @@ int hbt_wave_scale_sum_ordered(const hbt_device_table* table, int64_t n, const i
   b.work = workspace;
   b.segment_start = segment_start;
   b.out_sum = out_sum;
-  hipLaunchKernelGGL(segment_sum_ordered_kernel,
-                     dim3((unsigned)((n_segments + kBlock - 1) / kBlock), (unsigned)table->n_dest),
-                     dim3(kBlock), 0, stream, b);
+  b.out = out;
+  b.out_total = out_total;
+  b.out_bad = out_bad;
+  b.constant_ms = constant_ms;
+  hipLaunchKernelGGL(segment_sum_ordered_kernel, dim3((unsigned)table->n_dest), dim3(kBlock), 0,
+                     stream, b);
   return hipGetLastError() == hipSuccess ? HBT_OK : HBT_EHIP;
+}
+
+int hbt_wave_scale_sum_ordered(const hbt_device_table* table, int64_t n, const int32_t* num_blocks,
+                               const int32_t* block_size, const int32_t* dynamic_smem,
+                               const int32_t* static_smem, const int32_t* regs,
+                               const int32_t* dest_regs, const double* run_time_ns,
+                               const double* flop_sp_efficiency, const double* dram_read_bytes,
+                               const double* dram_write_bytes, const uint8_t* has_metrics,
+                               const int64_t* segment_start, int32_t n_segments, double* workspace,
+                               double* out_sum, int32_t* out_bad, void* hip_stream) {
+  return hbt_wave_scale_sum_totals(table, n, num_blocks, block_size, dynamic_smem, static_smem, regs,
+                                   dest_regs, run_time_ns, flop_sp_efficiency, dram_read_bytes,
+                                   dram_write_bytes, has_metrics, segment_start, n_segments,
+                                   workspace, nullptr, table != nullptr ? table->n_dest : 0, 0.0,
+                                   out_sum, out_bad, nullptr, hip_stream);
 }
 
 int hbt_roofline_gamma(const hbt_device_spec* origin, const hbt_device_spec* dest, int64_t n,
@@ -511,7 +606,37 @@ int hbt_ratio_scale(const float* pred, int32_t n_dest, int32_t n_rows, const int
       (out_ms == nullptr && out_total == nullptr && out_clamped == nullptr))
     return HBT_EINVAL;
   if (n_rows == 0) return HBT_EINVAL;
-  RatioArgs a{pred, run_time_ms, op_row, n_dest, n_rows, n_ops, out_ms, out_total, out_clamped};
+  RatioArgs a{};
+  a.kinds[0] = {pred, op_row, run_time_ms, out_ms, n_rows, n_ops};
+  a.n_kinds = 1;
+  a.n_dest = n_dest;
+  a.out_total = out_total;
+  a.out_clamped = out_clamped;
+  a.add_clamped = true;
+  hipLaunchKernelGGL(ratio_scale_kernel, dim3((unsigned)n_dest), dim3(kBlock), 0,
+                     static_cast<hipStream_t>(hip_stream), a);
+  return hipGetLastError() == hipSuccess ? HBT_OK : HBT_EHIP;
+}
+
+int hbt_ratio_scale_kinds(const hbt_ratio_kind* kinds, int32_t n_kinds, int32_t n_dest,
+                          double* out_total, int32_t* out_clamped, void* hip_stream) {
+  using namespace hbt;
+  if (n_dest < 0 || n_kinds < 0 || n_kinds > HBT_RATIO_MAX_KINDS || (n_kinds > 0 && !kinds))
+    return HBT_EINVAL;
+  for (int k = 0; k < n_kinds; ++k) {
+    const hbt_ratio_kind& kind = kinds[k];
+    if (kind.n_ops < 0 || kind.n_rows < 0) return HBT_EINVAL;
+    if (kind.n_ops > 0 && (kind.pred == nullptr || kind.run_time_ms == nullptr || kind.n_rows == 0 ||
+                           (kind.op_row == nullptr && kind.n_rows != kind.n_ops)))
+      return HBT_EINVAL;
+  }
+  if (n_dest == 0) return HBT_OK;
+  RatioArgs a{};
+  for (int k = 0; k < n_kinds; ++k) a.kinds[k] = kinds[k];
+  a.n_kinds = n_kinds;
+  a.n_dest = n_dest;
+  a.out_total = out_total;
+  a.out_clamped = out_clamped;
   hipLaunchKernelGGL(ratio_scale_kernel, dim3((unsigned)n_dest), dim3(kBlock), 0,
                      static_cast<hipStream_t>(hip_stream), a);
   return hipGetLastError() == hipSuccess ? HBT_OK : HBT_EHIP;

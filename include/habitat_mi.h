@@ -266,6 +266,25 @@ int hbt_wave_scale_sum_ordered(const hbt_device_table *table, int64_t n, const i
                                double *out_sum, int32_t *out_bad, void *hip_stream);
 
 /*
+ * hbt_wave_scale_sum_ordered for part of a sweep's destinations, and with their totals:
+ * destination d's results go to row out_rows[d] (device, int32 [n_dest]; nullable = row d,
+ * then n_rows must be the table's size) of out_sum [n_rows][n_segments], out_bad [n_rows]
+ * and out_total [n_rows]; a destination whose row is outside [0, n_rows) is left out.
+ * out_total (nullable; with it out_bad is not) = constant_ms + the sum of its segments /
+ * 1e6, or NaN where a record was bad.
+ */
+int hbt_wave_scale_sum_totals(const hbt_device_table *table, int64_t n, const int32_t *num_blocks,
+                              const int32_t *block_size, const int32_t *dynamic_smem,
+                              const int32_t *static_smem, const int32_t *regs,
+                              const int32_t *dest_regs, const double *run_time_ns,
+                              const double *flop_sp_efficiency, const double *dram_read_bytes,
+                              const double *dram_write_bytes, const uint8_t *has_metrics,
+                              const int64_t *segment_start, int32_t n_segments, double *workspace,
+                              const int32_t *out_rows, int32_t n_rows, double constant_ms,
+                              double *out_sum, int32_t *out_bad, double *out_total,
+                              void *hip_stream);
+
+/*
  * The roofline exponent alone, _roofline_gamma
  * (analysis/wave_scaling/roofline.py:68-104) with _ridge_point (:107-108), for n
  * records that all have their three metrics: out_gamma[n] fp64, NaN where the
@@ -293,6 +312,24 @@ int hbt_roofline_gamma(const hbt_device_spec *origin, const hbt_device_spec *des
 int hbt_ratio_scale(const float *pred, int32_t n_dest, int32_t n_rows, const int32_t *op_row,
                     int32_t n_ops, const double *run_time_ms, double *out_ms, double *out_total,
                     int32_t *out_clamped, void *hip_stream);
+
+/*
+ * The same for several kinds of operation at once, each with a network's predictions and
+ * operations of its own: out_total[d] += the kinds' sums, one after the other;
+ * out_clamped[d] = the number of negative values (both nullable).  n_kinds is at most
+ * HBT_RATIO_MAX_KINDS; the array of kinds is host memory.
+ */
+#define HBT_RATIO_MAX_KINDS 8
+typedef struct hbt_ratio_kind {
+  const float *pred;          /* [(n_dest + 1)][n_rows] */
+  const int32_t *op_row;      /* [n_ops], nullable */
+  const double *run_time_ms;  /* [n_ops] */
+  double *out_ms;             /* [n_dest][n_ops], nullable */
+  int32_t n_rows;
+  int32_t n_ops;
+} hbt_ratio_kind;
+int hbt_ratio_scale_kinds(const hbt_ratio_kind *kinds, int32_t n_kinds, int32_t n_dest,
+                          double *out_total, int32_t *out_clamped, void *hip_stream);
 
 /*
  * Per-operation MLP (fc1 -> ReLU -> hidden x (Linear, ReLU) -> fc2), the

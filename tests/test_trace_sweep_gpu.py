@@ -8,7 +8,8 @@ from conftest import oracle_device
 from habitat_amd import Device, DeviceProperties, _lib, synthetic
 from habitat_amd.analysis.mlp.mlp import RuntimePredictor
 from habitat_amd.analysis.predictor import Predictor
-from habitat_amd.analysis.wave_scaling.batch import (DeviceTable, KernelRecords, ratio_scale,
+from habitat_amd.analysis.wave_scaling.batch import (DeviceTable, KernelRecords, TotalsCall,
+                                                     ratio_scale, ratio_scale_kinds,
                                                      wave_scale, wave_scale_sum)
 from oracle import lib as olib
 from oracle import mlp as omlp
@@ -364,3 +365,60 @@ def test_device_table_argument_checks():
     with pytest.raises(_lib.HabitatLibraryError) as e:
         DeviceTable(Device.V100, [Device.T4, bad])
     assert e.value.code == _lib.HBT_ESPEC
+
+
+@pytest.mark.parametrize("n", [1, 255, 2048, 2049, 5000])
+def test_totals_of_some_rows(n):
+    """hbt_wave_scale_sum_totals: segments at the edges of its stages of 2048 records and of
+    256 segments, empty, repeated and out of order; rows of a larger sweep, and none."""
+    rng = np.random.default_rng(n)
+    rec, _ = synthetic.kernel_records(n, Device.V100, seed=n)
+    records = KernelRecords.from_numpy(rec, "cuda:0")
+    dests = [Device.T4, Device.P100, Device.RTX2070]
+    table = DeviceTable(Device.V100, dests)
+    start = np.sort(rng.integers(0, n + 1, 301))
+    start[[0, 300]] = 0, n
+    start[100:103] = start[200]          # a run that goes back, and an empty one
+    start = torch.from_numpy(start).cuda()
+    work = torch.empty((3, n), dtype=torch.float64, device="cuda")
+    want, bad = wave_scale_sum(records, table, n_segments=300, segment_start=start, workspace=work)
+    times = work.cpu().numpy()           # (what the kernel before left to be added)
+    edges = start.cpu().numpy()
+    for d in range(3):
+        for s in range(300):
+            total = 0.0
+            for t in times[d][edges[s]:edges[s + 1]]:
+                total += t
+            assert float(want[d, s]) == total
+    sums = torch.full((5, 300), -1.0, dtype=torch.float64, device="cuda")
+    n_bad = torch.full((5,), -1, dtype=torch.int32, device="cuda")
+    totals = torch.full((5,), -1.0, dtype=torch.float64, device="cuda")
+    rows = torch.tensor([3, 7, 0], dtype=torch.int32, device="cuda")   # P100 has none
+    call = TotalsCall(records, table, start, 300, work, rows, 5, 2.5)
+    for _ in range(2):
+        call(sums, n_bad, totals, torch.cuda.current_stream())
+        for row, d in ((3, 0), (0, 2)):
+            assert torch.equal(sums[row], want[d]) and n_bad[row] == bad[d]
+            expected = float("nan") if int(bad[d]) else 2.5 + float(want[d].sum()) / 1e6
+            assert np.isclose(float(totals[row]), expected, rtol=1e-13, equal_nan=True)
+        for row in (1, 2, 4):
+            assert torch.all(sums[row] == -1) and n_bad[row] == -1 and totals[row] == -1
+
+
+@pytest.mark.parametrize("kinds", [0, 1, 2, 8])
+def test_ratios_of_several_kinds_in_one_launch(kinds):
+    rng = np.random.default_rng(kinds)
+    D = 37
+    parts, totals = [], torch.arange(D, dtype=torch.float64, device="cuda")
+    want_totals, want_clamped = totals.clone(), torch.zeros(D, dtype=torch.int32, device="cuda")
+    want = {}
+    for k in range(kinds):
+        ops, rows = [2, 300, 54, 1, 256, 257, 8, 3][k], [5, 1, 23, 1, 64, 256, 8, 2][k]
+        pred = torch.from_numpy(rng.normal(1.0, 1.0, (D + 1, rows)).astype(np.float32)).cuda()
+        ms = torch.from_numpy(rng.random(ops)).cuda()
+        op_row = torch.from_numpy(rng.integers(0, rows, ops).astype(np.int32)).cuda()
+        parts.append((str(k), pred, ms, op_row))
+        want[str(k)] = ratio_scale(pred, ms, D, totals=want_totals, op_row=op_row, clamped=want_clamped)
+    out, clamped = ratio_scale_kinds(parts, D, totals, torch.cuda.current_stream())
+    assert torch.equal(totals, want_totals) and torch.equal(clamped, want_clamped)
+    assert all(torch.equal(out[k], want[k]) for k in want)
