@@ -133,12 +133,14 @@ class MeasuredKernel:
         a kernel found WITHOUT its metrics is looked at again when raw metrics
         have been added to its metric kernels since."""
         packed = self._packed
-        if packed is not None:
-            if packed[1] or packed[2] == sum(len(k.metrics) for k in self._metrics_kernels):
-                return packed
-        record, has = pack_record(self)
-        self._packed = packed = (record, has,
-                                 sum(len(k.metrics) for k in self._metrics_kernels))
+        if packed is not None and packed[1]:
+            return packed
+        raw = 0
+        for k in self._metrics_kernels:
+            raw += len(k.metrics)
+        if packed is None or packed[2] != raw:
+            record, has = pack_record(self)
+            self._packed = packed = (record, has, raw)
         return packed
 
     def __getattr__(self, name):

@@ -55,10 +55,11 @@ class Trace:
         # is returned as it is and a predicted one refuses; the measured ones
         # that do need predicting go to the GPU together.
         operations = list(self._operations)
-        batch = [i for i, op in enumerate(operations)
-                 if isinstance(op, MeasuredOperation) and op.device.name != dest_device.name]
+        dest_name, batch = dest_device.name, []
         for i, op in enumerate(operations):
-            if not isinstance(op, MeasuredOperation) or op.device.name == dest_device.name:
+            if isinstance(op, MeasuredOperation) and op.device.name != dest_name:
+                batch.append(i)
+            else:
                 operations[i] = op.to_device(dest_device, predictor)
         predicted = predictor.predict_operations([operations[i] for i in batch], dest_device)
         for i, op in zip(batch, predicted):

@@ -132,11 +132,14 @@ class DeferredPredictedKernel(PredictedKernel):
     @property
     def run_time_ns(self):
         pending = self._set
-        if pending.times is None:
+        times = pending.times
+        if times is None:
             pending.flush()
-        if pending.failed is not None and self._index in pending.failed:
-            raise_for_status(pending.failed[self._index])
-        return pending.times[self._index]
+            times = pending.times
+        failed = pending.failed
+        if failed is not None and self._index in failed:
+            raise_for_status(failed[self._index])
+        return times[self._index]
 
 
 class _State(threading.local):
@@ -166,8 +169,9 @@ def _strategy(mode, name, doc, needs_metrics=False):
             pending = _state.pending = PendingSet(origin_device, dest_device, metadata_manager,
                                                   mode)
         kernels = pending.kernels
+        index = len(kernels)
         kernels.append(kernel)
-        return DeferredPredictedKernel(kernel, pending, len(kernels) - 1)
+        return DeferredPredictedKernel(kernel, pending, index)
 
     strategy.__name__ = strategy.__qualname__ = name
     strategy.__doc__ = doc

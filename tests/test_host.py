@@ -513,3 +513,17 @@ def test_a_traces_quotients_are_of_fp32_sums(batches):
         pred.predict_batch(np.zeros((rows, 12)))
         assert pred._gpu.calls[2:] == [("hbt_mlp_forward", rows)]
         assert make is RuntimePredictor or pred.seen == 3
+
+
+def test_device_attributes_are_plain_once_the_table_is_read():
+    """Device.<name> stays the one object of the table, unknown names raise KeyError as
+    before, and no device takes the place of a method."""
+    from habitat_amd.device import _Device
+    table = _Device()
+    first = table.V100
+    assert table.__dict__["V100"] is first and table.V100 is first
+    assert [table.__dict__[n] for n in table.names()] == [getattr(table, n) for n in table.names()]
+    with pytest.raises(KeyError):
+        table.NoSuchDevice
+    with pytest.raises(AttributeError):
+        table.__wrapped__
