@@ -20,7 +20,7 @@ origin -> MI355X-like destination), inputs resident in HBM.  Prints ONE JSON lin
   large         the same kernel at 64 M records (beyond the 256 MB last-level cache);
                 large_16M: at 16 M records
   mlp           the MLP (conv2d, 1 M rows): rows/s, its roofline
-                against the bf16 matrix peak at six products per fp32 product and a torch-CPU fp32 baseline
+                against the 16-bit matrix peak at three products per fp32 product and a torch-CPU fp32 baseline
   scalar_strategy  the reference's one-kernel strategy call through the same kernel
   host_records  the same records as an array of structures in HOST memory, results
                 back in host memory, copies and wait included
@@ -43,9 +43,9 @@ if ROOT not in sys.path:
 HBM_PEAK_GBS = 8000.0          # MI355X HBM3E, published
 MFMA_FP32_PEAK_TFLOPS = 157.3  # MI355X dense fp32 matrix, published
 BYTES_PER_RECORD = 68          # 5 x i32 + 4 x f64 read, f64 + 2 x i32 written
-# Large batches run on the bf16 matrix cores (2516.6 TFLOP/s dense, published) with six
-# products of bf16 pieces per fp32 product: 419 TFLOP/s of fp32 work.
-MFMA_SPLIT_PEAK_TFLOPS = 2516.6 / 6
+# Large batches run on the fp16 matrix cores (2516.6 TFLOP/s dense, published) with three
+# products of fp16 pairs per fp32 product: 839 TFLOP/s of fp32 work.
+MFMA_SPLIT_PEAK_TFLOPS = 2516.6 / 3
 # Measured L2<->fabric bytes per record (rocprofv3 FETCH_SIZE + WRITE_SIZE, scaled
 # on a copy kernel of known size; profiles/wave_scale_kernel_1M_and_64M_records.md):
 # 52.07 read + 17.13 written (the status byte is the 69th).
@@ -171,7 +171,7 @@ def mlp_bench(args):
            "roofline": {"bound": "mfma", "achieved": tflops, "peak": MFMA_SPLIT_PEAK_TFLOPS,
                         "unit": "TFLOP/s", "frac": tflops / MFMA_SPLIT_PEAK_TFLOPS,
                         "fp32_matrix_peak": MFMA_FP32_PEAK_TFLOPS,
-                        "kernel": "split::large_kernel",
+                        "kernel": "pairs::wide_kernel",
                         "launch_ms": m_launch, "flops_per_row": flops_per_row}}
     if not args.no_cpu:
         from oracle import mlp as omlp
@@ -235,7 +235,7 @@ def mlp_bench(args):
                          "against": "oracle/mlp.py forward_fp64 on the first %d rows" % m}
     few["note"] = ("rows_N_us: GPU time of one forward (HIP events); up to 4 rows one launch "
                    "(chain_kernel), above that one per layer over the whole GPU "
-                   "(mlp_layer_kernel up to 128 rows, split:: kernels above); predict_wall_us: wall time of one "
+                   "(mlp_layer_kernel up to 128 rows, split:: kernels to 1024, pairs:: above); predict_wall_us: wall time of one "
                    "RuntimePredictor.predict call, predict_again_wall_us: of one with arguments "
                    "asked before; cpu_rows_1_us: torch CPU fp32, batch 1, as the reference "
                    "predicts")

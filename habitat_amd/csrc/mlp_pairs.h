@@ -252,9 +252,9 @@ __device__ __forceinline__ void finish_tile(const LayerArgs& a, const T (&sums)[
 // of RING k-steps of registers; the activations, which all want, go through LDS by direct
 // loads, KS k-steps at a time (a slab, one barrier), NBUF slabs.  With weights in LDS too,
 // and four or two waves reading each fragment of both, LDS was busy 1280 of a step's 1536
-// cycles of MFMAs (256 x 256 per workgroup: 93 us a layer of 16 384 rows, 86 this way, 81
-// with buffer loads throughout; 128 x 192: 36 and 32 us at 5911 rows).  The direct loads are
-// buffer loads: among global ones the compiler waits for all of the ring at each slab.
+// cycles of MFMAs (whole forwards, 128 x 192 per workgroup: 5911 rows 300 us, 286 this way;
+// 256 x 256: 12 288 rows 594 us, 2 x 4 tiles this way 567).  The direct loads are buffer loads:
+// among global ones the compiler waits for all of the ring at each slab (5911 rows 303 us).
 //
 // Order of the sum.  The matrix core adds eight products and rounds the running sum, and a
 // rounding costs half an ulp of what the sum has grown to (errors in 2^-24 of the output's
@@ -270,7 +270,7 @@ __device__ __forceinline__ void finish_tile(const LayerArgs& a, const T (&sums)[
 //     none 6.0 and 2.5 % less time, with all 3.7.
 //
 //   TN x TM  rows of a round  us a layer  PFLOP/s of fp16  three bf16 pieces
-//   1 x 1 double  2048           16-18        0.7            19-24
+//   1 x 1 double  2048           16-18        0.74           19-24
 //   1 x 2         4096           24            1.1            34
 //   1 x 3         6144           32            1.2            52
 //   2 x 4        16384           81            1.27          143

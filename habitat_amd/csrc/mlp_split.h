@@ -31,6 +31,9 @@
 // fp32 matrix cores 6.7, the six products of each step in turn 7.9, the five
 // small products of all steps before the leading ones 2.4.
 //
+// Batches of 1025 rows and more come here only where the network is not for fp16 pairs
+// (mlp_pairs.h), which take half the products; the ranges named below are such networks'.
+//
 // Included by mlp.hip only.
 #pragma once
 

@@ -359,14 +359,17 @@ hbt_mlp *hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
  * or partial sums in scratch memory that belongs to the handle (allocated by
  * hbt_mlp_create, 13 KiB for each of 64 rows per compute unit: 0.21 GB on 256;
  * longer batches are taken in chunks.  With its weights a handle of eight hidden
- * layers holds 0.29 GB of device memory from the start):
+ * layers holds 0.33 GB of device memory from the start):
  * calls on ONE handle must therefore not overlap, on any streams; different
  * handles are independent.  Results are reproducible for a given n and position
  * of the row; the kernels for different row counts sum in different orders and
  * agree to fp32 rounding.  From 129 rows on the hidden layers' products are formed
- * from bf16 pieces (see hbt_mlp_forward_fp32), unless a hidden weight is infinite,
- * NaN or 2^7 or more in magnitude, or a hidden unit has 1 to 191 nonzero weights:
- * such a network is hbt_mlp_forward_fp32 at any n.
+ * from three bf16 pieces of each number, from 1025 rows on from a pair of fp16 numbers
+ * (see hbt_mlp_forward_fp32); neither if a hidden weight is infinite, NaN or 2^7 or
+ * more in magnitude, or a hidden unit has 1 to 191 nonzero weights: such a network is
+ * hbt_mlp_forward_fp32 at any n.  A network in which a unit is made of few of its inputs
+ * (the sum of its weights times their sizes, squared, is below 256 times the sum of the
+ * squares) or of units beyond 2^120 keeps the bf16 pieces at any n.
  */
 int hbt_mlp_forward(hbt_mlp *mlp, const double *raw_features, int64_t n, float *out,
                     void *hip_stream);
@@ -374,9 +377,12 @@ int hbt_mlp_forward(hbt_mlp *mlp, const double *raw_features, int64_t n, float *
 /*
  * hbt_mlp_forward with fp32 products and sums at any n; their order, and so the
  * last bits, depends on n and on the position of the row.  (hbt_mlp_forward takes
- * batches from 129 rows on in bf16 pieces: faster, sums of some hundred products
- * and more closer to an exact evaluation, other last bits; a single product is held
- * to 2^-23, a weight or activation below 2^-110 to 2^-134.)  For callers that divide
+ * batches from 129 rows on in bf16 pieces or fp16 pairs: faster, sums of some hundred
+ * products and more closer to an exact evaluation, other last bits.  A single product is
+ * held to 2^-23 in pieces and 2^-21 in pairs; a weight or activation below 2^-110 to
+ * 2^-134 in pieces; in pairs a weight to 2^-40 of the largest of its unit, an activation
+ * to 2^-40 of a bound on its row's largest, both relative to their units' sizes.)  For
+ * callers that divide
  * predictions by each other and hold the quotients against earlier ones, as a trace
  * and a device sweep do: where predictions cancel, a quotient shows another order of
  * sums in its fifth digit.  Arguments, limits and scratch as hbt_mlp_forward.

@@ -132,3 +132,51 @@ def test_units_on_few_inputs_are_not_for_pairs():
     want = forward_fp64(rp, x)
     y = rp.predict_batch(x).double().cpu().numpy()
     assert np.max(np.abs(y / want - 1)) <= 6 * 2 * 8 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("features", [1, 16, 17, 60])
+@pytest.mark.parametrize("rows", [1500, 3000, 5000, 13000])
+def test_any_number_of_features(rows, features):
+    """fc1 of 5 to 64 inputs: its two kernels, and the bound on what it makes of them."""
+    from habitat_amd.analysis.mlp.mlp import _OperationMLP, _DeviceMLP
+
+    class Network(_OperationMLP):
+        features = ["f%d" % i for i in range(60)]
+
+    Network.features = Network.features[:features]
+    torch.manual_seed(features)
+    model = Network(2, 1024)
+    with torch.no_grad():
+        for name, p in model.named_parameters():
+            if name.endswith("weight") and not name.startswith("fc2"):
+                p.mul_(6.0 ** 0.5)
+    x = np.random.default_rng(rows).normal(size=(rows, features + 4))
+    x[::7] *= 2.0 ** 30
+    handle = _DeviceMLP(model, np.zeros(features + 4), np.ones(features + 4))
+    y = handle.forward(torch.from_numpy(x).cuda()).double().cpu().numpy()
+    rp = RuntimePredictor("bmm", 2, 1024)
+    rp.model, rp.mu, rp.sigma = model, np.zeros(features + 4), np.ones(features + 4)
+    want = forward_fp64(rp, x)
+    for part in (slice(0, None, 7), np.arange(rows) % 7 != 0):
+        # the bound of tests/test_mlp_split_gpu.py, for rows of each size
+        assert np.sqrt(np.mean((y[part] - want[part]) ** 2)) <= \
+            3 * 8 * 2.0 ** -24 * np.sqrt(np.mean(want[part] ** 2))
+
+
+@pytest.mark.parametrize("rows", [1500, 5911, 16384 + 3000])
+def test_replays_of_a_captured_forward(rows):
+    rp = network("linear", 3)
+    x, mu, sigma = synthetic.mlp_features("linear", rows, seed=4)
+    rp.set_normalization(mu, sigma)
+    raw, out = torch.from_numpy(x).cuda(), torch.empty(rows, device="cuda")
+    want = rp.predict_batch(raw).clone()
+    other = rp.predict_batch(raw * 1.5).clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        rp.predict_batch(raw, out=out)
+    for _ in range(4):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        assert torch.equal(rp.predict_batch(raw * 1.5), other)   # eager work between the replays
