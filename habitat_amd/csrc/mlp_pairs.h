@@ -465,6 +465,11 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const LayerArgs a) {
 // products, and below its largest weights 2^-15 a row loses bits.
 constexpr double kLeastShare = 256.;
 
+// Units whose size is beyond 2^+-kUnitRange are not for pairs: their activations would leave
+// fp32, where layers that make nearly nothing of their inputs follow each other, while
+// their scaled ones do not.
+constexpr int kUnitRange = 100;
+
 struct PrepareArgs {
   const float* w_stream;   // packed fp32 weights (mlp.hip)
   int32_t groups_total;    // k-groups per wave stream
@@ -484,7 +489,7 @@ struct PrepareArgs {
 // Size of a unit: what it is for inputs of their sizes and either sign, and its bias.
 __device__ __forceinline__ void put_size(const PrepareArgs& a, int n, double squares) {
   const double u = sqrt(squares) + fabs((double)a.bias[n]);
-  if (!(u < 0x1p120)) *a.outside = 1;
+  if (u != 0. && !(u >= ldexp(1., -kUnitRange) && u < ldexp(1., kUnitRange))) *a.outside = 1;
   const int e = u > 0. ? __builtin_amdgcn_frexp_exp(u) - 1 : 0;
   a.G[n] = -e;
   a.size[n] = (float)ldexp(u, -e);
@@ -504,14 +509,14 @@ __global__ __launch_bounds__(256) void prepare_first(const PrepareArgs a) {
 
 // One workgroup per n-tile, K over its 16 waves.
 __global__ __launch_bounds__(1024) void prepare_layer(const PrepareArgs a) {
-  __shared__ double sums[3][16][32];
-  __shared__ float largest[16][32];
+  __shared__ double sums[2][16][32];
+  __shared__ double largest[16][32];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, tile = blockIdx.x;
   const int m = lane & 31, h = lane >> 5;
   const f32x4* in = reinterpret_cast<const f32x4*>(a.w_stream) +
                     ((size_t)(tile >> 3) * a.groups_total + a.g0) * (8 * 64) + (tile & 7) * 64 + lane;
-  double s[3] = {0., 0., 0.};
-  float most = 0.f;
+  double s[2] = {0., 0.};
+  double most = 0.;   // (2^-149 of a weight times a unit's 2^-100 is no fp32 number)
 #pragma unroll
   for (int i = 0; i < kWidth / 8 / 16; ++i) {
     const int g = wave * (kWidth / 8 / 16) + i, k = 8 * g + 4 * h;
@@ -522,7 +527,7 @@ __global__ __launch_bounds__(1024) void prepare_layer(const PrepareArgs a) {
       const double x = w * a.size_in[k + e];
       s[0] += fabs(x);
       s[1] += x * x;
-      most = fmaxf(most, (float)fabs(w));
+      most = fmax(most, fabs(w));
     }
   }
 #pragma unroll
@@ -530,19 +535,19 @@ __global__ __launch_bounds__(1024) void prepare_layer(const PrepareArgs a) {
     s[t] += __shfl_xor(s[t], 32);
     sums[t][wave][m] = s[t];
   }
-  largest[wave][m] = fmaxf(most, __shfl_xor(most, 32));
+  largest[wave][m] = fmax(most, __shfl_xor(most, 32));
   __syncthreads();
   if (threadIdx.x >= 32) return;
   double total = 0., squares = 0.;
   for (int w = 0; w < 16; ++w) {
     total += sums[0][w][m];
     squares += sums[1][w][m];
-    most = fmaxf(most, largest[w][m]);
+    most = fmax(most, largest[w][m]);
   }
   // (a weight that is not finite has been found by check_kernel)
-  if (!(total * total >= kLeastShare * squares) || !(most < 0x1p120f)) *a.outside = 1;
+  if (!(total * total >= kLeastShare * squares)) *a.outside = 1;
   const int n = tile * 32 + m;
-  a.F[n] = most > 0.f ? __builtin_amdgcn_frexp_expf(most) - kTop : 0;
+  a.F[n] = most > 0. ? __builtin_amdgcn_frexp_exp(most) - kTop : 0;
   put_size(a, n, squares);
 }
 

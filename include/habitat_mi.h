@@ -369,7 +369,7 @@ hbt_mlp *hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
  * more in magnitude, or a hidden unit has 1 to 191 nonzero weights: such a network is
  * hbt_mlp_forward_fp32 at any n.  A network in which a unit is made of few of its inputs
  * (the sum of its weights times their sizes, squared, is below 256 times the sum of the
- * squares) or of units beyond 2^120 keeps the bf16 pieces at any n.
+ * squares), or with a unit whose size is beyond 2^+-100, keeps the bf16 pieces at any n.
  */
 int hbt_mlp_forward(hbt_mlp *mlp, const double *raw_features, int64_t n, float *out,
                     void *hip_stream);

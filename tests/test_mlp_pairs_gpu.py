@@ -180,3 +180,27 @@ def test_replays_of_a_captured_forward(rows):
         torch.cuda.synchronize()
         assert torch.equal(out, want)
         assert torch.equal(rp.predict_batch(raw * 1.5), other)   # eager work between the replays
+
+
+def layers_of(rp):
+    """(weight, bias) of fc1 and the hidden layers."""
+    names = ["fc1"] + ["mlp.layers.%d" % (2 * i) for i in range(rp.layers)]
+    params = dict(rp.model.named_parameters())
+    return [(params[n + ".weight"], params[n + ".bias"]) for n in names]
+
+
+@pytest.mark.parametrize("rows", [1024, 1025, 3000, 5911, 13000])
+@pytest.mark.parametrize("exponents", [(40, 40), (60, 60), (76, 80), (100, 100), (120, 120)])
+def test_collapsed_layers(rows, exponents):
+    """Two layers that make next to nothing of their inputs, one after the other: the
+    prediction is what the biases after them make, at any number of rows."""
+    rp = network("lstm", 4)
+    with torch.no_grad():
+        for (weight, bias), e in zip(layers_of(rp)[1:], exponents + (0, 0)):
+            weight.mul_(2.0 ** -e)
+            bias.zero_()
+        layers_of(rp)[0][1].zero_()
+        rp.model.fc2.bias.fill_(4.0)
+    x, mu, sigma = synthetic.mlp_features("lstm", rows, seed=rows)
+    rp.set_normalization(mu, sigma)
+    assert np.allclose(rp.predict_batch(x).double().cpu().numpy(), forward_fp64(rp, x), rtol=2.0 ** -22)
