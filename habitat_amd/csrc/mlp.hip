@@ -1586,6 +1586,7 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
       k.groups_total = a.groups_total;
       k.g0 = p.g0;
       k.G_in = p.G_in;
+      k.size_in = p.size_in;
       k.F = p.F;
       k.w = reinterpret_cast<char*>(base) + off_pairs + (size_t)l * kPairsLayerBytes;
       hipLaunchKernelGGL(pairs::pack_kernel, dim3((kWidth / 32) * split::kSteps / 4), dim3(256), 0,

@@ -527,7 +527,8 @@ __global__ __launch_bounds__(1024) void prepare_layer(const PrepareArgs a) {
       const double x = w * a.size_in[k + e];
       s[0] += fabs(x);
       s[1] += x * x;
-      most = fmax(most, fabs(w));
+      // (a unit of size 0 is always 0 or NaN: its weights take no part, and are packed as 0)
+      if (a.size_in[k + e] > 0.f) most = fmax(most, fabs(w));
     }
   }
 #pragma unroll
@@ -557,6 +558,7 @@ struct PackArgs {
   int32_t groups_total;
   int32_t g0;
   const int32_t* G_in;
+  const float* size_in;
   const int32_t* F;
   char* w;
 };
@@ -573,8 +575,9 @@ __global__ __launch_bounds__(256) void pack_kernel(const PackArgs a) {
   for (int g = 0; g < 2; ++g)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float w = in[g * (8 * 64)][e];
-      const float v = ldexpf(w, -a.G_in[16 * step + 8 * g + 4 * (lane >> 5) + e] - F);
+      const int k = 16 * step + 8 * g + 4 * (lane >> 5) + e;
+      const float w = a.size_in[k] > 0.f ? in[g * (8 * 64)][e] : 0.f;
+      const float v = ldexpf(w, -a.G_in[k] - F);
       _Float16 p = (_Float16)v, q = (_Float16)(v - (float)p);
       if (p == (_Float16)0.f && w != 0.f) {  // keeps its sign for an infinite activation
         p = (_Float16)(w > 0.f ? 0x1p-24f : -0x1p-24f);

@@ -204,3 +204,28 @@ def test_collapsed_layers(rows, exponents):
     x, mu, sigma = synthetic.mlp_features("lstm", rows, seed=rows)
     rp.set_normalization(mu, sigma)
     assert np.allclose(rp.predict_batch(x).double().cpu().numpy(), forward_fp64(rp, x), rtol=2.0 ** -22)
+
+
+@pytest.mark.parametrize("rows", [1500, 3000, 5911, 13000])
+@pytest.mark.parametrize("size", [0, -20, -30, -40])
+def test_units_of_zeros_beside_small_ones(rows, size):
+    """Units without weights or bias, as pruning leaves them, beside units of any size: their
+    outgoing weights, which meet nothing but zeros, take no bits of the others'."""
+    rp = network("lstm", 3)
+    with torch.no_grad():
+        for weight, bias in layers_of(rp):
+            bias.mul_(2.0 ** size)
+        layers_of(rp)[0][0].mul_(2.0 ** size)
+        for (weight, bias), unit in zip(layers_of(rp)[:2], (3, 700)):
+            weight[unit], bias[unit] = 0.0, 0.0
+        rp.model.fc2.bias.zero_()
+    x, mu, sigma = synthetic.mlp_features("lstm", rows, seed=rows)
+    rp.set_normalization(mu, sigma)
+    y, want = rp.predict_batch(x).double().cpu().numpy(), forward_fp64(rp, x)
+    rms = np.sqrt(np.mean((want - want.mean()) ** 2)) + abs(want.mean())
+    # the bound of tests/test_mlp_split_gpu.py
+    assert np.sqrt(np.mean((y - want) ** 2)) <= 4 * 8 * 2.0 ** -24 * rms
+    x[::5, 2] = np.nan                        # a unit of zeros hands a NaN on
+    x[1::5, 3] = np.inf
+    got, fp32 = rp.predict_batch(x).cpu().numpy(), rp.predict_batch_fp32(x).cpu().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(fp32)) and np.isnan(got).sum() >= 2 * (rows // 5)
