@@ -202,6 +202,8 @@ __device__ __forceinline__ void finish_half(const LayerArgs& a, const T (&sums)[
       if constexpr (std::is_same_v<T, double>) {
         double y = __builtin_ldexp(sums[4 * g + e], F[e] - e_in) + (double)b[e];
         y = y < 0. ? 0. : y;
+        // what is infinite in fp32 is so here
+        y = (float)y < __builtin_inff() ? y : (double)(float)y;
         if (!LAST) y = __builtin_ldexp(y, G[e] + e_out);
         v[4 * g + e] = (float)y;
         rest[4 * g + e] = (float)(y - (double)v[4 * g + e]);

@@ -94,7 +94,7 @@ def test_whole_numbers_are_exact(rows):
     assert np.array_equal(rp.predict_batch(x).double().cpu().numpy(), forward_fp64(rp, x))
 
 
-@pytest.mark.parametrize("rows", [2100, 5000, 13000])
+@pytest.mark.parametrize("rows", [1500, 2100, 4500, 5000, 10000, 13000])
 def test_infinities_and_nan_among_finite_rows(rows):
     """Where fp32 gives an infinity, zero or NaN for a row, and nothing in the rows beside it."""
     rp = network("conv2d", 3)
@@ -229,3 +229,31 @@ def test_units_of_zeros_beside_small_ones(rows, size):
     x[1::5, 3] = np.inf
     got, fp32 = rp.predict_batch(x).cpu().numpy(), rp.predict_batch_fp32(x).cpu().numpy()
     assert np.array_equal(np.isnan(got), np.isnan(fp32)) and np.isnan(got).sum() >= 2 * (rows // 5)
+
+
+@pytest.mark.parametrize("signs", ["either", "positive"])
+@pytest.mark.parametrize("rows", [1025, 1500, 2048, 2500, 4500, 5911, 10000, 13000])
+def test_sums_beyond_fp32_are_infinite(rows, signs):
+    """A hidden layer's output of 2^128 and more is an infinity, at any number of rows, and
+    does not come back as a number where the next layer's weights are small."""
+    rp = network("bmm", 3)
+    with torch.no_grad():
+        for (weight, bias), e in zip(layers_of(rp), (0, 6, 6, -40)):
+            if signs == "positive":
+                weight.abs_()
+            weight.mul_(2.0 ** e)
+        if signs == "positive":
+            rp.model.fc2.weight.abs_()
+    rp.set_normalization(np.zeros(8), np.ones(8))
+    x = np.abs(np.random.default_rng(rows).normal(size=(rows, 8))) + 0.1
+    plain = rp.predict_batch(x).cpu().numpy()
+    x[::7] *= 2.0 ** (110 if signs == "positive" else 118)
+    h = torch.from_numpy(x[::7]).cuda()
+    with torch.no_grad():
+        for weight, bias in layers_of(rp)[:3]:
+            h = torch.relu(h @ weight.double().cuda().t() + bias.double().cuda())
+    assert bool(((h > 2.0 ** 129).sum(1) > 100).all())      # far beyond, in every such row
+    got = rp.predict_batch(x).cpu().numpy()
+    assert np.all(np.isposinf(got[::7]) if signs == "positive" else np.isnan(got[::7]))
+    others = np.arange(rows) % 7 != 0
+    assert np.array_equal(got[others], plain[others])
