@@ -56,6 +56,10 @@ constexpr int kMaxInPadded = 64;  // in_features padded to a multiple of 32, at 
 // (hbt_mlp_forward_fp32): one workgroup takes 32 rows through the whole
 // network, with the activations in LDS.  Bound by the fp32 matrix cores: a
 // round of 8192 rows takes 0.94 ms, 146 TFLOP/s of 157.
+//
+// FINISH: after the layers of mlp_pairs.h, the sum of a row's shares of the final dot
+// product, and for the rows that are marked what this kernel makes of them.  A workgroup
+// without a marked row is one trip to memory and two rows of 32 threads.
 struct MlpArgs {
   const double* raw;     // [n][in_features]
   float* out;            // [n]
@@ -69,6 +73,9 @@ struct MlpArgs {
   const float* bias;     // [(hidden + 1)][kWidth]: fc1 bias, then hidden biases
   const float* w_last;   // fc2.weight [kWidth]
   float b_last;
+  const float* part;     // FINISH: split::FinishArgs'
+  int32_t rows_pad;
+  const int32_t* redo;   // FINISH: [rows_pad] rows to be taken through the network here
 };
 
 // Fragments travel through a ring of four register slots.  Weight fragments are
@@ -163,7 +170,7 @@ __device__ __forceinline__ void layer_k_loop(Ring<TPW>& r, const WeightStream& s
   }
 }
 
-template <int WAVES>
+template <int WAVES, bool FINISH>
 __global__ __launch_bounds__(WAVES * 64, 1) void mlp_fused_kernel(const MlpArgs a) {
   constexpr int TPW = (kWidth / 32) / WAVES;  // n-tiles per wave
   constexpr int THREADS = WAVES * 64;
@@ -177,6 +184,21 @@ __global__ __launch_bounds__(WAVES * 64, 1) void mlp_fused_kernel(const MlpArgs 
   const int lane = tid & 63, wave = tid >> 6;
   const int m = lane & 31, h = lane >> 5;
   const int64_t row0 = (int64_t)blockIdx.x * kRows;
+
+  bool again = true;   // this thread's row of the tile, of the first 32 threads
+  if (FINISH) {
+    again = false;
+    if (tid < kRows && row0 + tid < a.n) {
+      again = a.redo[row0 + tid] != 0;
+      a.out[row0 + tid] = split::sum_of_shares(a.part, a.rows_pad, row0 + tid, a.b_last);
+    }
+    if (wave == 0) {
+      const bool any = __any(again);
+      if (lane == 0) red[0] = any ? 1.f : 0.f;
+    }
+    __syncthreads();
+    if (red[0] == 0.f) return;
+  }
 
   // ---- stage standardised inputs: act[r][k], zero beyond in_features / n ----
   for (int idx = tid; idx < kRows * a.in_padded; idx += THREADS) {
@@ -269,7 +291,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void mlp_fused_kernel(const MlpArgs 
     }
     red[part * 32 + r] = s;
     __syncthreads();
-    if (tid < 32 && row0 + tid < a.n) {
+    if (tid < 32 && row0 + tid < a.n && again) {
       float total = a.b_last;
 #pragma unroll
       for (int p = 0; p < PARTS; ++p) total += red[p * 32 + tid];
@@ -858,6 +880,7 @@ struct hbt_mlp {
   bool takes_pairs;
   int32_t* row_scales[2];   // of a layer's rows and of the next one's: [chunk_rows]
   int32_t* row_most[2];     // [kWidth / 32][chunk_rows]
+  int32_t* redo;            // [chunk_rows] rows that the pairs do not hold
   int64_t chunk_rows;  // rows the split path takes at a time
   // the words of chain::Args of hbt_mlp_forward and hbt_mlp_predict_one, and of
   // hbt_mlp_forward_static; the counter of tickets comes first, in a block of its own
@@ -1076,11 +1099,8 @@ int forward_layers(hbt_mlp* mlp, const double* raw_features, int64_t n, float* o
 }
 
 // The fused kernel: one workgroup per 32 rows.
-int forward_fused(hbt_mlp* mlp, const double* raw_features, int64_t n, float* out,
-                  hipStream_t stream) {
-  using namespace hbt;
-  const int64_t blocks = (n + kRows - 1) / kRows;
-  MlpArgs a{};
+hbt::MlpArgs fused_args(const hbt_mlp* mlp, const double* raw_features, int64_t n, float* out) {
+  hbt::MlpArgs a{};
   a.raw = raw_features;
   a.out = out;
   a.n = n;
@@ -1093,8 +1113,15 @@ int forward_fused(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
   a.bias = mlp->bias;
   a.w_last = mlp->w_last;
   a.b_last = mlp->b_last;
-  hipLaunchKernelGGL(mlp_fused_kernel<kWaves>, dim3((unsigned)blocks), dim3(kWaves * 64),
-                     kLdsBytes, stream, a);
+  return a;
+}
+
+int forward_fused(hbt_mlp* mlp, const double* raw_features, int64_t n, float* out,
+                  hipStream_t stream) {
+  using namespace hbt;
+  const MlpArgs a = fused_args(mlp, raw_features, n, out);
+  hipLaunchKernelGGL((mlp_fused_kernel<kWaves, false>), dim3((unsigned)((n + kRows - 1) / kRows)),
+                     dim3(kWaves * 64), kLdsBytes, stream, a);
   return hipGetLastError() == hipSuccess ? HBT_OK : HBT_EHIP;
 }
 
@@ -1319,6 +1346,7 @@ int forward_pairs(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
   f.units = {mlp->bias, nullptr, mlp->G, mlp->bias_most};
   f.in_features = mlp->in_features; f.n = n;
   f.y = buffers[0]; f.e_out = mlp->row_scales[0]; f.most_out = mlp->row_most[0];
+  f.redo = mlp->redo;
   const dim3 first_grid((unsigned)m_tiles, split::kFirstSlices);
   if (mlp->in_features <= kFirstFmaMaxIn)
     hipLaunchKernelGGL(pairs::first_kernel<kFirstFmaMaxIn>, first_grid, dim3(256), 0, stream, f);
@@ -1330,6 +1358,7 @@ int forward_pairs(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
   l.part = mlp->part;
   l.m_tiles = m_tiles;
   l.most_count = pairs::kFirstParts;
+  l.redo = mlp->redo;
   for (int layer = 0; layer < mlp->hidden; ++layer) {
     const int in = layer & 1, to = in ^ 1;
     l.w = mlp->w_pairs + (size_t)layer * kPairsLayerBytes;
@@ -1340,13 +1369,12 @@ int forward_pairs(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
     kernel.launch(l, layer + 1 == mlp->hidden, stream);
     l.most_count = kernel.parts;
   }
-  split::FinishArgs z{};
+  MlpArgs z = fused_args(mlp, raw_features, n, out);
   z.part = mlp->part;
   z.rows_pad = m_tiles * kRows;
-  z.b_last = mlp->b_last;
-  z.n = n;
-  z.out = out;
-  hipLaunchKernelGGL(split::finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, z);
+  z.redo = mlp->redo;
+  hipLaunchKernelGGL((mlp_fused_kernel<kWaves, true>), dim3((unsigned)m_tiles), dim3(kWaves * 64),
+                     kLdsBytes, stream, z);
   return hipGetLastError() == hipSuccess ? HBT_OK : HBT_EHIP;
 }
 
@@ -1462,6 +1490,7 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
   const size_t off_sizes = off; off = align_up(off + sizeof(float) * unit_ints, 256);
   const size_t off_row_scales = off;
   off = align_up(off + sizeof(int32_t) * 2 * (1 + kWidth / 32) * (size_t)chunk_rows, 256);
+  const size_t off_redo = off; off = align_up(off + sizeof(int32_t) * (size_t)chunk_rows, 256);
   const size_t off_scratch0 = off; off = align_up(off + scratch_bytes, 256);
   const size_t off_scratch1 = off; off = align_up(off + scratch_bytes, 256);
   const size_t off_part = off;
@@ -1509,7 +1538,10 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
     *err = HBT_EHIP;
     return nullptr;
   }
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&mlp_fused_kernel<kWaves>),
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&mlp_fused_kernel<kWaves, false>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize,
+                          (int)kLdsBytes) != hipSuccess ||
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&mlp_fused_kernel<kWaves, true>),
                           hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)kLdsBytes) != hipSuccess ||
       !split_ready<SplitSmall1x1, SplitSmall1x2, SplitSmall2x2, SplitSmall2x3, SplitSmall2x4,
@@ -1639,6 +1671,7 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
     m->row_scales[i] = rows;
     m->row_most[i] = rows + chunk_rows;
   }
+  m->redo = reinterpret_cast<int32_t*>(base + off_redo);
   m->chunk_rows = chunk_rows;
   for (int i = 0; i < 2; ++i)
     m->chain[i] = reinterpret_cast<uint64_t*>(base + off_chain + i * chain_bytes);

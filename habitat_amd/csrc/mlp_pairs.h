@@ -17,9 +17,13 @@
 //   row m of a batch by 2^e[m], chosen by the kernel that computes a layer, from the
 //     largest of the row's (scaled) inputs and a bound on what the layer makes of it;
 //   row n of a layer's weights by 2^-F[n], its largest weight to [2^14, 2^15).
-// A number below 2^-2 of that scale is held to 2^-25 of it: 2^-40 of the largest weight
-// of its row, 2^-30 or so of the row's activations.  Networks in which a unit hangs on
-// few of its inputs, so that this would show, do not come here (kLeastShare).  An
+// A scaled number below kHeldFrom is held to 2^-25: a weight to 2^-40 of its row's largest,
+// an activation to 2^-40 of the bound on its row's, some 2^-32 of the row's usual ones.
+// Where that is the loss of more than kMostLost numbers of a sum, they are not summed here:
+// a network with such a row of weights, or with a unit that hangs on few of its inputs
+// (kLeastShare), keeps the bf16 pieces; a row of a batch with such activations, as where a
+// few units are 2^10 times the others, is marked while the layers run and goes through the
+// network again on the fp32 matrix cores (mlp_fused_kernel).  An
 // infinite activation is the second number of its pair, so that it meets nothing but
 // the other operand's first number, whose sign is the weight's; a NaN stays one.
 //
@@ -55,6 +59,13 @@ constexpr int kFragBytes = split::kFragBytes;
 constexpr int kStepBytes = 2 * kFragBytes;
 constexpr int kTileBytes = kSteps * kStepBytes;
 constexpr int kTop = 15;  // scaled numbers are below 2^kTop
+// From here on a scaled number is held to 2^-22 of itself, below to 2^-25.
+constexpr float kHeldFrom = 0x1p-3f;
+// Numbers below that in a row of weights or activations.  Of 1024 activations that are of one
+// size 0 to 20 are (networks of eight layers, any gain), and with one unit 2^8, 2^10 and 2^12
+// times the others 46-262, 185-527 and 472-551 (all that are not 0): errors of 4e-7, 6e-7 and
+// 2e-6 where fp32 sums have 1e-6.
+constexpr int kMostLost = 128;
 
 __device__ __forceinline__ size_t tile_offset(int tile, int step) {
   return (size_t)tile * kTileBytes + (size_t)step * kStepBytes;
@@ -129,8 +140,9 @@ struct LayerArgs {
   const char* x;          // activations in, [m_tiles] tiles
   Units units;
   const int32_t* e_in;    // [m_tiles * 32] exponents of the rows' scales
-  const int32_t* most_in; // [most_count][m_tiles * 32] exponent_of a row's largest inputs, by parts
+  const int32_t* most_in; // [most_count][m_tiles * 32] part_of a row's inputs
   int32_t most_count;
+  int32_t* redo;          // [m_tiles * 32] set where the inputs are not held
   char* y;                // not LAST: activations out, and what goes with them
   int32_t* e_out;
   int32_t* most_out;
@@ -138,6 +150,27 @@ struct LayerArgs {
   float* part;            // LAST: [kWidth / 32][m_tiles * 32] shares of the final dot product
   int32_t m_tiles;
 };
+
+// A part of a row's outputs: exponent_of the largest, and how many are below kHeldFrom.
+__device__ __forceinline__ int32_t part_of(int exponent, int lost) { return exponent * 256 + lost; }
+__device__ __forceinline__ int part_exponent(int32_t part) { return part >> 8; }
+__device__ __forceinline__ int part_lost(int32_t part) { return part & 255; }
+__device__ __forceinline__ int32_t both_parts(int32_t a, int32_t b) {
+  return (a > b ? a & -256 : b & -256) + part_lost(a) + part_lost(b);
+}
+__device__ __forceinline__ int is_lost(bool positive, float scaled) { return positive && scaled < kHeldFrom; }
+
+// v of 4, 8 or 16 lanes together (in registers: a step through LDS is 100 cycles, and these
+// come before the first MFMA).
+template <int LANES, class Op>
+__device__ __forceinline__ int over_lanes(int v, Op op) {
+  static_assert(LANES == 4 || LANES == 8 || LANES == 16, "a row of lanes or a part of it");
+  v = op(v, __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true));                    // 1 0 3 2
+  v = op(v, __builtin_amdgcn_mov_dpp(v, 0x4E, 0xf, 0xf, true));                    // 2 3 0 1
+  if (LANES > 4) v = op(v, __builtin_amdgcn_mov_dpp(v, 0x141, 0xf, 0xf, true));    // half mirror
+  if (LANES > 8) v = op(v, __builtin_amdgcn_mov_dpp(v, 0x140, 0xf, 0xf, true));    // mirror
+  return v;
+}
 
 // The exponents of a block's rows, in and out, into LDS.  Some lanes to a row, each with its
 // share of the parts, all loads at once: this comes before the first MFMA.
@@ -151,71 +184,95 @@ __device__ __forceinline__ void row_scales(const LayerArgs& a, int m_tile0, bool
   const int r = threadIdx.x / kLanes, part = threadIdx.x % kLanes;
   const int row = m_tile0 * kRows + r < rows ? m_tile0 * kRows + r : rows - 1;
   const int e_in = a.e_in[row];
-  int most = -kNotFinite;
-  if (!LAST) {
-    int v[kLoads];
+  int32_t v[kLoads];
 #pragma unroll
-    for (int j = 0; j < kLoads; ++j) {
-      const int p = part + j * kLanes < a.most_count ? part + j * kLanes : 0;
-      v[j] = a.most_in[(size_t)p * rows + row];
-    }
-#pragma unroll
-    for (int j = 0; j < kLoads; ++j) most = v[j] > most ? v[j] : most;
-#pragma unroll
-    for (int d = 1; d < kLanes; d *= 2) {
-      const int other = __shfl_xor(most, d);
-      most = other > most ? other : most;
-    }
+  for (int j = 0; j < kLoads; ++j) {
+    const int p = part + j * kLanes;
+    v[j] = a.most_in[(size_t)(p < a.most_count ? p : 0) * rows + row];
   }
+  int most = v[0], lost = 0;
+#pragma unroll
+  for (int j = 0; j < kLoads; ++j) {
+    most = v[j] > most ? v[j] : most;
+    lost += part + j * kLanes < a.most_count ? part_lost(v[j]) : 0;
+  }
+  most = part_exponent(over_lanes<kLanes>(most, [](int x, int y) { return x > y ? x : y; }));
+  lost = over_lanes<kLanes>(lost, [](int x, int y) { return x + y; });
   if (part != 0 || r >= ROWS) return;
   const int e = row_exponent(most, bias_most);
   scales[r][0] = e_in;
   scales[r][1] = e;
-  if (!LAST && store_out && m_tile0 * kRows + r < rows) a.e_out[row] = e;
+  if (!store_out || m_tile0 * kRows + r >= rows) return;
+  if (!LAST) a.e_out[row] = e;
+  if (lost > kMostLost) a.redo[row] = 1;
 }
 
-// The largest of a row's outputs in part `part` of them.
-__device__ __forceinline__ void put_most(const LayerArgs& a, int part, int m_tile, int lane,
-                                         float most, int e_out) {
-  most = __builtin_elementwise_maximum(most, __shfl_xor(most, 32));
-  if (lane < 32)
-    a.most_out[(size_t)part * (a.m_tiles * kRows) + m_tile * kRows + lane] = exponent_of(most, e_out);
+// Part `part` of a row's outputs: the largest, and how many are not held.
+__device__ __forceinline__ void put_part(const LayerArgs& a, int part, int m_tile, int lane,
+                                         float most, int lost, int e_out) {
+  int32_t v = part_of(exponent_of(most, e_out), lost);
+  v = both_parts(v, __shfl_xor(v, 32));
+  if (lane < 32) a.most_out[(size_t)part * (a.m_tiles * kRows) + m_tile * kRows + lane] = v;
 }
+
+// What goes with a lane's 16 units of an n-tile, loaded once for all m-tiles: between the
+// stores of one m-tile and the next the compiler would load it again and wait (1 x 3 tiles
+// 0.7 us a layer, which is what counting is_lost takes).  Loaded before the k-steps it costs
+// 1 x 1 tiles their second workgroup on a compute unit (1500 rows 146 -> 150 us).
+template <bool LAST>
+struct LaneUnits {
+  f32x4 bias[4], w_last[4];
+  i32x4 F[4], G[4];
+  __device__ __forceinline__ LaneUnits(const LayerArgs& a, int n_tile, int lane) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int n = n_tile * 32 + 8 * g + 4 * (lane >> 5);
+      bias[g] = *reinterpret_cast<const f32x4*>(a.units.bias + n);
+      F[g] = *reinterpret_cast<const i32x4*>(a.units.F + n);
+      if (LAST) w_last[g] = *reinterpret_cast<const f32x4*>(a.w_last + n);
+      else G[g] = *reinterpret_cast<const i32x4*>(a.units.G + n);
+    }
+  }
+};
 
 // A lane's 8 outputs of a k-step of the next layer, registers 8 kk .. 8 kk + 7 of a tile,
-// from their sums.  most: the largest of a row's so far; share (LAST): of the final dot
-// product.  Sums in double leave the pair one rounding, not an fp32 number's and its own.
+// from their sums.  most: the largest of a row's so far; lost: those not held; share (LAST):
+// of the final dot product.  Sums in double leave the pair one rounding, not an fp32 number's
+// and its own.
 template <bool LAST, class T>
-__device__ __forceinline__ void finish_half(const LayerArgs& a, const T (&sums)[8], int n_tile, int kk,
-                                            int m_tile, int lane, int e_in, int e_out, float& most,
+__device__ __forceinline__ void finish_half(const LayerArgs& a, const LaneUnits<LAST>& units,
+                                            const T (&sums)[8], int n_tile, int kk, int m_tile,
+                                            int lane, int e_in, int e_out, float& most, int& lost,
                                             float& share) {
-  const int h = lane >> 5;
   float v[8], rest[8], largest = 0.f;
 #pragma unroll
   for (int g = 0; g < 2; ++g) {
-    const int n = n_tile * 32 + 16 * kk + 8 * g + 4 * h;
-    const f32x4 b = *reinterpret_cast<const f32x4*>(a.units.bias + n);
-    const i32x4 F = *reinterpret_cast<const i32x4*>(a.units.F + n);
-    const i32x4 G = *reinterpret_cast<const i32x4*>(a.units.G + n);
+    const f32x4 b = units.bias[2 * kk + g];
+    const i32x4 F = units.F[2 * kk + g], G = units.G[2 * kk + g];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       if constexpr (std::is_same_v<T, double>) {
-        double y = __builtin_ldexp(sums[4 * g + e], F[e] - e_in) + (double)b[e];
-        y = y < 0. ? 0. : y;
-        // what is infinite in fp32 is so here
-        y = (float)y < __builtin_inff() ? y : (double)(float)y;
-        if (!LAST) y = __builtin_ldexp(y, G[e] + e_out);
-        v[4 * g + e] = (float)y;
-        rest[4 * g + e] = (float)(y - (double)v[4 * g + e]);
+        const double y = __builtin_ldexp(sums[4 * g + e], F[e] - e_in) + (double)b[e];
+        const float whole = (float)y;
+        if (LAST) {
+          v[4 * g + e] = relu_nan(whole);
+          continue;
+        }
+        const double scaled = __builtin_ldexp(y, G[e] + e_out);
+        const bool positive = whole > 0.f;
+        // (what is infinite in fp32 is so here)
+        v[4 * g + e] = relu_nan(whole < __builtin_inff() ? (float)scaled : whole);
+        rest[4 * g + e] = positive ? (float)(scaled - (double)v[4 * g + e]) : 0.f;
+        lost += is_lost(positive, v[4 * g + e]);
       } else {
         const float y = relu_nan(__builtin_ldexpf(sums[4 * g + e], F[e] - e_in) + b[e]);
         v[4 * g + e] = LAST ? y : __builtin_ldexpf(y, G[e] + e_out);
+        if (!LAST) lost += is_lost(y > 0.f, v[4 * g + e]);
       }
     }
     if (LAST) {
-      const f32x4 wl = *reinterpret_cast<const f32x4*>(a.w_last + n);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) share = fmaf(v[4 * g + e], wl[e], share);
+      for (int e = 0; e < 4; ++e) share = fmaf(v[4 * g + e], units.w_last[2 * kk + g][e], share);
     }
   }
   if (LAST) return;
@@ -228,16 +285,16 @@ __device__ __forceinline__ void finish_half(const LayerArgs& a, const T (&sums)[
 
 // Outputs of one tile from its sums.
 template <bool LAST, class T>
-__device__ __forceinline__ void finish_tile(const LayerArgs& a, const T (&sums)[16], int n_tile,
-                                            int m_tile, int lane, int e_in, int e_out,
-                                            float& most) {
+__device__ __forceinline__ void finish_tile(const LayerArgs& a, const LaneUnits<LAST>& units,
+                                            const T (&sums)[16], int n_tile, int m_tile, int lane,
+                                            int e_in, int e_out, float& most, int& lost) {
   float share = 0.f;
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) {
     T half[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) half[e] = sums[8 * kk + e];
-    finish_half<LAST, T>(a, half, n_tile, kk, m_tile, lane, e_in, e_out, most, share);
+    finish_half<LAST, T>(a, units, half, n_tile, kk, m_tile, lane, e_in, e_out, most, lost, share);
   }
   if (LAST) {
     share += __shfl_xor(share, 32);
@@ -290,6 +347,7 @@ struct Wide {
   static constexpr int kUnits = kSteps + SPLIT_STEPS / 2, SLABS = kUnits / KS;
   static_assert(FLUSH % KS == 0 && kSteps % FLUSH == 0, "whole slabs to a part of the sum");
   static_assert(SPLIT_STEPS % (2 * KS) == 0, "whole slabs");
+  static_assert(TN * 32 < 256, "part_of holds the count of a part's numbers");
   static_assert(KS % RING == 0 && KS % XB == 0, "the rings turn a whole number of times in a slab");
 };
 
@@ -441,21 +499,26 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const LayerArgs a) {
   wait_fetches<0>();
 
   const int m = lane & 31;
+  float most[TM] = {};
+  int lost[TM] = {};
 #pragma unroll
-  for (int j = 0; j < TM; ++j) {
-    const int m_tile = m_tile0 + j;
-    if (m_tile >= a.m_tiles) continue;
-    const int* const e = scales[j * kRows + m];
-    const int e_in = e[0], e_out = LAST ? 0 : e[1];
-    float most = 0.f;
+  for (int i = 0; i < TN; ++i) {
+    const LaneUnits<LAST> units(a, n_tile0 + i, lane);
 #pragma unroll
-    for (int i = 0; i < TN; ++i) {
+    for (int j = 0; j < TM; ++j) {
+      if (m_tile0 + j >= a.m_tiles) continue;
+      const int* const e = scales[j * kRows + m];
 #pragma unroll
       for (int r = 0; r < 16; ++r) total[i][j][r] += (T)small[i][j][r];
-      finish_tile<LAST, T>(a, total[i][j], n_tile0 + i, m_tile, lane, e_in, e_out, most);
+      finish_tile<LAST, T>(a, units, total[i][j], n_tile0 + i, m_tile0 + j, lane, e[0],
+                           LAST ? 0 : e[1], most[j], lost[j]);
     }
-    if (!LAST) put_most(a, n_blk * S::WAVES + wave, m_tile, lane, most, e_out);
   }
+  if (LAST) return;
+#pragma unroll
+  for (int j = 0; j < TM; ++j)
+    if (m_tile0 + j < a.m_tiles)
+      put_part(a, n_blk * S::WAVES + wave, m_tile0 + j, lane, most[j], lost[j], scales[j * kRows + m][1]);
 }
 
 // ---------------------------------------------------------------------------
@@ -464,7 +527,7 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const LayerArgs a) {
 // Least share that a unit's inputs have together in what it is made of: (sum of its
 // weights times the inputs' sizes)^2 over the sum of their squares, 768 for 1024
 // weights of one spread.  A pair's error does not average out over a sum of few
-// products, and below its largest weights 2^-15 a row loses bits.
+// products; and of 256 inputs at least half are held in any row that is not marked.
 constexpr double kLeastShare = 256.;
 
 // Units whose size is beyond 2^+-kUnitRange are not for pairs: their activations would leave
@@ -513,6 +576,7 @@ __global__ __launch_bounds__(256) void prepare_first(const PrepareArgs a) {
 __global__ __launch_bounds__(1024) void prepare_layer(const PrepareArgs a) {
   __shared__ double sums[2][16][32];
   __shared__ double largest[16][32];
+  __shared__ int lost_of[16][32];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, tile = blockIdx.x;
   const int m = lane & 31, h = lane >> 5;
   const f32x4* in = reinterpret_cast<const f32x4*>(a.w_stream) +
@@ -540,17 +604,32 @@ __global__ __launch_bounds__(1024) void prepare_layer(const PrepareArgs a) {
   }
   largest[wave][m] = fmax(most, __shfl_xor(most, 32));
   __syncthreads();
-  if (threadIdx.x >= 32) return;
   double total = 0., squares = 0.;
   for (int w = 0; w < 16; ++w) {
     total += sums[0][w][m];
     squares += sums[1][w][m];
     most = fmax(most, largest[w][m]);
   }
+  const int F = most > 0. ? __builtin_amdgcn_frexp_exp(most) - kTop : 0;
+  int lost = 0;
+  for (int i = 0; i < kWidth / 8 / 16; ++i) {
+    const int g = wave * (kWidth / 8 / 16) + i, k = 8 * g + 4 * h;
+    const f32x4 v = in[(size_t)g * (8 * 64)];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      lost += a.size_in[k + e] > 0.f && v[e] != 0.f &&
+              ldexp(fabs((double)v[e]), -a.G_in[k + e] - F) < kHeldFrom;
+  }
+  lost += __shfl_xor(lost, 32);
+  lost_of[wave][m] = lost;
+  __syncthreads();
+  if (threadIdx.x >= 32) return;
+  lost = 0;
+  for (int w = 0; w < 16; ++w) lost += lost_of[w][m];
   // (a weight that is not finite has been found by check_kernel)
-  if (!(total * total >= kLeastShare * squares)) *a.outside = 1;
+  if (!(total * total >= kLeastShare * squares) || lost > kMostLost) *a.outside = 1;
   const int n = tile * 32 + m;
-  a.F[n] = most > 0. ? __builtin_amdgcn_frexp_exp(most) - kTop : 0;
+  a.F[n] = F;
   put_size(a, n, squares);
 }
 
@@ -604,6 +683,7 @@ struct FirstArgs {
   char* y;               // activations out, [m_tiles] tiles, and what goes with them
   int32_t* e_out;
   int32_t* most_out;     // [kFirstParts][m_tiles * 32]
+  int32_t* redo;         // [m_tiles * 32] cleared
 };
 constexpr int kFirstParts = 4 * split::kFirstSlices;
 
@@ -634,8 +714,12 @@ __global__ __launch_bounds__(256) void first_kernel(const FirstArgs a) {
   for (int k = 0; k < a.in_features; ++k)
     most_in = __builtin_elementwise_maximum(most_in, fabsf(xs[m][k]));
   const int e_out = row_exponent(exponent_of(most_in, 0), *a.units.bias_most);
-  if (blockIdx.y == 0 && wave == 0 && h == 0) a.e_out[m_tile * kRows + m] = e_out;
+  if (blockIdx.y == 0 && wave == 0 && h == 0) {
+    a.e_out[m_tile * kRows + m] = e_out;
+    a.redo[m_tile * kRows + m] = 0;
+  }
   float most = 0.f;
+  int lost = 0;
   for (int s = wave; s < kSlice / 16; s += 4) {
     float v[8];
 #pragma unroll
@@ -659,17 +743,20 @@ __global__ __launch_bounds__(256) void first_kernel(const FirstArgs a) {
       const i32x4 G = *reinterpret_cast<const i32x4*>(a.units.G + n_base + 16 * s + 8 * g + 4 * h);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        v[4 * g + e] = __builtin_ldexpf(relu_nan(v[4 * g + e]), G[e] + e_out);
+        const float y = relu_nan(v[4 * g + e]);
+        v[4 * g + e] = __builtin_ldexpf(y, G[e] + e_out);
+        lost += is_lost(y > 0.f, v[4 * g + e]);
         largest = __builtin_elementwise_maximum(largest, v[4 * g + e]);
       }
     }
     store_pairs(a.y + tile_offset(m_tile, n_base / 16 + s) + lane * 16, v, nullptr, largest);
     most = __builtin_elementwise_maximum(most, largest);
   }
-  most = __builtin_elementwise_maximum(most, __shfl_xor(most, 32));
+  int32_t part = part_of(exponent_of(most, e_out), lost);
+  part = both_parts(part, __shfl_xor(part, 32));
   if (h == 0)
     a.most_out[(size_t)((int)blockIdx.y * 4 + wave) * ((size_t)gridDim.x * kRows) + m_tile * kRows + m] =
-        exponent_of(most, e_out);
+        part;
 }
 
 }  // namespace pairs

@@ -875,16 +875,20 @@ struct FinishArgs {
 
 // fc2: the shares of the final dot product that the last hidden layer left, added in
 // n-tile order, in double: in fp32 these 32 sums were half of a prediction's error.
-__global__ __launch_bounds__(256) void finish_kernel(const FinishArgs a) {
-  const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (row >= a.n) return;
+__device__ __forceinline__ float sum_of_shares(const float* part, int32_t rows_pad, int64_t row,
+                                               float b_last) {
   float v[kWidth / 32];
 #pragma unroll
-  for (int t = 0; t < kWidth / 32; ++t) v[t] = a.part[(size_t)t * a.rows_pad + row];
-  double sum = a.b_last;
+  for (int t = 0; t < kWidth / 32; ++t) v[t] = part[(size_t)t * rows_pad + row];
+  double sum = b_last;
 #pragma unroll
   for (int t = 0; t < kWidth / 32; ++t) sum += (double)v[t];
-  a.out[row] = (float)sum;
+  return (float)sum;
+}
+
+__global__ __launch_bounds__(256) void finish_kernel(const FinishArgs a) {
+  const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (row < a.n) a.out[row] = sum_of_shares(a.part, a.rows_pad, row, a.b_last);
 }
 
 }  // namespace split

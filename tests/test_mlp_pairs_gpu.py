@@ -257,3 +257,78 @@ def test_sums_beyond_fp32_are_infinite(rows, signs):
     assert np.all(np.isposinf(got[::7]) if signs == "positive" else np.isnan(got[::7]))
     others = np.arange(rows) % 7 != 0
     assert np.array_equal(got[others], plain[others])
+
+
+@pytest.mark.parametrize("rows", [1025, 2048, 3000, 4500, 5911, 10000, 13001, 16384 + 3001])
+def test_rows_that_one_unit_dominates(rows):
+    """A unit that is large in some rows and hardly read by the next layer: what the other
+    units make is held as fp32 holds it, and the rows beside such a row are left alone."""
+    rp = network("conv2d", 3)
+    with torch.no_grad():
+        for _, bias in layers_of(rp):
+            bias.zero_()
+        rp.model.fc2.bias.zero_()
+        first = rp.model.fc1.weight
+        first[:, 0] = 0.0
+        first[40] = 0.0
+        first[40, 0] = 1.0                                  # unit 40 is feature 0 alone
+        layers_of(rp)[1][0][:, 40] *= 2.0 ** -60
+    inputs = first.shape[1]
+    rp.set_normalization(np.zeros(inputs), np.ones(inputs))
+    rng = np.random.default_rng(rows)
+    x = rng.normal(size=(rows, inputs))
+    x[:, 0] = 1.0
+    plain = rp.predict_batch(x).cpu().numpy()
+    want = forward_fp64(rp, x)                              # (feature 0 is 2^-60 of it)
+    rms = np.sqrt(np.mean(want ** 2))
+    at = np.sort(rng.choice(rows, rows // 40, replace=False))
+    for k in (4, 8, 10, 12, 16, 20, 32):
+        x[at, 0] = 2.0 ** k
+        y = rp.predict_batch(x).cpu().numpy()
+        # the bound of tests/test_mlp_split_gpu.py
+        assert np.sqrt(np.mean((y[at] - want[at]) ** 2)) <= 4 * 8 * 2.0 ** -24 * rms, k
+        others = np.setdiff1d(np.arange(rows), at)
+        assert np.array_equal(y[others], plain[others]), k
+        if k >= 12:   # (whole rounds of the fused fp32 kernel)
+            whole = np.resize(x[at], (8192, inputs))
+            assert np.array_equal(y[at], rp.predict_batch_fp32(whole).cpu().numpy()[:at.size])
+    graph, out = torch.cuda.CUDAGraph(), torch.empty(rows, device="cuda")
+    raw = torch.from_numpy(x).cuda()
+    with torch.cuda.graph(graph):
+        rp.predict_batch(raw, out=out)
+    raw[:, 0] = 1.0                          # what was marked in one pass is not in the next
+    for _ in range(2):
+        out.zero_()
+        graph.replay()
+        assert np.array_equal(out.cpu().numpy(), plain)
+        assert np.array_equal(rp.predict_batch(x).cpu().numpy(), y)
+
+
+@pytest.mark.parametrize("rows", [1500, 3000, 5911, 13000])
+def test_small_weights_that_are_all_that_counts(rows):
+    """Half of the inputs with ordinary weights, the other half with 2^-24 of them, and rows
+    in which the first half is off."""
+    rp = network("linear", 2)
+    with torch.no_grad():
+        for _, bias in layers_of(rp):
+            bias.zero_()
+        rp.model.fc2.bias.zero_()
+        rp.model.fc1.weight.abs_()
+        rp.model.fc1.weight[::2, 0] = 0.0
+        rp.model.fc1.weight[1::2, 1:] = 0.0               # every second unit is feature 0 alone
+        layers_of(rp)[1][0][:, ::2] *= 2.0 ** -24
+    rp.set_normalization(np.zeros(8), np.ones(8))
+    x = np.abs(np.random.default_rng(rows).normal(size=(rows, 8)))
+    x[::2, 0] = 0.0
+    y, want = rp.predict_batch(x).double().cpu().numpy(), forward_fp64(rp, x)
+    h = torch.from_numpy(x).cuda()
+    with torch.no_grad():
+        for weight, _ in layers_of(rp):
+            h = torch.relu(h @ weight.double().cuda().t())
+        size = (h * rp.model.fc2.weight.double().cuda()).norm(dim=1).cpu().numpy()
+    for part in (slice(0, None, 2), slice(1, None, 2)):
+        # The bound of tests/test_mlp_split_gpu.py, for either kind of row.  All activations of
+        # a second row are multiples of one feature, so that what the last sum cancels to is
+        # the same part of it in all of them: its terms' root sum of squares stands for it.
+        assert np.sqrt(np.mean((y[part] - want[part]) ** 2)) <= \
+            3 * 8 * 2.0 ** -24 * np.sqrt(np.mean(size[part] ** 2))
