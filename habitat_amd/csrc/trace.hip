@@ -204,6 +204,8 @@ struct OrderedSumArgs {
   double* out_total;             // [rows], nullable
   const int32_t* out_bad;        // [rows], with out_total
   double constant_ms;
+  int32_t per_block;             // segments that a workgroup takes at a time, up to kBlock
+  bool totals_here;              // kBlock at a time, and all of a destination's
 };
 
 // Sum of `v` over the workgroup, in one order; for thread 0.
@@ -219,14 +221,27 @@ __device__ __forceinline__ double block_sum(double v, double (&part)[kBlock / 64
   return total;
 }
 
-// One workgroup per destination, a thread per segment: it adds the segment's scaled times
-// one after the other in the records' order, as the reference adds a pass's kernels
-// (run_time.py:50-58).  No floating-point atomics: the sum is the same every time, and the
-// same as a sequential sum of the per-record kernel's times.  Bound by that chain of
-// additions for the longest segment (an optimizer pass is several hundred kernels): the
-// times come through LDS, kStage of them at a time, so that no addition waits for memory
-// (256 destinations of a ResNet-50's records: 21 us with loads of their own, 8 us).
+__device__ __forceinline__ void put_total(const OrderedSumArgs& a, int row, double mine,
+                                          double (&part)[kBlock / 64]) {
+  const double total = block_sum(mine, part);
+  if (threadIdx.x == 0)
+    a.out_total[row] = a.out_bad[row] > 0 ? __builtin_nan("") : a.constant_ms + total / 1e6;
+}
+
+// A thread per segment, up to 256 of them and a destination (blockIdx.x) to a workgroup: a
+// thread adds its segment's scaled times one after the other in the records' order, as the
+// reference adds a pass's kernels (run_time.py:50-58).  No floating-point atomics: the sum is
+// the same every time, and the same as a sequential sum of the per-record kernel's times.
+// Bound by that chain of additions for the longest segment (an optimizer pass is several
+// hundred kernels): the times come through LDS, kStage of them at a time, so that no addition
+// waits for memory (256 destinations of a ResNet-50's records: 21 us with loads of their own,
+// 8 us).  A workgroup takes segments for about one stage (per_block), since those of the next
+// stages would wait for them, and the workgroups of a destination are spread over gridDim.y
+// where the destinations alone do not fill the GPU: one destination, a million records in
+// 100 000 segments 28 us with the scaling and in 1000 segments 32, by one workgroup
+// 3660 and 5390.
 constexpr int kStage = 2048;
+constexpr int kFillGrid = 1024;   // workgroups that fill the GPU
 __global__ __launch_bounds__(kBlock) void segment_sum_ordered_kernel(const OrderedSumArgs a) {
   __shared__ double staged[kStage];
   __shared__ double part[kBlock / 64];
@@ -235,8 +250,9 @@ __global__ __launch_bounds__(kBlock) void segment_sum_ordered_kernel(const Order
   if (row < 0) return;
   const double* v = a.work + (int64_t)d * a.n;
   double mine = 0.0;
-  for (int s0 = 0; s0 < a.n_segments; s0 += kBlock) {
-    const int s = s0 + (int)threadIdx.x;
+  for (int64_t s0 = (int64_t)blockIdx.y * a.per_block; s0 < a.n_segments;
+       s0 += (int64_t)gridDim.y * a.per_block) {
+    const int64_t s = (int)threadIdx.x < a.per_block ? s0 + (int)threadIdx.x : a.n_segments;
     // (clamped to the columns: a wrong boundary must not become a stray read)
     int64_t begin = 0, end = 0;
     if (s < a.n_segments) {
@@ -271,10 +287,20 @@ __global__ __launch_bounds__(kBlock) void segment_sum_ordered_kernel(const Order
     mine += sum;
     __syncthreads();   // range is read above and set again
   }
-  if (a.out_total == nullptr) return;
-  const double total = block_sum(mine, part);
-  if (threadIdx.x == 0)
-    a.out_total[row] = a.out_bad[row] > 0 ? __builtin_nan("") : a.constant_ms + total / 1e6;
+  if (!a.totals_here) return;
+  put_total(a, row, mine, part);
+}
+
+// The totals of destinations whose segments were spread, in the order of a workgroup that
+// has them 256 at a time.
+__global__ __launch_bounds__(kBlock) void segment_totals_kernel(const OrderedSumArgs a) {
+  __shared__ double part[kBlock / 64];
+  const int row = a.out.of(blockIdx.x);
+  if (row < 0) return;
+  double mine = 0.0;
+  for (int64_t s = threadIdx.x; s < a.n_segments; s += kBlock)
+    mine += a.out_sum[(int64_t)row * a.n_segments + s];
+  put_total(a, row, mine, part);
 }
 
 struct GammaArgs {
@@ -544,8 +570,16 @@ int hbt_wave_scale_sum_totals(const hbt_device_table* table, int64_t n, const in
   b.out_total = out_total;
   b.out_bad = out_bad;
   b.constant_ms = constant_ms;
-  hipLaunchKernelGGL(segment_sum_ordered_kernel, dim3((unsigned)table->n_dest), dim3(kBlock), 0,
-                     stream, b);
+  const int64_t stage = n > 0 ? (int64_t)kStage * n_segments / n : kBlock;
+  b.per_block = (int32_t)(stage > kBlock || stage >= n_segments ? kBlock : stage > 0 ? stage : 1);
+  const int64_t blocks_all = ((int64_t)n_segments + b.per_block - 1) / b.per_block;
+  const int64_t fill = table->n_dest < kFillGrid ? kFillGrid / table->n_dest : 1;
+  const dim3 sum_grid((unsigned)table->n_dest, (unsigned)(blocks_all < fill ? blocks_all : fill));
+  b.totals_here = out_total != nullptr && b.per_block == kBlock && sum_grid.y == 1;
+  hipLaunchKernelGGL(segment_sum_ordered_kernel, sum_grid, dim3(kBlock), 0, stream, b);
+  if (out_total != nullptr && !b.totals_here)
+    hipLaunchKernelGGL(segment_totals_kernel, dim3((unsigned)table->n_dest), dim3(kBlock), 0, stream,
+                       b);
   return hipGetLastError() == hipSuccess ? HBT_OK : HBT_EHIP;
 }
 

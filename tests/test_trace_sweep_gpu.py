@@ -422,3 +422,70 @@ def test_ratios_of_several_kinds_in_one_launch(kinds):
     out, clamped = ratio_scale_kinds(parts, D, totals, torch.cuda.current_stream())
     assert torch.equal(totals, want_totals) and torch.equal(clamped, want_clamped)
     assert all(torch.equal(out[k], want[k]) for k in want)
+
+
+@pytest.mark.parametrize("segments", [1000, 100_000])
+def test_ordered_sums_of_a_million_records_fill_the_gpu(segments):
+    """Passes of a database of traces, on one destination: a segment's chain of additions is
+    short, so the sums take about what those of any order take."""
+    n = 1_000_000
+    rec, _ = synthetic.kernel_records(n, Device.V100, seed=5)
+    records = KernelRecords.from_numpy(rec, "cuda:0")
+    table = DeviceTable(Device.V100, [Device.T4])
+    start = torch.arange(segments + 1, dtype=torch.int64, device="cuda") * (n // segments)
+    segment = torch.arange(n, device="cuda").div(n // segments, rounding_mode="floor").int()
+    work = torch.empty((1, n), dtype=torch.float64, device="cuda")
+
+    def ms(call):
+        times = []
+        for _ in range(8):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            for _ in range(5):
+                call()
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end) / 5)
+        return min(times)
+
+    ordered = ms(lambda: wave_scale_sum(records, table, n_segments=segments, segment_start=start,
+                                        workspace=work))
+    any_order = ms(lambda: wave_scale_sum(records, table, segment, n_segments=segments))
+    # measured: 28 to 32 us beside 20; one workgroup for all segments, 3600 to 5400
+    assert ordered <= 10 * any_order, (ordered, any_order)
+
+
+@pytest.mark.parametrize("n,segments,dests", [(1, 1, 1), (5000, 3, 1), (5000, 255, 1), (5000, 257, 1),
+                                              (5000, 5000, 1), (300, 70_000, 1), (40_000, 1000, 3),
+                                              (40_000, 9, 1100), (3000, 600, 1100)])
+def test_ordered_sums_and_totals_at_any_shape(n, segments, dests):
+    """Segments to a workgroup from one to 256, destinations that fill the GPU and that do
+    not, and more segments than records."""
+    rng = np.random.default_rng(segments)
+    rec, _ = synthetic.kernel_records(n, Device.V100, seed=n)
+    records = KernelRecords.from_numpy(rec, "cuda:0")
+    pool = [Device.T4, Device.P100, Device.RTX2070]
+    table = DeviceTable(Device.V100, [pool[d % 3] for d in range(dests)])
+    edges = np.sort(rng.integers(0, n + 1, segments + 1))
+    edges[0], edges[-1] = 0, n
+    work = torch.empty((dests, n), dtype=torch.float64, device="cuda")
+    call = TotalsCall(records, table, torch.from_numpy(edges).cuda(), segments, work, None, dests, 2.5)
+    sums = torch.full((dests, segments), -1.0, dtype=torch.float64, device="cuda")
+    bad = torch.full((dests,), -1, dtype=torch.int32, device="cuda")
+    totals = torch.full((dests,), -1.0, dtype=torch.float64, device="cuda")
+    call(sums, bad, totals, torch.cuda.current_stream())
+    for d in range(min(dests, 3)):
+        times = work[d].cpu().numpy()
+        want = np.zeros(segments)
+        for s in range(segments):
+            for t in times[edges[s]:edges[s + 1]]:
+                want[s] += t
+        assert np.array_equal(sums[d].cpu().numpy(), want)
+    for d in range(dests):
+        assert torch.equal(sums[d], sums[d % 3]) and bad[d] == bad[d % 3]
+        assert int(bad[d]) or totals[d] == totals[d % 3]
+    # (a total adds at most 70 000 numbers in some order)
+    want = 2.5 + sums.sum(dim=1) / 1e6
+    ok = bad == 0
+    assert torch.allclose(totals[ok], want[ok], rtol=1e-11, atol=0)
+    assert bool(torch.isnan(totals[~ok]).all())
