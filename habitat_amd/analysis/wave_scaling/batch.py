@@ -263,6 +263,11 @@ def wave_scale_sum(records, table, segment=None, n_segments=1, stream=None, segm
     return sums, bad
 
 
+def _is_buffer(t, dtype, shape, device):
+    """Whether a kernel can write (or read) `t` as [shape] of dtype from its first element."""
+    return t.dtype == dtype and t.shape == shape and t.device == device and t.is_contiguous()
+
+
 class TotalsCall:
     """hbt_wave_scale_sum_totals for records and destinations that stay the same: what the
     call is made of is looked over and laid out once.  `rows`: int32 GPU tensor naming each
@@ -297,11 +302,11 @@ class TotalsCall:
     def __call__(self, sums, bad, totals, stream):
         """sums float64 [n_rows, n_segments], bad int32 [n_rows], totals float64 [n_rows]:
         contiguous GPU tensors; only the rows of this call are written."""
-        if (sums.shape != self.shape or bad.shape != self.shape[:1] or totals.shape != bad.shape
-                or sums.dtype != torch.float64 or bad.dtype != torch.int32
-                or totals.dtype != torch.float64):
-            raise TypeError("sums must be float64 %s, bad int32 and totals float64 of its rows"
-                            % (list(self.shape),))
+        if not (_is_buffer(sums, torch.float64, self.shape, self._device)
+                and _is_buffer(bad, torch.int32, self.shape[:1], self._device)
+                and _is_buffer(totals, torch.float64, self.shape[:1], self._device)):
+            raise TypeError("sums must be float64 %s, bad int32 and totals float64 of its rows, "
+                            "contiguous on the records' GPU" % (list(self.shape),))
         with torch.cuda.device(self._device):
             rc = _lib.lib().hbt_wave_scale_sum_totals(
                 *self._args, sums.data_ptr(), bad.data_ptr(), totals.data_ptr(),
@@ -312,7 +317,10 @@ class TotalsCall:
 def ratio_scale_kinds(kinds, n_dest, totals, stream):
     """ratio_scale for several kinds of operation in one launch.  kinds: (name, pred,
     run_time_ms, op_row) each, as there.  Adds to `totals`; returns ({name: ms [n_dest,
-    n_ops]}, clamped int32 [n_dest])."""
+    n_ops]}, clamped int32 [n_dest]).  All tensors are on one GPU, `totals` is contiguous."""
+    device = totals.device
+    if not totals.is_cuda or not _is_buffer(totals, torch.float64, (n_dest,), device):
+        raise TypeError("totals must be a contiguous float64 GPU tensor [%d]" % n_dest)
     clamped = torch.empty((n_dest,), dtype=torch.int32, device=totals.device)
     array = (_lib.RatioKind * max(len(kinds), 1))()
     out, keep = {}, []
@@ -323,6 +331,8 @@ def ratio_scale_kinds(kinds, n_dest, totals, stream):
         if (run_time_ms.dtype != torch.float64 or op_row.dtype != torch.int32
                 or op_row.shape != (n_ops,)):
             raise TypeError("run_time_ms must be float64 and op_row int32, both [%d]" % n_ops)
+        if any(t.device != device for t in (pred, run_time_ms, op_row)):
+            raise ValueError("pred, run_time_ms and op_row must live on the totals' GPU")
         pred, run_time_ms, op_row = pred.contiguous(), run_time_ms.contiguous(), op_row.contiguous()
         out[name] = torch.empty((n_dest, n_ops), dtype=torch.float64, device=pred.device)
         keep.append((pred, run_time_ms, op_row))
@@ -357,6 +367,9 @@ def ratio_scale(pred, run_time_ms, n_dest, totals=None, want_ms=True, stream=Non
         raise TypeError("run_time_ms and totals must be float64")
     if clamped is not None and (clamped.dtype != torch.int32 or clamped.shape != (n_dest,)):
         raise TypeError("clamped must be int32 [%d]" % n_dest)
+    if any(t is not None and (t.device != pred.device or not t.is_contiguous())
+           for t in (totals, clamped)):
+        raise TypeError("totals and clamped must be contiguous, on the predictions' GPU")
     pred = pred.contiguous()
     out = (torch.empty((n_dest, n_ops), dtype=torch.float64, device=pred.device)
            if want_ms else None)

@@ -489,3 +489,44 @@ def test_ordered_sums_and_totals_at_any_shape(n, segments, dests):
     ok = bad == 0
     assert torch.allclose(totals[ok], want[ok], rtol=1e-11, atol=0)
     assert bool(torch.isnan(totals[~ok]).all())
+
+
+def test_outputs_that_a_kernel_cannot_write_are_refused():
+    """TotalsCall, ratio_scale_kinds and ratio_scale hand their outputs to a kernel as they
+    are: another type, shape, stride or device is refused before."""
+    rec, _ = synthetic.kernel_records(100, Device.V100, seed=1)
+    records = KernelRecords.from_numpy(rec, "cuda:0")
+    table = DeviceTable(Device.V100, [Device.T4, Device.P100])
+    start = torch.tensor([0, 40, 100], device="cuda")
+    call = TotalsCall(records, table, start, 2, torch.empty((2, 100), dtype=torch.float64,
+                                                            device="cuda"), None, 2, 0.0)
+    stream = torch.cuda.current_stream()
+    f64 = dict(dtype=torch.float64, device="cuda")
+    right = [torch.zeros((2, 2), **f64), torch.zeros(2, dtype=torch.int32, device="cuda"),
+             torch.zeros(2, **f64)]
+    wrong = [[torch.zeros((2, 2), **f64).t(), torch.zeros((2, 2), dtype=torch.float64),
+              torch.zeros((1, 2), **f64), torch.zeros((2, 2), device="cuda")],
+             [torch.zeros(4, dtype=torch.int32, device="cuda")[::2],
+              torch.zeros(2, dtype=torch.int32), torch.zeros(1, dtype=torch.int32, device="cuda")],
+             [torch.zeros(4, **f64)[::2], torch.zeros(2, dtype=torch.float64),
+              torch.zeros(3, **f64), torch.zeros(2, device="cuda")]]
+    for i, outputs in enumerate(wrong):
+        for t in outputs:
+            with pytest.raises(TypeError):
+                call(*right[:i], t, *right[i + 1:], stream)
+    pred, ms = torch.ones((3, 4), device="cuda"), torch.ones(4, **f64)
+    op_row = torch.arange(4, dtype=torch.int32, device="cuda")
+    for t in wrong[2]:
+        with pytest.raises(TypeError):
+            ratio_scale_kinds([("bmm", pred, ms, op_row)], 2, t, stream)
+        with pytest.raises(TypeError):
+            ratio_scale(pred, ms, 2, totals=t, op_row=op_row)
+    for t in wrong[1]:
+        with pytest.raises(TypeError):
+            ratio_scale(pred, ms, 2, op_row=op_row, clamped=t)
+    for kind in (("bmm", pred.cpu(), ms, op_row), ("bmm", pred, ms.cpu(), op_row),
+                 ("bmm", pred, ms, op_row.cpu())):
+        with pytest.raises(ValueError):
+            ratio_scale_kinds([kind], 2, right[2], stream)
+    call(*right, stream)
+    ratio_scale_kinds([("bmm", pred, ms, op_row)], 2, right[2], stream)
