@@ -153,7 +153,6 @@ def wave_scale(records, origin, dests, out=None, stream=None, waves=True, status
 
 def _enqueue_wave_scale(records, origin, specs, n_dest, out, stream):
     c, regs, metrics = records.columns, records.dest_regs, records.has_metrics
-    waves, status = out.wave_origin, out.status
     return _lib.lib().hbt_wave_scale(
         ctypes.byref(origin.spec), specs, n_dest, records.n,
         c["num_blocks"].data_ptr(), c["block_size"].data_ptr(), c["dynamic_smem"].data_ptr(),
@@ -162,10 +161,8 @@ def _enqueue_wave_scale(records, origin, specs, n_dest, out, stream):
         c["run_time_ns"].data_ptr(), c["flop_sp_efficiency"].data_ptr(),
         c["dram_read_bytes"].data_ptr(), c["dram_write_bytes"].data_ptr(),
         None if metrics is None else metrics.data_ptr(),
-        out.time_ns.data_ptr(), out.occ_origin.data_ptr(), out.occ_dest.data_ptr(),
-        None if waves is None else waves.data_ptr(),
-        None if out.wave_dest is None else out.wave_dest.data_ptr(),
-        None if status is None else status.data_ptr(), stream)
+        _ptr(out.time_ns), _ptr(out.occ_origin), _ptr(out.occ_dest), _ptr(out.wave_origin),
+        _ptr(out.wave_dest), _ptr(out.status), stream)
 
 
 class DeviceTable:

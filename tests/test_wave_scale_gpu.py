@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from conftest import GOLDEN, oracle_device
-from habitat_amd import Device, DeviceProperties, synthetic
+from habitat_amd import Device, DeviceProperties, _lib, synthetic
 from habitat_amd.analysis.wave_scaling.batch import KernelRecords, WaveScaleOutput, wave_scale
 from oracle import lib as olib
 
@@ -622,3 +622,20 @@ def test_bad_specs_are_rejected_not_launched():
     with pytest.raises(_lib.HabitatLibraryError) as e:
         wave_scale(kr, Device.V100, [zero_bw])
     assert e.value.code == _lib.HBT_ESPEC
+
+
+@pytest.mark.parametrize("missing", ["occ_origin", "occ_dest", "wave_origin", "wave_dest", "status"])
+def test_an_output_that_is_not_wanted(missing):
+    """Every output but the times may be None."""
+    rec, _ = synthetic.kernel_records(1000, Device.V100, seed=1)
+    records = KernelRecords.from_numpy(rec, "cuda:0")
+    want = wave_scale(records, Device.V100, [Device.T4])
+    out = WaveScaleOutput(1000, 1, records.device)
+    setattr(out, missing, None)
+    assert wave_scale(records, Device.V100, [Device.T4], out=out) is out
+    for name in ("time_ns", "occ_origin", "occ_dest", "wave_origin", "wave_dest", "status"):
+        if name != missing:
+            assert torch.equal(getattr(out, name), getattr(want, name)), name
+    out.time_ns = None
+    with pytest.raises(_lib.HabitatLibraryError):
+        wave_scale(records, Device.V100, [Device.T4], out=out)
