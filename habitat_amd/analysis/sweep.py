@@ -189,11 +189,12 @@ class SweepCall:
                     [op_feats.unsqueeze(0).expand(D + 1, U, -1),
                      dev_feats.unsqueeze(1).expand(D + 1, U, 4)], dim=2).reshape((D + 1) * U, -1)
 
-        # The kind with the most rows runs on the caller's stream, so that what decides the
-        # time waits for no other stream, each other kind beside it on one of its own (of
-        # default priority).  The passes' sums come before them: 25 us with the GPU to
-        # themselves; beside a network's launches they are as slow as those (256 devices:
-        # 836 us a sweep and 878, 60: 274 and 314).
+        # The kind with the most rows runs on the caller's stream, after the passes' sums, so
+        # that what decides the time waits for no other stream; each other kind runs on a
+        # stream of its own (of default priority), beside the sums and beside that one.  (The
+        # sums beside the largest kind take as long as its launches: 256 devices 878 us a sweep
+        # and not 838, 60 devices 314 and 274.  The other kinds after the sums: 2 devices 164
+        # us and not 126, 16 devices 192 and 154, 1024 devices 3140 and 3100.)
         kinds = sorted(self.rows, key=lambda kind: -self.rows[kind].shape[0])
         self.kinds = [(kind, torch.cuda.Stream(plan.gpu) if i else None)
                       for i, kind in enumerate(kinds)]
@@ -205,7 +206,7 @@ class SweepCall:
         res.pass_overhead_ns = plan.pass_overhead_ns
         res.pass_owner = plan.pass_owner
         main = torch.cuda.current_stream(plan.gpu)
-        for side in self.streams:
+        for side in self.streams:   # (before the sums: the other kinds do not wait for them)
             side.wait_stream(main)
         if self.groups:
             total = torch.empty((D,), dtype=torch.float64, device=plan.gpu)
