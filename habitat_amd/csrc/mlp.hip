@@ -1198,31 +1198,28 @@ void split_launch(const split::LayerArgs& a, bool last, hipStream_t stream) {
 //
 // Where mid_kernel and the 4 x 3 and 4 x 4 tiles are within 2 %, it is taken for its
 // second set of sums (errors of 0.8 and 1.2 in 2^-24 of a layer's output).
-struct SplitKernel {
-  void (*launch)(const split::LayerArgs&, bool, hipStream_t);
-  bool nearest;   // its sums are the nearest to exact ones (1.3 in 2^-24 of a layer's output)
-};
-SplitKernel split_kernel_for(int m_tiles, int compute_units) {
-  SplitKernel best{};
+using SplitLaunch = void (*)(const split::LayerArgs&, bool, hipStream_t);
+SplitLaunch split_kernel_for(int m_tiles, int compute_units) {
+  SplitLaunch best = nullptr;
   float best_us = 0.f;
-  const auto consider = [&](auto kernel, float start, float round_us, bool nearest) {
+  const auto consider = [&](auto kernel, float start, float round_us) {
     using C = decltype(kernel);
     const int per_round = C::S::BM * (compute_units / C::S::NBLK > 0 ? compute_units / C::S::NBLK : 1);
     const float us = start + round_us * (float)((m_tiles + per_round - 1) / per_round);
-    if (best.launch == nullptr || us < best_us) {
-      best = {split_launch<C>, nearest};
+    if (best == nullptr || us < best_us) {
+      best = split_launch<C>;
       best_us = us;
     }
   };
-  consider(SplitSmall1x1(), 2.7f, 4.05f, true);   // rounds of 256 rows
-  consider(SplitSmall1x2(), 2.f, 6.9f, true);     // 512
-  consider(SplitSmall2x2(), 3.5f, 10.f, true);    // 1024
-  consider(SplitSmall2x3(), 2.5f, 13.5f, true);   // 1536
-  consider(SplitSmall2x4(), 4.f, 18.f, true);     // 2048
-  consider(SplitSmall4x3(), 4.f, 24.5f, false);   // 3072
-  consider(SplitSmall4x4(), 3.f, 32.f, false);    // 4096
-  consider(SplitMid192(), 6.f, 44.f, false);      // 6144
-  consider(SplitLarge(), 0.f, 122.f, false);      // 16 384
+  consider(SplitSmall1x1(), 2.7f, 4.05f);   // rounds of 256 rows
+  consider(SplitSmall1x2(), 2.f, 6.9f);     // 512
+  consider(SplitSmall2x2(), 3.5f, 10.f);    // 1024
+  consider(SplitSmall2x3(), 2.5f, 13.5f);   // 1536
+  consider(SplitSmall2x4(), 4.f, 18.f);     // 2048
+  consider(SplitSmall4x3(), 4.f, 24.5f);   // 3072
+  consider(SplitSmall4x4(), 3.f, 32.f);    // 4096
+  consider(SplitMid192(), 6.f, 44.f);      // 6144
+  consider(SplitLarge(), 0.f, 122.f);      // 16 384
   return best;
 }
 
@@ -1245,7 +1242,7 @@ int forward_split(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
     hipLaunchKernelGGL(split::first_kernel<kFirstFmaMaxIn>, first_grid, dim3(256), 0, stream, f);
   else
     hipLaunchKernelGGL(split::first_kernel<kMaxInPadded>, first_grid, dim3(256), 0, stream, f);
-  const SplitKernel kernel = split_kernel_for(m_tiles, mlp->compute_units);
+  const SplitLaunch launch = split_kernel_for(m_tiles, mlp->compute_units);
   split::LayerArgs l{};
   l.w_last = mlp->w_last;
   l.part = part;
@@ -1256,7 +1253,7 @@ int forward_split(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
     l.x = buffers[layer & 1];
     l.y = buffers[(layer + 1) & 1];
     const bool last = layer + 1 == mlp->hidden;
-    kernel.launch(l, last, stream);
+    launch(l, last, stream);
   }
   split::FinishArgs z{};
   z.part = part;
@@ -1305,16 +1302,26 @@ void pairs_launch(const pairs::LayerArgs& a, bool last, hipStream_t stream) {
 //   16384         814   803   686    1196
 //
 // At 9217 to 12 288 rows 2 x 4 tiles are 2 % faster than 1 x 3; the sums of these are nearer.
-// 1 x 1 tiles, with totals in double, are for the batches whose bf16 pieces have their
-// nearest sums (split_kernel_for): errors of a prediction (eight networks, 2-norm, relative)
-// 4.8e-8 both; 1 x 2 and 1 x 3 have 5.8e-8 (mid_kernel 6.5e-8, one set of pieces' sums
-// 1.07e-7), 2 x 4 1.17e-7 (large_kernel 1.41e-7).
+//
+// 1 x 1 tiles, with totals in double, have the nearest sums: errors of a prediction (eight
+// networks, 2-norm, relative) 4.8e-8; 1 x 2 and 1 x 3 have 5.8e-8, 2 x 4 1.17e-7.  They are
+// taken for a batch of up to one round, where they are the fastest too, and in two ranges in
+// which the three bf16 pieces have their nearest sums, 4.8e-8 as well (in the others 6.5e-8,
+// one set of sums 1.07e-7, large_kernel 1.41e-7), so that no batch is further from exact
+// sums in pairs than in pieces: 2 to 2 1/4 rounds (4097 to 4608 rows; 4500: 370 us, 1 x 3 in
+// one round of its own 293) and 4 1/2 to 5 (9217 to 10 240; 10 000: 631 and 570).
+bool pairs_nearest(int m_tiles, int compute_units) {
+  constexpr int kBlocks = PairsWide1x1::S::NBLK;
+  const int round = compute_units / kBlocks > 0 ? compute_units / kBlocks : 1;   // of m-tiles
+  return m_tiles <= round || (m_tiles > 2 * round && 4 * m_tiles <= 9 * round) ||
+         (2 * m_tiles > 9 * round && m_tiles <= 5 * round);
+}
 struct PairsKernel {
   void (*launch)(const pairs::LayerArgs&, bool, hipStream_t);
   int parts;   // in which a layer leaves the rows' largest outputs
 };
 PairsKernel pairs_kernel_for(int m_tiles, int compute_units) {
-  if (split_kernel_for(m_tiles, compute_units).nearest)
+  if (pairs_nearest(m_tiles, compute_units))
     return {pairs_launch<PairsWide1x1>, PairsWide1x1::S::PARTS};
   PairsKernel best{};
   float best_us = 0.f;
