@@ -1268,16 +1268,16 @@ int forward_split(hbt_mlp* mlp, const double* raw_features, int64_t n, float* ou
 // The pairs' hidden layers (mlp_pairs.h).
 constexpr size_t kPairsLayerBytes = (size_t)(kWidth / 32) * pairs::kTileBytes;
 
-template <class T, int TN, int TM, int KS, int NBUF, int RING, int XB, int FLUSH, int SPLIT>
+template <class T, int TN, int TM, int KS, int NBUF, int RING, int FLUSH, int SPLIT>
 struct PairsWide {
-  using S = pairs::Wide<TN, TM, KS, NBUF, RING, XB, FLUSH, SPLIT>;
-  static constexpr auto kHidden = &pairs::wide_kernel<T, TN, TM, KS, NBUF, RING, XB, FLUSH, SPLIT, false>;
-  static constexpr auto kLast = &pairs::wide_kernel<T, TN, TM, KS, NBUF, RING, XB, FLUSH, SPLIT, true>;
+  using S = pairs::Wide<TN, TM, KS, NBUF, RING, FLUSH, SPLIT>;
+  static constexpr auto kHidden = &pairs::wide_kernel<T, TN, TM, KS, NBUF, RING, FLUSH, SPLIT, false>;
+  static constexpr auto kLast = &pairs::wide_kernel<T, TN, TM, KS, NBUF, RING, FLUSH, SPLIT, true>;
 };
-using PairsWide1x1 = PairsWide<double, 1, 1, 4, 3, 4, 2, 4, 0>;
-using PairsWide1x2 = PairsWide<float, 1, 2, 4, 3, 4, 2, 8, 0>;
-using PairsWide1x3 = PairsWide<float, 1, 3, 8, 2, 4, 2, 8, 0>;
-using PairsWide2x4 = PairsWide<float, 2, 4, 4, 3, 2, 2, 64, 24>;
+using PairsWide1x1 = PairsWide<double, 1, 1, 4, 3, 4, 4, 0>;
+using PairsWide1x2 = PairsWide<float, 1, 2, 4, 3, 4, 8, 0>;
+using PairsWide1x3 = PairsWide<float, 1, 3, 8, 2, 4, 8, 0>;
+using PairsWide2x4 = PairsWide<float, 2, 4, 4, 3, 2, 64, 24>;
 
 template <class C>
 void pairs_launch(const pairs::LayerArgs& a, bool last, hipStream_t stream) {
@@ -1552,7 +1552,8 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
                           hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)kLdsBytes) != hipSuccess ||
       !split_ready<SplitSmall1x1, SplitSmall1x2, SplitSmall2x2, SplitSmall2x3, SplitSmall2x4,
-                   SplitSmall4x3, SplitSmall4x4, SplitMid192, SplitLarge, PairsWide1x1, PairsWide1x2, PairsWide1x3, PairsWide2x4>()) {
+                   SplitSmall4x3, SplitSmall4x4, SplitMid192, SplitLarge, PairsWide1x1, PairsWide1x2,
+                   PairsWide1x3, PairsWide2x4>()) {
     (void)hipGetLastError();
     (void)hipFree(blob);
     *err = HBT_EHIP;

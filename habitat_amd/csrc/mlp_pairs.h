@@ -333,7 +333,7 @@ __device__ __forceinline__ void finish_tile(const LayerArgs& a, const LaneUnits<
 //   1 x 2         4096           24            1.1            34
 //   1 x 3         6144           32            1.2            52
 //   2 x 4        16384           81            1.27          143
-template <int TN, int TM, int KS, int NBUF, int RING, int XB, int FLUSH, int SPLIT_STEPS>
+template <int TN, int TM, int KS, int NBUF, int RING, int FLUSH, int SPLIT_STEPS>
 struct Wide {
   static constexpr int WAVES = 8, BN = WAVES * TN, BM = TM;
   static constexpr int THREADS = WAVES * 64;
@@ -348,13 +348,12 @@ struct Wide {
   static_assert(FLUSH % KS == 0 && kSteps % FLUSH == 0, "whole slabs to a part of the sum");
   static_assert(SPLIT_STEPS % (2 * KS) == 0, "whole slabs");
   static_assert(TN * 32 < 256, "part_of holds the count of a part's numbers");
-  static_assert(KS % RING == 0 && KS % XB == 0, "the rings turn a whole number of times in a slab");
+  static_assert(KS % RING == 0 && KS % 2 == 0, "the rings turn a whole number of times in a slab");
 };
 
-template <class T, int TN, int TM, int KS, int NBUF, int RING, int XB, int FLUSH, int SPLIT_STEPS,
-          bool LAST>
+template <class T, int TN, int TM, int KS, int NBUF, int RING, int FLUSH, int SPLIT_STEPS, bool LAST>
 __global__ __launch_bounds__(512, 2) void wide_kernel(const LayerArgs a) {
-  using S = Wide<TN, TM, KS, NBUF, RING, XB, FLUSH, SPLIT_STEPS>;
+  using S = Wide<TN, TM, KS, NBUF, RING, FLUSH, SPLIT_STEPS>;
   constexpr bool PARTED = FLUSH < kSteps;   // three sets of sums
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   int(*const scales)[2] = reinterpret_cast<int(*)[2]>(lds + S::SLAB * NBUF);
@@ -408,7 +407,7 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const LayerArgs a) {
   row_scales<S::BM * kRows, S::THREADS, LAST>(a, m_tile0, n_blk == 0, scales);
 
   f32x16 sums[PARTED ? 2 : 1][TN][TM];   // leading products', small ones'
-  T total[TN][TM][16];                   // PARTED: finished parts'
+  T total[PARTED ? TN : 1][PARTED ? TM : 1][16] = {};   // PARTED: finished parts'
   f32x16(&leading)[TN][TM] = sums[0], (&small)[TN][TM] = sums[PARTED ? 1 : 0];
 #pragma unroll
   for (int t = 0; t < (PARTED ? 2 : 1); ++t)
@@ -417,12 +416,9 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const LayerArgs a) {
 #pragma unroll
       for (int j = 0; j < TM; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          sums[t][i][j][r] = 0.f;
-          total[i][j][r] = 0;
-        }
+        for (int r = 0; r < 16; ++r) sums[t][i][j][r] = 0.f;
 
-  half8 x[XB][2][TM];
+  half8 x[2][2][TM];
   auto load_x = [&](half8(&d)[2][TM], int buf, int k) {
     const char* at = lds + buf * S::SLAB + k * kStepBytes + lane * 16;
 #pragma unroll
@@ -440,7 +436,7 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const LayerArgs a) {
   };
   wait_fetches<0>();
   __builtin_amdgcn_s_barrier();
-  if (XB == 2) load_x(x[0], 0, 0);
+  load_x(x[0], 0, 0);
   int buf = 0;
   // phase 0: the small products, 1: all, 2: the leading ones of two steps
   auto slab_body = [&](auto phase, int s) {
@@ -449,21 +445,20 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const LayerArgs a) {
 #pragma unroll
     for (int k = 0; k < KS; ++k) {
       load_w((k + RING - 1) % RING, s * KS + k + RING - 1);
-      if (XB == 1) load_x(x[0], buf, k);
       if (k == KS - 1) {
         // (what may be on its way: the weights ahead, and later slabs)
         wait_fetches<2 * TN * (RING - 1) + 2>();
         __builtin_amdgcn_s_barrier();
         fetch(s + NBUF, buf);
         HBT_FENCE;
-        if (XB == 2) load_x(x[(k + 1) % XB], next, 0);
-      } else if (XB == 2) {
-        load_x(x[(k + 1) % XB], buf, k + 1);
+        load_x(x[(k + 1) % 2], next, 0);
+      } else {
+        load_x(x[(k + 1) % 2], buf, k + 1);
       }
       // (2 x 4 tiles 0.8 % slower without it, the others 1 to 2 % slower with it)
       if (!PARTED) HBT_FENCE;
       half8(&wk)[2][TN] = w[k % RING];
-      half8(&xk)[2][TM] = x[k % XB];
+      half8(&xk)[2][TM] = x[k % 2];
       if (P != 0) mm(leading, wk[0], xk[0]);
       if (P == 2) mm(leading, wk[1], xk[1]);
       if (P != 2) mm(small, wk[0], xk[1]);
@@ -508,9 +503,13 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const LayerArgs a) {
     for (int j = 0; j < TM; ++j) {
       if (m_tile0 + j >= a.m_tiles) continue;
       const int* const e = scales[j * kRows + m];
+      T sum[16];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) total[i][j][r] += (T)small[i][j][r];
-      finish_tile<LAST, T>(a, units, total[i][j], n_tile0 + i, m_tile0 + j, lane, e[0],
+      for (int r = 0; r < 16; ++r) {
+        sum[r] = (T)small[i][j][r];
+        if constexpr (PARTED) sum[r] += total[i][j][r];
+      }
+      finish_tile<LAST, T>(a, units, sum, n_tile0 + i, m_tile0 + j, lane, e[0],
                            LAST ? 0 : e[1], most[j], lost[j]);
     }
   }
