@@ -24,6 +24,20 @@ def network(kind, hidden, seed=0):
     return rp
 
 
+def without_pairs(rp):
+    """Keeps `rp` from the fp16 pairs (mlp_pairs.h), from 1025 rows on: the last unit of the
+    last hidden layer, which fc2 no longer reads, hangs on one of its inputs.  Returns a
+    predictor without that weight, for which a batch of some rows gives the same numbers in
+    other roundings if and only if one of the two runs in pairs and the other does not."""
+    rp.model.fc2.weight.data[0, 1023] = 0.0
+    other = RuntimePredictor(rp.model_name, rp.layers, 1024)
+    other.model.load_state_dict(rp.model.state_dict())
+    other.set_normalization(rp.mu, rp.sigma)
+    rp.model.mlp.layers[2 * (rp.layers - 1)].weight.data[1023, 5] = 100.0
+    rp.refresh()
+    return other
+
+
 def forward_fp64(rp, x):
     """oracle.mlp.forward_fp64 on the GPU (float64 matrix products)."""
     sd = {k: v.double().cuda() for k, v in rp.model.state_dict().items()}
@@ -47,6 +61,11 @@ def test_rows_around_the_kernels_edges(rows, hidden):
     rp = network("lstm", hidden)
     x, mu, sigma = synthetic.mlp_features("lstm", rows, seed=rows)
     rp.set_normalization(mu, sigma)
+    check_against_fp64(rp, x)
+
+
+def check_against_fp64(rp, x):
+    hidden = rp.layers
     y = rp.predict_batch(x).cpu().numpy().astype(np.float64)
     want = forward_fp64(rp, x)
     # Per layer a sum of 1024 products in fp32: an error of at most 8 x 2^-24 of the
@@ -58,6 +77,21 @@ def test_rows_around_the_kernels_edges(rows, hidden):
     assert err <= (hidden + 1) * 8 * 2.0 ** -24 * rms
     assert float(np.max(np.abs(y - want))) <= 6 * (hidden + 1) * 8 * 2.0 ** -24 * rms
     assert np.array_equal(y, rp.predict_batch(x).cpu().numpy().astype(np.float64))
+
+
+# The kernels of split_kernel_for from 1025 rows on, where other networks take the pairs.
+@pytest.mark.parametrize("rows", [1025, 1500, 1536, 1537, 2048, 2049, 2177, 3071, 3072, 3073, 4000, 4096,
+                                  4097, 4608, 4609, 5911, 6144, 6145, 7300, 8192, 8193, 9216, 9217,
+                                  10240, 10241, 11000, 12288, 12289, 13000, 16384, 16385 + 1024, 32769])
+@pytest.mark.parametrize("hidden", [1, 2])
+def test_rows_around_the_kernels_edges_in_pieces(rows, hidden):
+    rp = network("lstm", hidden)
+    x, mu, sigma = synthetic.mlp_features("lstm", rows, seed=rows)
+    rp.set_normalization(mu, sigma)
+    pairs = without_pairs(rp)
+    check_against_fp64(rp, x)
+    assert not torch.equal(rp.predict_batch(x), pairs.predict_batch(x))
+    assert torch.equal(rp.predict_batch(x[:1024]), pairs.predict_batch(x[:1024]))
 
 
 @pytest.mark.parametrize("rows", [200, 400, 800, 1400, 2000, 3000, 4000, 6000, 9000, 20000])
@@ -231,23 +265,23 @@ def test_sparse_weights_keep_fp32_sums(rows):
 
 
 def whole_numbers(seed):
-    """Two dense hidden layers of whole numbers, 11 bits wide in the first, whose sums
-    are exact in any order: below 2^24 in every partial sum, activations of up to
-    three pieces and weights of two."""
+    """Two dense hidden layers of sixteenths, 11 bits wide in the first, whose sums are exact
+    in any order: below 2^24 sixteenths in every partial sum, activations of up to three
+    pieces and weights of two."""
     rng = np.random.default_rng(seed)
     rp = RuntimePredictor("bmm", 2, 1024)
-    first = rng.integers(1, 2048, (1024, 1024)) * rng.choice([-1, 1], (1024, 1024))
+    first = rng.integers(1, 2048, (1024, 1024)) * rng.choice([-1, 1], (1024, 1024)) / 16
     second = rng.choice([-1, 1], (1024, 1024)) * (rng.random((1024, 1024)) < 0.3)
     last = np.zeros(1024)
-    last[rng.choice(1024, 16, replace=False)] = rng.choice([-1, 1], 16)
+    last[rng.choice(1023, 16, replace=False)] = rng.choice([-1, 1], 16)
     with torch.no_grad():
         for p in rp.model.parameters():
             p.zero_()
         rp.model.fc1.weight.copy_(torch.from_numpy(rng.integers(-1, 2, (1024, 8))))
         rp.model.mlp.layers[0].weight.copy_(torch.from_numpy(first))
         rp.model.mlp.layers[2].weight.copy_(torch.from_numpy(second))
-        rp.model.mlp.layers[0].bias.copy_(torch.from_numpy(rng.integers(-2048, 2048, 1024)))
-        rp.model.mlp.layers[2].bias.copy_(torch.from_numpy(rng.integers(-2048, 2048, 1024)))
+        rp.model.mlp.layers[0].bias.copy_(torch.from_numpy(rng.integers(-2048, 2048, 1024) / 16))
+        rp.model.mlp.layers[2].bias.copy_(torch.from_numpy(rng.integers(-2048, 2048, 1024) / 16))
         rp.model.fc2.weight.copy_(torch.from_numpy(last)[None])
     rp.set_normalization(np.zeros(8), np.ones(8))
     return rp, rng
@@ -262,17 +296,32 @@ def whole_numbers(seed):
                                   16351, 16384, 16384 + 12500])
 def test_every_weight_position_is_wired_in_pieces(rows):
     rp, rng = whole_numbers(rows)
+    other = without_pairs(rp)     # (its last unit is not summed exactly, and not read)
     x = rng.integers(-1, 2, (rows, 8)).astype(np.float64)
     sd = {k: v.double().cuda() for k, v in rp.model.state_dict().items()}
     h = torch.relu(torch.from_numpy(x).cuda() @ sd["fc1.weight"].t())
     for name in ("mlp.layers.0", "mlp.layers.2", "fc2"):
         w = sd[name + ".weight"]
-        assert float((h @ w.abs().t()).max()) + 2048 < 2 ** 24
+        assert 16 * float((h @ w.abs().t())[:, :1023].max()) + 2048 < 2 ** 24
         h = h @ w.t() + sd[name + ".bias"]
         h = torch.relu(h) if name != "fc2" else h
     pieces, fp32 = rp.predict_batch(x).double(), rp.predict_batch_fp32(x).double()
     assert torch.equal(fp32, h.reshape(-1))
     assert torch.equal(pieces, h.reshape(-1))
+    # neither the fp32 kernels nor, from 1025 rows on, the pairs
+    x = rng.normal(size=(rows, 8))
+    pieces, fp32 = rp.predict_batch(x), rp.predict_batch_fp32(x)
+    assert not torch.equal(pieces, fp32)
+    if rows > 1024:
+        # (the other one's second layer is near what the pairs ask of a sum's terms: it is one
+        # of +-1 and 0; with every weight +-1 it takes them)
+        with torch.no_grad():
+            for m in (rp.model, other.model):
+                w = m.mlp.layers[2].weight
+                w[:1023][w[:1023] == 0] = 1.0
+            other.model.mlp.layers[2].weight[1023] = 1.0
+        rp.refresh(), other.refresh()
+        assert not torch.equal(rp.predict_batch(x), other.predict_batch(x))
 
 
 # hbt_mlp_forward_fp32 (device sweeps): around its per-layer path's end at 7168 rows, the
