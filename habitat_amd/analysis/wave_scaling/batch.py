@@ -284,9 +284,10 @@ class TotalsCall:
                             "int32 [%d], on the records' GPU"
                             % (n_segments + 1, len(table) * records.n, len(table)))
         self.shape = (n_rows, n_segments)
-        self._keep = (records, table, segment_start, workspace, rows)
         self._device = records.device
-        c = records.columns
+        c = dict(records.columns)
+        # what the pointers point into, whatever becomes of the objects they came in
+        self._keep = (c, records.dest_regs, records.has_metrics, table, segment_start, workspace, rows)
         self._args = (
             table.handle, records.n,
             _ptr(c["num_blocks"]), _ptr(c["block_size"]), _ptr(c["dynamic_smem"]),

@@ -530,3 +530,23 @@ def test_outputs_that_a_kernel_cannot_write_are_refused():
             ratio_scale_kinds([kind], 2, right[2], stream)
     call(*right, stream)
     ratio_scale_kinds([("bmm", pred, ms, op_row)], 2, right[2], stream)
+
+
+def test_a_totals_call_keeps_what_it_points_into():
+    import gc
+    import weakref
+    rec, _ = synthetic.kernel_records(100, Device.V100, seed=1, metrics_fraction=0.5)
+    records = KernelRecords.from_numpy(rec, "cuda:0")
+    records.dest_regs = torch.full((100,), -1, dtype=torch.int32, device="cuda")
+    call = TotalsCall(records, DeviceTable(Device.V100, [Device.T4]),
+                      torch.tensor([0, 40, 100], device="cuda"), 2,
+                      torch.empty((1, 100), dtype=torch.float64, device="cuda"), None, 1, 0.0)
+    inside = [weakref.ref(t) for t in (*records.columns.values(), records.dest_regs,
+                                       records.has_metrics)]
+    records.columns.clear()
+    records.dest_regs = records.has_metrics = None
+    gc.collect()
+    assert all(t() is not None for t in inside)
+    del call
+    gc.collect()
+    assert not any(t() is not None for t in inside)
