@@ -1484,6 +1484,8 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
   const size_t off_first_t = off;
   off = align_up(off + sizeof(float) * first_t_rows * kWidth, 256);
   const size_t off_bias_most = off; off = align_up(off + sizeof(int32_t) * (hidden_layers + 1), 256);
+  const size_t off_column_lost = off;
+  off = align_up(off + sizeof(int32_t) * (size_t)hidden_layers * kWidth, 256);
   const size_t image = off;  // what is copied from the host; scratch follows
   const int64_t chunk_rows = kSplitRowsPerUnit * compute_units;
   size_t scratch_bytes = (size_t)(chunk_rows / kRows) * split::kTileBytes;
@@ -1616,6 +1618,7 @@ hbt_mlp* hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
       p.G_in = p.G;
       p.size_in = p.size;
       p.F = reinterpret_cast<int32_t*>(base + off_F) + (size_t)l * kWidth;
+      p.column_lost = reinterpret_cast<int32_t*>(base + off_column_lost) + (size_t)l * kWidth;
       p.G += kWidth;
       p.size += kWidth;
       p.bias += kWidth;

@@ -19,10 +19,11 @@
 //   row n of a layer's weights by 2^-F[n], its largest weight to [2^14, 2^15).
 // A scaled number below kHeldFrom is held to 2^-25: a weight to 2^-40 of its row's largest,
 // an activation to 2^-40 of the bound on its row's, some 2^-32 of the row's usual ones.
-// Where that is the loss of more than kMostLost numbers of a sum, they are not summed here:
-// a network with such a row of weights, or with a unit that hangs on few of its inputs
-// (kLeastShare), keeps the bf16 pieces; a row of a batch with such activations, as where a
-// few units are 2^10 times the others, is marked while the layers run and goes through the
+// Where sums may hang on such numbers they are not made here: a network with many such
+// weights in a row or column (kMostLostWeights), or with a unit that hangs on few of its
+// inputs (kLeastShare), keeps the bf16 pieces; a row of a batch with many such activations,
+// as where a few units are 2^10 times the others, or with hardly any above them
+// (rows_lost), is marked while the layers run and goes through the
 // network again on the fp32 matrix cores (mlp_fused_kernel).  An
 // infinite activation is the second number of its pair, so that it meets nothing but
 // the other operand's first number, whose sign is the weight's; a NaN stays one.
@@ -61,11 +62,13 @@ constexpr int kTileBytes = kSteps * kStepBytes;
 constexpr int kTop = 15;  // scaled numbers are below 2^kTop
 // From here on a scaled number is held to 2^-22 of itself, below to 2^-25.
 constexpr float kHeldFrom = 0x1p-3f;
-// Numbers below that in a row of weights or activations.  Of 1024 activations that are of one
-// size 0 to 20 are (networks of eight layers, any gain), and with one unit 2^8, 2^10 and 2^12
-// times the others 46-262, 185-527 and 472-551 (all that are not 0): errors of 4e-7, 6e-7 and
-// 2e-6 where fp32 sums have 1e-6.
+// Activations of a row below that.  Of 1024 that are of one size 0 to 20 are (networks of
+// eight layers, any gain), and with one unit 2^4, 2^8, 2^10 and 2^12 times the others 1-21,
+// 46-262, 185-527 and 472-551 (all that are not 0): errors of 5e-7, 4e-7, 6e-7 and 2e-6 where
+// fp32 sums have 1e-6.
 constexpr int kMostLost = 128;
+// Weights of a row or column below that: of 1024 of one spread 0 to 2.
+constexpr int kMostLostWeights = 16;
 
 __device__ __forceinline__ size_t tile_offset(int tile, int step) {
   return (size_t)tile * kTileBytes + (size_t)step * kStepBytes;
@@ -158,6 +161,12 @@ __device__ __forceinline__ int part_lost(int32_t part) { return part & 255; }
 __device__ __forceinline__ int32_t both_parts(int32_t a, int32_t b) {
   return (a > b ? a & -256 : b & -256) + part_lost(a) + part_lost(b);
 }
+// Whether a sum may hang on what a row has lost: there is much of it, or nothing is larger
+// than 1 (all but some of the row's units are 0, and the bound was far from the others).
+// most: part_exponent of the row, e: of its scale.
+__device__ __forceinline__ bool rows_lost(int lost, int most, int e) {
+  return lost > kMostLost || (lost > 0 && (most <= -kNotFinite || most + e <= 0));
+}
 __device__ __forceinline__ int is_lost(bool positive, float scaled) { return positive && scaled < kHeldFrom; }
 
 // v of 4, 8 or 16 lanes together (in registers: a step through LDS is 100 cycles, and these
@@ -204,7 +213,7 @@ __device__ __forceinline__ void row_scales(const LayerArgs& a, int m_tile0, bool
   scales[r][1] = e;
   if (!store_out || m_tile0 * kRows + r >= rows) return;
   if (!LAST) a.e_out[row] = e;
-  if (lost > kMostLost) a.redo[row] = 1;
+  if (rows_lost(lost, most, e_in)) a.redo[row] = 1;
 }
 
 // Part `part` of a row's outputs: the largest, and how many are not held.
@@ -547,6 +556,7 @@ struct PrepareArgs {
   int32_t* G;
   float* size;
   int32_t* bias_most;      // of the layer; at the least there is before
+  int32_t* column_lost;    // [kWidth] weights below kHeldFrom of an input; zeroes before
   uint32_t* outside;       // set where the layer is not for pairs
 };
 
@@ -616,8 +626,11 @@ __global__ __launch_bounds__(1024) void prepare_layer(const PrepareArgs a) {
     const f32x4 v = in[(size_t)g * (8 * 64)];
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      lost += a.size_in[k + e] > 0.f && v[e] != 0.f &&
-              ldexp(fabs((double)v[e]), -a.G_in[k + e] - F) < kHeldFrom;
+      if (a.size_in[k + e] > 0.f && v[e] != 0.f &&
+          ldexp(fabs((double)v[e]), -a.G_in[k + e] - F) < kHeldFrom) {
+        ++lost;
+        if (atomicAdd(a.column_lost + k + e, 1) >= kMostLostWeights) *a.outside = 1;
+      }
   }
   lost += __shfl_xor(lost, 32);
   lost_of[wave][m] = lost;
@@ -626,7 +639,7 @@ __global__ __launch_bounds__(1024) void prepare_layer(const PrepareArgs a) {
   lost = 0;
   for (int w = 0; w < 16; ++w) lost += lost_of[w][m];
   // (a weight that is not finite has been found by check_kernel)
-  if (!(total * total >= kLeastShare * squares) || lost > kMostLost) *a.outside = 1;
+  if (!(total * total >= kLeastShare * squares) || lost > kMostLostWeights) *a.outside = 1;
   const int n = tile * 32 + m;
   a.F[n] = F;
   put_size(a, n, squares);

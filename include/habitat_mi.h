@@ -369,12 +369,13 @@ hbt_mlp *hbt_mlp_create(int32_t in_features, int32_t width, int32_t hidden_layer
  * more in magnitude, or a hidden unit has 1 to 191 nonzero weights: such a network is
  * hbt_mlp_forward_fp32 at any n.  A network in which a unit is made of few of its inputs
  * (the sum of its weights times their sizes, squared, is below 256 times the sum of the
- * squares), with a unit whose size is beyond 2^+-100, or with more than 128 nonzero weights
- * of a unit below 2^-17 of its largest (relative to their inputs' sizes) keeps the bf16 pieces
- * at any n.  A row of a batch in which more than 128 units of a layer are positive and below
- * 2^-18 of the bound on the row's largest, as where few of them are 2^10 times the others, is
- * computed with the sums of hbt_mlp_forward_fp32 (0.9 ms for up to 32 rows per compute unit,
- * whatever they hold); the rows beside it are as they are without it.
+ * squares), with a unit whose size is beyond 2^+-100, or in which more than 16 nonzero
+ * weights of a unit, or of an input, are below 2^-17 of their units' largest (relative to the
+ * inputs' sizes) keeps the bf16 pieces at any n.  A row of a batch in which more than 128 units
+ * of a layer are positive and below 2^-18 of the bound on the row's largest, as where few of
+ * them are 2^10 times the others, or some are and none is above 2^-15 of it, is computed with
+ * the sums of hbt_mlp_forward_fp32 (0.9 ms for up to 32 rows per compute unit, whatever they
+ * hold); the rows beside it are as they are without it.
  */
 int hbt_mlp_forward(hbt_mlp *mlp, const double *raw_features, int64_t n, float *out,
                     void *hip_stream);

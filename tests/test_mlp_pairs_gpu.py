@@ -260,34 +260,37 @@ def test_sums_beyond_fp32_are_infinite(rows, signs):
 
 
 @pytest.mark.parametrize("rows", [1025, 2048, 3000, 4500, 5911, 10000, 13001, 16384 + 3001])
-def test_rows_that_one_unit_dominates(rows):
-    """A unit that is large in some rows and hardly read by the next layer: what the other
-    units make is held as fp32 holds it, and the rows beside such a row are left alone."""
+def test_rows_that_some_units_dominate(rows):
+    """Two networks of 512 units side by side, of which fc2 reads the second and feature 0
+    feeds the first: where that one is large, what the second makes is held as fp32 holds it,
+    and the rows beside such a row are left alone."""
     rp = network("conv2d", 3)
+    inputs = rp.model.fc1.weight.shape[1]
     with torch.no_grad():
-        for _, bias in layers_of(rp):
+        for weight, bias in layers_of(rp):
             bias.zero_()
+            if weight.shape[1] == 1024:
+                weight[:512, 512:] = 0.0
+                weight[512:, :512] = 0.0
+                weight.mul_(2.0 ** 0.5)
+            else:
+                weight[:512, 1:] = 0.0
+                weight[512:, 0] = 0.0
+        rp.model.fc2.weight[0, :512] = 0.0
         rp.model.fc2.bias.zero_()
-        first = rp.model.fc1.weight
-        first[:, 0] = 0.0
-        first[40] = 0.0
-        first[40, 0] = 1.0                                  # unit 40 is feature 0 alone
-        layers_of(rp)[1][0][:, 40] *= 2.0 ** -60
-    inputs = first.shape[1]
     rp.set_normalization(np.zeros(inputs), np.ones(inputs))
     rng = np.random.default_rng(rows)
     x = rng.normal(size=(rows, inputs))
-    x[:, 0] = 1.0
     plain = rp.predict_batch(x).cpu().numpy()
-    want = forward_fp64(rp, x)                              # (feature 0 is 2^-60 of it)
+    want = forward_fp64(rp, x)                              # (feature 0 is no part of it)
     rms = np.sqrt(np.mean(want ** 2))
     at = np.sort(rng.choice(rows, rows // 40, replace=False))
+    others = np.setdiff1d(np.arange(rows), at)
     for k in (4, 8, 10, 12, 16, 20, 32):
         x[at, 0] = 2.0 ** k
         y = rp.predict_batch(x).cpu().numpy()
         # the bound of tests/test_mlp_split_gpu.py
         assert np.sqrt(np.mean((y[at] - want[at]) ** 2)) <= 4 * 8 * 2.0 ** -24 * rms, k
-        others = np.setdiff1d(np.arange(rows), at)
         assert np.array_equal(y[others], plain[others]), k
         if k >= 12:   # (whole rounds of the fused fp32 kernel)
             whole = np.resize(x[at], (8192, inputs))
@@ -296,12 +299,71 @@ def test_rows_that_one_unit_dominates(rows):
     raw = torch.from_numpy(x).cuda()
     with torch.cuda.graph(graph):
         rp.predict_batch(raw, out=out)
-    raw[:, 0] = 1.0                          # what was marked in one pass is not in the next
+    raw[:, 0] = 0.5                          # what was marked in one pass is not in the next
+    want = rp.predict_batch(raw).cpu().numpy()
+    assert not np.array_equal(want[at], y[at])
     for _ in range(2):
         out.zero_()
         graph.replay()
-        assert np.array_equal(out.cpu().numpy(), plain)
+        assert np.array_equal(out.cpu().numpy(), want)
         assert np.array_equal(rp.predict_batch(x).cpu().numpy(), y)
+
+
+@pytest.mark.parametrize("rows", [1500, 3000, 4500, 5911, 13000])
+def test_rows_in_which_few_units_are_on(rows):
+    """Features that switch all but twenty units off, whatever they would have made of them,
+    and the others' activations far below what the features bound them by."""
+    rp = network("linear", 2)
+    with torch.no_grad():
+        for _, bias in layers_of(rp):
+            bias.zero_()
+        rp.model.fc2.bias.zero_()
+        first = rp.model.fc1.weight
+        first.copy_(-first.abs())
+        first[:, 0] = 0.0
+        first[300:320] = 0.0
+        first[300:320, 0] = torch.rand(20) + 0.5
+    rp.set_normalization(np.zeros(8), np.ones(8))
+    x = np.abs(np.random.default_rng(rows).normal(size=(rows, 8))) + 0.1
+    x[::3, 1:] *= 2.0 ** 30
+    y, want = rp.predict_batch(x).double().cpu().numpy(), forward_fp64(rp, x)
+    # All rows are multiples of one, so one sum's chance is all rows'; the bound of
+    # tests/test_mlp_split_gpu.py on the last sum's terms (sums of 20 products have less)
+    h = torch.from_numpy(x).cuda()
+    with torch.no_grad():
+        for weight, _ in layers_of(rp):
+            h = torch.relu(h @ weight.double().cuda().t())
+        size = (h * rp.model.fc2.weight.double().cuda()).norm(dim=1).cpu().numpy()
+    for part in (slice(0, None, 3), slice(1, None, 3)):
+        assert np.max(np.abs(y[part] - want[part]) / size[part]) <= 6 * 3 * 8 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("rows", [1500, 3000, 4500, 5911, 13000])
+def test_an_input_of_tiny_weights_alone(rows):
+    """A unit whose outgoing weights are 2^-60 of the others', large, and alone in being on:
+    its weights are not for pairs, and the network is not."""
+    rp = network("linear", 2)
+    with torch.no_grad():
+        for _, bias in layers_of(rp):
+            bias.zero_()
+        rp.model.fc2.bias.zero_()
+        first = rp.model.fc1.weight
+        first.copy_(-first.abs())
+        first[:, 0] = 0.0
+        first[40] = 0.0
+        first[40, 0] = 1.0
+        layers_of(rp)[1][0][:, 40] *= 2.0 ** -60
+    rp.set_normalization(np.zeros(8), np.ones(8))
+    x = np.abs(np.random.default_rng(rows).normal(size=(rows, 8))) + 0.1
+    x[:, 0] *= 2.0 ** 32
+    y, want = rp.predict_batch(x).double().cpu().numpy(), forward_fp64(rp, x)
+    h = torch.from_numpy(x).cuda()
+    with torch.no_grad():
+        for weight, _ in layers_of(rp):
+            h = torch.relu(h @ weight.double().cuda().t())
+        size = (h * rp.model.fc2.weight.double().cuda()).norm(dim=1).cpu().numpy()
+    # as above
+    assert np.max(np.abs(y - want) / size) <= 6 * 3 * 8 * 2.0 ** -24
 
 
 @pytest.mark.parametrize("rows", [1500, 3000, 5911, 13000])
