@@ -193,8 +193,8 @@ class SweepCall:
         # that what decides the time waits for no other stream; each other kind runs on a
         # stream of its own (of default priority), beside the sums and beside that one.  (The
         # sums beside the largest kind take as long as its launches: 256 devices 878 us a sweep
-        # and not 838, 60 devices 314 and 274.  The other kinds after the sums: 2 devices 164
-        # us and not 126, 16 devices 192 and 154, 1024 devices 3140 and 3100.)
+        # and not 838, 60 devices 314 and 274.  The other kinds after the sums: 256 devices 837
+        # and not 833, 1024 devices 3131 and 3096, 2 and 16 the same; six runs of each in turn.)
         kinds = sorted(self.rows, key=lambda kind: -self.rows[kind].shape[0])
         self.kinds = [(kind, torch.cuda.Stream(plan.gpu) if i else None)
                       for i, kind in enumerate(kinds)]
